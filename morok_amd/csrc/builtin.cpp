@@ -141,8 +141,11 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         while (p.size() < 4) p.push_back(1);
         if (p.size() < 5) p.push_back(0);
         if (p[4] < 0) return fail(kInvalidArgument, k + ": negative workspace size");
-        if (!gemm_bf16_nt_supported(p[0], p[1], p[2], p[3]))
-            return fail(kInvalidArgument, k + ": shape not covered (K a multiple of 8; at most 64 rows, or N a multiple of 8)");
+        // (operand rows that are no whole 16-byte chunks need the scratch their padded copies go to)
+        if (!gemm_bf16_nt_supported(p[0], p[1], p[2], p[3]) &&
+            !(gemm_bf16_nt_padded_supported(p[0], p[1], p[2], p[3]) &&
+              static_cast<size_t>(p[4]) >= gemm_bf16_nt_workspace_bytes(p[0], p[1], p[2], p[3])))
+            return fail(kInvalidArgument, k + ": shape not covered without scratch (K a multiple of 8; at most 64 rows, or N a multiple of 8)");
         std::string name = k + "_" + std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]);
         if (p[3] > 1) name += "_x" + std::to_string(p[3]);
         if (p[4] > 0) {  // a fourth buffer of p[4] bytes: scratch for the split-K partial results
@@ -161,29 +164,33 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
     }
     // c = a b + r in the product's own kernels: r a matrix of c's shape ("_residual") or one row [N] ("_bias");
     // {M, N, K}, {M, N, K, batch} or {M, N, K, batch, workspace bytes}; buffers {c, a, b, r[, scratch]}
-    if (k == "gemm_bf16_bias" || k == "gemm_bf16_nt_bias" || k == "gemm_bf16_residual" || k == "gemm_bf16_nt_residual") {
+    if (k == "gemm_bf16_bias" || k == "gemm_bf16_nt_bias" || k == "gemm_bf16_residual" || k == "gemm_bf16_nt_residual" || k == "gemm_f16_bias" ||
+        k == "gemm_f16_nt_bias" || k == "gemm_f16_residual" || k == "gemm_f16_nt_residual") {
+        const bool f16 = k.compare(0, 8, "gemm_f16") == 0;
         const bool nt = k.find("_nt_") != std::string::npos, row = k.find("_bias") != std::string::npos;
         if (nparams < 3 || nparams > 5)
             return failf(kInvalidArgument, "builtin '%s' takes 3 to 5 parameters, got %zu", k.c_str(), nparams);
         while (p.size() < 4) p.push_back(1);
         if (p.size() < 5) p.push_back(0);
         if (p[4] < 0) return fail(kInvalidArgument, k + ": negative workspace size");
-        if (!gemm_bf16_bias_launchable(p[0], p[1], p[2], p[3], nt))
-            return failf(kInvalidArgument, "%s: shape not covered (N and K multiples of 8%s)", k.c_str(),
+        const bool whole = gemm_bf16_residual_supported(p[0], p[1], p[2], p[3]) || (nt && gemm_nt_bias_streamed(p[0], p[1], p[2], p[3]));
+        const size_t want = nt ? gemm_bf16_nt_workspace_bytes(p[0], p[1], p[2], p[3]) : gemm_bf16_workspace_bytes(p[0], p[1], p[2], p[3]);
+        if (!gemm_bf16_bias_launchable(p[0], p[1], p[2], p[3], nt) || (!whole && static_cast<size_t>(p[4]) < want))
+            return failf(kInvalidArgument, "%s: shape not covered (without scratch: N and K multiples of 8%s)", k.c_str(),
                          nt ? "; or up to 64 rows with K a multiple of 8" : "");
         std::string name = k + "_" + std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]);
         if (p[3] > 1) name += "_x" + std::to_string(p[3]);
         if (p[4] > 0) {  // a fifth buffer of p[4] bytes: scratch for the partial results of a product spread along K
             out->reset(new BuiltinProgram(device_id, stream, name + "_splitk", 5, p,
-                                          [nt, row](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+                                          [nt, row, f16](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                               return launch_gemm_bf16_residual(s, b[1], b[2], b[3], b[0], q[0], q[1], q[2], q[3], nt, row, b[4],
-                                                                               static_cast<size_t>(q[4]));
+                                                                               static_cast<size_t>(q[4]), f16);
                                           }));
             return kOk;
         }
         out->reset(new BuiltinProgram(device_id, stream, name, 4, p,
-                                      [nt, row](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
-                                          return launch_gemm_bf16_residual(s, b[1], b[2], b[3], b[0], q[0], q[1], q[2], q[3], nt, row);
+                                      [nt, row, f16](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+                                          return launch_gemm_bf16_residual(s, b[1], b[2], b[3], b[0], q[0], q[1], q[2], q[3], nt, row, nullptr, 0, f16);
                                       }));
         return kOk;
     }

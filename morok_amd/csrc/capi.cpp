@@ -961,7 +961,7 @@ int mrk_hip_gemm_bf16_noalloc(int device_id, const void* a, const void* b, void*
     if (!d)
         return failf(kInvalidArgument, "gemm_bf16_noalloc: device HIP:%d has not been created; call mrk_hip_device_create "
                                        "during set-up (this entry point allocates nothing, device creation does)", device_id);
-    const size_t need = gemm_bf16_workspace_bytes(m, n, k, 1);
+    const size_t need = gemm_bf16_static_workspace_need(m, n, k);
     if (need > gemm_bf16_static_workspace_capacity())
         return failf(kInvalidArgument, "gemm_bf16_noalloc: %lldx%lldx%lld needs %zu bytes of split-K scratch, the built-in "
                                        "scratch holds %zu; use mrk_hip_gemm_bf16", (long long)m, (long long)n, (long long)k,

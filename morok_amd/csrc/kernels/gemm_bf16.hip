@@ -31,11 +31,15 @@
 // barrier to sit there every fragment of tile kt must have been read by then: fragments are
 // read a sub-step ahead of their MFMAs into two register slots (one per 32-deep sub-step).
 //
-// Shapes.  M is arbitrary, N and K multiples of 8: edge tiles redirect out-of-range rows and
-// column chunks to the last valid one and mask their stores; a partial last K step is copied
-// from zeros beyond K.  A second instance of the same body with a 128x256 workgroup tile serves
-// shapes that would otherwise leave most compute units idle; a leading batch dimension runs as
-// grid.y.  Everything else takes the any-shape kernel at the end of this file.
+// Shapes.  Any M, N and K: edge tiles redirect out-of-range rows and column chunks to the last
+// valid one and mask their stores; a partial last K step is copied from zeros beyond K.  The
+// 16-byte copies need operand rows that start on 16 bytes: an operand whose row length is no
+// multiple of 8 elements is first written out with padded rows (gemm_repitch), and C, whose rows
+// cannot be padded, is stored with 16-byte stores of 2-byte alignment.  A second instance of the
+// same body with a 128x256 workgroup tile serves shapes that would otherwise leave most compute
+// units idle; a leading batch dimension runs as grid.y.  The kernel at the end of this file, one
+// wave per 32x32 tile straight from global memory, is left for callers that bring no scratch for
+// the padded operands and for unaligned base pointers.
 #include <hip/hip_runtime.h>
 #include <atomic>
 
@@ -53,6 +57,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+// the same in memory where a row of 16-bit (of 32-bit) elements may start on any element
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 #define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
 
@@ -84,9 +91,12 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
 // lanes whose k lies beyond K.
 __device__ __attribute__((aligned(16))) const unsigned g_zero16[4] = {0u, 0u, 0u, 0u};
 
-// kRaggedK: K is not a multiple of 64 (but of 8).  The copies of the last, partial K step use
+// kAny: K is not a multiple of 64, or N not of 8.  The copies of a partial last K step use
 // per-lane 64-bit addresses so that chunks beyond K can be redirected to g_zero16: zero
 // operands on both sides contribute nothing.  Every other step is copied as in the full case.
+// The operands have row pitches of their own (lda, ldb elements, multiples of 8, zeros from K on
+// inside a row's padding), and C and R rows may start on any element: they are accessed in
+// 16-byte pieces of 2-byte alignment, the last piece of a row element by element.
 //
 // kJ: 32-column blocks (two MFMA tile columns each) per wave.  kJ = 4: 256x256 workgroup tile, waves 2x2, each 128x128.
 // kJ = 2: 128x256 workgroup tile, waves 1x4, each 128x64 (half the accumulators, an A stage of
@@ -125,6 +135,17 @@ __device__ __forceinline__ bf16x4 round_to_elem(const f32x4& v) {
     if constexpr (kF16) return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, f16x4));
     else return __builtin_convertvector(v, bf16x4);
 }
+// the sum of two chunks of eight 16-bit elements, taken in f32 and rounded once
+template <bool kF16>
+__device__ __forceinline__ u32x4 add_elems(const u32x4& a, const u32x4& b) {
+    if constexpr (kF16) {
+        const f32x8 s = __builtin_convertvector(__builtin_bit_cast(f16x8, a), f32x8) + __builtin_convertvector(__builtin_bit_cast(f16x8, b), f32x8);
+        return __builtin_bit_cast(u32x4, __builtin_convertvector(s, f16x8));
+    } else {
+        const f32x8 s = __builtin_convertvector(__builtin_bit_cast(bf16x8, a), f32x8) + __builtin_convertvector(__builtin_bit_cast(bf16x8, b), f32x8);
+        return __builtin_bit_cast(u32x4, __builtin_convertvector(s, bf16x8));
+    }
+}
 //
 // kRope (256-row tile only): the product of a packed projection whose first `split` columns are
 // attention heads of 128 columns each (q | k of a fused QKV product).  The epilogue applies the
@@ -141,14 +162,14 @@ struct RopeEpilogue {
     __bf16* rest;  // [M, N - split]: the columns from `split` on
     int seq, split;
 };
-template <bool kRaggedK, int kJ, bool kSplitK = false, bool kResidual = false, bool kSwiGLU = false, bool kBT = false, bool kF16 = false,
+template <bool kAny, int kJ, bool kSplitK = false, bool kResidual = false, bool kSwiGLU = false, bool kBT = false, bool kF16 = false,
           bool kRope = false>
 __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                                __bf16* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
                                                float* __restrict__ W = nullptr, int kt_per_split = 0,
                                                const __bf16* __restrict__ R = nullptr, const RopeEpilogue& rope = RopeEpilogue{},
-                                               int ldr = -1) {
-    static_assert(!kF16 || (!kResidual && !kSwiGLU && !kRope), "the fused epilogues exist for bf16 only");
+                                               int ldr = -1, int lda = 0, int ldb = 0) {
+    static_assert(!kF16 || (!kSwiGLU && !kRope), "the gated and the rotary epilogue exist for bf16 only");
     static_assert(!kRope || (kJ == 4 && !kSplitK && !kResidual && !kSwiGLU), "the rotary epilogue exists for the plain 256-row tile only");
     constexpr int kTM = kJ == 4 ? 256 : 128;      // rows of the workgroup tile
     constexpr int kAq = kTM / 32;                 // 1 KB A chunks (8 rows) each wave copies per K step
@@ -164,9 +185,12 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     __shared__ __attribute__((aligned(1024))) char smem[kSmemT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = kJ == 4 ? wave >> 1 : 0, wn = kJ == 4 ? (wave & 1) : wave;
+    // row pitches of the operands in elements
+    const size_t a_pitch = kAny ? (size_t)lda : (size_t)K;
+    const size_t b_pitch = kAny ? (size_t)ldb : kBT ? (size_t)K : (size_t)N;
     // blockIdx.y: which of the back-to-back stored products
-    A += (size_t)blockIdx.y * M * K;
-    B += (size_t)blockIdx.y * K * N;
+    A += (size_t)blockIdx.y * M * a_pitch;
+    B += (size_t)blockIdx.y * (kBT ? N : K) * b_pitch;
     if (!kSplitK) C += (size_t)blockIdx.y * M * N;
     // row pitch of R in elements: N for a matrix of C's shape, 0 for one row added to every row of C (a bias)
     const size_t r_pitch = ldr < 0 ? (size_t)N : (size_t)ldr;
@@ -196,7 +220,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         size_t row = m0 + wave * (kAq * 8) + q * 8 + (lane >> 3);
         row = row < (size_t)M ? row : (size_t)M - 1;
         const int chunk = (lane & 7) ^ ((q & 1) * 4 + (lane >> 4));
-        a_voff[q] = (unsigned)(((row - m0) * K + (chunk << 3)) * 2);
+        a_voff[q] = (unsigned)(((row - m0) * a_pitch + (chunk << 3)) * 2);
     }
     const int b_h = lane & 1, b_g = (lane & 31) >> 1, b_r = lane >> 5;
     // kBT: B^T chunk q (1 KB = 8 n-rows of 128 B), copied and swizzled exactly like an A chunk;
@@ -217,7 +241,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                 row = row < (size_t)N ? row : (size_t)N - 1;
             }
             const int chunk = (lane & 7) ^ ((q & 1) * 4 + (lane >> 4));
-            bt_voff[q] = (unsigned)(((row - n0) * K + (chunk << 3)) * 2);
+            bt_voff[q] = (unsigned)(((row - n0) * b_pitch + (chunk << 3)) * 2);
         }
     }
     unsigned b_voff[2];
@@ -230,17 +254,17 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             col = n0 + (lc & 127);
             col = (col + 8 <= F ? col : F - 8) + half * F;
         } else {
-            col = col + 8 <= (size_t)N ? col : (size_t)N - 8;
+            col = col + 8 <= b_pitch ? col : b_pitch - 8;
         }
-        b_voff[par] = (unsigned)(((size_t)(wave * 16 + b_r) * N + (col - n0)) * 2);
+        b_voff[par] = (unsigned)(((size_t)(wave * 16 + b_r) * b_pitch + (col - n0)) * 2);
     }
     const int KT_all = (K + kBK - 1) / kBK;
     const int kt0 = kSplitK ? (int)blockIdx.z * kt_per_split : 0;  // first K step of this workgroup
     const int KT = kSplitK ? (KT_all - kt0 < kt_per_split ? KT_all - kt0 : kt_per_split) : KT_all;
     const bool has_last = kt0 + KT == KT_all;  // the (possibly partial) last K step is in this range
-    const char* a_tile = reinterpret_cast<const char*>(A + m0 * K) + (size_t)kt0 * kBK * 2;
-    const char* b_tile = kBT ? reinterpret_cast<const char*>(B + n0 * K) + (size_t)kt0 * kBK * 2
-                             : reinterpret_cast<const char*>(B + n0) + (size_t)kt0 * kBK * N * 2;
+    const char* a_tile = reinterpret_cast<const char*>(A + m0 * a_pitch) + (size_t)kt0 * kBK * 2;
+    const char* b_tile = kBT ? reinterpret_cast<const char*>(B + n0 * b_pitch) + (size_t)kt0 * kBK * 2
+                             : reinterpret_cast<const char*>(B + n0) + (size_t)kt0 * kBK * b_pitch * 2;
     const unsigned lds_a = (unsigned)(uintptr_t)LDS_PTR(char, sA0) + wave * (kAq * 1024);
     const unsigned lds_b = (unsigned)(uintptr_t)LDS_PTR(char, sB0) + wave * 8192;
     // One direct copy: 64 lanes x 16 B land at LDS [m0, m0 + 1 KB); the compiler is not told
@@ -255,11 +279,11 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     auto dma_from = [&](unsigned lds_addr, const char* addr) {  // per-lane 64-bit source address
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(addr) : "m0");
     };
-    const int k_last = K - (KT_all - 1) * kBK;  // depth of the last K step: 64, or 8..56 when ragged
+    const int k_last = K - (KT_all - 1) * kBK;  // depth of the last K step: 64, or 1..63
     const char* zero16 = reinterpret_cast<const char*>(g_zero16);
     // (stage_off: byte offset of the stage inside the A or B part of the LDS)
     auto dma_a = [&](int q, int kt, unsigned stage_off) {
-        if (kRaggedK && has_last && kt == KT - 1) {
+        if (kAny && has_last && kt == KT - 1) {
             const int chunk = (lane & 7) ^ ((q & 1) * 4 + (lane >> 4));  // logical 8-deep k chunk of this lane
             dma_from(lds_a + stage_off + q * 1024,
                      chunk * 8 < k_last ? a_tile + (size_t)kt * kBK * 2 + a_voff[q] : zero16);
@@ -269,7 +293,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     };
     auto dma_b = [&](int q, int kt, unsigned stage_off) {
         if constexpr (kBT) {
-            if (kRaggedK && has_last && kt == KT - 1) {
+            if (kAny && has_last && kt == KT - 1) {
                 const int chunk = (lane & 7) ^ ((q & 1) * 4 + (lane >> 4));
                 dma_from(lds_b + stage_off + q * 1024,
                          chunk * 8 < k_last ? b_tile + (size_t)kt * kBK * 2 + bt_voff[q] : zero16);
@@ -278,12 +302,12 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             }
             return;
         }
-        if (kRaggedK && has_last && kt == KT - 1) {
+        if (kAny && has_last && kt == KT - 1) {
             dma_from(lds_b + stage_off + q * 1024,
-                     wave * 16 + q * 2 + b_r < k_last ? b_tile + ((size_t)kt * kBK + q * 2) * N * 2 + b_voff[q & 1] : zero16);
+                     wave * 16 + q * 2 + b_r < k_last ? b_tile + ((size_t)kt * kBK + q * 2) * b_pitch * 2 + b_voff[q & 1] : zero16);
             return;
         }
-        dma(lds_b + stage_off + q * 1024, b_voff[q & 1], b_tile + ((size_t)kt * kBK + q * 2) * N * 2);
+        dma(lds_b + stage_off + q * 1024, b_voff[q & 1], b_tile + ((size_t)kt * kBK + q * 2) * b_pitch * 2);
     };
 
     f32x4 acc[kI16][kJ16];
@@ -371,9 +395,9 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         const char* b_src;  // B tile kt2: k-row 0 of it ([K, N] form) or n-row 0 (B^T form)
         unsigned sb_cur, sb_nxt, sb_fill;
     } ls;
-    const unsigned b_step32 = kBT ? (unsigned)(kBK * 2) : (unsigned)kBK * (unsigned)N * 2u;  // bytes from one B tile to the next (N < 2^25)
+    const unsigned b_step32 = kBT ? (unsigned)(kBK * 2) : (unsigned)kBK * (unsigned)b_pitch * 2u;  // bytes from one B tile to the next (N < 2^25)
     unsigned adv = 0;
-    const size_t b_row2 = (size_t)N * 4;                                // [K, N] form: bytes from one 1 KB chunk (2 k-rows) to the next
+    const size_t b_row2 = b_pitch * 4;                                  // [K, N] form: bytes from one 1 KB chunk (2 k-rows) to the next
     ls.kt2 = KT > 2 ? 2 : KT - 1;
     ls.a_src = a_tile + (size_t)ls.kt2 * kBK * 2;
     ls.b_src = b_tile + (size_t)ls.kt2 * b_step32;
@@ -431,7 +455,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         constexpr int kEvery = (kSlots - kFirst - kTail) / kCopies;  // slots per copy (address, then copy)
         static_assert(kEvery >= 2, "a copy needs two slots");
         const unsigned lds_dst = p < 2 ? lds_b + ls.sb_fill : lds_a + cur * kAStageT;
-        const bool ragged_now = kRaggedK && has_last && ls.kt2 == KT - 1;  // this step copies the partial last tile
+        const bool ragged_now = kAny && has_last && ls.kt2 == KT - 1;  // this step copies the partial last tile
         const char* src = p < 2 ? ls.b_src : ls.a_src;
         if (p == 1 && !kBT) src += 4 * b_row2;
 #pragma unroll
@@ -447,7 +471,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             const int c = copy_range ? (n - kFirst) / kEvery : 0, part = copy_range ? (n - kFirst) % kEvery : -1;
             const int q = (p & 1) * kCopies + c;  // chunk of the tile
             // a copy slot: the MFMA and the copy as one statement; where a step may have to copy
-            // the partial last tile instead (kRaggedK) the choice is made at run time, and the MFMA
+            // the partial last tile instead (kAny) the choice is made at run time, and the MFMA
             // stays outside that branch: an accumulator that flows through a branch would be moved
             // by the compiler, which does not know that it has to wait for the matrix pipe first
             auto with_q = [&](auto&& f) {
@@ -466,7 +490,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                 constexpr int qq = decltype(q_c)::value;
                 return p >= 2 ? a_voff[qq < kAq ? qq : 0] : kBT ? bt_voff[kBT ? qq : 0] : b_voff[qq & 1];
             };
-            if (part == 1 && !kRaggedK) {
+            if (part == 1 && !kAny) {
                 with_q([&](auto q_c) { mfma_dma(acc[mi][mj], fb[slot][mj], fa[slot][mi], lds_dst, q_c, voff_of(q_c), src); });
             } else {
                 mfma(acc[mi][mj], fb[slot][mj], fa[slot][mi]);
@@ -556,13 +580,41 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     const int lr = lane / kChunks, lc = lane % kChunks;
     const int rows_here = row0 >= (size_t)M ? 0 : (size_t)M - row0 < 128 ? (int)((size_t)M - row0) : 128;  // rows of the wave's tile inside C
     const bool col_ok = col0 + lc * 8 + 8 <= (size_t)N;
+    // columns of this lane's chunk inside C when the chunk is the partial last one of a row (kAny: N % 8 of them), else 0
+    const int col_tail = kAny && !col_ok && col0 + lc * 8 < (size_t)N ? (int)((size_t)N - (col0 + lc * 8)) : 0;
+    auto store_chunk = [&](__bf16* dst, const u32x4& v, bool row_ok) {
+        if constexpr (kAny) {
+            if (col_ok && row_ok) *reinterpret_cast<u32x4_any*>(dst) = v;
+            else if (row_ok) {
+                const bf16x8 e8 = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+                for (int e = 0; e < 7; e++)
+                    if (e < col_tail) dst[e] = e8[e];
+            }
+        } else {
+            if (col_ok && row_ok) *reinterpret_cast<u32x4*>(dst) = v;
+        }
+    };
     u32x4 res[kResidual ? kIts : 1];
     auto fetch_residual = [&](int first, int last) {
         const __bf16* Rl = R + (row0 + lr) * r_pitch + col0 + lc * 8;
 #pragma unroll
         for (int it = first; it < last; it++) {
             res[it] = u32x4{0u, 0u, 0u, 0u};
-            if (col_ok && it * kRowsPerIt + lr < rows_here) res[it] = *reinterpret_cast<const u32x4*>(Rl + (size_t)(it * kRowsPerIt) * r_pitch);
+            const bool row_ok = it * kRowsPerIt + lr < rows_here;
+            const __bf16* src = Rl + (size_t)(it * kRowsPerIt) * r_pitch;
+            if constexpr (kAny) {
+                if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
+                else if (row_ok) {
+                    bf16x8 e8 = __builtin_bit_cast(bf16x8, res[it]);
+#pragma unroll
+                    for (int e = 0; e < 7; e++)
+                        if (e < col_tail) e8[e] = src[e];
+                    res[it] = __builtin_bit_cast(u32x4, e8);
+                }
+            } else {
+                if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4*>(src);
+            }
         }
     };
     {
@@ -595,7 +647,16 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
 #pragma unroll
             for (int j = 0; j < kJ16; j++) {
                 const size_t row = row0 + i * 16 + (lane & 15), col = col0 + j * 16 + 4 * (lane >> 4);
-                if (row < (size_t)M && col + 4 <= (size_t)N) *reinterpret_cast<f32x4*>(Wt + row * N + col) = acc[i][j];
+                if constexpr (kAny) {
+                    if (row < (size_t)M && col + 4 <= (size_t)N) *reinterpret_cast<f32x4_any*>(Wt + row * N + col) = acc[i][j];
+                    else if (row < (size_t)M) {
+#pragma unroll
+                        for (int e = 0; e < 3; e++)
+                            if (col + e < (size_t)N) Wt[row * N + col + e] = acc[i][j][e];
+                    }
+                } else {
+                    if (row < (size_t)M && col + 4 <= (size_t)N) *reinterpret_cast<f32x4*>(Wt + row * N + col) = acc[i][j];
+                }
             }
         return;
     }
@@ -667,9 +728,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             for (int t = 0; t < kPerRow; t++) {
                 const int r = i * 16 + t * kRowsPerIt;
                 if constexpr (kResidual) {
-                    const f32x8 sum = __builtin_convertvector(__builtin_bit_cast(bf16x8, v[t]), f32x8) +
-                                      __builtin_convertvector(__builtin_bit_cast(bf16x8, res[i * kPerRow + t]), f32x8);
-                    v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(sum, bf16x8));
+                    v[t] = add_elems<kF16>(v[t], res[i * kPerRow + t]);
                 }
                 if constexpr (kRope) {
                     if (rotate) {
@@ -681,7 +740,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
-                if (col_ok && r + lr < rows_here) *reinterpret_cast<u32x4*>(Cl + (size_t)r * ldc) = v[t];
+                store_chunk(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
             }
         }
         return;
@@ -722,66 +781,71 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     }
 }
 
-__global__ __launch_bounds__(256) void gemm_bf16_tile256(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                         __bf16* __restrict__ C, int M, int N, int K, int tiles_m,
-                                                         int tiles_n) {
-    gemm_tile_body<false, 4>(A, B, C, M, N, K, tiles_m, tiles_n);
-}
-// B^T variants: the second operand is Bt[N, K] row-major (k contiguous, the layout of a Linear
-// layer's weight), C = A Bt^T; for the gated epilogue Bt is [2F, K], gate rows first.
-#define MRK_GEMM_NT_KERNEL(name, ...)                                                                                      \
-    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ Bt,              \
-                                                __bf16* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n) { \
-        gemm_tile_body<__VA_ARGS__>(A, Bt, C, M, N, K, tiles_m, tiles_n);                                                  \
+// Instantiations.  B is [K, N], or ("_nt") Bt [N, K] row-major (k contiguous, the layout of a Linear layer's weight),
+// C = A Bt^T; for the gated epilogue B is [K, 2F] or Bt [2F, K], gate first.  lda / ldb are read by the "_any" kernels.
+#define MRK_GEMM_KERNEL(name, ...)                                                                                                    \
+    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ B, __bf16* __restrict__ C,   \
+                                                int M, int N, int K, int tiles_m, int tiles_n, int lda, int ldb) {                    \
+        gemm_tile_body<__VA_ARGS__>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, nullptr, RopeEpilogue{}, -1, lda, ldb);            \
     }
-#define MRK_GEMM_NT_RESIDUAL_KERNEL(name, ...)                                                                          \
-    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ Bt,           \
-                                                const __bf16* __restrict__ R, __bf16* __restrict__ C, int M, int N,    \
-                                                int K, int tiles_m, int tiles_n, int ldr) {                            \
-        gemm_tile_body<__VA_ARGS__>(A, Bt, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr);           \
+#define MRK_GEMM_RESIDUAL_KERNEL(name, ...)                                                                                           \
+    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ B,                           \
+                                                const __bf16* __restrict__ R, __bf16* __restrict__ C, int M, int N, int K,            \
+                                                int tiles_m, int tiles_n, int ldr, int lda, int ldb) {                                \
+        gemm_tile_body<__VA_ARGS__>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr, lda, ldb);                 \
     }
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile256, false, 4, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile256_ragged_k, true, 4, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile128, false, 2, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile128_ragged_k, true, 2, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile256_swiglu, false, 4, false, false, true, true)
-MRK_GEMM_NT_KERNEL(gemm_bf16_nt_tile256_swiglu_ragged_k, true, 4, false, false, true, true)
-MRK_GEMM_NT_RESIDUAL_KERNEL(gemm_bf16_nt_tile256_residual, false, 4, false, true, false, true)
-MRK_GEMM_NT_RESIDUAL_KERNEL(gemm_bf16_nt_tile256_residual_ragged_k, true, 4, false, true, false, true)
-MRK_GEMM_NT_RESIDUAL_KERNEL(gemm_bf16_nt_tile128_residual, false, 2, false, true, false, true)
-MRK_GEMM_NT_RESIDUAL_KERNEL(gemm_bf16_nt_tile128_residual_ragged_k, true, 2, false, true, false, true)
-// half-precision instantiations (plain product; [K, N] and [N, K] second operand)
-MRK_GEMM_NT_KERNEL(gemm_f16_tile256, false, 4, false, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_tile256_ragged_k, true, 4, false, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_tile128, false, 2, false, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_tile128_ragged_k, true, 2, false, false, false, false, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_nt_tile256, false, 4, false, false, false, true, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_nt_tile256_ragged_k, true, 4, false, false, false, true, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_nt_tile128, false, 2, false, false, false, true, true)
-MRK_GEMM_NT_KERNEL(gemm_f16_nt_tile128_ragged_k, true, 2, false, false, false, true, true)
-#undef MRK_GEMM_NT_KERNEL
-#undef MRK_GEMM_NT_RESIDUAL_KERNEL
-__global__ __launch_bounds__(256) void gemm_f16_tile128_splitk(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                               float* __restrict__ W, int M, int N, int K, int tiles_m,
-                                                               int tiles_n, int kt_per_split) {
-    gemm_tile_body<false, 2, true, false, false, false, true>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split);
-}
-__global__ __launch_bounds__(256) void gemm_f16_tile128_splitk_ragged_k(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                                        float* __restrict__ W, int M, int N, int K, int tiles_m,
-                                                                        int tiles_n, int kt_per_split) {
-    gemm_tile_body<true, 2, true, false, false, false, true>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split);
-}
-// split-K over a second operand stored [N, K]
-#define MRK_GEMM_NT_SPLITK_KERNEL(name, ragged, f16)                                                                                   \
-    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ B, float* __restrict__ W, int M, \
-                                                int N, int K, int tiles_m, int tiles_n, int kt_per_split) {                             \
-        gemm_tile_body<ragged, 2, true, false, false, true, f16>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split);            \
+#define MRK_GEMM_SPLITK_KERNEL(name, ...)                                                                                             \
+    __global__ __launch_bounds__(256) void name(const __bf16* __restrict__ A, const __bf16* __restrict__ B, float* __restrict__ W,    \
+                                                int M, int N, int K, int tiles_m, int tiles_n, int kt_per_split, int lda, int ldb) {  \
+        gemm_tile_body<__VA_ARGS__>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split, nullptr, RopeEpilogue{}, -1, lda, ldb); \
     }
-MRK_GEMM_NT_SPLITK_KERNEL(gemm_bf16_nt_tile128_splitk, false, false)
-MRK_GEMM_NT_SPLITK_KERNEL(gemm_bf16_nt_tile128_splitk_ragged_k, true, false)
-MRK_GEMM_NT_SPLITK_KERNEL(gemm_f16_nt_tile128_splitk, false, true)
-MRK_GEMM_NT_SPLITK_KERNEL(gemm_f16_nt_tile128_splitk_ragged_k, true, true)
-#undef MRK_GEMM_NT_SPLITK_KERNEL
+MRK_GEMM_KERNEL(gemm_bf16_tile256, false, 4, false, false, false, false, false)
+MRK_GEMM_KERNEL(gemm_bf16_tile256_any, true, 4, false, false, false, false, false)
+MRK_GEMM_KERNEL(gemm_bf16_tile128, false, 2, false, false, false, false, false)
+MRK_GEMM_KERNEL(gemm_bf16_tile128_any, true, 2, false, false, false, false, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_tile256_residual, false, 4, false, true, false, false, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_tile256_residual_any, true, 4, false, true, false, false, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_tile128_residual, false, 2, false, true, false, false, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_tile128_residual_any, true, 2, false, true, false, false, false)
+MRK_GEMM_SPLITK_KERNEL(gemm_bf16_tile128_splitk, false, 2, true, false, false, false, false)
+MRK_GEMM_SPLITK_KERNEL(gemm_bf16_tile128_splitk_any, true, 2, true, false, false, false, false)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile256, false, 4, false, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile256_any, true, 4, false, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile128, false, 2, false, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile128_any, true, 2, false, false, false, true, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_nt_tile256_residual, false, 4, false, true, false, true, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_nt_tile256_residual_any, true, 4, false, true, false, true, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_nt_tile128_residual, false, 2, false, true, false, true, false)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_bf16_nt_tile128_residual_any, true, 2, false, true, false, true, false)
+MRK_GEMM_SPLITK_KERNEL(gemm_bf16_nt_tile128_splitk, false, 2, true, false, false, true, false)
+MRK_GEMM_SPLITK_KERNEL(gemm_bf16_nt_tile128_splitk_any, true, 2, true, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_f16_tile256, false, 4, false, false, false, false, true)
+MRK_GEMM_KERNEL(gemm_f16_tile256_any, true, 4, false, false, false, false, true)
+MRK_GEMM_KERNEL(gemm_f16_tile128, false, 2, false, false, false, false, true)
+MRK_GEMM_KERNEL(gemm_f16_tile128_any, true, 2, false, false, false, false, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_tile256_residual, false, 4, false, true, false, false, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_tile256_residual_any, true, 4, false, true, false, false, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_tile128_residual, false, 2, false, true, false, false, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_tile128_residual_any, true, 2, false, true, false, false, true)
+MRK_GEMM_SPLITK_KERNEL(gemm_f16_tile128_splitk, false, 2, true, false, false, false, true)
+MRK_GEMM_SPLITK_KERNEL(gemm_f16_tile128_splitk_any, true, 2, true, false, false, false, true)
+MRK_GEMM_KERNEL(gemm_f16_nt_tile256, false, 4, false, false, false, true, true)
+MRK_GEMM_KERNEL(gemm_f16_nt_tile256_any, true, 4, false, false, false, true, true)
+MRK_GEMM_KERNEL(gemm_f16_nt_tile128, false, 2, false, false, false, true, true)
+MRK_GEMM_KERNEL(gemm_f16_nt_tile128_any, true, 2, false, false, false, true, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_nt_tile256_residual, false, 4, false, true, false, true, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_nt_tile256_residual_any, true, 4, false, true, false, true, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_nt_tile128_residual, false, 2, false, true, false, true, true)
+MRK_GEMM_RESIDUAL_KERNEL(gemm_f16_nt_tile128_residual_any, true, 2, false, true, false, true, true)
+MRK_GEMM_SPLITK_KERNEL(gemm_f16_nt_tile128_splitk, false, 2, true, false, false, true, true)
+MRK_GEMM_SPLITK_KERNEL(gemm_f16_nt_tile128_splitk_any, true, 2, true, false, false, true, true)
+MRK_GEMM_KERNEL(gemm_bf16_tile256_swiglu, false, 4, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_bf16_tile256_swiglu_any, true, 4, false, false, true, false)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile256_swiglu, false, 4, false, false, true, true)
+MRK_GEMM_KERNEL(gemm_bf16_nt_tile256_swiglu_any, true, 4, false, false, true, true)
+#undef MRK_GEMM_KERNEL
+#undef MRK_GEMM_RESIDUAL_KERNEL
+#undef MRK_GEMM_SPLITK_KERNEL
 __global__ __launch_bounds__(256) void gemm_bf16_tile256_rope(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                                               __bf16* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
                                                               RopeEpilogue rope) {
@@ -792,72 +856,53 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_tile256_rope(const __bf16* _
                                                               RopeEpilogue rope) {
     gemm_tile_body<false, 4, false, false, false, true, false, true>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, nullptr, rope);
 }
-__global__ __launch_bounds__(256) void gemm_bf16_tile256_ragged_k(const __bf16* __restrict__ A,
-                                                                  const __bf16* __restrict__ B, __bf16* __restrict__ C,
-                                                                  int M, int N, int K, int tiles_m, int tiles_n) {
-    gemm_tile_body<true, 4>(A, B, C, M, N, K, tiles_m, tiles_n);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile256_residual(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                                  const __bf16* __restrict__ R, __bf16* __restrict__ C, int M,
-                                                                  int N, int K, int tiles_m, int tiles_n, int ldr) {
-    gemm_tile_body<false, 4, false, true>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile256_residual_ragged_k(const __bf16* __restrict__ A,
-                                                                           const __bf16* __restrict__ B,
-                                                                           const __bf16* __restrict__ R, __bf16* __restrict__ C,
-                                                                           int M, int N, int K, int tiles_m, int tiles_n, int ldr) {
-    gemm_tile_body<true, 4, false, true>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile256_swiglu(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                                __bf16* __restrict__ C, int M, int N2, int K, int tiles_m,
-                                                                int tiles_n) {
-    gemm_tile_body<false, 4, false, false, true>(A, B, C, M, N2, K, tiles_m, tiles_n);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile256_swiglu_ragged_k(const __bf16* __restrict__ A,
-                                                                         const __bf16* __restrict__ B, __bf16* __restrict__ C,
-                                                                         int M, int N2, int K, int tiles_m, int tiles_n) {
-    gemm_tile_body<true, 4, false, false, true>(A, B, C, M, N2, K, tiles_m, tiles_n);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128_residual(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                                  const __bf16* __restrict__ R, __bf16* __restrict__ C, int M,
-                                                                  int N, int K, int tiles_m, int tiles_n, int ldr) {
-    gemm_tile_body<false, 2, false, true>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128_residual_ragged_k(const __bf16* __restrict__ A,
-                                                                           const __bf16* __restrict__ B,
-                                                                           const __bf16* __restrict__ R, __bf16* __restrict__ C,
-                                                                           int M, int N, int K, int tiles_m, int tiles_n, int ldr) {
-    gemm_tile_body<true, 2, false, true>(A, B, C, M, N, K, tiles_m, tiles_n, nullptr, 0, R, RopeEpilogue{}, ldr);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
-                                                         __bf16* __restrict__ C, int M, int N, int K, int tiles_m,
-                                                         int tiles_n) {
-    gemm_tile_body<false, 2>(A, B, C, M, N, K, tiles_m, tiles_n);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128_ragged_k(const __bf16* __restrict__ A,
-                                                                  const __bf16* __restrict__ B, __bf16* __restrict__ C,
-                                                                  int M, int N, int K, int tiles_m, int tiles_n) {
-    gemm_tile_body<true, 2>(A, B, C, M, N, K, tiles_m, tiles_n);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128_splitk(const __bf16* __restrict__ A,
-                                                                const __bf16* __restrict__ B, float* __restrict__ W,
-                                                                int M, int N, int K, int tiles_m, int tiles_n,
-                                                                int kt_per_split) {
-    gemm_tile_body<false, 2, true>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split);
-}
-__global__ __launch_bounds__(256) void gemm_bf16_tile128_splitk_ragged_k(const __bf16* __restrict__ A,
-                                                                         const __bf16* __restrict__ B,
-                                                                         float* __restrict__ W, int M, int N, int K,
-                                                                         int tiles_m, int tiles_n, int kt_per_split) {
-    gemm_tile_body<true, 2, true>(A, B, nullptr, M, N, K, tiles_m, tiles_n, W, kt_per_split);
+
+// dst[rows][pitch] = src[rows][cols] with zeros from cols to pitch (a multiple of 8): an operand whose rows start on odd
+// elements, laid out for the 16-byte copies of the tiled kernels.  A wave walks one row in 16-byte pieces (the loads
+// aligned to 2 bytes only).  Bound by HBM: 2 (cols + pitch) bytes a row.
+__global__ __launch_bounds__(256) void gemm_repitch(const unsigned short* __restrict__ src, unsigned short* __restrict__ dst, long rows,
+                                                    int cols, int pitch) {
+    const int lane = threadIdx.x & 63;
+    for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < rows; row += (long)gridDim.x * 4) {
+        const unsigned short* s = src + (size_t)row * cols;
+        u32x4* d = reinterpret_cast<u32x4*>(dst + (size_t)row * pitch);
+        for (int p = lane; p < pitch / 8; p += 64) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (p * 8 + 8 <= cols) v = *reinterpret_cast<const u32x4_any*>(s + p * 8);
+            else {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (p * 8 + e < cols) v[e >> 1] |= (unsigned)s[p * 8 + e] << (16 * (e & 1));
+            }
+            d[p] = v;
+        }
+    }
 }
 // C[i] = bf16(W[0][i] + W[1][i] + ... + W[splits-1][i]), 8 elements per work-item, partials added
 // in the order of their K ranges so the result does not depend on timing.  R, when given, is added to the rounded
 // sum and the result rounded again (the bits of the product followed by an elementwise add): a matrix of C's shape
 // (r_period 0) or one row repeated every r_period elements (a bias).
-template <bool kF16>
+// kAny: total (or r_period) is no multiple of 8: one element per work-item and the row of R element by element.
+template <bool kF16, bool kAny>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restrict__ W, __bf16* __restrict__ C, long total,
                                                           int splits, const __bf16* __restrict__ R, long r_period) {
+    if constexpr (kAny) {
+        const long i = (long)blockIdx.x * 256 + threadIdx.x;
+        if (i >= total) return;
+        float s = 0.0f;
+        for (int k = 0; k < splits; k++) s += W[(size_t)k * total + i];
+        const __bf16* r = R ? R + (r_period ? i % r_period : i) : nullptr;
+        if constexpr (kF16) {
+            _Float16 h = (_Float16)s;
+            if (r) h = (_Float16)((float)h + (float)__builtin_bit_cast(_Float16, *r));
+            C[i] = __builtin_bit_cast(__bf16, h);
+        } else {
+            __bf16 h = (__bf16)s;
+            if (r) h = (__bf16)((float)h + (float)*r);
+            C[i] = h;
+        }
+        return;
+    }
     const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
     if (i >= total) return;
     f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
@@ -947,7 +992,7 @@ SplitPlan plan_split_k(long M, long N, long K, long batch) {
     // at most a quarter of the CUs busy; with up to 64 rows (the weight is streamed once, the partial results are
     // small) up to half of them, and then two or three ranges already pay (16 x 22016 x 4096: 86 tiles)
     const bool few_rows = M <= 64;
-    if (K % 8 != 0 || N % 8 != 0 || tiles > (few_rows ? 128 : 64) || kt_all < 8) return p;
+    if (tiles > (few_rows ? 128 : 64) || kt_all < 8) return p;
     long want = 256 / tiles;                 // ranges that would put one workgroup on every CU
     if (want > kt_all / 2) want = kt_all / 2;  // at least two K steps per range
     // the partial results are written and read back once per range: worth it only while that
@@ -961,6 +1006,44 @@ SplitPlan plan_split_k(long M, long N, long K, long batch) {
     if (p.splits < 2) p.splits = 1;
     return p;
 }
+size_t split_k_bytes(long M, long N, long K, long batch) {
+    const SplitPlan p = plan_split_k(M, N, K, batch);
+    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
+}
+
+// shapes the tiled kernels address (32-bit offsets inside a tile); without scratch the operands' rows have to be whole
+// 16-byte chunks, see operand_padding
+bool tile_addressable(long M, long N, long K, long batch) {
+    if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || batch > 65535) return false;
+    if (M > 0x7fffffffL || N > 0x7fffffffL || K > (1L << 23) || N >= (1L << 25)) return false;
+    const long tn = (N + mrk::dev::kBN - 1) / mrk::dev::kBN, tm128 = (M + 127) / 128;
+    return tm128 * tn <= 0x7fffffffL;
+}
+// The operands whose rows are no whole 16-byte chunks, and the scratch their padded copies take (in front of the
+// split-K partials).  Copying costs twice the operand's bytes on top of the product's own traffic; what it replaces (one
+// wave per 32x32 tile, 2-byte loads straight from global memory) ran at 0.036 PFLOP/s on every shape: a projection of 512
+// rows onto 50257 columns at K = 768, weight [N, K], took 1560 us with the transposed copy that kernel needs and takes 50
+// (only C's rows are odd there: nothing is padded).
+struct OperandPadding {
+    bool a = false, b = false;
+    long lda = 0, ldb = 0;            // row pitches in elements as the kernel reads the operands
+    size_t a_bytes = 0, b_bytes = 0;  // scratch for the padded copies, multiples of 256
+};
+OperandPadding operand_padding(long M, long N, long K, long batch, bool b_transposed) {
+    OperandPadding o;
+    // A small [K, N] product stays with the kernel that needs no padding: it is one launch of at most one wave per SIMD
+    // and a few steps of K there (6.4-6.9 us from 33 x 7 x 19 to 256 x 255 x 63), two or three launches here (12-13 us);
+    // at K = 515 it is 20 against 15.  There is no such kernel for a [N, K] operand.
+    if (!b_transposed && (K % 8 || N % 8) && K <= 128 && ((M + 31) / 32) * ((N + 31) / 32) * batch <= 1024) return o;
+    const long row_b = b_transposed ? K : N, rows_b = batch * (b_transposed ? N : K);
+    o.a = K % 8 != 0;
+    o.b = row_b % 8 != 0;
+    o.lda = (K + 7) / 8 * 8;
+    o.ldb = (row_b + 7) / 8 * 8;
+    if (o.a) o.a_bytes = ((size_t)batch * M * o.lda * 2 + 255) / 256 * 256;
+    if (o.b) o.b_bytes = ((size_t)rows_b * o.ldb * 2 + 255) / 256 * 256;
+    return o;
+}
 }  // namespace
 
 size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch) {
@@ -969,8 +1052,10 @@ size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch) {
     // a handful of rows: streamed (one row on the vector ALUs where that kernel's plan takes the shape, more on the matrix pipes)
     if (gemm_kn_skinny_plan(M, N, K, batch, &ks, &kr)) return (size_t)ks * M * N * sizeof(float);
     if (gemm_kn_rows_plan(M, N, K, batch, &ks, &kr)) return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
-    const SplitPlan p = plan_split_k(M, N, K, batch);
-    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
+    if (!tile_addressable(M, N, K, batch)) return 0;
+    const OperandPadding pad = operand_padding(M, N, K, batch, false);
+    if (!pad.lda) return 0;
+    return pad.a_bytes + pad.b_bytes + split_k_bytes(M, N, K, batch);
 }
 
 int gemm_bf16_static_workspace_init(int device_id) {
@@ -986,9 +1071,15 @@ int gemm_bf16_static_workspace_init(int device_id) {
 
 size_t gemm_bf16_static_workspace_capacity() { return kStaticWsBytes; }
 
+size_t gemm_bf16_static_workspace_need(long M, long N, long K) {
+    const size_t need = gemm_bf16_workspace_bytes(M, N, K, 1);
+    // padded operands that do not fit: the kernel that needs no scratch
+    return need > kStaticWsBytes && (N % 8 || K % 8) ? 0 : need;
+}
+
 int launch_gemm_bf16_static_ws(void* stream, int device_id, const void* A, const void* B, void* C, long M, long N, long K) {
     if (device_id < 0 || device_id >= kMaxDevices) return (int)hipErrorInvalidDevice;
-    const size_t need = gemm_bf16_workspace_bytes(M, N, K, 1);
+    const size_t need = gemm_bf16_static_workspace_need(M, N, K);
     if (need > kStaticWsBytes) return (int)hipErrorInvalidValue;
     void* ws = g_static_ws[device_id].load(std::memory_order_acquire);
     if (!ws) return (int)hipErrorNotInitialized;
@@ -1000,13 +1091,8 @@ int launch_gemm_bf16_static_ws(void* stream, int device_id, const void* A, const
 bool gemm_bf16_residual_supported(long M, long N, long K, long batch);  // (defined behind tiled_shape)
 
 namespace {
-// shapes the tiled kernels address (any M; N and K in whole 16-byte chunks; 32-bit offsets inside a tile)
-bool tiled_shape(long M, long N, long K, long batch) {
-    if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || batch > 65535) return false;
-    if (M > 0x7fffffffL || N > 0x7fffffffL || N % 8 || K % 8 || K > (1L << 23) || N >= (1L << 25)) return false;
-    const long tn = (N + mrk::dev::kBN - 1) / mrk::dev::kBN, tm128 = (M + 127) / 128;
-    return tm128 * tn <= 0x7fffffffL;
-}
+// shapes the tiled kernels take without scratch for padded operands (any M; N and K in whole 16-byte chunks)
+bool tiled_shape(long M, long N, long K, long batch) { return tile_addressable(M, N, K, batch) && N % 8 == 0 && K % 8 == 0; }
 }  // namespace
 
 bool gemm_bf16_residual_supported(long M, long N, long K, long batch) { return tiled_shape(M, N, K, batch); }
@@ -1017,54 +1103,30 @@ bool gemm_bf16_nt_supported(long M, long N, long K, long batch) {
     return tiled_shape(M, N, K, batch) || gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch);
 }
 
+bool gemm_bf16_nt_padded_supported(long M, long N, long K, long batch) {
+    return gemm_bf16_nt_supported(M, N, K, batch) || tile_addressable(M, N, K, batch);
+}
+
 size_t gemm_bf16_nt_workspace_bytes(long M, long N, long K, long batch) {
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
     if (gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch)) return 0;  // streamed in one launch
-    const SplitPlan p = plan_split_k(M, N, K, batch);
-    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
+    if (!tile_addressable(M, N, K, batch)) return 0;
+    const OperandPadding pad = operand_padding(M, N, K, batch, true);
+    return pad.a_bytes + pad.b_bytes + split_k_bytes(M, N, K, batch);
 }
 
 int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
                       size_t workspace_bytes, bool b_transposed, bool f16, const void* add, bool add_is_row);
 
-namespace {
-// the tiled kernels with the residual epilogue (one pass of output tiles; variant 3 / 4 force the tile)
-int launch_tiled_residual(void* stream, const void* A, const void* B, const void* R, void* C, long M, long N, long K, long batch,
-                          bool b_transposed, bool r_is_row, int variant) {
-    using namespace mrk::dev;
-    if (M <= 0 || N <= 0 || batch <= 0) return 0;
-    if (!tiled_shape(M, N, K, batch)) return (int)hipErrorInvalidValue;
-    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(R)) % 16)
-        return (int)hipErrorInvalidValue;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    (void)hipGetLastError();
-    const long tn = (N + kBN - 1) / kBN, tm128 = (M + 127) / 128;
-    const bool small = variant == 4 || (variant != 3 && tm128 * tn * batch <= 256);
-    const long tm = small ? tm128 : (M + kBM - 1) / kBM;
-    const dim3 grid((unsigned)(tm * tn), (unsigned)batch);
-    const __bf16* a = static_cast<const __bf16*>(A);
-    const __bf16* b = static_cast<const __bf16*>(B);
-    const __bf16* r = static_cast<const __bf16*>(R);
-    __bf16* c = static_cast<__bf16*>(C);
-    const bool ragged_k = K % kBK != 0;
-    auto kernel = b_transposed ? (small ? (ragged_k ? gemm_bf16_nt_tile128_residual_ragged_k : gemm_bf16_nt_tile128_residual)
-                                        : (ragged_k ? gemm_bf16_nt_tile256_residual_ragged_k : gemm_bf16_nt_tile256_residual))
-                               : (small ? (ragged_k ? gemm_bf16_tile128_residual_ragged_k : gemm_bf16_tile128_residual)
-                                        : (ragged_k ? gemm_bf16_tile256_residual_ragged_k : gemm_bf16_tile256_residual));
-    kernel<<<grid, 256, 0, s>>>(a, b, r, c, (int)M, (int)N, (int)K, (int)tm, (int)tn, r_is_row ? 0 : -1);
-    return (int)hipGetLastError();
-}
-}  // namespace
-
 int launch_gemm_bf16_residual(void* stream, const void* A, const void* B, const void* R, void* C, long M, long N, long K, long batch,
-                              bool b_transposed, bool r_is_row, void* workspace, size_t workspace_bytes) {
+                              bool b_transposed, bool r_is_row, void* workspace, size_t workspace_bytes, bool f16) {
     if (!R) return (int)hipErrorInvalidValue;
-    return launch_gemm_16bit(stream, A, B, C, M, N, K, 0, batch, workspace, workspace_bytes, b_transposed, false, R, r_is_row);
+    return launch_gemm_16bit(stream, A, B, C, M, N, K, 0, batch, workspace, workspace_bytes, b_transposed, f16, R, r_is_row);
 }
 
 bool gemm_bf16_bias_supported(long M, long N, long K, long batch, bool b_transposed) {
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return false;
-    return (b_transposed && gemm_nt_bias_streamed(M, N, K, batch)) || tiled_shape(M, N, K, batch);
+    return (b_transposed && gemm_nt_bias_streamed(M, N, K, batch)) || (tile_addressable(M, N, K, batch) && operand_padding(M, N, K, batch, b_transposed).lda);
 }
 
 bool gemm_bf16_bias_launchable(long M, long N, long K, long batch, bool b_transposed) { return gemm_bf16_bias_supported(M, N, K, batch, b_transposed); }
@@ -1097,10 +1159,10 @@ int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C,
     const __bf16* a = static_cast<const __bf16*>(A);
     const __bf16* b = static_cast<const __bf16*>(B);
     __bf16* c = static_cast<__bf16*>(C);
-    const bool ragged_k = K % kBK != 0;
-    auto kernel = b_transposed ? (ragged_k ? gemm_bf16_nt_tile256_swiglu_ragged_k : gemm_bf16_nt_tile256_swiglu)
-                               : (ragged_k ? gemm_bf16_tile256_swiglu_ragged_k : gemm_bf16_tile256_swiglu);
-    kernel<<<grid, 256, 0, s>>>(a, b, c, (int)M, (int)(2 * F), (int)K, (int)tm, (int)tn);
+    const bool any = K % kBK != 0;
+    auto kernel = b_transposed ? (any ? gemm_bf16_nt_tile256_swiglu_any : gemm_bf16_nt_tile256_swiglu)
+                               : (any ? gemm_bf16_tile256_swiglu_any : gemm_bf16_tile256_swiglu);
+    kernel<<<grid, 256, 0, s>>>(a, b, c, (int)M, (int)(2 * F), (int)K, (int)tm, (int)tn, (int)K, b_transposed ? (int)K : (int)(2 * F));
     return (int)hipGetLastError();
 }
 
@@ -1128,11 +1190,64 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
 }
 
 namespace {
-int launch_tiled_residual(void* stream, const void* A, const void* B, const void* R, void* C, long M, long N, long K, long batch,
-                          bool b_transposed, bool r_is_row, int variant);
+// Output tiles over the chip: the K loop spread over ranges when the shape has a split plan and the caller brought the
+// scratch for the partial results, else one pass of 256-row or 128-row tiles.  Operands aligned to 16 bytes; those whose
+// rows are no whole 16-byte chunks are padded into the scratch first.  False when the scratch for that is missing.
+bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
+                  size_t workspace_bytes, bool b_transposed, bool f16, const __bf16* add, bool add_is_row) {
+    using namespace mrk::dev;
+    const OperandPadding pad = operand_padding(M, N, K, batch, b_transposed);
+    const __bf16 *a = static_cast<const __bf16*>(A), *b = static_cast<const __bf16*>(B);
+    __bf16* c = static_cast<__bf16*>(C);
+    char* ws = static_cast<char*>(workspace);
+    size_t ws_left = reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace ? workspace_bytes : 0;
+    if (pad.a_bytes + pad.b_bytes > ws_left || !pad.lda) return false;
+    auto padded = [&](const __bf16* src, long rows, long cols, long pitch, size_t bytes) {
+        const long groups = (rows + 3) / 4;
+        gemm_repitch<<<(unsigned)(groups < (1L << 20) ? groups : (1L << 20)), 256, 0, s>>>(
+            reinterpret_cast<const unsigned short*>(src), reinterpret_cast<unsigned short*>(ws), rows, (int)cols, (int)pitch);
+        const __bf16* at = reinterpret_cast<const __bf16*>(ws);
+        ws += bytes;
+        ws_left -= bytes;
+        return at;
+    };
+    if (pad.a) a = padded(a, batch * M, K, pad.lda, pad.a_bytes);
+    if (pad.b) b = padded(b, batch * (b_transposed ? N : K), b_transposed ? K : N, pad.ldb, pad.b_bytes);
+    const bool any = K % kBK != 0 || N % 8 != 0;
+    const int pitch_a = (int)pad.lda, pitch_b = (int)pad.ldb;
+    const long tn = (N + kBN - 1) / kBN, tm128 = (M + 127) / 128;
+#define MRK_PICK(stem) (f16 ? (b_transposed ? (any ? gemm_f16_nt_##stem##_any : gemm_f16_nt_##stem) : (any ? gemm_f16_##stem##_any : gemm_f16_##stem)) \
+                            : (b_transposed ? (any ? gemm_bf16_nt_##stem##_any : gemm_bf16_nt_##stem) : (any ? gemm_bf16_##stem##_any : gemm_bf16_##stem)))
+    const SplitPlan sp = variant == 0 || variant == 5 ? plan_split_k(M, N, K, batch) : SplitPlan();
+    if (sp.splits > 1 && ws_left >= (size_t)sp.splits * batch * M * N * sizeof(float) && batch * sp.splits <= 65535) {
+        float* w = reinterpret_cast<float*>(ws);
+        MRK_PICK(tile128_splitk)<<<dim3((unsigned)(tm128 * tn), (unsigned)batch, (unsigned)sp.splits), 256, 0, s>>>(
+            a, b, w, (int)M, (int)N, (int)K, (int)tm128, (int)tn, (int)sp.kt_per_split, pitch_a, pitch_b);
+        const long total = batch * M * N;
+        const bool each = total % 8 != 0 || (add_is_row && N % 8 != 0);
+        auto reduce_kernel = f16 ? (each ? gemm_splitk_reduce<true, true> : gemm_splitk_reduce<true, false>)
+                                 : (each ? gemm_splitk_reduce<false, true> : gemm_splitk_reduce<false, false>);
+        reduce_kernel<<<(unsigned)(((each ? total : total / 8) + 255) / 256), 256, 0, s>>>(w, c, total, (int)sp.splits, add, add_is_row ? N : 0);
+        return true;
+    }
+    // the 128-row tile when all its workgroups are resident at once (at most one per compute unit): twice the
+    // workgroups of the 256-row tile for the same work.  3 / 4 force one.
+    const bool small = variant == 4 || (variant != 3 && tm128 * tn * batch <= 256);
+    const long tm = small ? tm128 : (M + kBM - 1) / kBM;
+    const dim3 grid((unsigned)(tm * tn), (unsigned)batch);
+    if (add) {
+        auto kernel = small ? MRK_PICK(tile128_residual) : MRK_PICK(tile256_residual);
+        kernel<<<grid, 256, 0, s>>>(a, b, add, c, (int)M, (int)N, (int)K, (int)tm, (int)tn, add_is_row ? 0 : -1, pitch_a, pitch_b);
+    } else {
+        auto kernel = small ? MRK_PICK(tile128) : MRK_PICK(tile256);
+        kernel<<<grid, 256, 0, s>>>(a, b, c, (int)M, (int)N, (int)K, (int)tm, (int)tn, pitch_a, pitch_b);
+    }
+#undef MRK_PICK
+    return true;
 }
+}  // namespace
 
-// The product, with `add` (a matrix of C's shape or, add_is_row, one row [N]; bf16) added to the rounded result by
+// The product, with `add` (a matrix of C's shape or, add_is_row, one row [N]; of C's type) added to the rounded result by
 // whichever kernel writes it: the streaming kernels, the split-K reduction or the tiled kernels' residual epilogue.
 int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
                       size_t workspace_bytes, bool b_transposed, bool f16, const void* add, bool add_is_row) {
@@ -1140,23 +1255,17 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
     if (M <= 0 || N <= 0 || batch <= 0) return 0;
     if (add && reinterpret_cast<uintptr_t>(add) % 16) return (int)hipErrorInvalidValue;
     const __bf16* addp = static_cast<const __bf16*>(add);
-    const long add_period = add_is_row ? N : 0;
     if (batch > 65535) return (int)hipErrorInvalidValue;  // grid y extent
     if (M > 0x7fffffffL || N > 0x7fffffffL || K > 0x7fffffffL || K < 0) return (int)hipErrorInvalidValue;
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
     const bool aligned = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16) == 0;
-    // the tiled kernel addresses a tile's rows with 32-bit byte offsets from the tile origin:
-    // 255 rows of A (K elements each) and 49 rows of B (N elements each) must stay below 4 GiB
-    const bool offsets_fit = K <= (1L << 23) && N < (1L << 25);
     if (b_transposed) {
-        // B given as Bt[N, K]: the tiled kernels, or nothing (variant 3 / 4 force a tile size)
-        if (!aligned || !gemm_bf16_nt_supported(M, N, K, batch)) return (int)hipErrorInvalidValue;
-        const bool choose = variant == 0 || variant == 5;  // 3 / 4 force a tile where the shape has one
-        const bool tiled = tiled_shape(M, N, K, batch);
+        // B given as Bt[N, K]: the streaming or the tiled kernels, or nothing (variant 3 / 4 force a tile size)
+        if (!aligned || !gemm_bf16_nt_padded_supported(M, N, K, batch)) return (int)hipErrorInvalidValue;
         // up to 64 rows: one pass over the weight streams it faster than any tile (one or two rows on the
         // vector ALUs, more on the matrix pipes with 16-row blocks staged through LDS)
-        if (choose || !tiled) {
+        if (variant == 0 || variant == 5 || !tiled_shape(M, N, K, batch)) {
             if (add) {
                 if (gemm_nt_bias_streamed(M, N, K, batch)) return launch_gemm_nt_bias_streamed(stream, A, B, add, C, M, N, K, f16, add_is_row);
             } else {
@@ -1164,37 +1273,9 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
                 if (gemm_nt_rows_supported(M, N, K, batch)) return launch_gemm_nt_rows(stream, A, B, C, M, N, K, batch, f16);
             }
         }
-        if (!tiled) return (int)hipErrorInvalidValue;
-        const long tn = (N + kBN - 1) / kBN, tm128 = (M + 127) / 128;
-        const SplitPlan sp = choose ? plan_split_k(M, N, K, batch) : SplitPlan();
-        if (sp.splits > 1) {
-            // few output tiles against a long K: the K loop spread over the chip when the caller
-            // brought the workspace for the partial results
-            // (without one the plain tiled kernel runs on the few workgroups it has)
-            if (workspace && workspace_bytes >= (size_t)sp.splits * batch * M * N * sizeof(float) &&
-                reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && batch * sp.splits <= 65535) {
-                const dim3 grid((unsigned)(tm128 * tn), (unsigned)batch, (unsigned)sp.splits);
-                float* w = static_cast<float*>(workspace);
-                auto split_kernel = f16 ? (K % kBK == 0 ? gemm_f16_nt_tile128_splitk : gemm_f16_nt_tile128_splitk_ragged_k)
-                                        : (K % kBK == 0 ? gemm_bf16_nt_tile128_splitk : gemm_bf16_nt_tile128_splitk_ragged_k);
-                split_kernel<<<grid, 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B), w, (int)M, (int)N, (int)K,
-                                                  (int)tm128, (int)tn, (int)sp.kt_per_split);
-                const long total = batch * M * N;
-                auto reduce_kernel = f16 ? gemm_splitk_reduce<true> : gemm_splitk_reduce<false>;
-                reduce_kernel<<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>(w, static_cast<__bf16*>(C), total, (int)sp.splits, addp, add_period);
-                return (int)hipGetLastError();
-            }
-        }
-        if (add) return f16 ? (int)hipErrorInvalidValue : launch_tiled_residual(stream, A, B, add, C, M, N, K, batch, true, add_is_row, variant);
-        const bool small = variant == 4 || (variant != 3 && tm128 * tn * batch <= 256);
-        const long tm = small ? tm128 : (M + kBM - 1) / kBM;
-        const bool ragged_k = K % kBK != 0;
-        auto kernel = f16 ? (small ? (ragged_k ? gemm_f16_nt_tile128_ragged_k : gemm_f16_nt_tile128)
-                                   : (ragged_k ? gemm_f16_nt_tile256_ragged_k : gemm_f16_nt_tile256))
-                          : (small ? (ragged_k ? gemm_bf16_nt_tile128_ragged_k : gemm_bf16_nt_tile128)
-                                   : (ragged_k ? gemm_bf16_nt_tile256_ragged_k : gemm_bf16_nt_tile256));
-        kernel<<<dim3((unsigned)(tm * tn), (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
-                                                                          static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tm, (int)tn);
+        if (!tile_addressable(M, N, K, batch) ||
+            !launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, true, f16, addp, add_is_row))
+            return (int)hipErrorInvalidValue;
         return (int)hipGetLastError();
     }
     // up to 16 rows: one streaming pass over the weight into f32 partial sums, then their sum
@@ -1209,54 +1290,17 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
             return launch_gemm_kn_rows(stream, A, B, C, workspace, M, N, K, ks, kr, f16, add, add_is_row);
         }
     }
-    // any M; N and K in whole 16-byte chunks
-    if (variant != 2 && aligned && offsets_fit && K > 0 && N % 8 == 0 && K % 8 == 0) {
-        const long tn = (N + kBN - 1) / kBN;
-        const long tm128 = (M + 127) / 128;
-        // a handful of rows against a large weight matrix: spread the K loop over the chip when
-        // the caller brought the workspace for the partial results
-        const SplitPlan sp = variant == 0 || variant == 5 ? plan_split_k(M, N, K, batch) : SplitPlan();
-        if (sp.splits > 1 && workspace && workspace_bytes >= (size_t)sp.splits * batch * M * N * sizeof(float) &&
-            reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && batch * sp.splits <= 65535) {
-            const dim3 grid((unsigned)(tm128 * tn), (unsigned)batch, (unsigned)sp.splits);
-            float* w = static_cast<float*>(workspace);
-            const __bf16* a = static_cast<const __bf16*>(A);
-            const __bf16* b = static_cast<const __bf16*>(B);
-            auto split_kernel = f16 ? (K % kBK == 0 ? gemm_f16_tile128_splitk : gemm_f16_tile128_splitk_ragged_k)
-                                    : (K % kBK == 0 ? gemm_bf16_tile128_splitk : gemm_bf16_tile128_splitk_ragged_k);
-            split_kernel<<<grid, 256, 0, s>>>(a, b, w, (int)M, (int)N, (int)K, (int)tm128, (int)tn, (int)sp.kt_per_split);
-            const long total = batch * M * N;
-            auto reduce_kernel = f16 ? gemm_splitk_reduce<true> : gemm_splitk_reduce<false>;
-            reduce_kernel<<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>(w, static_cast<__bf16*>(C), total, (int)sp.splits, addp, add_period);
-            return (int)hipGetLastError();
-        }
-        // variant 0: the 128-row tile when all its workgroups are resident at once (at most one per
-        // compute unit): twice the workgroups of the 256-row tile for the same work.  3 / 4 force one.
-        if (add) return f16 ? (int)hipErrorInvalidValue : launch_tiled_residual(stream, A, B, add, C, M, N, K, batch, false, add_is_row, variant);
-        const bool small = variant == 4 || (variant != 3 && tm128 * tn * batch <= 256);
-        const long tm = small ? tm128 : (M + kBM - 1) / kBM;
-        if (tm * tn > 0x7fffffffL) return (int)hipErrorInvalidValue;
-        const dim3 grid((unsigned)(tm * tn), (unsigned)batch);
-        const __bf16* a = static_cast<const __bf16*>(A);
-        const __bf16* b = static_cast<const __bf16*>(B);
-        __bf16* c = static_cast<__bf16*>(C);
-        const bool ragged_k = K % kBK != 0;
-        auto kernel = f16 ? (small ? (ragged_k ? gemm_f16_tile128_ragged_k : gemm_f16_tile128)
-                                   : (ragged_k ? gemm_f16_tile256_ragged_k : gemm_f16_tile256))
-                          : (small ? (ragged_k ? gemm_bf16_tile128_ragged_k : gemm_bf16_tile128)
-                                   : (ragged_k ? gemm_bf16_tile256_ragged_k : gemm_bf16_tile256));
-        kernel<<<grid, 256, 0, s>>>(a, b, c, (int)M, (int)N, (int)K, (int)tm, (int)tn);
-    } else {
-        if (add) return (int)hipErrorInvalidValue;  // (the any-shape kernel has no epilogue)
-        const long tm = (M + 31) / 32, tn = (N + 31) / 32;
-        const long total = tm * tn;
-        const long blocks = (total + 3) / 4;
-        if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
-        auto generic = f16 ? gemm_bf16_generic<true> : gemm_bf16_generic<false>;
-        generic<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
-                                                           static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn,
-                                                           total);
-    }
+    if (variant != 2 && aligned && tile_addressable(M, N, K, batch) &&
+        launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, false, f16, addp, add_is_row))
+        return (int)hipGetLastError();
+    if (add) return (int)hipErrorInvalidValue;  // (the kernel below has no epilogue)
+    const long tm = (M + 31) / 32, tn = (N + 31) / 32;
+    const long total = tm * tn;
+    const long blocks = (total + 3) / 4;
+    if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
+    auto generic = f16 ? gemm_bf16_generic<true> : gemm_bf16_generic<false>;
+    generic<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
+                                                                   static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn, total);
     return (int)hipGetLastError();
 }
 

@@ -19,16 +19,18 @@ int launch_softmax_f32(void* stream, const void* x, void* y, long rows, long col
 // [batch, N, K] for batch > 1).  Same products in the same order, so the same bits as the [K, N]
 // form (split-K included, given the workspace).  Up to 64 rows with K a multiple of 8 take the
 // streaming kernels below (any N, no workspace), whose sums run in another order.  Shapes outside
-// gemm_bf16_nt_supported (K not a multiple of 8; N not a multiple of 8 with more than 64 rows)
-// are refused with hipErrorInvalidValue.
+// gemm_bf16_nt_supported (K not a multiple of 8; N not a multiple of 8 with more than 64 rows) need a
+// workspace of gemm_bf16_nt_workspace_bytes for padded operands (gemm_bf16_nt_padded_supported) and are
+// refused with hipErrorInvalidValue without one.
 // f16: operands and result are IEEE half precision instead of bf16 (the same kernels around
-// v_mfma_f32_16x16x32_f16; plain product only, the fused epilogues are bf16).
+// v_mfma_f32_16x16x32_f16; the gated and the rotary epilogue are bf16 only).
 int launch_gemm_bf16(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant,
                      long batch = 1, void* workspace = nullptr, size_t workspace_bytes = 0, bool b_transposed = false,
                      bool f16 = false);
 bool gemm_bf16_nt_supported(long M, long N, long K, long batch);
-// Scratch bytes launch_gemm_bf16 wants for the Bt[N, K] form: 0 for up to 64 rows (streamed), else the split-K
-// plan's as for the [K, N] form.
+bool gemm_bf16_nt_padded_supported(long M, long N, long K, long batch);
+// Scratch bytes launch_gemm_bf16 wants for the Bt[N, K] form: 0 for up to 64 rows (streamed), else what the [K, N]
+// form wants: padded copies of operands whose rows are no whole 16-byte chunks, and the split-K plan's partials.
 size_t gemm_bf16_nt_workspace_bytes(long M, long N, long K, long batch);
 // C[M, N] = A[M, K] @ Bt[N, K]^T for one or two rows (a decode step against a Linear layer's weight): one
 // pass over the weight with packed dot products, no matrix pipe, no scratch memory.  K a multiple
@@ -61,11 +63,13 @@ int launch_gemm_kn_rows(void* stream, const void* A, const void* B, void* C, voi
 // Linear layer's bias, tensor/src/nn/linear.rs:39-41): the same bits as the product followed by an elementwise add.  The
 // product takes the route launch_gemm_bf16 would take (same workspace: gemm_bf16[_nt]_workspace_bytes) and r is added by
 // whichever kernel writes the result: the tiled kernels' residual epilogue, the split-K reduction, the streaming kernels.
-// gemm_bf16_residual_supported: N and K multiples of 8 (the tiled kernels' shapes); with the second operand stored
-// [N, K] also every shape the streaming kernels take (gemm_bf16_bias_supported / _launchable tell, for either operand).
+// gemm_bf16_residual_supported: N and K multiples of 8 (what runs without a workspace); gemm_bf16_bias_supported /
+// _launchable: with the workspace, any shape the tiled kernels address, and with the second operand stored [N, K] also
+// every shape the streaming kernels take.
 bool gemm_bf16_residual_supported(long M, long N, long K, long batch);
 int launch_gemm_bf16_residual(void* stream, const void* a, const void* b, const void* r, void* c, long M, long N, long K, long batch,
-                              bool b_transposed = false, bool r_is_row = false, void* workspace = nullptr, size_t workspace_bytes = 0);
+                              bool b_transposed = false, bool r_is_row = false, void* workspace = nullptr, size_t workspace_bytes = 0,
+                              bool f16 = false);
 bool gemm_bf16_bias_supported(long M, long N, long K, long batch, bool b_transposed);
 bool gemm_bf16_bias_launchable(long M, long N, long K, long batch, bool b_transposed);
 int launch_gemm_bf16_bias(void* stream, const void* a, const void* b, const void* bias, void* c, long M, long N, long K, long batch,
@@ -95,10 +99,11 @@ int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c,
 bool gemm_bf16_rope_supported(long M, long N, long K, long split, long seq);
 int launch_gemm_bf16_rope(void* stream, const void* a, const void* b, void* c_rot, void* c_rest, long M, long N, long K, long split,
                           const void* cos, const void* sin, long seq, bool b_transposed = false);
-// Bytes of f32 scratch with which launch_gemm_bf16 spreads the K loop of this shape over the
-// chip (split-K: partial products per K range, added up in a fixed order by a second kernel);
-// 0 when the shape has enough output tiles by itself.  Without the workspace the same shape
-// runs unsplit.
+// Bytes of scratch launch_gemm_bf16 wants for this shape: padded copies of operands whose rows are
+// no whole 16-byte chunks (K, or N, no multiple of 8), and f32 partial results with which the K
+// loop is spread over the chip (split-K: partial products per K range, added up in a fixed order by a
+// second kernel); 0 for whole chunks and enough output tiles.  Without the workspace the same shape
+// runs unsplit, and one with odd rows on a kernel that reads them element by element.
 size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch);
 // The same product with the split-K partials in a file-scope device array instead of a
 // caller's workspace, for callers that must not allocate.  gemm_bf16_static_workspace_init
@@ -108,6 +113,7 @@ size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch);
 // when the address has not been resolved for device_id.  Calls on one device share the array.
 int gemm_bf16_static_workspace_init(int device_id);
 size_t gemm_bf16_static_workspace_capacity();
+size_t gemm_bf16_static_workspace_need(long M, long N, long K);  // (0 where the kernel without scratch takes over)
 int launch_gemm_bf16_static_ws(void* stream, int device_id, const void* A, const void* B, void* C, long M, long N, long K);
 
 // The attention kernels form the byte offset of a row inside one (batch, head) in 32 bits:

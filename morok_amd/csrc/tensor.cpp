@@ -1416,21 +1416,21 @@ struct Scheduler {
         if (gemm_bf16_workspace_bytes(M, N, K, batch) || gemm_kn_rows_plan(M, N, K, batch, &splits, &per)) return true;
         return transposed_weight(mm) && (gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch));
     }
-    // x + (a @ w) in bf16 where nothing else reads the product: the product kernel adds x in its
+    // x + (a @ w) in bf16 or f16 where nothing else reads the product: the product kernel adds x in its
     // epilogue (same bits as the product followed by the add).  Returns the product node and the
     // other operand.
     TensorNode* residual_matmul(TensorNode* n, TensorNode** other, bool* is_row = nullptr) const {
         if (is_row) *is_row = false;
-        if (!g_fusion || n->kind != TKind::Binary || static_cast<BinaryOp>(n->sub) != BinaryOp::Add || n->dtype != Scalar::BFloat16 ||
-            n->numel() == 0 || n->src.size() != 2)
+        if (!g_fusion || n->kind != TKind::Binary || static_cast<BinaryOp>(n->sub) != BinaryOp::Add ||
+            (n->dtype != Scalar::BFloat16 && n->dtype != Scalar::Float16) || n->numel() == 0 || n->src.size() != 2)
             return nullptr;
         for (int side = 0; side < 2; side++) {
             TensorNode* mm = n->src[side].get();
             TensorNode* r = n->src[1 - side].get();
-            if (mm->buffer || mm->hint != HintKind::Matmul || !fusable(mm) || mm->dtype != Scalar::BFloat16) continue;
+            if (mm->buffer || mm->hint != HintKind::Matmul || !fusable(mm) || mm->dtype != n->dtype) continue;
             auto u = uses.find(mm);
             if (u == uses.end() || u->second != 1) continue;
-            if (r->dtype != Scalar::BFloat16 || r->shape != n->shape || mm->shape != n->shape) continue;
+            if (r->dtype != n->dtype || r->shape != n->shape || mm->shape != n->shape) continue;
             int64_t M, N, K, batch;
             matmul_extents(mm, &M, &N, &K, &batch);
             // a bias (x @ w + b, tensor/src/nn/linear.rs:39-41): one row [N] that is in memory, broadcast over the
@@ -1439,7 +1439,7 @@ struct Scheduler {
             if (!r->buffer && (r->kind == TKind::Expand || (M * batch == 1 && r->kind == TKind::Reshape))) {
                 TensorNode* b = r->kind == TKind::Expand ? r->src[0].get() : r;
                 while (!b->buffer && b->kind == TKind::Reshape) b = b->src[0].get();
-                if (!b->buffer || b->dtype != Scalar::BFloat16 || b->numel() != N || n->shape.back() != N || b->buffer->offset() % 16) continue;
+                if (!b->buffer || b->dtype != n->dtype || b->numel() != N || n->shape.back() != N || b->buffer->offset() % 16) continue;
                 if (!gemm_bf16_bias_supported(M, N, K, batch, transposed_weight(mm) != nullptr)) continue;
                 *other = b;
                 if (is_row) *is_row = true;
@@ -1558,7 +1558,7 @@ struct Scheduler {
         MRK_TRY(weight_operand(mm, true, &wbuf, &nt));  // (the residual epilogue exists for exactly the shapes the B^T kernels take)
         MRK_TRY(materialize(r));
         auto out = new_buffer(n);
-        const std::string kind = std::string(nt ? "gemm_bf16_nt_" : "gemm_bf16_") + (is_row ? "bias" : "residual");
+        const std::string kind = std::string(n->dtype == Scalar::Float16 ? "gemm_f16_" : "gemm_bf16_") + (nt ? "nt_" : "") + (is_row ? "bias" : "residual");
         // few output tiles against a long K: scratch for the partial results, an intermediate of the plan like any other
         const size_t ws = nt ? gemm_bf16_nt_workspace_bytes(M, N, K, batch) : gemm_bf16_workspace_bytes(M, N, K, batch);
         if (ws) {
@@ -2139,7 +2139,7 @@ struct Scheduler {
             int64_t M, N, K, batch;
             matmul_extents(n, &M, &N, &K, &batch);
             MRK_TRY(materialize(n->hint_inputs[0].get()));
-            MRK_TRY(weight_operand(n, gemm_bf16_nt_supported(M, N, K, batch), &wbuf, &nt));
+            MRK_TRY(weight_operand(n, gemm_bf16_nt_padded_supported(M, N, K, batch), &wbuf, &nt));
         } else {
             for (const TensorRef& in : n->hint_inputs) MRK_TRY(materialize(in.get()));
         }
@@ -2154,8 +2154,9 @@ struct Scheduler {
             int64_t M = a->shape[a->shape.size() - 2], batch = 1;
             for (size_t i = 0; i + 2 < a->shape.size(); i++) (w->shape.size() == 2 ? M : batch) *= a->shape[i];
             if (a->dtype == Scalar::BFloat16 || a->dtype == Scalar::Float16) {
-                // few output tiles against a long K: scratch for split-K partials, an intermediate
-                // of the plan like any other (lazily allocated, placed by the memory planner)
+                // few output tiles against a long K, or operand rows that are no whole 16-byte chunks: scratch for
+                // split-K partials and padded operands, an intermediate of the plan like any other (lazily
+                // allocated, placed by the memory planner)
                 // (up to 64 rows against an [N, K] weight stream it in one pass and need no scratch)
                 const size_t ws = nt ? gemm_bf16_nt_workspace_bytes(M, N, K, batch) : gemm_bf16_workspace_bytes(M, N, K, batch);
                 const std::string kind = a->dtype == Scalar::Float16 ? "gemm_f16" : "gemm_bf16";

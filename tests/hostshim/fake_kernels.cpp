@@ -18,6 +18,7 @@ int launch_gemm_bf16(void* stream, const void*, const void*, void*, long, long, 
 bool gemm_bf16_nt_supported(long M, long N, long K, long batch) {
     return M > 0 && N > 0 && K > 0 && batch > 0 && N % 8 == 0 && K % 8 == 0;
 }
+bool gemm_bf16_nt_padded_supported(long M, long N, long K, long batch) { return gemm_bf16_nt_supported(M, N, K, batch); }
 bool gemm_nt_skinny_supported(long M, long N, long K, long batch) { return M >= 1 && M <= 2 && N >= 1 && K >= 8 && K % 8 == 0 && batch >= 1; }
 int launch_gemm_nt_skinny(void* stream, const void*, const void*, void*, long, long, long, long, bool f16) {
     mrk_shim_note_launch(stream, f16 ? "gemm_f16_nt" : "gemm_bf16_nt");
@@ -40,6 +41,7 @@ int launch_gemm_kn_skinny(void* stream, const void*, const void*, void*, void*, 
 }
 int gemm_bf16_static_workspace_init(int) { return 0; }
 size_t gemm_bf16_static_workspace_capacity() { return size_t(32) << 20; }
+size_t gemm_bf16_static_workspace_need(long, long, long) { return 0; }
 int launch_gemm_bf16_static_ws(void* stream, int, const void*, const void*, void*, long, long, long) {
     mrk_shim_note_launch(stream, "gemm_bf16");
     return 0;
@@ -55,7 +57,11 @@ int launch_gemm_bf16_bias(void* stream, const void*, const void*, const void*, v
 bool gemm_bf16_residual_supported(long M, long N, long K, long batch) {
     return M > 0 && N > 0 && K > 0 && batch > 0 && N % 8 == 0 && K % 8 == 0;
 }
-int launch_gemm_bf16_residual(void* stream, const void*, const void*, const void*, void*, long, long, long, long, bool b_transposed, bool r_is_row, void*, size_t) {
+int launch_gemm_bf16_residual(void* stream, const void*, const void*, const void*, void*, long, long, long, long, bool b_transposed, bool r_is_row, void*, size_t, bool f16) {
+    if (f16) {
+        mrk_shim_note_launch(stream, r_is_row ? (b_transposed ? "gemm_f16_nt_bias" : "gemm_f16_bias") : b_transposed ? "gemm_f16_nt_residual" : "gemm_f16_residual");
+        return 0;
+    }
     if (r_is_row) {
         mrk_shim_note_launch(stream, b_transposed ? "gemm_bf16_nt_bias" : "gemm_bf16_bias");
         return 0;
