@@ -133,6 +133,26 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                       }));
         return kOk;
     }
+    // f32 products on the f32 matrix instructions: {M, N, K}, buffers {c, a, b[, r]}, b [K, N] or ("_nt") [N, K], r one row
+    // ("_bias") or a matrix ("_residual").  The plain product carries the name the generated kernel of the same product has:
+    // which of the two runs is a matter of the shape.
+    if (k.compare(0, 8, "gemm_f32") == 0) {
+        const std::string rest = k.substr(8);
+        const bool nt = rest.compare(0, 3, "_nt") == 0;
+        const std::string tail = nt ? rest.substr(3) : rest;
+        const bool row = tail == "_bias", add = row || tail == "_residual";
+        if (tail.empty() || add) {
+            MRK_TRY(need(3));
+            if (!gemm_f32_supported(p[0], p[1], p[2])) return fail(kInvalidArgument, k + ": shape not covered");
+            const std::string dims = std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]);
+            const std::string name = !nt && !add ? "r_" + dims : k + "_" + dims;
+            out->reset(new BuiltinProgram(device_id, stream, name, add ? 4 : 3, p,
+                                          [nt, row, add](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+                                              return launch_gemm_f32(s, b[1], b[2], b[0], add ? b[3] : nullptr, row, q[0], q[1], q[2], nt, 0);
+                                          }));
+            return kOk;
+        }
+    }
     // the "_nt" kinds take the second operand as B^T [N, K] (a Linear layer's weight as it is stored)
     if (k == "gemm_bf16_nt" || k == "gemm_f16_nt") {  // {M, N, K}, {M, N, K, batch} or {M, N, K, batch, workspace bytes}; buffers {c, a, bt[, scratch]}
         const bool f16 = k == "gemm_f16_nt";

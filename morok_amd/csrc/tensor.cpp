@@ -1143,6 +1143,7 @@ struct Scheduler {
     RealizeStats stats;
     std::vector<TensorNode*> produced;  // nodes this realization gave a buffer
     std::vector<TensorNode*> produced_host;  // CPU nodes this realization gave host memory (device -> CPU copies)
+    const int beam = std::getenv("MOROK_BEAM") ? std::atoi(std::getenv("MOROK_BEAM")) : 0;
     std::unordered_map<const TensorNode*, int> uses;  // consumers of a node within the realised graph
 
     std::unordered_map<const TensorNode*, std::vector<TensorNode*>> matmul_readers;  // who reads each product node
@@ -1291,9 +1292,8 @@ struct Scheduler {
                     return batch <= 65535;
                 }
                 if (a->shape.size() != 2 || w->shape.size() != 2) return false;
-                if (a->dtype == Scalar::Float32)
-                    return a->shape[0] % 64 == 0 && w->shape[1] % 64 == 0 && a->shape[0] > 0 && w->shape[1] > 0;
-                return false;
+                if (a->dtype != Scalar::Float32) return false;
+                return matrix_f32(n) || (a->shape[0] % 64 == 0 && w->shape[1] % 64 == 0 && a->shape[0] > 0 && w->shape[1] > 0);
             }
             case HintKind::Sdpa: {
                 const TensorNode* q = n->hint_inputs[0].get();
@@ -1320,6 +1320,15 @@ struct Scheduler {
             }
             default: return false;
         }
+    }
+
+    // An f32 product of two matrices that the hand-written f32 kernels take (any shape above a few thousand multiply-adds per
+    // output tile).  Under MOROK_BEAM products stay with the generated kernels, whose choices it searches.
+    bool matrix_f32(const TensorNode* mm) const {
+        if (beam > 0 || mm->hint != HintKind::Matmul || mm->dtype != Scalar::Float32) return false;
+        const TensorNode *a = mm->hint_inputs[0].get(), *w = mm->hint_inputs[1].get();
+        return a->dtype == Scalar::Float32 && w->dtype == Scalar::Float32 && a->shape.size() == 2 && w->shape.size() == 2 &&
+               gemm_f32_supported(a->shape[0], w->shape[1], a->shape[1]);
     }
 
     // With the hand-written kernels switched off, a bf16 matmul whose shape fits still takes the
@@ -1416,14 +1425,15 @@ struct Scheduler {
         if (gemm_bf16_workspace_bytes(M, N, K, batch) || gemm_kn_rows_plan(M, N, K, batch, &splits, &per)) return true;
         return transposed_weight(mm) && (gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch));
     }
-    // x + (a @ w) in bf16 or f16 where nothing else reads the product: the product kernel adds x in its
+    // x + (a @ w) in bf16, f16 or f32 where nothing else reads the product: the product kernel adds x in its
     // epilogue (same bits as the product followed by the add).  Returns the product node and the
     // other operand.
     TensorNode* residual_matmul(TensorNode* n, TensorNode** other, bool* is_row = nullptr) const {
         if (is_row) *is_row = false;
         if (!g_fusion || n->kind != TKind::Binary || static_cast<BinaryOp>(n->sub) != BinaryOp::Add ||
-            (n->dtype != Scalar::BFloat16 && n->dtype != Scalar::Float16) || n->numel() == 0 || n->src.size() != 2)
+            (n->dtype != Scalar::BFloat16 && n->dtype != Scalar::Float16 && n->dtype != Scalar::Float32) || n->numel() == 0 || n->src.size() != 2)
             return nullptr;
+        const bool f32 = n->dtype == Scalar::Float32;
         for (int side = 0; side < 2; side++) {
             TensorNode* mm = n->src[side].get();
             TensorNode* r = n->src[1 - side].get();
@@ -1431,6 +1441,7 @@ struct Scheduler {
             auto u = uses.find(mm);
             if (u == uses.end() || u->second != 1) continue;
             if (r->dtype != n->dtype || r->shape != n->shape || mm->shape != n->shape) continue;
+            if (f32 && !matrix_f32(mm)) continue;
             int64_t M, N, K, batch;
             matmul_extents(mm, &M, &N, &K, &batch);
             // a bias (x @ w + b, tensor/src/nn/linear.rs:39-41): one row [N] that is in memory, broadcast over the
@@ -1440,7 +1451,7 @@ struct Scheduler {
                 TensorNode* b = r->kind == TKind::Expand ? r->src[0].get() : r;
                 while (!b->buffer && b->kind == TKind::Reshape) b = b->src[0].get();
                 if (!b->buffer || b->dtype != n->dtype || b->numel() != N || n->shape.back() != N || b->buffer->offset() % 16) continue;
-                if (!gemm_bf16_bias_supported(M, N, K, batch, transposed_weight(mm) != nullptr)) continue;
+                if (!f32 && !gemm_bf16_bias_supported(M, N, K, batch, transposed_weight(mm) != nullptr)) continue;
                 *other = b;
                 if (is_row) *is_row = true;
                 return mm;
@@ -1452,7 +1463,7 @@ struct Scheduler {
             if (!(rb->buffer || is_boundary_kind(rb) || fusable(rb))) continue;
             // (whichever kernel writes the product adds the operand: a tiled kernel's epilogue, the sum of a product spread
             // along K, a streaming kernel for a handful of rows)
-            if (!gemm_bf16_bias_supported(M, N, K, batch, transposed_weight(mm) != nullptr)) continue;
+            if (!f32 && !gemm_bf16_bias_supported(M, N, K, batch, transposed_weight(mm) != nullptr)) continue;
             *other = r;
             return mm;
         }
@@ -1498,8 +1509,8 @@ struct Scheduler {
     TensorNode* transposed_weight(const TensorNode* mm) const {
         if (!g_fusion) return nullptr;
         TensorNode* w = mm->hint_inputs[1].get();
-        if (w->buffer || w->kind != TKind::Permute || (w->dtype != Scalar::BFloat16 && w->dtype != Scalar::Float16) || w->shape.size() != 2 ||
-            w->arg.size() != 2 ||
+        if (w->buffer || w->kind != TKind::Permute || (w->dtype != Scalar::BFloat16 && w->dtype != Scalar::Float16 && !matrix_f32(mm)) ||
+            w->shape.size() != 2 || w->arg.size() != 2 ||
             w->arg[0] != 1 || w->arg[1] != 0)
             return nullptr;
         TensorNode* wt = w->src[0].get();
@@ -1558,6 +1569,13 @@ struct Scheduler {
         MRK_TRY(weight_operand(mm, true, &wbuf, &nt));  // (the residual epilogue exists for exactly the shapes the B^T kernels take)
         MRK_TRY(materialize(r));
         auto out = new_buffer(n);
+        if (n->dtype == Scalar::Float32) {
+            const std::string kind = std::string("gemm_f32") + (nt ? "_nt" : "") + (is_row ? "_bias" : "_residual");
+            MRK_TRY(builtin(kind.c_str(), {M, N, K}, {out, mm->hint_inputs[0]->buffer, wbuf, r->buffer}));
+            n->buffer = out;
+            produced.push_back(n);
+            return kOk;
+        }
         const std::string kind = std::string(n->dtype == Scalar::Float16 ? "gemm_f16_" : "gemm_bf16_") + (nt ? "nt_" : "") + (is_row ? "bias" : "residual");
         // few output tiles against a long K: scratch for the partial results, an intermediate of the plan like any other
         const size_t ws = nt ? gemm_bf16_nt_workspace_bytes(M, N, K, batch) : gemm_bf16_workspace_bytes(M, N, K, batch);
@@ -2140,6 +2158,9 @@ struct Scheduler {
             matmul_extents(n, &M, &N, &K, &batch);
             MRK_TRY(materialize(n->hint_inputs[0].get()));
             MRK_TRY(weight_operand(n, gemm_bf16_nt_padded_supported(M, N, K, batch), &wbuf, &nt));
+        } else if (n->hint == HintKind::Matmul && matrix_f32(n)) {
+            MRK_TRY(materialize(n->hint_inputs[0].get()));
+            MRK_TRY(weight_operand(n, true, &wbuf, &nt));
         } else {
             for (const TensorRef& in : n->hint_inputs) MRK_TRY(materialize(in.get()));
         }
@@ -2171,6 +2192,8 @@ struct Scheduler {
                 } else {
                     rc = batch == 1 ? builtin(kind.c_str(), {M, N, K}, {out, a->buffer, wbuf}) : builtin(kind.c_str(), {M, N, K, batch}, {out, a->buffer, wbuf});
                 }
+            } else if (matrix_f32(n)) {
+                rc = builtin(nt ? "gemm_f32_nt" : "gemm_f32", {M, N, K}, {out, a->buffer, wbuf});
             } else {
                 // MOROK_BEAM=<width> selects the LOCAL/UPCAST/UNROLL choices by timed search
                 // (cached on disk) instead of the fixed heuristic (tensor/src/realize.rs:1160-1250)
@@ -2185,8 +2208,6 @@ struct Scheduler {
                     opts = c;
                     if ((M / (c.local_y * c.up_m)) * (N / (c.local_x * c.up_n)) >= 512) break;
                 }
-                int beam = 0;
-                if (const char* e = std::getenv("MOROK_BEAM")) beam = std::atoi(e);
                 if (beam > 0) MRK_TRY(beam_search_matmul_f32(*dev, M, N, K, beam, &opts, nullptr, nullptr, nullptr));
                 LinearKernel k = build_matmul_f32_kernel(M, N, K, opts);
                 std::shared_ptr<CachedKernel> ck;

@@ -99,6 +99,11 @@ int launch_flash_fwd_bf16_ext(void* stream, const void*, const void*, const void
     mrk_shim_note_launch(stream, mask_kind == 0 && !(softcap > 0.0f) ? "flash_fwd_bf16_strided" : ws ? "flash_fwd_bf16_ext_splitkv" : "flash_fwd_bf16_ext");
     return 0;
 }
+bool gemm_f32_supported(long M, long N, long K) { return M > 0 && N > 0 && K >= 64 && M * N * K >= (1L << 18); }
+int launch_gemm_f32(void* stream, const void*, const void*, void*, const void* add, bool add_is_row, long, long, long, bool b_transposed, int) {
+    mrk_shim_note_launch(stream, add ? (add_is_row ? "gemm_f32_bias" : "gemm_f32_residual") : b_transposed ? "gemm_f32_nt" : "gemm_f32");
+    return 0;
+}
 int launch_fill(void* stream, void*, size_t, int, int, unsigned long long, unsigned long long, float, float) {
     mrk_shim_note_launch(stream, "fill");
     return 0;
