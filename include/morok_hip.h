@@ -666,6 +666,9 @@ int mrk_hip_tensor_expand(const mrk_tensor* t, const int64_t* shape, size_t ndim
 int mrk_hip_tensor_shrink(const mrk_tensor* t, const int64_t* begin, const int64_t* end, size_t ndim,
                           mrk_tensor** out);
 int mrk_hip_tensor_contiguous(const mrk_tensor* t, mrk_tensor** out);                         /* lib.rs:548 */
+/* A realization that computes `t` on the way to another tensor keeps its data: `t` is realized with it (a decode step's grown
+ * keys and values beside its output).  Plans from mrk_hip_tensor_prepare keep their root alone. */
+int mrk_hip_tensor_keep(const mrk_tensor* t);
 int mrk_hip_tensor_cat(const mrk_tensor* const* parts, size_t nparts, int64_t axis, mrk_tensor** out);
 /* elementwise, with broadcasting and dtype promotion (dtype/src/cast.rs:88) */
 int mrk_hip_tensor_cast(const mrk_tensor* t, int dtype, mrk_tensor** out);                    /* lib.rs:495 */

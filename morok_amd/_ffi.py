@@ -210,6 +210,7 @@ _SIGS = {
     "mrk_hip_tensor_transpose": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, c_void_pp]),
     "mrk_hip_tensor_expand": (C.c_int, [C.c_void_p, c_i64_p, C.c_size_t, c_void_pp]),
     "mrk_hip_tensor_shrink": (C.c_int, [C.c_void_p, c_i64_p, c_i64_p, C.c_size_t, c_void_pp]),
+    "mrk_hip_tensor_keep": (C.c_int, [C.c_void_p]),
     "mrk_hip_tensor_contiguous": (C.c_int, [C.c_void_p, c_void_pp]),
     "mrk_hip_tensor_cat": (C.c_int, [c_void_pp, C.c_size_t, C.c_int64, c_void_pp]),
     "mrk_hip_tensor_cast": (C.c_int, [C.c_void_p, C.c_int, c_void_pp]),

@@ -1344,6 +1344,10 @@ int mrk_hip_tensor_contiguous(const mrk_tensor* t, mrk_tensor** out) {
     MRK_T1(t);
     return wrap_tensor(t->t.contiguous(), out);
 }
+int mrk_hip_tensor_keep(const mrk_tensor* t) {
+    MRK_NONNULL(t);
+    return t->t.keep();
+}
 int mrk_hip_tensor_cat(const mrk_tensor* const* parts, size_t nparts, int64_t axis, mrk_tensor** out) {
     MRK_NONNULL(parts);
     MRK_NONNULL(out);

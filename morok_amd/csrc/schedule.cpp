@@ -366,7 +366,6 @@ uint32_t KernelBuilder::add(Op op, DType dt, std::vector<uint32_t> src, int64_t 
                             std::string str, std::vector<int64_t> extra) {
     // Common-subexpression elimination for side-effect-free value nodes: an identical node
     // that is still in scope is returned instead of a new one.
-    std::string key;
     bool pure = false;
     if (cse_) {
         switch (op) {
@@ -382,27 +381,42 @@ uint32_t KernelBuilder::add(Op op, DType dt, std::vector<uint32_t> src, int64_t 
             default: break;
         }
     }
+    uint64_t hash = 0;
     if (pure) {
-        auto put = [&](const void* p, size_t n) { key.append(static_cast<const char*>(p), n); };
-        uint16_t head[6] = {static_cast<uint16_t>(op), static_cast<uint16_t>(dt.scalar), dt.vcount,
-                            static_cast<uint16_t>(dt.is_ptr), static_cast<uint16_t>(dt.space), sub};
-        put(head, sizeof head);
-        put(&dt.ptr_size, sizeof dt.ptr_size);
-        put(&arg_i, sizeof arg_i);
-        put(&arg_f, sizeof arg_f);
-        for (uint32_t v : src) put(&v, sizeof v);
-        key.push_back('|');
-        for (int64_t v : extra) put(&v, sizeof v);
-        key.push_back('|');
-        key += str;
-        auto it = cse_map_.find(key);
-        if (it != cse_map_.end()) return it->second;
+        uint64_t f_bits;
+        std::memcpy(&f_bits, &arg_f, sizeof f_bits);
+        auto mix = [&](uint64_t v) {
+            hash ^= v;
+            hash *= 0x9e3779b97f4a7c15ull;
+            hash ^= hash >> 29;
+        };
+        mix(static_cast<uint64_t>(op) | static_cast<uint64_t>(dt.scalar) << 16 | static_cast<uint64_t>(dt.vcount) << 32 | static_cast<uint64_t>(sub) << 48);
+        mix(static_cast<uint64_t>(dt.ptr_size) ^ (dt.is_ptr ? 1ull << 63 : 0) ^ static_cast<uint64_t>(dt.space) << 60);
+        mix(static_cast<uint64_t>(arg_i));
+        mix(f_bits);
+        for (uint32_t v : src) mix(v);
+        for (int64_t v : extra) mix(static_cast<uint64_t>(v));
+        const auto same = cse_map_.equal_range(hash);
+        for (auto it = same.first; it != same.second; ++it) {
+            const UOp& u = node(it->second);
+            if (u.op == op && u.dtype.scalar == dt.scalar && u.dtype.vcount == dt.vcount && u.dtype.is_ptr == dt.is_ptr && u.dtype.space == dt.space &&
+                u.dtype.ptr_size == dt.ptr_size && u.sub == sub && u.arg_i == arg_i && std::memcmp(&u.arg_f, &arg_f, sizeof arg_f) == 0 && u.src == src &&
+                u.extra == extra && u.str == str)
+                return it->second;
+        }
     }
     // scopes: values defined inside a loop or a conditional are not visible after it closes
     if (cse_ && (op == Op::End || op == Op::EndIf)) {
         size_t closes = op == Op::End ? std::max<size_t>(src.size(), 1) : 1;
         for (size_t i = 0; i < closes && !cse_scopes_.empty(); i++) {
-            for (const std::string& k : cse_scopes_.back()) cse_map_.erase(k);
+            for (const auto& [h, node_id] : cse_scopes_.back()) {
+                const auto range = cse_map_.equal_range(h);
+                for (auto it = range.first; it != range.second; ++it)
+                    if (it->second == node_id) {
+                        cse_map_.erase(it);
+                        break;
+                    }
+            }
             cse_scopes_.pop_back();
         }
     }
@@ -419,8 +433,8 @@ uint32_t KernelBuilder::add(Op op, DType dt, std::vector<uint32_t> src, int64_t 
     k_.nodes.push_back(std::move(u));
     const uint32_t id = k_.nodes.back().id;
     if (pure) {
-        cse_map_.emplace(key, id);
-        if (!cse_scopes_.empty()) cse_scopes_.back().push_back(std::move(key));
+        cse_map_.emplace(hash, id);
+        if (!cse_scopes_.empty()) cse_scopes_.back().emplace_back(hash, id);
     }
     if (cse_ && (op == Op::Range || op == Op::If)) cse_scopes_.emplace_back();
     return id;
@@ -470,6 +484,7 @@ uint32_t KernelBuilder::imod(uint32_t a, int64_t c) {
 
 std::vector<uint8_t> KernelBuilder::serialize() const {
     std::vector<uint8_t> out;
+    out.reserve(12 + k_.nodes.size() * 64);
     auto put = [&](const void* p, size_t n) {
         const uint8_t* b = static_cast<const uint8_t*>(p);
         out.insert(out.end(), b, b + n);
@@ -504,7 +519,7 @@ std::vector<uint8_t> KernelBuilder::serialize() const {
 LinearKernel KernelBuilder::finish() {
     std::vector<uint8_t> bytes = serialize();
     k_.content_hash = fnv1a64(bytes.data(), bytes.size());
-    return k_;
+    return std::move(k_);  // (the builder is done with)
 }
 
 // ============================================================================ matmul kernels

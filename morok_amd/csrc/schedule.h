@@ -190,8 +190,8 @@ class KernelBuilder {
   private:
     LinearKernel k_;
     bool cse_ = false;
-    std::unordered_map<std::string, uint32_t> cse_map_;
-    std::vector<std::vector<std::string>> cse_scopes_;
+    std::unordered_multimap<uint64_t, uint32_t> cse_map_;  // hash of a node's contents -> its id
+    std::vector<std::vector<std::pair<uint64_t, uint32_t>>> cse_scopes_;
 };
 
 // Linearized kernels for the matmul shapes on the hot path.

@@ -2975,19 +2975,23 @@ int prepare_locked(const TensorRef& root, std::unique_ptr<ExecutionPlan>* out, s
         s.plan->set_outputs({s.plan->add_buffer(root->src[0]->buffer)});  // the device side of the copy stays whole
     } else {
         if (!root->buffer) MRK_TRY(s.materialize(root.get()));
-        s.plan->set_outputs({s.plan->add_buffer(root->buffer)});
+        std::vector<size_t> outputs{s.plan->add_buffer(root->buffer)};
+        // (a prepared plan is executed later, or never: only its root is promised to its caller)
+        for (TensorNode* t : s.produced)
+            if (kept && t->keep && t->buffer && t != root.get()) outputs.push_back(s.plan->add_buffer(t->buffer));
+        s.plan->set_outputs(outputs);
     }
     if (deferred && !deferred->empty()) return kCompileFirst;  // (the rollback returns every touched node to its lazy state)
     // Intermediates share blocks by liveness (tensor/src/memory_planner.rs); their contents do
-    // not outlive the plan's execution, so their nodes go back to being lazy: only the root
-    // keeps its buffer.  MOROK_NO_MEMORY_PLANNER=1 keeps every intermediate resident.
+    // not outlive the plan's execution, so their nodes go back to being lazy: only the root, and
+    // what the caller asked to keep of a realization, stay in memory.  MOROK_NO_MEMORY_PLANNER=1 keeps every intermediate resident.
     const char* no_planner = std::getenv("MOROK_NO_MEMORY_PLANNER");
     const bool planner = !(no_planner && no_planner[0] && no_planner[0] != '0');
     if (planner) s.plan->enable_memory_planner();
     MRK_TRY(s.plan->build());
     rollback.armed = false;
     for (TensorNode* t : s.produced) {
-        if (planner && t != root.get()) t->buffer = nullptr;
+        if (planner && t != root.get() && !(kept && t->keep && !to_cpu)) t->buffer = nullptr;
         else if (kept) kept->push_back(t);
     }
     if (kept) kept->insert(kept->end(), s.produced_host.begin(), s.produced_host.end());
@@ -3034,6 +3038,13 @@ int prepare_compiling_unlocked(const TensorRef& root, std::unique_lock<std::recu
     return prepare_locked(root, out, kept, nullptr, &fresh);
 }
 }  // namespace
+
+int Tensor::keep() const {
+    if (!n_) return fail(kInvalidArgument, "keep: invalid tensor");
+    std::lock_guard<std::recursive_mutex> lock(g_graph_mutex);
+    n_->keep = true;
+    return kOk;
+}
 
 int Tensor::prepare(std::unique_ptr<ExecutionPlan>* out) const {
     if (!n_) return fail(kInvalidArgument, "prepare: invalid tensor");

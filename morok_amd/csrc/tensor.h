@@ -57,6 +57,8 @@ struct TensorNode {
     // stream must be synchronized before the bytes of such a copy are read (kCpuDevice: none).
     std::shared_ptr<std::vector<uint8_t>> host;
     int host_from = kCpuDevice;
+    // Tensor::keep(): a realization that computes this node on the way to its root keeps its data
+    bool keep = false;
     // fused-kernel hint: the node is the root of a composed graph a hand-written kernel covers
     HintKind hint = HintKind::None;
     std::vector<TensorRef> hint_inputs;
@@ -117,6 +119,9 @@ class Tensor {
     Tensor try_unsqueeze(int64_t axis) const;
     Tensor try_squeeze(int64_t axis) const;
     Tensor contiguous() const;  // lib.rs:548
+    // A realization that computes this tensor on the way to another one keeps its data (this tensor is realized with it)
+    // instead of giving its memory to later intermediates.  A prepared plan keeps its root alone.
+    int keep() const;
     static Tensor cat(const std::vector<Tensor>& parts, int64_t axis);
 
     // ---- elementwise

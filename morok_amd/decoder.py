@@ -8,6 +8,7 @@ back to bfloat16 that rms_norm's f32 promotion requires placed at each stage out
 import numpy as np
 
 from . import synth, uop
+from .device import Buffer
 from .tensor import Tensor
 
 WEIGHT_NAMES = ("emb", "w_an", "Wq", "Wk", "Wv", "Wo", "w_fn", "W1", "W3", "W2")
@@ -52,6 +53,7 @@ class DecoderBlock:
         self.batch, self.seq, self.hidden, self.heads, self.ffn, self.eps = batch, seq, hidden, heads, ffn, eps
         self.dim = hidden // heads
         self.linear_layout = bool(linear_layout)
+        self.theta, self.device_id, self._rope = theta, device_id, None
         projections = ("Wq", "Wk", "Wv", "Wo", "W1", "W2", "W3")
         stored = {k: (np.ascontiguousarray(weights[k].T) if self.linear_layout and k in projections else np.ascontiguousarray(weights[k]))
                   for k in WEIGHT_NAMES}
@@ -116,6 +118,19 @@ class DecoderBlock:
         out = h2.try_add(self._proj(g, "W2"))
         return (out, k.contiguous(), v.contiguous()) if with_cache else out
 
+    def _rope_row(self, pos):
+        """cos and sin of one position as [1, 1, 1, dim/2] tensors: views of tables in device memory, made for the next
+        power of two of positions at a time (a step's own row costs no trigonometry, no upload and no wait)."""
+        half = self.dim // 2
+        pitch = -(-half // 16) * 16  # rows start on 64 bytes
+        tables = self._rope
+        if tables is None or pos >= tables[0]:
+            rows = max(256, 1 << pos.bit_length())
+            padded = np.zeros((2, rows, pitch), np.float32)
+            padded[0, :, :half], padded[1, :, :half] = rope_tables(rows, self.dim, self.theta)
+            tables = self._rope = (rows, Buffer.from_numpy(padded[0], self.device_id), Buffer.from_numpy(padded[1], self.device_id))
+        return [Tensor.from_buffer(t.view(pos * pitch * 4, half * 4), (1, 1, 1, half), uop.F32) for t in tables[1:]]
+
     def decode_step(self, tokens, past_k, past_v, pos):
         """One new token per sequence against the keys and values of the `pos` tokens before it, the way the reference
         carries a cache through its attention operator (onnx/src/registry/transformer.rs:74-75: K = cat(past, new) along
@@ -126,9 +141,7 @@ class DecoderBlock:
         once, and the attention is one query per head over pos + 1 keys."""
         assert self.fused, "decode_step uses the packed projections"
         w, B, H, D = self.w, self.batch, self.heads, self.dim
-        cos, sin = rope_tables(pos + 1, D)
-        cos_p = Tensor.from_numpy(np.ascontiguousarray(cos[pos].reshape(1, 1, 1, D // 2)))
-        sin_p = Tensor.from_numpy(np.ascontiguousarray(sin[pos].reshape(1, 1, 1, D // 2)))
+        cos_p, sin_p = self._rope_row(pos)
         h = w["emb"].embedding(tokens).contiguous()
         xn = self._norm(h, w["w_an"])
         qkv = self._proj(xn, "Wqkv")
@@ -138,8 +151,9 @@ class DecoderBlock:
         q = qk.try_shrink([(0, B), (0, 1), (0, H), (0, D)]).try_permute([0, 2, 1, 3])
         k_new = qk.try_shrink([(0, B), (0, 1), (H, 2 * H), (0, D)]).try_permute([0, 2, 1, 3])
         v_new = xv.try_reshape([B, 1, H, D]).try_permute([0, 2, 1, 3])
-        k_all = Tensor.cat([past_k, k_new], 2).contiguous()
-        v_all = Tensor.cat([past_v, v_new], 2).contiguous()
+        # kept: whoever realizes the output has the grown cache with it, and realizing those finds them done
+        k_all = Tensor.cat([past_k, k_new], 2).contiguous().keep()
+        v_all = Tensor.cat([past_v, v_new], 2).contiguous().keep()
         a = q.scaled_dot_product_attention(k_all, v_all)
         a = a.try_permute([0, 2, 1, 3]).try_reshape([B, self.hidden])
         h2 = h.try_add(self._proj(a, "Wo")).contiguous()

@@ -191,6 +191,11 @@ class Tensor:
     def contiguous(self):
         return self._new(lib.mrk_hip_tensor_contiguous)
 
+    def keep(self):
+        """A realization that computes this tensor on the way to another one keeps its data."""
+        check(lib.mrk_hip_tensor_keep(self._h))
+        return self
+
     @staticmethod
     def cat(parts, axis):
         arr = (C.c_void_p * len(parts))(*[p._h for p in parts])

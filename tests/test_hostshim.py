@@ -775,6 +775,45 @@ def test_planned_intermediates_become_lazy_again(T, shim):
     assert len(c.kernels()) == 1
 
 
+def test_kept_intermediates_are_realized_with_the_root(T, shim):
+    x = zeros(T, (64, 64))
+    mid = x.try_add(1.0).contiguous().keep()
+    other = mid.try_add(2.0).contiguous()          # not kept
+    plan = other.try_mul(2.0).sum(1).prepare()     # a prepared plan keeps its root alone
+    assert plan.kernel_count >= 2
+    assert len(mid.try_mul(3.0).realize().kernels()) == 2
+    a = other.try_mul(2.0).sum(1).realize()        # computed on the way to mid.try_mul above: read from now on
+    n = len(a.kernels())
+    assert mid.realize().kernels() == [] and mid.to_numpy().shape == (64, 64)
+    assert len(other.realize().kernels()) == 1 and n == 2
+    # a realization that fails while launching leaves a kept tensor lazy like the rest
+    k2 = x.try_sub(5.0).contiguous().keep()
+    shim.mrk_shim_fail_module_load_after(1)
+    with pytest.raises(MorokHipError):
+        k2.try_mul(x).sum(0).realize()
+    shim.mrk_shim_fail_module_load_after(-1)
+    assert len(k2.realize().kernels()) == 1
+
+
+def test_decode_step_is_one_realization(T, shim):
+    """The grown keys and values come with the output, and a step's rotary row is a view of tables that grow by powers of
+    two: equal to the row computed for that position alone, with no upload and no wait per step."""
+    from morok_amd import decoder, uop
+
+    blk = decoder.DecoderBlock(decoder.synthetic_weights(256, 512, 100, seed=1), 2, 1, 256, 2, 512, linear_layout=True)
+    ids = T.Tensor.from_numpy(np.zeros(2, np.int32))
+    for pos in (255, 256, 700):
+        past = T.Tensor.from_numpy(np.zeros((2, 2, pos, 128), np.uint16), uop.BF16)
+        cos, sin = decoder.rope_tables(pos + 1, 128)
+        got = blk._rope_row(pos)
+        assert np.array_equal(got[0].to_numpy().reshape(-1), cos[pos]) and np.array_equal(got[1].to_numpy().reshape(-1), sin[pos])
+        syncs = shim.mrk_shim_syncs()
+        out, k, v = blk.decode_step(ids, past, past, pos)
+        out.realize()
+        assert shim.mrk_shim_syncs() == syncs
+        assert k.realize().kernels() == [] and v.realize().kernels() == [] and k.shape == (2, 2, pos + 1, 128)
+
+
 def test_failed_schedule_leaves_the_graph_lazy(T, shim):
     """A kernel that fails to load in the middle of a realization must not leave provisional
     buffers on the nodes scheduled before it: the next realization of the same graph has to
