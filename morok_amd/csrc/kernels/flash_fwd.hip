@@ -45,6 +45,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQT = 128;       // queries per workgroup
 constexpr int kKT = 64;        // keys per tile
+constexpr int kMaxMaskTiles = 1024;  // key tiles of the row-mask kernels (8 KB of words)
 
 // max(x of lane l, x of lane l ^ 32): the swap exchanges the upper 32 lanes of its first
 // register with the lower 32 lanes of its second, which leaves one register holding the
@@ -82,7 +83,14 @@ struct FlashExt {
 // chunks; with 128-byte rows two consecutive rows span the banks, so the K swizzle uses
 // (row >> 1) & 7 over the 8 chunks of a row and the V granule swizzle (row & 3 over 32-byte
 // granules) needs no change.
-// kMask: 0 none, 1 Bool (one byte per element, nonzero = attend), 2 additive bf16.  kCap: softcap.
+// kMask: 0 none, 1 Bool (one byte per element, nonzero = attend), 2 additive bf16, 3 a Bool mask that is one row for every
+// query (a key-padding mask).  kCap: softcap.
+// The row mask is read once per workgroup, into one word of 64 bits per key tile: tiles behind the last visible key are
+// not visited, tiles before the first masked one take the unmasked body, and the others test a bit per score.  The
+// general Bool kernel reads eight groups of mask bytes per tile and lane and waits for them (and, the counter being one,
+// for the next tiles' copies) in every tile.  Measured against it, lengths between half and all of the keys: 8 x 16 heads,
+// 1000 x 1000, D = 64: 59.0 -> 40.7 us; 15 x 32, 2439 x 1592, D = 128: 1152 -> 842; 10 x 16, 973 x 1080, D = 256: 277 -> 204;
+// 2 x 8, 783 x 2680, D = 64 (112 workgroups): 48.8 -> 35.0.  Bound by the exponentials beside the matrix pipe.
 template <int kD, bool kStrided, int kMask = 0, bool kCap = false>
 __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, const __bf16* __restrict__ K,
                                                const __bf16* __restrict__ V, __bf16* __restrict__ O, int BH, int Sq, int Sk,
@@ -90,10 +98,13 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
                                                const FlashExt& ext = FlashExt{}) {
     static_assert(kD == 256 || kD == 128 || kD == 64, "head dims with an instantiation: 256, 128 and 64");
     static_assert(kStrided || (kMask == 0 && !kCap), "the extended kernels take their operands as views");
+    static_assert(kMask != 3 || !kCap, "under a softcap masked keys take part: no key tile may be left out");
     // The extended kernels turn every score into its final value in exp2 units (scale, masks,
     // softcap, log2 e) as soon as the score product has drained; from there on the online softmax
     // is the plain kernel's with a scale of one.
-    constexpr bool kExt = kMask != 0 || kCap;
+    constexpr bool kBits = kMask == 3;  // raw scores, as in the plain kernel
+    constexpr bool kExt = (kMask != 0 && !kBits) || kCap;
+    constexpr bool kEmptyRows = kExt || kBits;  // a query may have no visible key (yet)
     const float sc = kExt ? 1.0f : scale_log2e;
     constexpr int kRow = kD * 2;          // bytes per K/V row in LDS: 256 (128)
     constexpr int kTile = kKT * kRow;     // 16 KB (8 KB)
@@ -103,6 +114,7 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
     constexpr int kRowsPerDma = 64 / kCh; // rows one 1 KB copy covers: 4 (8)
     constexpr int kDmaPerWave = 16 / kRowsPerDma;  // copies per wave and tile: 4 (2)
     __shared__ __attribute__((aligned(1024))) char smem[4 * kTile];
+    __shared__ unsigned long long visible[kBits ? kMaxMaskTiles : 1];  // bit i of word t: key 64 t + i is visible
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Workgroup ids congruent mod 8 run on the same XCD and share its L2.  Each XCD walks
     // its own heads one after another, all work units of a head back to back, so the units
@@ -146,13 +158,37 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
     }
     const char* Kh = reinterpret_cast<const char*>(Kh_);
     const char* Vh = reinterpret_cast<const char*>(Vh_);
+    // kBits: the tiles up to the last one with a visible key (at least one: a row that sees nothing comes out as NaN),
+    // and the first one with a masked key
+    int key_tiles = (Sk + kKT - 1) / kKT, first_partial = key_tiles;
+    if constexpr (kBits) {
+        const int all = key_tiles;
+        for (int t = wave; t < all; t += 4) {
+            const int key = t * kKT + lane;
+            const bool on = key < Sk && mask_row[key] != 0;
+            const unsigned long long word = __builtin_amdgcn_ballot_w64(on);
+            if (lane == 0) visible[t] = word;
+        }
+        __syncthreads();
+        key_tiles = 1;
+        for (int t0 = all - 1 & ~63; t0 >= 0; t0 -= 64) {
+            const unsigned long long word = t0 + lane < all ? visible[t0 + lane] : 0;
+            const unsigned long long some = __builtin_amdgcn_ballot_w64(word != 0);
+            const unsigned long long partial = __builtin_amdgcn_ballot_w64(t0 + lane < all && word != ~0ull);
+            if (some && key_tiles == 1) key_tiles = t0 + 64 - __builtin_clzll(some);
+            if (partial) first_partial = t0 + __builtin_ctzll(partial);
+        }
+        key_tiles = __builtin_amdgcn_readfirstlane(key_tiles);
+        first_partial = __builtin_amdgcn_readfirstlane(first_partial);
+    }
     const int first_qt = causal ? q_tiles - 1 - unit : unit;
     const int npass = (causal && unit != first_qt) ? 2 : 1;
     // key tiles a query tile visits
     auto tiles_of = [&](int qt) {
         int kend = Sk;
         if (causal && qt * kQT + kQT < kend) kend = qt * kQT + kQT;
-        return (kend + kKT - 1) / kKT;
+        const int n = (kend + kKT - 1) / kKT;
+        return kBits && key_tiles < n ? key_tiles : n;
     };
     // The key tiles of the (up to) two passes form one sequence g = 0 .. ntot-1; the copies run
     // two (K) and one (V) tiles ahead along that sequence, across the pass boundary, and tile
@@ -254,7 +290,7 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
 
     // first tile that needs masking for this wave: the causal diagonal (a tile is clear of
     // it iff its last key <= the wave's first query) or the ragged tail of the keys
-    int first_masked = (Sk % kKT) ? Sk / kKT : ntiles;
+    int first_masked = kBits ? first_partial : (Sk % kKT) ? Sk / kKT : ntiles;
     if ((causal || (kExt && ext.causal_elem)) && qw0 / kKT < first_masked) first_masked = qw0 / kKT;
     const int qidx = qw0 + lq;
     const int lim = causal ? (qidx < Sk - 1 ? qidx : Sk - 1) : Sk - 1;  // last visible key
@@ -268,9 +304,9 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
         MaskGroup g[2][4];
     };
     const char* mask_q = nullptr;  // this lane's query row of the mask (of this pass)
-    if constexpr (kMask != 0) mask_q = mask_row + (long long)(qidx < Sq ? qidx : Sq - 1) * ext.row * (kMask == 2 ? 2 : 1);
+    if constexpr (kMask == 1 || kMask == 2) mask_q = mask_row + (long long)(qidx < Sq ? qidx : Sq - 1) * ext.row * (kMask == 2 ? 2 : 1);
     auto load_mask = [&](int key0, MaskTile& mt) {
-        if constexpr (kMask != 0) {
+        if constexpr (kMask == 1 || kMask == 2) {
 #pragma unroll
             for (int kb = 0; kb < 2; kb++)
 #pragma unroll
@@ -280,6 +316,23 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
                     mt.g[kb][g] = *reinterpret_cast<const MaskGroup*>(mask_q + (long long)key * (kMask == 2 ? 2 : 1));
                 }
         }
+    };
+    // kBits: bit 8 * (e / 4) + e % 4 of word kb tells whether this lane's score e of block kb counts
+    struct TileBits {
+        unsigned w[2];
+    };
+    auto tile_bits = [&](int j) {
+        TileBits b{};
+        if constexpr (kBits) {
+            unsigned long long v = visible[j];
+            if (causal) {
+                const int n = lim - j * kKT + 1;  // keys of the tile up to the diagonal
+                v &= n >= 64 ? ~0ull : n <= 0 ? 0ull : (1ull << n) - 1;
+            }
+            b.w[0] = (unsigned)v >> (4 * lg);
+            b.w[1] = (unsigned)(v >> 32) >> (4 * lg);
+        }
+        return b;
     };
     const int lim_causal = ext.causal_elem ? qidx : 0x7fffffff;  // reference mask: -inf before the softcap
     constexpr float kLog2e = 1.4426950408889634f;
@@ -341,6 +394,13 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
 #pragma unroll
                 for (int e = 0; e < 16; e++)
                     st[kb][e] = ext_score(st[kb][e], key0 + kb * 32 + 8 * (e >> 2) + 4 * lg + (e & 3), mt, kb, e, mask);
+        } else if (kBits && mask) {
+            const TileBits tb = tile_bits(key0 / kKT);
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    if (!(tb.w[kb] >> (8 * (e >> 2) + (e & 3)) & 1u)) st[kb][e] = -INFINITY;
         } else if (mask) {
 #pragma unroll
             for (int kb = 0; kb < 2; kb++)
@@ -376,7 +436,7 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
         if (__builtin_amdgcn_ballot_w64(mx_cur > m_run + lazy_thresh) != 0) {
             const float m_new = fmaxf(m_run, mx_cur);
             // (a row with nothing visible yet keeps -inf: its empty accumulators are left as they are)
-            const float alpha = kExt && m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * sc);
+            const float alpha = kEmptyRows && m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * sc);
             m_run = m_new;
             l_run *= alpha;
 #pragma unroll
@@ -393,7 +453,7 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
         const char* sKn = smem + ((g + 1) & 1) * kTile;
         const char* sV = smem + 2 * kTile + (g & 1) * kTile;
         // (a row whose keys so far are all masked has m_run = -inf: its probabilities must come out as 0, not NaN)
-        const float mb = kExt && m_run == -INFINITY ? 0.0f : m_run * sc;
+        const float mb = kEmptyRows && m_run == -INFINITY ? 0.0f : m_run * sc;
 
         // (the wave asks for the SIMD's issue slots first while it is in this phase, the one with the
         // exponentials: with two waves per SIMD that measured +0.5 to +2 % at D = 128 and up to +3.7 % at D = 64
@@ -470,6 +530,8 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
             vf[0] = vfrag(0);
             vf[1] = vfrag(1);
             const int key0n = (j + 1) * kKT;
+            TileBits tb{};
+            if constexpr (kBits && !kLast && decltype(mask_next)::value) tb = tile_bits(j + 1 < key_tiles ? j + 1 : j);
 #pragma unroll
             for (int n = 0; n < kNB; n++) {
                 if (n + 2 < kNB) vf[(n + 2) % 3] = vfrag(n + 2);
@@ -482,6 +544,8 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
                     for (int e = e0; e < e0 + kRegs; e++) {
                         if constexpr (kExt) {
                             nxt[kb][e] = ext_score(nxt[kb][e], key0n + kb * 32 + 8 * (e >> 2) + 4 * lg + (e & 3), mt, kb, e, decltype(mask_next)::value);
+                        } else if (kBits && decltype(mask_next)::value) {
+                            if (!(tb.w[kb] >> (8 * (e >> 2) + (e & 3)) & 1u)) nxt[kb][e] = -INFINITY;
                         } else if (decltype(mask_next)::value) {
                             const int key = key0n + kb * 32 + 8 * (e >> 2) + 4 * lg + (e & 3);
                             if (key > lim) nxt[kb][e] = -INFINITY;
@@ -641,6 +705,9 @@ MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d128_add, 128, 2, 2, false)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d128_cap, 128, 2, 0, true)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d128_bool_cap, 128, 2, 1, true)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d128_add_cap, 128, 2, 2, true)
+MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d128_rowmask, 128, 2, 3, false)
+MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d64_rowmask, 64, 2, 3, false)
+MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d256_rowmask, 256, 1, 3, false)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d64_bool, 64, 2, 1, false)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d64_add, 64, 2, 2, false)
 MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d64_cap, 64, 2, 0, true)
@@ -831,7 +898,12 @@ int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const 
         {{nullptr, flash_fwd_ext_d64_cap}, {flash_fwd_ext_d64_bool, flash_fwd_ext_d64_bool_cap}, {flash_fwd_ext_d64_add, flash_fwd_ext_d64_add_cap}},
         {{nullptr, flash_fwd_ext_d128_cap}, {flash_fwd_ext_d128_bool, flash_fwd_ext_d128_bool_cap}, {flash_fwd_ext_d128_add, flash_fwd_ext_d128_add_cap}},
         {{nullptr, flash_fwd_ext_d256_cap}, {flash_fwd_ext_d256_bool, flash_fwd_ext_d256_bool_cap}, {flash_fwd_ext_d256_add, flash_fwd_ext_d256_add_cap}}};
-    const Kernel kernel = table[D == 64 ? 0 : D == 128 ? 1 : 2][mask_kind][cap ? 1 : 0];
+    static const Kernel row_table[3] = {flash_fwd_ext_d64_rowmask, flash_fwd_ext_d128_rowmask, flash_fwd_ext_d256_rowmask};
+    const int dim = D == 64 ? 0 : D == 128 ? 1 : 2;
+    // one row of the mask for every query (its words are made once per workgroup; no query count was found at which the
+    // general kernel is ahead), as long as the words fit their 8 KB
+    const bool row_mask = mask_kind == 1 && !cap && (ext.row == 0 || Sq == 1) && Sk <= (long)kMaxMaskTiles * kKT;
+    const Kernel kernel = row_mask ? row_table[dim] : table[dim][mask_kind][cap ? 1 : 0];
     kernel<<<(unsigned)blocks, 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const __bf16*>(q), static_cast<const __bf16*>(k), static_cast<const __bf16*>(v), static_cast<__bf16*>(o), (int)BH,
         (int)Sq, (int)Sk, scale_log2e, causal_tiles, (int)q_tiles, (int)units, lay, ext);
