@@ -108,6 +108,16 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                       }));
         return kOk;
     }
+    if (k == "softmax_bf16" || k == "softmax_f16") {
+        MRK_TRY(need(2));
+        if (!softmax_half_supported(p[0], p[1])) return fail(kInvalidArgument, k + ": rows of 1 to 65536 elements");
+        const bool f16 = k == "softmax_f16";
+        out->reset(new BuiltinProgram(device_id, stream, k + "_" + std::to_string(p[0]) + "_" + std::to_string(p[1]), 2, p,
+                                      [f16](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+                                          return launch_softmax_half(s, b[1], b[0], q[0], q[1], f16);
+                                      }));
+        return kOk;
+    }
     // "gemm_f16" / "gemm_f16_nt": the same kernels on IEEE half precision operands and result
     if (k == "gemm_bf16" || k == "gemm_f16") {  // {M, N, K}, {M, N, K, batch} or {M, N, K, batch, workspace bytes}
         const bool f16 = k == "gemm_f16";

@@ -8,7 +8,9 @@ namespace mrk {
 
 // y = softmax(x, axis=-1), x and y f32 [rows, cols] row-major.  variant 0 = default.
 int launch_softmax_f32(void* stream, const void* x, void* y, long rows, long cols, int variant);
-
+// the same over bf16 (f16: IEEE half) rows of up to 65536 elements, f32 inside, one rounding
+bool softmax_half_supported(long rows, long cols);
+int launch_softmax_half(void* stream, const void* x, void* y, long rows, long cols, bool f16);
 
 // C[M,N] = A[M,K] * B[K,N]; bf16 row-major operands, f32 accumulate, bf16 result.
 // variant 0 = choose by shape, 2 = force the any-shape kernel, 3 / 4 = force the 256-row /

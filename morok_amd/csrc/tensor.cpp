@@ -1273,8 +1273,11 @@ struct Scheduler {
             case HintKind::Swish: return false;  // no kernel of its own: only matched as part of swiglu_matmul
             case HintKind::Rope: return false;   // likewise: only matched as the epilogue of a packed projection (rope_matmul)
             case HintKind::Softmax:
-                return n->dtype == Scalar::Float32 && !n->shape.empty() &&
-                       n->arg[0] == static_cast<int64_t>(n->shape.size()) - 1 && n->numel() > 0;
+                if (n->shape.empty() || n->arg[0] != static_cast<int64_t>(n->shape.size()) - 1 || n->numel() <= 0) return false;
+                if (n->dtype == Scalar::Float32) return true;
+                // half rows of whole waves of vectors are one row-resident generated kernel, which can take what is
+                // around the softmax in as well; all others would be three kernels
+                return is_half(n->dtype) && !row_fused_block(n) && softmax_half_supported(n->numel() / n->shape.back(), n->shape.back());
             case HintKind::Matmul: {
                 const TensorNode *a = n->hint_inputs[0].get(), *w = n->hint_inputs[1].get();
                 if (a->dtype != w->dtype) return false;
@@ -2168,7 +2171,8 @@ struct Scheduler {
         int rc = kOk;
         if (n->hint == HintKind::Softmax) {
             const int64_t cols = n->shape.back(), rows = n->numel() / cols;
-            rc = builtin("softmax_f32", {rows, cols}, {out, n->hint_inputs[0]->buffer});
+            const char* kind = n->dtype == Scalar::Float32 ? "softmax_f32" : n->dtype == Scalar::BFloat16 ? "softmax_bf16" : "softmax_f16";
+            rc = builtin(kind, {rows, cols}, {out, n->hint_inputs[0]->buffer});
         } else if (n->hint == HintKind::Matmul) {
             const TensorNode *a = n->hint_inputs[0].get(), *w = n->hint_inputs[1].get();
             const int64_t K = a->shape.back(), N = w->shape.back();
@@ -2335,6 +2339,28 @@ struct Scheduler {
     // Up to three such reductions may feed the kernel, one building on another (softmax: the row
     // maximum, then the sum of exp(x - max); layer norm: the mean, then the variance of the centred
     // row): they are returned in an order in which each one's own expression only needs earlier ones.
+    // Work-items that share a row of `n` in a row-resident kernel; 0: rows of this shape are not kept in registers.
+    static int64_t row_fused_block(const TensorNode* n) {
+        const int64_t C = n->shape.back(), rows = n->numel() / C;
+        int64_t width = 1;
+        for (int64_t w = 16 / static_cast<int64_t>(scalar_size(n->dtype)); w > 1; w /= 2)
+            if (C % w == 0) {
+                width = w;
+                break;
+            }
+        const int64_t V = C / width;
+        int64_t block = 0;
+        for (int64_t c : {256, 128, 64})
+            if (V % c == 0) {
+                block = c;
+                break;
+            }
+        // whole waves, at most 8 vectors per work-item (the row stays in registers), enough rows to fill the chip; a
+        // handful of short rows (a decode step's activations: up to 1 MiB in all) is bound by launches, not by the
+        // chip, and one kernel instead of a reduction and an elementwise kernel is the faster form there
+        const bool tiny = n->numel() * static_cast<int64_t>(scalar_size(n->dtype)) <= (1 << 20);
+        return !block || V / block > 8 || (rows < 128 && !tiny) ? 0 : block;
+    }
     std::vector<TensorNode*> row_reduce_deps(const TensorNode* n, const std::vector<TensorNode*>& deps, int64_t* block_out) {
         const char* off = std::getenv("MOROK_NO_ROW_FUSION");
         if (off && off[0] && off[0] != '0') return {};
@@ -2443,25 +2469,8 @@ struct Scheduler {
         if (!keeps_row(n, true)) return {};
         for (TensorNode* R : ordered)
             if (!keeps_row(R->src[0].get(), true)) return {};
-        const int64_t C = n->shape.back(), rows = n->numel() / C;
-        int64_t width = 1;
-        for (int64_t w = 16 / static_cast<int64_t>(scalar_size(n->dtype)); w > 1; w /= 2)
-            if (C % w == 0) {
-                width = w;
-                break;
-            }
-        const int64_t V = C / width;
-        int64_t block = 0;
-        for (int64_t c : {256, 128, 64})
-            if (V % c == 0) {
-                block = c;
-                break;
-            }
-        // whole waves, at most 8 vectors per work-item (the row stays in registers), enough rows to fill the chip; a
-        // handful of short rows (a decode step's activations: up to 1 MiB in all) is bound by launches, not by the
-        // chip, and one kernel instead of a reduction and an elementwise kernel is the faster form there
-        const bool tiny = n->numel() * static_cast<int64_t>(scalar_size(n->dtype)) <= (1 << 20);
-        if (!block || V / block > 8 || (rows < 128 && !tiny)) return {};
+        const int64_t block = row_fused_block(n);
+        if (!block) return {};
         *block_out = block;
         return ordered;
     }

@@ -9,6 +9,11 @@ int launch_softmax_f32(void* stream, const void*, void*, long, long, int) {
     mrk_shim_note_launch(stream, "softmax_f32");
     return 0;
 }
+bool softmax_half_supported(long rows, long cols) { return rows > 0 && cols > 0 && cols <= 65536; }
+int launch_softmax_half(void* stream, const void*, void*, long, long, bool f16) {
+    mrk_shim_note_launch(stream, f16 ? "softmax_f16" : "softmax_bf16");
+    return 0;
+}
 size_t gemm_bf16_workspace_bytes(long, long, long, long) { return 0; }
 size_t gemm_bf16_nt_workspace_bytes(long, long, long, long) { return 0; }
 int launch_gemm_bf16(void* stream, const void*, const void*, void*, long, long, long, int, long, void*, size_t, bool b_transposed, bool f16) {
