@@ -2878,18 +2878,32 @@ struct Scheduler {
         uint32_t oc = P > 1 ? b.idiv(wc, P) : wc;
         uint32_t seg0 = P > 1 ? b.imul(b.imod(wc, P), chunk) : g.ci(0);  // first reduce index of the segment
         Coords coords = plain(unflatten(g, oc, n->shape));
-        const int64_t steps = (chunk + 64 * G - 1) / (64 * G);
+        // A long fold over the contiguous axis is read in groups of up to 16 bytes per lane (of the widest operand: eight
+        // elements of a half type) where the axis divides into them: one memory request and one loop step per group
+        // instead of one per element.  Small graphs keep the short kernel: they are bound by its latency and by
+        // the time it takes to emit.  Measured, RMSNorm with its second kernel unchanged, bf16: 4503 x 3608 31.5 -> 16.9 us,
+        // 2065 x 2128 11.7 -> 6.8, 16384 x 8184 231 -> 144.
+        int64_t W8 = 1;
+        if (n->arg.size() == 1 && n->arg[0] == static_cast<int64_t>(s->shape.size()) - 1 && Nout * R >= (1LL << 20) && P == 1)
+            for (int64_t c = 8; c > 1 && W8 == 1; c /= 2)
+                if (R % c == 0 && R >= 64 * G * c) W8 = c;
+        g.width = W8;
+        const int64_t steps = (chunk + 64 * G * W8 - 1) / (64 * G * W8);
         uint32_t rg = b.add(Op::Range, KernelBuilder::scalar(g.idx_t), {g.ci(steps)}, 0, 0, static_cast<uint16_t>(AxisType::Reduce));
-        // block rg * G + ly of the segment: the G waves read neighbouring 256-byte blocks
+        // block rg * G + ly of the segment: the G waves read neighbouring blocks of 64 groups
         uint32_t blk = G > 1 ? b.iadd(b.imul(rg, G), ly) : rg;
-        uint32_t in_seg = b.iadd(b.imul(blk, 64), lane);
+        uint32_t in_seg = b.imul(b.iadd(b.imul(blk, 64), lane), W8);
         uint32_t f = b.iadd(seg0, in_seg);
-        const bool exact = chunk % (64 * G) == 0 && chunk * P == R;
+        const bool exact = chunk % (64 * G * W8) == 0 && chunk * P == R;
         uint32_t fgate = b.binary(BinaryOp::And, b.binary(BinaryOp::Lt, in_seg, g.ci(chunk)), b.binary(BinaryOp::Lt, f, g.ci(R)));
-        uint32_t fc = exact ? f : b.where(fgate, f, g.ci(R - 1));
+        uint32_t fc = exact ? f : b.where(fgate, f, g.ci(R - W8));
         std::vector<uint32_t> rc = unflatten(g, fc, rdims);
-        for (size_t r = 0; r < n->arg.size(); r++) coords[n->arg[r]] = Cx{rc[r], 0, false};
-        uint32_t v = emit(g, s, coords);
+        uint32_t v = 0;
+        for (int64_t e = 0; e < W8; e++) {
+            for (size_t r = 0; r < n->arg.size(); r++) coords[n->arg[r]] = Cx{rc[r], e, W8 > 1, W8 > 1 ? W8 : 0};
+            uint32_t ve = emit(g, s, coords);
+            v = e == 0 ? ve : b.binary(op == ReduceOp::Add ? BinaryOp::Add : BinaryOp::Max, v, ve);
+        }
         if (!exact) v = b.where(fgate, v, identity());
         uint32_t red = b.reduce(op, v, {rg});
         b.end({rg});
