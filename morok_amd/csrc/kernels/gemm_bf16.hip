@@ -582,17 +582,13 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     const bool col_ok = col0 + lc * 8 + 8 <= (size_t)N;
     // columns of this lane's chunk inside C when the chunk is the partial last one of a row (kAny: N % 8 of them), else 0
     const int col_tail = kAny && !col_ok && col0 + lc * 8 < (size_t)N ? (int)((size_t)N - (col0 + lc * 8)) : 0;
-    auto store_chunk = [&](__bf16* dst, const u32x4& v, bool row_ok) {
-        if constexpr (kAny) {
-            if (col_ok && row_ok) *reinterpret_cast<u32x4_any*>(dst) = v;
-            else if (row_ok) {
-                const bf16x8 e8 = __builtin_bit_cast(bf16x8, v);
+    auto store_any = [&](__bf16* dst, const u32x4& v, bool row_ok) {
+        if (col_ok && row_ok) *reinterpret_cast<u32x4_any*>(dst) = v;
+        else if (row_ok) {
+            const bf16x8 e8 = __builtin_bit_cast(bf16x8, v);
 #pragma unroll
-                for (int e = 0; e < 7; e++)
-                    if (e < col_tail) dst[e] = e8[e];
-            }
-        } else {
-            if (col_ok && row_ok) *reinterpret_cast<u32x4*>(dst) = v;
+            for (int e = 0; e < 7; e++)
+                if (e < col_tail) dst[e] = e8[e];
         }
     };
     u32x4 res[kResidual ? kIts : 1];
@@ -601,9 +597,9 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
 #pragma unroll
         for (int it = first; it < last; it++) {
             res[it] = u32x4{0u, 0u, 0u, 0u};
-            const bool row_ok = it * kRowsPerIt + lr < rows_here;
             const __bf16* src = Rl + (size_t)(it * kRowsPerIt) * r_pitch;
             if constexpr (kAny) {
+                const bool row_ok = it * kRowsPerIt + lr < rows_here;
                 if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
                 else if (row_ok) {
                     bf16x8 e8 = __builtin_bit_cast(bf16x8, res[it]);
@@ -613,7 +609,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                     res[it] = __builtin_bit_cast(u32x4, e8);
                 }
             } else {
-                if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4*>(src);
+                if (col_ok && it * kRowsPerIt + lr < rows_here) res[it] = *reinterpret_cast<const u32x4*>(src);
             }
         }
     };
@@ -740,7 +736,8 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
-                store_chunk(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
+                if constexpr (kAny) store_any(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
+                else if (col_ok && r + lr < rows_here) *reinterpret_cast<u32x4*>(Cl + (size_t)r * ldc) = v[t];
             }
         }
         return;
