@@ -395,7 +395,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         const char* b_src;  // B tile kt2: k-row 0 of it ([K, N] form) or n-row 0 (B^T form)
         unsigned sb_cur, sb_nxt, sb_fill;
     } ls;
-    const unsigned b_step32 = kBT ? (unsigned)(kBK * 2) : (unsigned)kBK * (unsigned)b_pitch * 2u;  // bytes from one B tile to the next (N < 2^25)
+    const unsigned b_step32 = kBT ? (unsigned)(kBK * 2) : (unsigned)kBK * (unsigned)b_pitch * 2u;  // bytes from one B tile to the next (b_pitch < 2^25)
     unsigned adv = 0;
     const size_t b_row2 = b_pitch * 4;                                  // [K, N] form: bytes from one 1 KB chunk (2 k-rows) to the next
     ls.kt2 = KT > 2 ? 2 : KT - 1;
@@ -537,7 +537,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                 asm volatile("" : "+s"(ls.a_src));
             }
             if (p == 3 && n == kSlots - 1) {
-                ls.b_src += adv * b_step32;  // (32-bit product: a tile-to-tile step stays below 4 GiB)
+                ls.b_src += adv * b_step32;  // (a tile-to-tile step stays below 4 GiB: b_pitch < 2^25)
                 asm volatile("" : "+s"(ls.b_src));
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1008,11 +1008,12 @@ size_t split_k_bytes(long M, long N, long K, long batch) {
     return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
 }
 
-// shapes the tiled kernels address (32-bit offsets inside a tile); without scratch the operands' rows have to be whole
+// shapes the tiled kernels address (32-bit offsets inside a tile, and from one tile of B to the next 64 rows on: the limits
+// hold for the row pitches, which round N and K up to 8); without scratch the operands' rows have to be whole
 // 16-byte chunks, see operand_padding
 bool tile_addressable(long M, long N, long K, long batch) {
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || batch > 65535) return false;
-    if (M > 0x7fffffffL || N > 0x7fffffffL || K > (1L << 23) || N >= (1L << 25)) return false;
+    if (M > 0x7fffffffL || K > (1L << 23) || N > (1L << 25) - 8) return false;
     const long tn = (N + mrk::dev::kBN - 1) / mrk::dev::kBN, tm128 = (M + 127) / 128;
     return tm128 * tn <= 0x7fffffffL;
 }

@@ -82,3 +82,17 @@ def test_workspace_queries_are_host_side_and_bounded():
                     assert ws % ((d + 2) * 4 * 16) == 0 and ws <= 16 << 20, (b, sq, d, sk, ws)
     gemm = lib.mrk_hip_gemm_bf16_workspace_bytes
     assert gemm(4096, 4096, 4096, 1) == 0 and gemm(128, 4096, 11008, 1) > 0 and gemm(0, 4096, 4096, 1) == 0
+
+
+def test_padded_products_end_where_a_step_between_tiles_fits_32_bits():
+    """A [K, N] operand whose rows are no whole 16-byte chunks is laid out with N rounded up to 8, and the tiled kernels step from one
+    64-row tile of it to the next in 32 bits: the last pitch they take is 2^25 - 8.  Past it the kernel that indexes
+    in 64 bits runs, which wants no scratch."""
+    from morok_amd._ffi import lib
+
+    gemm = lib.mrk_hip_gemm_bf16_workspace_bytes
+    for m in (1, 200):
+        assert gemm(m, (1 << 25) - 15, 200, 1) >= 2 * 200 * ((1 << 25) - 8)
+        assert gemm(m, (1 << 25) - 8, 201, 1) > 0
+        for n in range((1 << 25) - 7, 1 << 25):
+            assert gemm(m, n, 200, 1) == 0, n
