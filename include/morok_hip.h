@@ -469,11 +469,13 @@ int mrk_hip_gemm_bf16_variant(int device_id, const void* a, const void* b, void*
 
 /* mrk_hip_gemm_bf16 for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
- * reference.  Same kernels and the same bits as mrk_hip_gemm_bf16, but the split-K partials go
+ * reference.  The same bits as mrk_hip_gemm_bf16, but the split-K partials and the padded copies of
+ * operands whose rows are no whole 16-byte chunks (N or K no multiple of 8) go
  * to a fixed 32 MiB device array inside the library (resolved per device by
  * mrk_hip_device_create) instead of a block from the allocator, and the call performs no
- * allocation or free of any kind.  The device must have been created before
- * (INVALID_ARGUMENT otherwise: creating it allocates).  A shape whose partials would exceed
+ * allocation or free of any kind.  Where those copies and partials do not fit the array the product
+ * runs on the kernel that needs no scratch, which takes the same sums in the same order and is slower.  The device must have been created before
+ * (INVALID_ARGUMENT otherwise: creating it allocates).  A shape of whole chunks whose partials would exceed
  * mrk_hip_gemm_bf16_noalloc_capacity() bytes is refused with INVALID_ARGUMENT and nothing is
  * launched.  All calls on one device share the array: calls that may overlap on one device
  * (different streams or threads without ordering between them) race; calls queued on the

@@ -52,7 +52,6 @@ namespace mrk::dev {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -923,11 +922,13 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restric
 
 // Any shape: one wave per 32x32 output tile, operands fetched straight from global memory
 // with bounds checks (zero fill), no LDS.  Correct for every M, N, K; used when the shape
-// does not fit the tiled kernel.
+// does not fit the tiled kernel.  The same instructions on the same k in the same order as the tiled
+// kernels', and sums of `k_range` deep ranges of K added up in order as the split-K reduction adds its partial
+// results: the same bits, whether or not there is scratch for padded operands and partial results.
 template <bool kF16>
 __global__ __launch_bounds__(256) void gemm_bf16_generic(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                                          __bf16* __restrict__ C, int M, int N, int K, int tiles_n,
-                                                         long total_tiles) {
+                                                         long total_tiles, int k_range) {
     const int lane = threadIdx.x & 63;
     const long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (tile >= total_tiles) return;
@@ -935,31 +936,50 @@ __global__ __launch_bounds__(256) void gemm_bf16_generic(const __bf16* __restric
     B += (size_t)blockIdx.y * K * N;
     C += (size_t)blockIdx.y * M * N;
     const long m0 = (tile / tiles_n) * 32, n0 = (tile % tiles_n) * 32;
-    const long m = m0 + (lane & 31), n = n0 + (lane & 31);
-    const int kg = 8 * (lane >> 5);
-    f32x16 acc;
+    const int lr = lane & 15, kg = 8 * (lane >> 4);
+    f32x4 sum[2][2] = {};
+    for (long first = 0; first < K; first += k_range) {
+        const long end = first + k_range < K ? first + k_range : K;
+        f32x4 acc[2][2] = {};
+        for (long k0 = first; k0 < end; k0 += 32) {
+            bf16x8 a[2], b[2];
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        bf16x8 a, b;
+            for (int t = 0; t < 2; t++) {
+                const long m = m0 + t * 16 + lr, n = n0 + t * 16 + lr;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int k = k0 + kg + e;
-            a[e] = (m < M && k < K) ? A[m * K + k] : (__bf16)0.0f;
-            b[e] = (n < N && k < K) ? B[(long)k * N + n] : (__bf16)0.0f;
+                for (int e = 0; e < 8; e++) {
+                    const long k = k0 + kg + e;
+                    a[t][e] = (m < M && k < K) ? A[m * K + k] : (__bf16)0.0f;
+                    b[t][e] = (n < N && k < K) ? B[k * N + n] : (__bf16)0.0f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    if constexpr (kF16)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[i]), __builtin_bit_cast(f16x8, b[j]), acc[i][j], 0, 0, 0);
+                    else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+                }
         }
-        if constexpr (kF16) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
-        else acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    // lane l register e: row 8*(e/4) + 4*(l/32) + e%4, column l%32
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const long r = m0 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-        if (r < M && n < N) {
-            if constexpr (kF16) C[r * N + n] = __builtin_bit_cast(__bf16, (_Float16)acc[e]);
-            else C[r * N + n] = (__bf16)acc[e];
-        }
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) sum[i][j] += acc[i][j];
     }
+    // lane l register e of tile (i, j): row 4*(l/16) + e, column l%16
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const long r = m0 + i * 16 + 4 * (lane >> 4) + e, n = n0 + j * 16 + lr;
+                if (r < M && n < N) {
+                    if constexpr (kF16) C[r * N + n] = __builtin_bit_cast(__bf16, (_Float16)sum[i][j][e]);
+                    else C[r * N + n] = (__bf16)sum[i][j][e];
+                }
+            }
 }
 
 }  // namespace mrk::dev
@@ -1071,7 +1091,7 @@ size_t gemm_bf16_static_workspace_capacity() { return kStaticWsBytes; }
 
 size_t gemm_bf16_static_workspace_need(long M, long N, long K) {
     const size_t need = gemm_bf16_workspace_bytes(M, N, K, 1);
-    // padded operands that do not fit: the kernel that needs no scratch
+    // padded operands and partial results that do not fit: the kernel that needs no scratch and gives the same bits
     return need > kStaticWsBytes && (N % 8 || K % 8) ? 0 : need;
 }
 
@@ -1296,9 +1316,12 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
     const long total = tm * tn;
     const long blocks = (total + 3) / 4;
     if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
+    // (the K ranges the tiled kernels would take: the result does not depend on whether there was scratch for them)
+    const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
+    const int k_range = sp.splits > 1 ? (int)sp.kt_per_split * kBK : 0x7fffffff;
     auto generic = f16 ? gemm_bf16_generic<true> : gemm_bf16_generic<false>;
     generic<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
-                                                                   static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn, total);
+                                                                   static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn, total, k_range);
     return (int)hipGetLastError();
 }
 

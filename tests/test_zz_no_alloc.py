@@ -76,3 +76,16 @@ def test_noalloc_argument_errors(dev):
     with pytest.raises(MorokHipError):
         morok_amd._ffi.check(lib.mrk_hip_gemm_bf16_noalloc(0, None, a.ptr, a.ptr, 4, 4, 2))
     morok_amd._ffi.check(lib.mrk_hip_gemm_bf16_noalloc(0, None, None, None, 0, 4, 2))  # empty product: nothing to do
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1001, 320), (17, 999, 2050),            # padded operands and partial results fit the array
+                                   (4097, 4097, 2060), (40, 4095, 4100),        # padded operands larger than the array, one and several ranges of K
+                                   (100, 513, 20001)])                          # padded operands fit, with the partial results they do not
+def test_noalloc_matches_where_operand_rows_are_odd(dev, M, N, K):
+    got, want, (a, b) = _pair(dev, M, N, K, 97)
+    assert np.array_equal(got, want)
+    # against f32 sums of the same products on the host: 2^-9 for the rounding to bf16, K 2^-24 |a| |b| for either order of the sums
+    af, bf = synth.from_bf16(a[:8]), synth.from_bf16(b)
+    ref = af.astype(np.float64) @ bf
+    bound = 2.0 ** -8 * np.abs(ref) + 2 * K * 2.0 ** -24 * (np.abs(af).astype(np.float64) @ np.abs(bf)) + 1e-30
+    assert np.all(np.abs(synth.from_bf16(got).reshape(M, N)[:8] - ref) <= bound)
