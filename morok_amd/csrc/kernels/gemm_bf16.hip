@@ -854,24 +854,31 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_tile256_rope(const __bf16* _
 }
 
 // dst[rows][pitch] = src[rows][cols] with zeros from cols to pitch (a multiple of 8): an operand whose rows start on odd
-// elements, laid out for the 16-byte copies of the tiled kernels.  A wave walks one row in 16-byte pieces (the loads
-// aligned to 2 bytes only).  Bound by HBM: 2 (cols + pitch) bytes a row.
+// elements, laid out for the 16-byte copies of the tiled kernels.  A wave moves up to 128 consecutive 16-byte pieces of a row
+// (the loads aligned to 2 bytes only); grid y counts such runs of long rows, so that few long
+// rows fill the chip too.
+constexpr int kRepitchRun = 128;
 __global__ __launch_bounds__(256) void gemm_repitch(const unsigned short* __restrict__ src, unsigned short* __restrict__ dst, long rows,
                                                     int cols, int pitch) {
-    const int lane = threadIdx.x & 63;
+    const int first = (int)blockIdx.y * kRepitchRun + (int)(threadIdx.x & 63);
     for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < rows; row += (long)gridDim.x * 4) {
         const unsigned short* s = src + (size_t)row * cols;
         u32x4* d = reinterpret_cast<u32x4*>(dst + (size_t)row * pitch);
-        for (int p = lane; p < pitch / 8; p += 64) {
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (p * 8 + 8 <= cols) v = *reinterpret_cast<const u32x4_any*>(s + p * 8);
-            else {
+        u32x4 v[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int c = (first + 64 * i) * 8;
+            v[i] = u32x4{0u, 0u, 0u, 0u};
+            if (c + 8 <= cols) v[i] = *reinterpret_cast<const u32x4_any*>(s + c);
+            else if (c < cols) {
 #pragma unroll
                 for (int e = 0; e < 8; e++)
-                    if (p * 8 + e < cols) v[e >> 1] |= (unsigned)s[p * 8 + e] << (16 * (e & 1));
+                    if (c + e < cols) v[i][e >> 1] |= (unsigned)s[c + e] << (16 * (e & 1));
             }
-            d[p] = v;
         }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            if (first + 64 * i < pitch / 8) d[first + 64 * i] = v[i];
     }
 }
 // C[i] = bf16(W[0][i] + W[1][i] + ... + W[splits-1][i]), 8 elements per work-item, partials added
@@ -1222,7 +1229,8 @@ bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, 
     if (pad.a_bytes + pad.b_bytes > ws_left || !pad.lda) return false;
     auto padded = [&](const __bf16* src, long rows, long cols, long pitch, size_t bytes) {
         const long groups = (rows + 3) / 4;
-        gemm_repitch<<<(unsigned)(groups < (1L << 20) ? groups : (1L << 20)), 256, 0, s>>>(
+        const dim3 grid((unsigned)(groups < (1L << 20) ? groups : (1L << 20)), (unsigned)((pitch / 8 + kRepitchRun - 1) / kRepitchRun));
+        gemm_repitch<<<grid, 256, 0, s>>>(
             reinterpret_cast<const unsigned short*>(src), reinterpret_cast<unsigned short*>(ws), rows, (int)cols, (int)pitch);
         const __bf16* at = reinterpret_cast<const __bf16*>(ws);
         ws += bytes;
