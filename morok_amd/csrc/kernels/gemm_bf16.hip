@@ -932,10 +932,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restric
 // does not fit the tiled kernel.  The same instructions on the same k in the same order as the tiled
 // kernels', and sums of `k_range` deep ranges of K added up in order as the split-K reduction adds its partial
 // results: the same bits, whether or not there is scratch for padded operands and partial results.
-template <bool kF16>
+// kBT: B is stored [N, K].  add (may be null): a matrix of C's shape or (add_pitch 0) one row, added to the rounded sums.
+template <bool kF16, bool kBT>
 __global__ __launch_bounds__(256) void gemm_bf16_generic(const __bf16* __restrict__ A, const __bf16* __restrict__ B,
                                                          __bf16* __restrict__ C, int M, int N, int K, int tiles_n,
-                                                         long total_tiles, int k_range) {
+                                                         long total_tiles, int k_range, const __bf16* __restrict__ add, long add_pitch) {
     const int lane = threadIdx.x & 63;
     const long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (tile >= total_tiles) return;
@@ -957,7 +958,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_generic(const __bf16* __restric
                 for (int e = 0; e < 8; e++) {
                     const long k = k0 + kg + e;
                     a[t][e] = (m < M && k < K) ? A[m * K + k] : (__bf16)0.0f;
-                    b[t][e] = (n < N && k < K) ? B[k * N + n] : (__bf16)0.0f;
+                    b[t][e] = (n < N && k < K) ? B[kBT ? n * K + k : k * N + n] : (__bf16)0.0f;
                 }
             }
 #pragma unroll
@@ -975,18 +976,27 @@ __global__ __launch_bounds__(256) void gemm_bf16_generic(const __bf16* __restric
             for (int j = 0; j < 2; j++) sum[i][j] += acc[i][j];
     }
     // lane l register e of tile (i, j): row 4*(l/16) + e, column l%16
+    auto store = [&](auto with_add) {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const long r = m0 + i * 16 + 4 * (lane >> 4) + e, n = n0 + j * 16 + lr;
-                if (r < M && n < N) {
-                    if constexpr (kF16) C[r * N + n] = __builtin_bit_cast(__bf16, (_Float16)sum[i][j][e]);
-                    else C[r * N + n] = (__bf16)sum[i][j][e];
+                for (int e = 0; e < 4; e++) {
+                    const long r = m0 + i * 16 + 4 * (lane >> 4) + e, n = n0 + j * 16 + lr;
+                    if (r >= M || n >= N) continue;
+                    using T = std::conditional_t<kF16, _Float16, __bf16>;
+                    T h = (T)sum[i][j][e];
+                    if constexpr (decltype(with_add)::value) h = (T)((float)h + (float)__builtin_bit_cast(T, add[r * add_pitch + n]));
+                    C[r * N + n] = __builtin_bit_cast(__bf16, h);
                 }
-            }
+    };
+    if (add) {
+        add += (size_t)blockIdx.y * M * add_pitch;
+        store(std::true_type{});
+    } else {
+        store(std::false_type{});
+    }
 }
 
 }  // namespace mrk::dev
@@ -1056,9 +1066,9 @@ struct OperandPadding {
 };
 OperandPadding operand_padding(long M, long N, long K, long batch, bool b_transposed) {
     OperandPadding o;
-    // A small [K, N] product stays with the kernel that needs no padding: it is one launch of at most one wave per SIMD
-    // and a few steps of K there (6.4-6.9 us from 33 x 7 x 19 to 256 x 255 x 63), two or three launches here (12-13 us);
-    // at K = 515 it is 20 against 15.  There is no such kernel for a [N, K] operand.
+    // A small [K, N] product asks for no scratch: it is one launch of at most one wave per SIMD and a few steps of K on the
+    // kernel that needs no padding (6.4-6.9 us from 33 x 7 x 19 to 256 x 255 x 63), two or three launches here (12-13 us).
+    // Which of the others run there although there is scratch: unpadded_faster.
     if (!b_transposed && (K % 8 || N % 8) && K <= 128 && ((M + 31) / 32) * ((N + 31) / 32) * batch <= 1024) return o;
     const long row_b = b_transposed ? K : N, rows_b = batch * (b_transposed ? N : K);
     o.a = K % 8 != 0;
@@ -1068,6 +1078,21 @@ OperandPadding operand_padding(long M, long N, long K, long batch, bool b_transp
     if (o.a) o.a_bytes = ((size_t)batch * M * o.lda * 2 + 255) / 256 * 256;
     if (o.b) o.b_bytes = ((size_t)rows_b * o.ldb * 2 + 255) / 256 * 256;
     return o;
+}
+// Whether a product that would have operands padded runs faster on the kernel that reads them as they are (also where there is
+// scratch): short K, or few rows against a wide weight.  Both times in us, from 445 shapes of 1 to 4096 rows, 9 to 50257
+// columns and K from 65 to 1032: one wave per 32 x 32 tile, four per CU at once (`rounds`; rows that are not there are not
+// loaded; tall products read B again; lanes along K of an [N, K] operand share fewer lines) against the tiles with their one
+// or two padding launches, whose traffic the last-level cache takes a part of.  On either side of the line the chosen kernel
+// was at most 20 % behind the other: 32 x 33 x 392 12.1 / 13.3, 256 x 255 x 257 11.0 / 15.2, 256 x 255 x 392 19.6 / 15.0,
+// 4 x 50257 x 769 29.4 / 40.9, 64 x 50257 x 513 74 / 33; [N, K] 256 x 255 x 129 9.6 / 13.8, 300 x 300 x 300 23.0 / 14.9.
+bool unpadded_faster(long M, long N, long K, long batch, const OperandPadding& pad, bool b_transposed) {
+    if (!pad.a && !pad.b) return false;
+    const double rounds = (double)(((M + 31) / 32) * ((N + 31) / 32) * batch) / 1024.0;
+    const double wait = rounds <= 1.0 ? 1.0 : M <= 4 ? 0.5 + 0.5 * rounds : M <= 128 && batch == 1 ? rounds : rounds + 1.25;
+    const double unpadded = 2.0 + K * wait * (M <= 4 ? 0.029 : M <= 16 ? 0.033 : 0.040) * (b_transposed ? 1.4 : 1.0);
+    const double padded = 8.5 + 3.5 * (pad.a + pad.b) + 6.0 * (double)batch * ((pad.a ? (double)M * K : 0.0) + (pad.b ? (double)K * N : 0.0)) / 8.5e6;
+    return unpadded < padded;
 }
 }  // namespace
 
@@ -1273,6 +1298,25 @@ bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, 
 }
 }  // namespace
 
+namespace {
+// The kernel that reads its operands as they are, whatever their rows and bases are aligned to.
+int launch_unpadded(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, long batch, bool b_transposed, bool f16,
+                    const __bf16* add, bool add_is_row) {
+    using namespace mrk::dev;
+    const long tn = (N + 31) / 32, total = ((M + 31) / 32) * tn, blocks = (total + 3) / 4;
+    if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
+    // (the K ranges the tiled kernels would take: the result does not depend on whether there was scratch for them)
+    const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
+    const int k_range = sp.splits > 1 ? (int)sp.kt_per_split * kBK : 0x7fffffff;
+    auto kernel = f16 ? (b_transposed ? gemm_bf16_generic<true, true> : gemm_bf16_generic<true, false>)
+                      : (b_transposed ? gemm_bf16_generic<false, true> : gemm_bf16_generic<false, false>);
+    kernel<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
+                                                                  static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn, total, k_range, add,
+                                                                  add_is_row ? 0 : N);
+    return (int)hipGetLastError();
+}
+}  // namespace
+
 // The product, with `add` (a matrix of C's shape or, add_is_row, one row [N]; of C's type) added to the rounded result by
 // whichever kernel writes it: the streaming kernels, the split-K reduction or the tiled kernels' residual epilogue.
 int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
@@ -1286,8 +1330,12 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
     const bool aligned = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16) == 0;
+    OperandPadding pad;
+    if (K > 0) pad = operand_padding(M, N, K, batch, b_transposed);
+    const bool unpadded = (variant == 0 || variant == 5) && aligned && unpadded_faster(M, N, K, batch, pad, b_transposed);
     if (b_transposed) {
-        // B given as Bt[N, K]: the streaming or the tiled kernels, or nothing (variant 3 / 4 force a tile size)
+        // B given as Bt[N, K]: the streaming or the tiled kernels, the unpadded one for small odd shapes, or nothing
+        // (variant 3 / 4 force a tile size)
         if (!aligned || !gemm_bf16_nt_padded_supported(M, N, K, batch)) return (int)hipErrorInvalidValue;
         // up to 64 rows: one pass over the weight streams it faster than any tile (one or two rows on the
         // vector ALUs, more on the matrix pipes with 16-row blocks staged through LDS)
@@ -1299,10 +1347,11 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
                 if (gemm_nt_rows_supported(M, N, K, batch)) return launch_gemm_nt_rows(stream, A, B, C, M, N, K, batch, f16);
             }
         }
-        if (!tile_addressable(M, N, K, batch) ||
-            !launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, true, f16, addp, add_is_row))
+        if (!tile_addressable(M, N, K, batch)) return (int)hipErrorInvalidValue;
+        if (!unpadded && !launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, true, f16, addp, add_is_row))
             return (int)hipErrorInvalidValue;
-        return (int)hipGetLastError();
+        if (!unpadded) return (int)hipGetLastError();
+        return launch_unpadded(s, A, B, C, M, N, K, batch, true, f16, addp, add_is_row);
     }
     // up to 16 rows: one streaming pass over the weight into f32 partial sums, then their sum
     {
@@ -1316,21 +1365,12 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
             return launch_gemm_kn_rows(stream, A, B, C, workspace, M, N, K, ks, kr, f16, add, add_is_row);
         }
     }
-    if (variant != 2 && aligned && tile_addressable(M, N, K, batch) &&
+    if (variant != 2 && aligned && tile_addressable(M, N, K, batch) && !unpadded &&
         launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, false, f16, addp, add_is_row))
         return (int)hipGetLastError();
-    if (add) return (int)hipErrorInvalidValue;  // (the kernel below has no epilogue)
-    const long tm = (M + 31) / 32, tn = (N + 31) / 32;
-    const long total = tm * tn;
-    const long blocks = (total + 3) / 4;
-    if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
-    // (the K ranges the tiled kernels would take: the result does not depend on whether there was scratch for them)
-    const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
-    const int k_range = sp.splits > 1 ? (int)sp.kt_per_split * kBK : 0x7fffffff;
-    auto generic = f16 ? gemm_bf16_generic<true> : gemm_bf16_generic<false>;
-    generic<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
-                                                                   static_cast<__bf16*>(C), (int)M, (int)N, (int)K, (int)tn, total, k_range);
-    return (int)hipGetLastError();
+    // (an addend is taken where there is scratch for the tiles, whichever kernel runs)
+    if (add && !(unpadded && pad.lda)) return (int)hipErrorInvalidValue;
+    return launch_unpadded(s, A, B, C, M, N, K, batch, false, f16, addp, add_is_row);
 }
 
 int launch_gemm_bf16(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,

@@ -55,6 +55,35 @@ def test_any_shape_exact(dev, shape, nt, f16):
         assert np.all(got[M * N:] == 0x1234), kind
 
 
+# short and long K around the line between the kernel that reads odd rows as they are and the padded tiles, in the classes of
+# rows the line is drawn for; wide weights; K in several ranges
+@pytest.mark.parametrize("shape", [(3, 33, 393), (4, 50257, 200), (16, 4097, 421), (33, 7, 19), (256, 255, 129), (256, 255, 337), (256, 255, 345),
+                                   (100, 513, 1001), (40, 257, 5003), (1030, 1001, 96)])
+def test_the_bits_do_not_depend_on_the_kernel(dev, shape):
+    M, N, K = shape
+    a, b, row = synth.normal_bf16((M, K), 8, 0), synth.normal_bf16((K, N), 8, 1), synth.normal_bf16((N,), 8, 2)
+    bufs = {nt: (_guarded(dev, a), _guarded(dev, np.ascontiguousarray(b.T) if nt else b)) for nt in (False, True)}
+    scratch = dev.buffer((M + 8) * (K + 8) * 2 + max((K + 8) * (N + 15), (N + 8) * (K + 15)) * 2 + 256 * 128 * 256 * 4)
+
+    def run(kind, nt, *more):
+        bc = morok_amd.Buffer.from_numpy(np.full(M * N + GUARD, 0x1234, np.uint16), dev.device_id)
+        morok_amd.Program.builtin(kind, [M, N, K, 1, scratch.size], dev.device_id).execute([bc, *bufs[nt], *more, scratch])
+        got = bc.copyout(np.uint16)
+        assert np.all(got[M * N:] == 0x1234), kind
+        return got[:M * N]
+
+    got = run("gemm_bf16", False)
+    any_shape = dev.buffer(M * N * 2)
+    morok_amd.ops.gemm_bf16(*bufs[False], any_shape, M, N, K, dev.device_id, variant=2)
+    assert np.array_equal(got, any_shape.copyout(np.uint16, nbytes=M * N * 2))
+    if M > 64 or K % 8:  # (up to 64 rows of whole chunks are streamed: another order)
+        assert np.array_equal(run("gemm_bf16_nt", True), got)
+        want = synth.to_bf16(synth.from_bf16(got).reshape(M, N) + synth.from_bf16(row)).reshape(-1)
+        assert np.array_equal(run("gemm_bf16_nt_bias", True, _guarded(dev, row)), want)
+        if K > 128:
+            assert np.array_equal(run("gemm_bf16_bias", False, _guarded(dev, row)), want)
+
+
 @pytest.mark.parametrize("f16", [False, True])
 def test_odd_linear_through_the_tensor_api(dev, f16):
     """A projection onto an odd number of outputs, weight [out, in]: one program, no transposed copy; with a bias as well."""
