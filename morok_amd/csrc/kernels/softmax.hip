@@ -185,7 +185,7 @@ __global__ __launch_bounds__(1024) void softmax_rows_streaming(const float* __re
 // bf16 / f16 rows of up to 65536 columns: read once into registers as f32, reduced like the f32 rows, rounded once on the
 // way out.  A row may start on any element: it is moved in 16-byte pieces of 2-byte alignment, the last cols % 8
 // elements one by one.  Bound by HBM at 4 bytes an element (the composed graph takes three kernels and reads the
-// matrix three times); small matrices are one launch instead of three.  Measured, bf16: 2859 x 712 10.1 -> 4.2 us,
+// matrix three times); small matrices are one launch instead of three.  Rows above 128 columns; measured, bf16: 2859 x 712 10.1 -> 4.2 us,
 // 8192 x 8190 126 -> 43.9 (6.1 TB/s), 600 x 30000 120 -> 19.0, 1024 x 65536 104 -> 66.4 (64 registers of row a work-item).
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
@@ -268,6 +268,57 @@ __global__ __launch_bounds__(kThreads* kRowsPerBlock) void softmax_half_rows_in_
     if (active && t < tail) yr[8 * nvec + t] = (unsigned short)to_half_bits<kF16>(last * inv);
 }
 
+// Rows of up to 128 columns: kLanes lanes share a row, eight consecutive elements each, so that a wave holds 64 / kLanes rows
+// (a wave to itself would leave a row of 16 with two busy lanes: 2^20 x 16 took 313 us that way, three generated kernels 28).
+// One lane's piece may be partial and is moved element by element.  Measured, bf16, against the three generated kernels: 2^20 x 2
+// 14.4 -> 6.1 us, 2^20 x 16 28.1 -> 11.9 (5.6 TB/s), 2^18 x 65 54.5 -> 22.0, 2^17 x 127 75.4 -> 19.5.
+template <int kLanes, bool kF16>
+__global__ __launch_bounds__(256) void softmax_half_short_rows(const unsigned short* __restrict__ x, unsigned short* __restrict__ y, long rows,
+                                                               int cols) {
+    const int t = threadIdx.x % kLanes;
+    const long row = (long)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
+    const int n = row >= rows ? 0 : cols - 8 * t;  // elements from this lane's first on
+    const unsigned short* xr = x + row * cols + 8 * t;
+    unsigned short* yr = y + row * cols + 8 * t;
+    float v[8];
+    if (n >= 8) {
+        const u32x4 w = *reinterpret_cast<const u32x4_any*>(xr);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = from_half_bits<kF16>(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = e < n ? from_half_bits<kF16>(xr[e]) : -INFINITY;
+    }
+    float m = v[0];
+#pragma unroll
+    for (int e = 1; e < 8; e++) m = fmaxf(m, v[e]);
+    m = lanes_reduce<MaxOp, kLanes>(m);
+    float s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        v[e] = expf(v[e] - m);  // (elements past the row hold -inf and contribute nothing)
+        s += v[e];
+    }
+    const float inv = 1.0f / lanes_reduce<SumOp, kLanes>(s);
+    if (n >= 8) {
+        u32x4 w;
+#pragma unroll
+        for (int q = 0; q < 4; q++) w[q] = to_half_bits<kF16>(v[2 * q] * inv) | to_half_bits<kF16>(v[2 * q + 1] * inv) << 16;
+        *reinterpret_cast<u32x4_any*>(yr) = w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+            if (e < n) yr[e] = (unsigned short)to_half_bits<kF16>(v[e] * inv);
+    }
+}
+
+template <int kLanes>
+static void launch_half_short(hipStream_t s, const unsigned short* x, unsigned short* y, long rows, int cols, bool f16) {
+    const unsigned grid = (unsigned)((rows + 256 / kLanes - 1) / (256 / kLanes));
+    if (f16) softmax_half_short_rows<kLanes, true><<<grid, 256, 0, s>>>(x, y, rows, cols);
+    else softmax_half_short_rows<kLanes, false><<<grid, 256, 0, s>>>(x, y, rows, cols);
+}
+
 template <int kThreads, int kVec, int kRowsPerBlock>
 static void launch_half_regs(hipStream_t s, const unsigned short* x, unsigned short* y, long rows, int cols, bool f16) {
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
@@ -330,8 +381,14 @@ int launch_softmax_half(void* stream, const void* x, void* y, long rows, long co
     const auto* xi = static_cast<const unsigned short*>(x);
     auto* yo = static_cast<unsigned short*>(y);
     const int c = (int)cols;
-    // as for f32: one wave (four rows a workgroup) for short rows, 256 to 1024 work-items per row for long ones
-    if (c <= 512 * 1) launch_half_regs<64, 1, 4>(s, xi, yo, rows, c, f16);
+    // up to 128 columns several rows a wave; then as for f32: one wave (four rows a workgroup) for short rows, 256 to 1024
+    // work-items per row for long ones
+    if (c <= 8) launch_half_short<1>(s, xi, yo, rows, c, f16);
+    else if (c <= 16) launch_half_short<2>(s, xi, yo, rows, c, f16);
+    else if (c <= 32) launch_half_short<4>(s, xi, yo, rows, c, f16);
+    else if (c <= 64) launch_half_short<8>(s, xi, yo, rows, c, f16);
+    else if (c <= 128) launch_half_short<16>(s, xi, yo, rows, c, f16);
+    else if (c <= 512 * 1) launch_half_regs<64, 1, 4>(s, xi, yo, rows, c, f16);
     else if (c <= 512 * 2) launch_half_regs<64, 2, 4>(s, xi, yo, rows, c, f16);
     else if (c <= 2048 * 1) launch_half_regs<256, 1, 1>(s, xi, yo, rows, c, f16);
     else if (c <= 2048 * 2) launch_half_regs<256, 2, 1>(s, xi, yo, rows, c, f16);

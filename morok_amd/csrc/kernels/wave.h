@@ -34,4 +34,15 @@ __device__ __forceinline__ float wave_reduce(float v) {
     return Op::apply(lo, hi);
 }
 
+// The same over groups of kLanes (1, 2, 4, 8 or 16) consecutive lanes.
+template <class Op, int kLanes>
+__device__ __forceinline__ float lanes_reduce(float v) {
+    static_assert(kLanes == 1 || kLanes == 2 || kLanes == 4 || kLanes == 8 || kLanes == 16, "groups inside a row of 16 lanes");
+    if constexpr (kLanes >= 2) v = Op::apply(v, dpp_move<0xB1>(v));
+    if constexpr (kLanes >= 4) v = Op::apply(v, dpp_move<0x4E>(v));
+    if constexpr (kLanes >= 8) v = Op::apply(v, dpp_move<0x141>(v));
+    if constexpr (kLanes >= 16) v = Op::apply(v, dpp_move<0x140>(v));
+    return v;
+}
+
 }  // namespace mrk::dev

@@ -45,3 +45,27 @@ def test_softmax_half_infinities_and_nan():
     got = synth.from_bf16(T.Tensor.from_numpy(synth.to_bf16(x), uop.BF16).softmax(-1).to_numpy())
     assert np.all(got[0, 5:] == 0) and np.allclose(got[0, :5], 0.2, atol=1e-3)
     assert np.all(np.isnan(got[1])) and np.all(np.isnan(got[2])) and np.allclose(got[3], 1 / 300, rtol=4e-3)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("cols", [1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 121, 127, 128, 129])
+def test_softmax_half_short_rows(dev, cols, f16):
+    """Several rows to a wave: rows that fill a workgroup and rows beyond, NaNs right behind the input and a pattern behind the
+    result, which has to stay."""
+    import morok_amd
+
+    rows = 1031
+    x = _half(synth.normal((rows, cols), cols, 7, sigma=3.0), f16)
+    guard = np.full(64, 0x7FFF, np.uint16)
+    bx = morok_amd.Buffer.from_numpy(np.concatenate([x.view(np.uint16).reshape(-1), guard]), dev.device_id)
+    by = morok_amd.Buffer.from_numpy(np.full(rows * cols + 64, 0x1234, np.uint16), dev.device_id)
+    morok_amd.Program.builtin("softmax_f16" if f16 else "softmax_bf16", [rows, cols], dev.device_id).execute([by, bx])
+    out = by.copyout(np.uint16)
+    assert np.all(out[rows * cols:] == 0x1234)
+    got = out[:rows * cols].reshape(rows, cols)
+    got = _wide(got.view(np.float16) if f16 else got, f16)
+    w = _wide(x, f16)
+    e = np.exp(w - w.max(1, keepdims=True))
+    ref = e / e.sum(1, keepdims=True)
+    u = 2.0 ** -11 if f16 else 2.0 ** -8  # (the bound of test_softmax_half)
+    assert np.all(np.abs(got - ref) <= ref * u * 1.01 + (2.0 ** -25 if f16 else 1e-38))
