@@ -1,4 +1,4 @@
-// f32 products on the matrix pipes: C[M, N] = A[M, K] B (+ a row or a matrix), every operand and every sum in f32
+// f32 products on the matrix pipes: C[M, N] = A[M, K] B (+ a row or a matrix), every operand in f32
 // (v_mfma_f32_32x32x2_f32: 64 flops per cycle and SIMD, twice the vector ALUs' rate without packed arithmetic).  B is
 // [K, N], or (kNT) [N, K] as a Linear layer stores its weight.  Any M, N, K.
 //
@@ -11,13 +11,23 @@
 //    such groups halve every K step and add their sums at the end: two waves per SIMD, so that one's reads of the
 //    local memory run under the other's matrix instructions, and two shorter chains of additions.  Global ->
 //    registers -> local memory, one step ahead, two stages, one barrier per step.
-//  - f32_direct: few output tiles.  A workgroup owns one 32 x 32 tile and its 4 (16) waves split K; a wave's operands
+//  - f32_direct: few output tiles.  A workgroup owns one 16 x 16 (32 x 32) tile and its 4 (16) waves split K; a wave's operands
 //    go from memory straight to registers, a batch of loads ahead of the matrix instructions, and the waves' sums
-//    meet in local memory, added in the waves' order.  No barrier until then: a small product is one trip to memory.
-// Both add in an order that depends on the shape alone.  Error against 64 bits (2-norm, uniform operands, K = 1024): tiled
-// 4.0e-7, direct 1.6e-7; one chain of K fused multiply-adds, as the generated kernel has, 5.8e-7.
-// Bound by the f32 matrix rate (157 TFLOP/s nominal).  Measured: 1024^3 25.9 us (83 TFLOP/s; generated kernel on the vector
-// ALUs 55.3), 4096^3 1.20 ms (114 TFLOP/s), 64 x 256 x 784 against a [N, K] weight 4.3 us (36.8 and a transposing copy before).
+//    meet in local memory.  No barrier until then: a small product is one trip to memory.
+//
+// The order of the additions depends on the shape, the layout of B and whether rows are whole aligned 16-byte chunks, and
+// on nothing else.  How far a sum is off grows with the root of the longest chain of additions.  The kernels these
+// took over from added 64 partial sums of K / 64 products for ragged sizes, and one chain of K for sizes of whole 64 x 64
+// tiles; neither loses precision here.  f32_direct chains 8 products, adds those sums up per wave, and the waves' in
+// 64 bits.  f32_tiled leaves whole tiles (and K < 128, where ragged sizes were one chain too) with a chain of K / 2 per
+// group; for ragged sizes a chain ends after 16 products (8 up to K of 192) and goes on in 64 bits, in registers: the vector
+// instructions for that do not run under f32 matrix instructions and cost 10 to 18 %.  (f32 totals cost as much:
+// short of the old error they need two levels of them.)  Error against 64 bits, 2-norm, uniform operands, in 1e-7, before and
+// now: 1000 x 1000 x K 0.77 / 0.59 at K = 130, 0.82 / 0.78 at 257, 1.04 / 0.78 at 1000, 1.62 / 0.78 at 4000; 130 x 200 x K
+// 0.77 / 0.74, 0.82 / 0.71, 1.04 / 0.77, 1.60 / 1.00; 1024 x 1024 x K 2.05 / 1.48, 2.88 / 2.06, 5.67 / 4.02, 11.3 / 8.0.
+// Bound by the f32 matrix rate (157 TFLOP/s nominal).  Measured: 1024^3 24.7 us (87 TFLOP/s; generated kernel on the vector
+// ALUs 55.3), [N, K] weight 22.3; 4096^3 1.11 ms (124 TFLOP/s); 1000^3 29.1 us (reduction 3500); 64 x 256 x 784 against
+// a [N, K] weight 4.3 us (36.8 and a transposing copy before).
 // What is left at 1024^3, one workgroup per CU: the fill and drain of sixteen steps, and the barrier in each.
 #include <hip/hip_runtime.h>
 
@@ -33,21 +43,18 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
-// Four elements of one row: p points at the row, k .. k + 3 of `n` elements; past the end zeros (kZero), or whatever
-// the last elements hold (columns that are not stored).  kVec: rows are whole 16-byte chunks, so a group is
-// inside or outside as a whole.
-template <bool kVec, bool kZero>
+// Four elements k .. k + 3 of a row of n elements at p, zeros past the end.  kVec: rows are whole 16-byte chunks, so a
+// group is inside or outside as a whole.
+template <bool kVec>
 __device__ __forceinline__ f32x4v load4(const float* p, long k, long n) {
     f32x4v v = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (kVec) {
         if (k < n) v = *reinterpret_cast<const f32x4v*>(p + k);
-        else if (!kZero) v = *reinterpret_cast<const f32x4v*>(p + n - 4);
     } else {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const long c = k + i < n ? k + i : n - 1;
-            const float x = p[c];
-            v[i] = kZero && k + i >= n ? 0.0f : x;
+            const float x = p[k + i < n ? k + i : n - 1];
+            v[i] = k + i >= n ? 0.0f : x;
         }
     }
     return v;
@@ -68,18 +75,23 @@ __device__ __forceinline__ int c_row(int e, int lane) { return 8 * (e >> 2) + 4 
 
 }  // namespace
 
-template <int kT, bool kNT, bool kVec, int kAdd>
+// kRun: products one accumulator chains before its sum goes on into 64 bits, 8 or 16; 0: all of a wave's share of K.
+template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
 __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                                                const float* __restrict__ add, long M, long N, long K, int tiles_m, int tiles_n) {
     constexpr int kBM = 64 * kT, kBN = 64 * kT;
-    constexpr int kBK = kT == 1 ? 64 : 32;   // K step of the workgroup; each group of four waves takes half of it
-    constexpr int kChunks = kBK / 16;        // 8-deep chunks per step and group
-    constexpr int kSlots = kBK / 4;          // 16-byte slots of a row of either tile in local memory, k contiguous
+    // Groups of four waves that share the tile and split every K step, and a wave's 32 x 32 blocks of C.  (The 128 tile with
+    // 64-bit totals is shared out over all eight waves instead: 128 x 128 totals twice do not fit the registers.)
+    constexpr int kGroups = kT == 2 && kRun ? 1 : 2, kMi = kT, kNj = kT == 2 && kRun ? 1 : kT;
+    constexpr int kBK = kT == 1 ? 64 : 32;        // K step of the workgroup
+    constexpr int kChunks = kBK / (8 * kGroups);  // 8-deep chunks per step and wave
+    constexpr int kSlots = kBK / 4;           // 16-byte slots of a row of either tile in local memory, k contiguous
     constexpr int kAF = kBM * kBK, kBF = kBN * kBK;
     constexpr int kStage = kAF + kBF;
     __shared__ __attribute__((aligned(16))) float smem[2 * kStage];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int group = kGroups == 2 ? wave >> 2 : 0;
+    const int wm = kGroups == 2 ? (wave >> 1) & 1 : wave >> 2, wn = kGroups == 2 ? wave & 1 : wave & 3;
     const int lr = lane & 31, lg = lane >> 5;
     // Workgroups congruent mod 8 share an L2: each such set takes a run of consecutive tiles, walked in bands of four
     // rows of tiles, so that it reads a few rows of A and of B many times instead of all of both.
@@ -104,104 +116,126 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     // four rows by four columns, which goes to local memory transposed, so that both fragments are read alike
     const bool moves_a = wave >= 4;
     const int tq = tid & 255;
-    // Group i of a step that starts at k0 lies at pr[i] + min(at + kr[i] * pitch, last * pitch) with at = k0 * pitch: the address
-    // of a group past the end of K is pulled back inside, and what it brought is cleared on the way to local memory.  No branch
+    // Addresses are a wave's own 64-bit base, advanced with the step, and 32-bit byte offsets from it (the launcher keeps the
+    // larger extents out).  Offset of group i: fixed[i] + k * pitch with k counted from the base's; k past the end of K is
+    // pulled back inside, and what it brought is cleared on the way to local memory.  No branch
     // around the loads: the compiler can only count how many are in flight in straight code.
     const bool transpose = !kNT && !moves_a;
-    const float* pr[4];
-    int kr[4], to[4];
-    const long bn = n0 + 4 * (tq % (kBN / 4));
-    const long pitch = transpose ? N : 1, last = (transpose || !kVec ? K - 1 : K - 4) * pitch;
-    const long step_pitch = kBK * pitch;
-    long at = 0, ofs[4];
+    const long first = moves_a ? m0 : n0, end = moves_a ? M : N;
+    const char* base = reinterpret_cast<const char*>(transpose ? B + n0 : (moves_a ? A : B) + first * K);
+    const unsigned pitch = transpose ? (unsigned)N * 4u : 4u;
+    unsigned fixed[4];
+    int kr, to[4];  // a group's first k in the step (transpose: + i)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         if (!transpose) {
-            const float* base = moves_a ? A : B;
-            const long first = moves_a ? m0 : n0, end = moves_a ? M : N;
             const int r = tq / kSlots + i * (256 / kSlots);
-            pr[i] = base + (first + r < end ? first + r : end - 1) * K;
-            kr[i] = 4 * (tq % kSlots);
-            ofs[i] = kr[i];
+            fixed[i] = (unsigned)(first + r < end ? r : end - 1 - first) * (unsigned)K * 4u;
+            kr = 4 * (tq % kSlots);
             to[i] = (moves_a ? 0 : kAF) + r * kBK + (((tq % kSlots) ^ swizzle(r)) << 2);
         } else {
-            const int r = 4 * (tq % (kBN / 4)) + i, k = 4 * (tq / (kBN / 4));
-            pr[i] = B + (bn + 4 <= N || !kVec ? bn : N - 4);
-            kr[i] = k + i;
-            ofs[i] = kr[i] * N;
-            to[i] = kAF + r * kBK + (((k >> 2) ^ swizzle(r)) << 2);
+            // (i: column, for element-wise loads)
+            const int r = 4 * (tq % (kBN / 4)), past = (int)(N - 1 - n0);
+            if (kVec) fixed[i] = 4u * (unsigned)(r + 3 <= past ? r : past - 3);
+            else fixed[i] = 4u * (unsigned)(r + i <= past ? r + i : past);
+            kr = 4 * (tq / (kBN / 4));
+            to[i] = kAF + (r + i) * kBK + (((kr >> 2) ^ swizzle(r + i)) << 2);
         }
     }
+    int k_next = 0;  // first k of the step to be fetched
     auto fetch = [&](f32x4v(&v)[4]) {
+        // (the base stays inside K: the steps fetched past the end read the last one again)
+        const int kb = k_next <= (int)K - kBK ? k_next : (int)K > kBK ? (int)K - kBK : 0;
+        const char* at = base + (long)kb * pitch;
+        const int k = kr + (k_next - kb), last = (int)K - 1 - kb;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const long o = at + ofs[i];
             if constexpr (kVec) {
-                v[i] = *reinterpret_cast<const f32x4v*>(pr[i] + (o < last ? o : last));
+                const int ki = transpose ? (k + i < last ? k + i : last) : (k < last - 3 ? k : last - 3);
+                v[i] = *reinterpret_cast<const f32x4v*>(at + (fixed[i] + (unsigned)ki * pitch));
             } else {
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
-                    const long c = bn + x < N ? x : N - 1 - bn, ox = transpose ? o : o + x;
-                    v[i][x] = pr[i][(ox < last ? ox : last) + (transpose ? c : 0)];
+                    const int kx = k + (transpose ? i : x);
+                    v[i][x] = *reinterpret_cast<const float*>(at + (fixed[transpose ? x : i] + (unsigned)(kx < last ? kx : last) * pitch));
                 }
             }
         }
-        at += step_pitch;
+        k_next += kBK;
         __builtin_amdgcn_sched_barrier(0);  // the loads set out before the step's matrix instructions, not after them
     };
-    auto stash = [&](float* st, long k0, const f32x4v(&v)[4]) {
+    auto stash = [&](float* st, int k0, const f32x4v(&v)[4]) {
+        const int left = (int)K - k0 - kr;
         f32x4v z[4];
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int x = 0; x < 4; x++) z[i][x] = k0 + kr[i] + (transpose || kVec ? 0 : x) < K ? v[i][x] : 0.0f;
+            for (int x = 0; x < 4; x++) z[i][x] = (transpose ? i : kVec ? 0 : x) < left ? v[i][x] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++)
             *reinterpret_cast<f32x4v*>(st + to[i]) = transpose ? f32x4v{z[0][i], z[1][i], z[2][i], z[3][i]} : z[i];
     };
 
-    f32x16 acc[kT][kT];
+    f32x16 acc[kMi][kNj];
+    using Total = std::conditional_t<kRun == 0, float, double>;
+    Total total[kRun ? kMi : 1][kRun ? kNj : 1][16];
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int i = 0; i < kT; i++)
+        for (int i = 0; i < kMi; i++)
 #pragma unroll
-        for (int j = 0; j < kT; j++)
+            for (int j = 0; j < kNj; j++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+                for (int e = 0; e < 16; e++) f(i, j, e);
+    };
+    each([&](int i, int j, int e) {
+        acc[i][j][e] = 0.0f;
+        if constexpr (kRun != 0) total[i][j][e] = 0.0;
+    });
 
-    const long steps = (K + kBK - 1) / kBK;
+    const int steps = (int)((K + kBK - 1) / kBK);
     // Step s multiplies stage s & 1 while step s + 1's operands are on their way to registers since step s - 1 (an L2 miss
     // takes longer than a step) and step s + 2's set out.
     f32x4v in0[4], in1[4];
-    auto step = [&](long s, f32x4v(&arriving)[4], f32x4v(&leaving)[4]) {
+    auto step = [&](int s, f32x4v(&arriving)[4], f32x4v(&leaving)[4]) {
         const float* st = smem + (s & 1) * kStage;
         fetch(leaving);
-        const int slot = group * (kSlots / 2) + lg;
-        f32x4v fa[2][kT], fb[2][kT];
+        const int slot = group * (kSlots / kGroups) + lg;
+        f32x4v fa[2][kMi], fb[2][kNj];
         auto fragments = [&](int c) {
 #pragma unroll
-            for (int i = 0; i < kT; i++) {
-                const int ra = (wm * kT + i) * 32 + lr, rb = (wn * kT + i) * 32 + lr;
+            for (int i = 0; i < kMi; i++) {
+                const int ra = (wm * kMi + i) * 32 + lr;
                 fa[c & 1][i] = *reinterpret_cast<const f32x4v*>(st + ra * kBK + (((slot + 2 * c) ^ swizzle(ra)) << 2));
-                fb[c & 1][i] = *reinterpret_cast<const f32x4v*>(st + kAF + rb * kBK + (((slot + 2 * c) ^ swizzle(rb)) << 2));
+            }
+#pragma unroll
+            for (int j = 0; j < kNj; j++) {
+                const int rb = (wn * kNj + j) * 32 + lr;
+                fb[c & 1][j] = *reinterpret_cast<const f32x4v*>(st + kAF + rb * kBK + (((slot + 2 * c) ^ swizzle(rb)) << 2));
             }
         };
         fragments(0);
 #pragma unroll
         for (int c = 0; c < kChunks; c++) {
             if (c + 1 < kChunks) fragments(c + 1);
+            const bool opens = kRun == 8 || (kRun == 16 && c % 2 == 0), closes = kRun == 8 || (kRun == 16 && c % 2 == 1);
 #pragma unroll
             for (int x = 0; x < 4; x++)
 #pragma unroll
-                for (int i = 0; i < kT; i++)
+                for (int i = 0; i < kMi; i++)
 #pragma unroll
-                    for (int j = 0; j < kT; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[c & 1][i][x], fb[c & 1][j][x], acc[i][j], 0, 0, 0);
-            // (a chunk's fragments are read under the matrix instructions of the chunk before)
-            if (c + 1 < kChunks) {
-                if (c == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
+                    for (int j = 0; j < kNj; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[c & 1][i][x], fb[c & 1][j][x], opens && x == 0 ? f32x16{} : acc[i][j], 0, 0, 0);
+            if constexpr (kRun == 0) {
+                // (a chunk's fragments are read under the matrix instructions of the chunk before)
+                if (c + 1 < kChunks) {
+                    if (c == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x8, 4 * kT * kT, 0);
+            } else if (closes) {
+                each([&](int i, int j, int e) { total[i][j][e] += (double)acc[i][j][e]; });
+                __builtin_amdgcn_sched_barrier(0);  // (one set of accumulators at a time: there are no registers for two)
             }
-            __builtin_amdgcn_sched_group_barrier(0x8, 4 * kT * kT, 0);
         }
         // (the other stage was last read in step s - 1, which every wave has left at the barrier before this step)
         stash(smem + ((s + 1) & 1) * kStage, (s + 1) * kBK, arriving);
@@ -211,39 +245,35 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     fetch(in1);
     stash(smem, 0, in0);
     __syncthreads();
-    for (long s = 0; s + 1 < steps; s += 2) {
+    for (int s = 0; s + 1 < steps; s += 2) {
         step(s, in1, in0);
         step(s + 1, in0, in1);
     }
     if (steps & 1) step(steps - 1, in1, in0);
-    // the second group hands its sums over through local memory (all reads of the stages are behind the last barrier)
-    static_assert(4 * kT * kT * 16 * 64 <= 2 * kStage, "the second group's sums fit into the stages");
-    float* x = smem + (wave & 3) * (kT * kT * 16 * 64) + lane;
-    if (group == 1) {
-#pragma unroll
-        for (int i = 0; i < kT; i++)
-#pragma unroll
-            for (int j = 0; j < kT; j++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) x[((i * kT + j) * 16 + e) * 64] = acc[i][j][e];
-    }
-    __syncthreads();
-    if (group == 0) {
-#pragma unroll
-        for (int i = 0; i < kT; i++)
-#pragma unroll
-            for (int j = 0; j < kT; j++)
-#pragma unroll
-                for (int e = 0; e < 16; e++)
-                    store_c<kAdd>(C, add, M, N, m0 + (wm * kT + i) * 32 + c_row(e, lane), n0 + (wn * kT + j) * 32 + lr,
-                                  acc[i][j][e] + x[((i * kT + j) * 16 + e) * 64]);
+    auto sum = [&](int i, int j, int e) -> Total {
+        if constexpr (kRun == 0) return acc[i][j][e];
+        else return total[i][j][e];
+    };
+    auto store = [&](int i, int j, int e, Total other) {
+        store_c<kAdd>(C, add, M, N, m0 + (wm * kMi + i) * 32 + c_row(e, lane), n0 + (wn * kNj + j) * 32 + lr, (float)(sum(i, j, e) + other));
+    };
+    if constexpr (kGroups == 2) {
+        // the second group hands its sums over through local memory (all reads of the stages are behind the last barrier)
+        constexpr int kWave = kMi * kNj * 16 * 64;
+        static_assert(4 * kWave * sizeof(Total) <= sizeof smem, "the second group's sums fit into the stages");
+        Total* x = reinterpret_cast<Total*>(smem) + (wave & 3) * kWave + lane;
+        if (group == 1) each([&](int i, int j, int e) { x[((i * kNj + j) * 16 + e) * 64] = sum(i, j, e); });
+        __syncthreads();
+        if (group == 0) each([&](int i, int j, int e) { store(i, j, e, x[((i * kNj + j) * 16 + e) * 64]); });
+    } else {
+        each([&](int i, int j, int e) { store(i, j, e, 0); });
     }
 }
 
-template <int kT, bool kNT, bool kVec, int kAdd>
+template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
 __global__ void __launch_bounds__(512, kT == 1 && kVec ? 4 : 2) f32_tiled(const float* A, const float* B, float* C, const float* add, long M, long N, long K, int tiles_m,
                                                  int tiles_n) {
-    f32_tiled_body<kT, kNT, kVec, kAdd>(A, B, C, add, M, N, K, tiles_m, tiles_n);
+    f32_tiled_body<kT, kNT, kVec, kAdd, kRun>(A, B, C, add, M, N, K, tiles_m, tiles_n);
 }
 
 // kWaves waves split K into runs of whole chunks (of eight for tiles of 32, of sixteen for tiles of 16, whose lane groups
@@ -253,6 +283,7 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
                                                           const float* __restrict__ add, long M, long N, long K, int tiles_n) {
     constexpr int kBatch = 4;  // chunks whose loads are in flight together
     constexpr int kDeep = 4 * (64 / kTile), kOut = kTile * kTile;
+    constexpr int kRun = kTile == 32 ? 4 : 2;  // matrix instructions in a row on one accumulator: 8 products
     using Acc = std::conditional_t<kTile == 32, f32x16, f32x4v>;
     __shared__ float sums[kWaves * kOut];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -264,18 +295,18 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
     const float* pb = kNT ? B + col * K : B + col;
     const long chunks = (K + kDeep - 1) / kDeep, per = (chunks + kWaves - 1) / kWaves;
     const long c0 = wave * per, c1 = c0 + per < chunks ? c0 + per : chunks;
-    Acc acc;
+    float total[kOut / 64];
 #pragma unroll
-    for (int e = 0; e < kOut / 64; e++) acc[e] = 0.0f;
+    for (int e = 0; e < kOut / 64; e++) total[e] = 0.0f;
     f32x4v fa[2][kBatch], fb[2][kBatch];
     auto fetch = [&](long c, f32x4v(&a)[kBatch], f32x4v(&b)[kBatch]) {
 #pragma unroll
         for (int i = 0; i < kBatch; i++) {
             // chunks past this wave's run multiply zeros
             const long k = c + i < c1 ? (c + i) * kDeep + 4 * lg : K;
-            a[i] = load4<kVec, true>(pa, k, K);
+            a[i] = load4<kVec>(pa, k, K);
             if constexpr (kNT) {
-                b[i] = load4<kVec, true>(pb, k, K);
+                b[i] = load4<kVec>(pb, k, K);
             } else {
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
@@ -287,12 +318,18 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
     };
     auto multiply = [&](f32x4v(&a)[kBatch], f32x4v(&b)[kBatch]) {
 #pragma unroll
-        for (int i = 0; i < kBatch; i++)
+        for (int i = 0; i < kBatch; i++) {
+            Acc run[4 / kRun];
 #pragma unroll
             for (int x = 0; x < 4; x++) {
+                Acc& acc = run[x / kRun];
+                if (x % kRun == 0) acc = Acc{};
                 if constexpr (kTile == 32) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][x], b[i][x], acc, 0, 0, 0);
                 else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][x], b[i][x], acc, 0, 0, 0);
             }
+#pragma unroll
+            for (int e = 0; e < kOut / 64; e++) total[e] += kRun == 4 ? run[0][e] : run[0][e] + run[4 / kRun - 1][e];
+        }
     };
     if (c0 < c1) {
         fetch(c0, fa[0], fb[0]);
@@ -306,15 +343,15 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
         }
     }
 #pragma unroll
-    for (int e = 0; e < kOut / 64; e++) sums[wave * kOut + e * 64 + lane] = acc[e];
+    for (int e = 0; e < kOut / 64; e++) sums[wave * kOut + e * 64 + lane] = total[e];
     __syncthreads();
 #pragma unroll
     for (int q = tid; q < kOut; q += kWaves * 64) {
-        float v = sums[q];
+        double v = sums[q];
 #pragma unroll
-        for (int w = 1; w < kWaves; w++) v += sums[w * kOut + q];
+        for (int w = 1; w < kWaves; w++) v += (double)sums[w * kOut + q];
         const int r = kTile == 32 ? c_row(q >> 6, q & 63) : 4 * ((q & 63) >> 4) + (q >> 6);
-        store_c<kAdd>(C, add, M, N, m0 + r, n0 + q % kTile, v);
+        store_c<kAdd>(C, add, M, N, m0 + r, n0 + q % kTile, (float)v);
     }
 }
 
@@ -334,6 +371,8 @@ int launch(hipStream_t s, const float* a, const float* b, float* c, const float*
     // 2048^3, 256 tiles: 169 against 196).  Element-wise loads need too many registers for 128 x 128.
     if (variant == 0) variant = t16 <= 512 ? 4 : t32 <= 384 ? 1 : kVec && t128 >= 256 ? 3 : 2;
     if (!kVec && variant == 3) variant = 2;
+    // (the tiled kernels' offsets inside a step are 32-bit: up to 128 rows of K floats, or 64 of N)
+    if ((variant == 2 || variant == 3) && (K > (1L << 22) || (!kNT && N > (1L << 22)))) variant = 4;
     if (t16 > 0x7fffffffL) return hipErrorInvalidValue;
     if (variant == 1) {
         const dim3 grid((unsigned)t32);
@@ -345,10 +384,25 @@ int launch(hipStream_t s, const float* a, const float* b, float* c, const float*
         const int tn = (int)((N + 15) / 16);
         if (K <= 256) dev::f32_direct<16, 4, kNT, kVec, kAdd><<<grid, 256, 0, s>>>(a, b, c, add, M, N, K, tn);
         else dev::f32_direct<16, 16, kNT, kVec, kAdd><<<grid, 1024, 0, s>>>(a, b, c, add, M, N, K, tn);
-    } else if (variant == 2) {
-        dev::f32_tiled<1, kNT, kVec, kAdd><<<dim3((unsigned)t64), 512, 0, s>>>(a, b, c, add, M, N, K, (int)((M + 63) / 64), (int)((N + 63) / 64));
-    } else if constexpr (kVec) {
-        dev::f32_tiled<2, kNT, kVec, kAdd><<<dim3((unsigned)t128), 512, 0, s>>>(a, b, c, add, M, N, K, (int)((M + 127) / 128), (int)((N + 127) / 128));
+    } else {
+        // Products of whole 64 x 64 tiles keep one chain per wave, see the head of the file.
+        const bool chain = (M % 64 == 0 && N % 64 == 0) || K < 128;
+        auto tiled = [&](auto t, auto run) {
+            constexpr int kT = decltype(t)::value, kB = 64 * kT;
+            const long tm = (M + kB - 1) / kB, tn = (N + kB - 1) / kB;
+            dev::f32_tiled<kT, kNT, kVec, kAdd, decltype(run)::value><<<dim3((unsigned)(tm * tn)), 512, 0, s>>>(a, b, c, add, M, N, K, (int)tm, (int)tn);
+        };
+        const std::integral_constant<int, 0> r0;
+        const std::integral_constant<int, 8> r8;
+        const std::integral_constant<int, 16> r16;
+        const std::integral_constant<int, 1> t1;
+        const std::integral_constant<int, 2> t2;
+        bool large = false;
+        if constexpr (kVec) {
+            large = variant == 3 && (chain || K >= 192);
+            if (large) chain ? tiled(t2, r0) : tiled(t2, r16);
+        }
+        if (!large) chain ? tiled(t1, r0) : K < 192 ? tiled(t1, r8) : tiled(t1, r16);
     }
     return hipGetLastError();
 }

@@ -72,3 +72,32 @@ def test_infinities_and_nan_stay_in_their_rows_and_columns():
     with np.errstate(invalid="ignore"):
         ref = a.astype(np.float64) @ b.astype(np.float64)
     assert np.array_equal(got, ref.astype(np.float32), equal_nan=True)
+
+
+def _sums_of_64(a, b):
+    """Row by column products the way the generated reduction adds them: lane l of a wave takes k = l, l + 64, ... one rounded
+    product and one addition after the other, and the 64 partial sums meet in a tree."""
+    parts = []
+    for lane in range(64):
+        acc = np.zeros((a.shape[0], b.shape[1]), np.float32)
+        for k in range(lane, a.shape[1], 64):
+            acc = acc + a[:, k:k + 1] * b[k:k + 1]
+        parts.append(acc)
+    while len(parts) > 1:
+        parts = [parts[i] + parts[i + 1] for i in range(0, len(parts), 2)]
+    return parts[0]
+
+
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("m,n,k", [(130, 200, 130), (130, 200, 1000), (481, 501, 257), (641, 703, 130), (641, 703, 192), (641, 704, 257),
+                                   (1001, 640, 777), (2049, 2052, 200), (2049, 2052, 515 + 1)])
+def test_ragged_products_are_no_less_exact_than_64_partial_sums(m, n, k, nt):
+    """2-norm against float64 over all outputs, against the same figure for 64 partial sums over 32 rows of it (at least 6400
+    outputs: the two figures are known to 1 %)."""
+    rng = np.random.default_rng(m + n + k)
+    a, b = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n)))
+    x = T.Tensor.from_numpy(a)
+    got = (x.linear(T.Tensor.from_numpy(np.ascontiguousarray(b.T))) if nt else x.matmul(T.Tensor.from_numpy(b))).to_numpy()
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    off = lambda y, r: np.linalg.norm(y - r) / np.linalg.norm(r)  # noqa: E731
+    assert off(got, ref) <= 1.02 * off(_sums_of_64(a[:32], b), ref[:32])
