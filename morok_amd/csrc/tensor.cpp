@@ -2339,6 +2339,44 @@ struct Scheduler {
     // Up to three such reductions may feed the kernel, one building on another (softmax: the row
     // maximum, then the sum of exp(x - max); layer norm: the mean, then the variance of the centred
     // row): they are returned in an order in which each one's own expression only needs earlier ones.
+    // Bytes of the widest operand that an expression reads element after element along its last axis (at least 1; operands that
+    // do not vary along it count nothing); 0 when some operand varies along it in another way.
+    static int64_t widest_along_rows(const TensorNode* root) {
+        std::unordered_map<const TensorNode*, int64_t> memo;
+        std::function<int64_t(const TensorNode*)> walk = [&](const TensorNode* m) -> int64_t {
+            if (m->shape.empty() || m->shape.back() == 1 || m->kind == TKind::Const || m->kind == TKind::Iota) return 1;
+            if (m->buffer) return static_cast<int64_t>(scalar_size(m->dtype));
+            const auto it = memo.find(m);
+            if (it != memo.end()) return it->second;
+            const TensorNode* c = m->src.empty() ? nullptr : m->src[0].get();
+            int64_t w = 0;
+            switch (m->kind) {
+                case TKind::Unary:
+                case TKind::Binary:
+                case TKind::Where:
+                case TKind::Cast:
+                case TKind::Contiguous:
+                    w = 1;
+                    for (const TensorRef& o : m->src) {
+                        const int64_t one = walk(o.get());
+                        w = one && w ? std::max(w, one) : 0;
+                    }
+                    break;
+                case TKind::Expand:
+                case TKind::Shrink: w = walk(c); break;
+                case TKind::Reshape:
+                    if (c->buffer) w = static_cast<int64_t>(scalar_size(c->dtype));
+                    else if (!c->shape.empty() && c->shape.back() == m->shape.back()) w = walk(c);
+                    break;
+                case TKind::Permute:
+                    if (m->arg.back() == static_cast<int64_t>(m->arg.size()) - 1) w = walk(c);
+                    break;
+                default: break;
+            }
+            return memo[m] = w;
+        };
+        return walk(root);
+    }
     // Work-items that share a row of `n` in a row-resident kernel; 0: rows of this shape are not kept in registers.
     static int64_t row_fused_block(const TensorNode* n) {
         const int64_t C = n->shape.back(), rows = n->numel() / C;
@@ -2879,14 +2917,20 @@ struct Scheduler {
         uint32_t seg0 = P > 1 ? b.imul(b.imod(wc, P), chunk) : g.ci(0);  // first reduce index of the segment
         Coords coords = plain(unflatten(g, oc, n->shape));
         // A long fold over the contiguous axis is read in groups of up to 16 bytes per lane (of the widest operand: eight
-        // elements of a half type) where the axis divides into them: one memory request and one loop step per group
-        // instead of one per element.  Small graphs keep the short kernel: they are bound by its latency and by
+        // elements of a half type, four of f32) where the axis divides into them: one memory request and one loop step per group
+        // instead of one per element.  Not where an operand is read across the lines of its memory (a transposed one: every
+        // element of a group is a request of its own) and not where the last, partial step would be most of the work: a wave
+        // takes 64 groups at a time.  Few outputs, few waves: eight elements of f32 too, for the requests in flight (log_softmax's
+        // folds over 400 x 9000 13.8 -> 12.5 us).  Small graphs keep the short kernel: they are bound by its latency and by
         // the time it takes to emit.  Measured, RMSNorm with its second kernel unchanged, bf16: 4503 x 3608 31.5 -> 16.9 us,
         // 2065 x 2128 11.7 -> 6.8, 16384 x 8184 231 -> 144.
         int64_t W8 = 1;
-        if (n->arg.size() == 1 && n->arg[0] == static_cast<int64_t>(s->shape.size()) - 1 && Nout * R >= (1LL << 20) && P == 1)
-            for (int64_t c = 8; c > 1 && W8 == 1; c /= 2)
-                if (R % c == 0 && R >= 64 * G * c) W8 = c;
+        const int64_t widest = n->arg.size() == 1 && n->arg[0] == static_cast<int64_t>(s->shape.size()) - 1 && Nout * R >= (1LL << 20) && P == 1
+                                   ? widest_along_rows(s) : 0;
+        for (int64_t c = !widest ? 1 : Nout <= 2048 ? 8 : std::min<int64_t>(8, 16 / widest); c > 1 && W8 == 1; c /= 2) {
+            const int64_t step = 64 * G * c;
+            if (R % c == 0 && R >= step && (R + step - 1) / step * step * 10 <= R * 13) W8 = c;
+        }
         g.width = W8;
         const int64_t steps = (chunk + 64 * G * W8 - 1) / (64 * G * W8);
         uint32_t rg = b.add(Op::Range, KernelBuilder::scalar(g.idx_t), {g.ci(steps)}, 0, 0, static_cast<uint16_t>(AxisType::Reduce));

@@ -1063,3 +1063,25 @@ def test_null_arguments_are_errors_not_crashes(T, dev, shim):
         rc = call()
         assert rc == 11, (i, rc, shim.mrk_hip_last_error())       # MRK_ERR_INVALID_ARGUMENT
         assert shim.mrk_hip_last_error()
+
+
+def test_folds_are_read_in_groups_where_that_is_one_request(T, shim):
+    """Long folds over the contiguous axis take 16 bytes per lane and step; operands that are read across the lines of their
+    memory, and rows whose last step would be mostly empty, one element."""
+    import re
+
+    from morok_amd import uop
+
+    def steps(t):
+        t.realize()
+        src = [s for s in T.last_kernel_sources() if "mrk_wave_reduce_add(acc" in s][0]
+        return int(re.search(r"ridx0 < (\d+)", src).group(1))
+
+    assert steps(zeros(T, (4096, 4096)).sum(1)) == 4096 // (64 * 4)
+    assert steps(zeros(T, (4096, 4096), np.uint16, uop.BF16).cast(uop.F32).sum(1)) == 4096 // (64 * 8)
+    assert steps(zeros(T, (4096, 4096)).try_mul(zeros(T, (4096,))).sum(1)) == 16              # a factor per column
+    assert steps(zeros(T, (4096, 4096)).try_sub(zeros(T, (4096, 1))).sum(1)) == 16            # and one per row
+    assert steps(zeros(T, (16384, 2049)).try_permute([1, 0]).sum(1)) == 16384 // 64           # transposed: one element
+    assert steps(zeros(T, (65536, 136)).sum(1)) == 3                                          # two steps of 128 would be half empty
+    assert steps(zeros(T, (65536, 264)).sum(1)) == 5
+    assert steps(zeros(T, (4096, 1000)).sum(1)) == 4                                          # 250 groups of four in steps of 64
