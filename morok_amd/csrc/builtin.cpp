@@ -158,7 +158,7 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
             const std::string name = !nt && !add ? "r_" + dims : k + "_" + dims;
             out->reset(new BuiltinProgram(device_id, stream, name, add ? 4 : 3, p,
                                           [nt, row, add](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
-                                              return launch_gemm_f32(s, b[1], b[2], b[0], add ? b[3] : nullptr, row, q[0], q[1], q[2], nt, 0);
+                                              return launch_gemm_f32(s, b[1], b[2], b[0], add ? b[3] : nullptr, row, q[0], q[1], q[2], nt);
                                           }));
             return kOk;
         }

@@ -360,76 +360,120 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
 namespace mrk {
 
 namespace {
-template <bool kNT, bool kVec, int kAdd>
-int launch(hipStream_t s, const float* a, const float* b, float* c, const float* add, long M, long N, long K, int variant) {
-    const long t16 = ((M + 15) / 16) * ((N + 15) / 16), t32 = ((M + 31) / 32) * ((N + 31) / 32);
-    const long t64 = ((M + 63) / 64) * ((N + 63) / 64), t128 = ((M + 127) / 128) * ((N + 127) / 128);
-    // Measured (us, [K, N] weight): up to two 16 x 16 tiles per CU they win (256 x 256 x 1536: 8.6, tiles of 32 16.4, of 64 35;
-    // 64 x 256 x 784: 5.1 / 9.8 / 20; 8192 x 10 x 784: 16.3 / 20.8 / 32), then 32 x 32 while they make one round
-    // (512^3: 6.8 against 17.8 and 14.7), at two rounds 64 x 64 draws level (512 x 1000 x 1024: 25.1 / 26.4) and
-    // ahead from there (768^3: 30.2 / 21.0); 128 x 128 from one tile per CU (1536^3, 144 tiles: 118 against 104;
-    // 2048^3, 256 tiles: 169 against 196).  Element-wise loads need too many registers for 128 x 128.
-    if (variant == 0) variant = t16 <= 512 ? 4 : t32 <= 384 ? 1 : kVec && t128 >= 256 ? 3 : 2;
-    if (!kVec && variant == 3) variant = 2;
-    // (the tiled kernels' offsets inside a step are 32-bit: up to 128 rows of K floats, or 64 of N)
-    if ((variant == 2 || variant == 3) && (K > (1L << 22) || (!kNT && N > (1L << 22)))) variant = 4;
-    if (t16 > 0x7fffffffL) return hipErrorInvalidValue;
-    if (variant == 1) {
-        const dim3 grid((unsigned)t32);
-        const int tn = (int)((N + 31) / 32);
-        if (K <= 256) dev::f32_direct<32, 4, kNT, kVec, kAdd><<<grid, 256, 0, s>>>(a, b, c, add, M, N, K, tn);
-        else dev::f32_direct<32, 16, kNT, kVec, kAdd><<<grid, 1024, 0, s>>>(a, b, c, add, M, N, K, tn);
-    } else if (variant == 4) {
-        const dim3 grid((unsigned)t16);
-        const int tn = (int)((N + 15) / 16);
-        if (K <= 256) dev::f32_direct<16, 4, kNT, kVec, kAdd><<<grid, 256, 0, s>>>(a, b, c, add, M, N, K, tn);
-        else dev::f32_direct<16, 16, kNT, kVec, kAdd><<<grid, 1024, 0, s>>>(a, b, c, add, M, N, K, tn);
+struct F32Call {
+    hipStream_t s;
+    const float *a, *b, *add;
+    float* c;
+    long M, N, K;
+};
+
+long tiles(long M, long N, long t) { return ((M + t - 1) / t) * ((N + t - 1) / t); }
+// What tiles of a size compute, whether it is stored or not: a product with a side of 1 to 32 in tiles of 128 is mostly
+// padding (65536 x 1 x 1024 144 us in tiles of 128, 62 in tiles of 16).
+double padded(long M, long N, long t) { return (double)tiles(M, N, t) * t * t; }
+
+// 16 and 32: f32_direct; 64: f32_tiled, which takes 128 where launch() says.
+// Measured (us, [K, N] weight): up to two 16 x 16 tiles per CU they win (256 x 256 x 1536: 8.6, tiles of 32 16.4, of 64 35;
+// 64 x 256 x 784: 5.1 / 9.8 / 20; 8192 x 10 x 784: 16.3 / 20.8 / 32), then 32 x 32 while they make one round
+// (512^3: 6.8 against 17.8 and 14.7), at two rounds 64 x 64 draws level (512 x 1000 x 1024: 25.1 / 26.4) and
+// ahead from there (768^3: 30.2 / 21.0).  A larger tile may pad as much more as it is faster: 1.4 from 32 to 64; tiles of
+// 16 read the longer operand's lines in halves and pay on long K only (65536 x 5 x 1024 68 us against 77 in tiles of 32,
+// 65536 x 8 x 500 47 / 41).  The tiled kernels' offsets inside a step are 32-bit: up to 128 rows of K floats, or 64 of N.
+int tile_size(long M, long N, long K, bool b_transposed) {
+    const bool narrow = padded(M, N, 64) > 1.4 * padded(M, N, 32), far = K > (1L << 22) || (!b_transposed && N > (1L << 22));
+    if (tiles(M, N, 16) <= 512 || far || (narrow && K >= 768 && padded(M, N, 32) > 1.4 * padded(M, N, 16))) return 16;
+    return tiles(M, N, 32) <= 384 || narrow ? 32 : 64;
+}
+
+// Times in us of f32_direct, and of the generated reduction that a product is without these kernels (K >= 128: one wave
+// per output; below: one work-item), fitted to 890 products with a side of 1 to 24 against 300 to 10^6, and of 17 to 600,
+// K from 64 to 4096.  Either is within a quarter of the measured time for most of them.
+double direct_us(double M, double N, double K, bool b_transposed, int tile, double area, long count) {
+    const double columns = b_transposed ? 0.0 : 0.2 + 3e-4 * K;
+    if (tile == 16) return columns + (count <= 512 ? 3.4 + 1.8e-3 * K + 2.2e-8 * area * K + 1.9e-7 * (M + N) * K : 6.2e-8 * area * K + 1.4e-5 * M * N);
+    return columns + (count <= 384 ? 3.0 + 7.4e-3 * K + 1.3e-6 * M * N : 2.8 + 3.7e-8 * area * K + 1.2e-6 * area);
+}
+double reduction_us(double M, double N, double K, bool b_transposed) {
+    const double x = M * N * K, edges = (M + N) * K;
+    if (K < 128) return 0.8 + 0.026 * K + (b_transposed ? 5e-7 : 2.5e-7) * x + (M < N ? 4e-7 : 3e-7) * edges;
+    // (a wide [N, K] operand is read again for every row)
+    if (b_transposed && M < N && N * K > (2 << 20)) return 8e-4 * K + 2.6e-7 * x + 6e-5 * M * N + 2e-7 * edges;
+    if (b_transposed) return 2.3 + 2e-4 * K + 1.9e-7 * x + 4.3e-5 * M * N + 1.2e-7 * edges;
+    // (a wave's lanes walk a column of a [K, N] operand, a line each)
+    if (N == 1) return 2.0 + 2e-4 * K + 4.5e-5 * M + 3.6e-7 * edges;
+    if (N <= 3) return 2.4 + 5e-7 * x + 2.4e-5 * M * N;
+    if (N <= 12) return 2.4 + (N >= 8 && K >= 1024 ? 2e-6 : 9e-7) * x + 1.5e-5 * M * N;
+    return N * K < (1 << 18) ? 1.8 + 1.5e-3 * K + 1.5e-6 * x : 1.8 + 1.5e-3 * K + 3.5e-6 * x + 2.5e-6 * edges;
+}
+
+template <int kTile, bool kNT, bool kVec, int kAdd>
+void launch_direct(const F32Call& p) {
+    const int tn = (int)((p.N + kTile - 1) / kTile);
+    const dim3 grid((unsigned)((p.M + kTile - 1) / kTile * tn));
+    if (p.K <= 256) dev::f32_direct<kTile, 4, kNT, kVec, kAdd><<<grid, 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+    else dev::f32_direct<kTile, 16, kNT, kVec, kAdd><<<grid, 1024, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+}
+
+template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
+void launch_tiled(const F32Call& p) {
+    constexpr int kB = 64 * kT;
+    const long tm = (p.M + kB - 1) / kB, tn = (p.N + kB - 1) / kB;
+    dev::f32_tiled<kT, kNT, kVec, kAdd, kRun><<<dim3((unsigned)(tm * tn)), 512, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, (int)tm, (int)tn);
+}
+
+template <bool kNT, int kAdd>
+int launch(const F32Call& p) {
+    const long M = p.M, N = p.N, K = p.K;
+    if (tiles(M, N, 16) > 0x7fffffffL) return hipErrorInvalidValue;
+    auto aligned = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+    // whole aligned 16-byte chunks along the rows that a kernel reads in them (f32_direct reads columns of a [K, N] operand)
+    const bool rows = K % 4 == 0 && aligned(p.a) && (!kNT || aligned(p.b)), vec = rows && (kNT || (N % 4 == 0 && aligned(p.b)));
+    const int tile = tile_size(M, N, K, kNT);
+    if (tile == 16) {
+        rows ? launch_direct<16, kNT, true, kAdd>(p) : launch_direct<16, kNT, false, kAdd>(p);
+    } else if (tile == 32) {
+        rows ? launch_direct<32, kNT, true, kAdd>(p) : launch_direct<32, kNT, false, kAdd>(p);
     } else {
-        // Products of whole 64 x 64 tiles keep one chain per wave, see the head of the file.
+        // 128 x 128 from one tile per CU (1536^3, 144 tiles: 118 us against 104; 2048^3, 256 tiles: 169 against 196) and where they
+        // pad no more than they gain.  Element-wise loads need too many registers for them.
+        // Products of whole 64 x 64 tiles, and short ones, keep one chain per wave, see the head of the file.
         const bool chain = (M % 64 == 0 && N % 64 == 0) || K < 128;
-        auto tiled = [&](auto t, auto run) {
-            constexpr int kT = decltype(t)::value, kB = 64 * kT;
-            const long tm = (M + kB - 1) / kB, tn = (N + kB - 1) / kB;
-            dev::f32_tiled<kT, kNT, kVec, kAdd, decltype(run)::value><<<dim3((unsigned)(tm * tn)), 512, 0, s>>>(a, b, c, add, M, N, K, (int)tm, (int)tn);
-        };
-        const std::integral_constant<int, 0> r0;
-        const std::integral_constant<int, 8> r8;
-        const std::integral_constant<int, 16> r16;
-        const std::integral_constant<int, 1> t1;
-        const std::integral_constant<int, 2> t2;
-        bool large = false;
-        if constexpr (kVec) {
-            large = variant == 3 && (chain || K >= 192);
-            if (large) chain ? tiled(t2, r0) : tiled(t2, r16);
-        }
-        if (!large) chain ? tiled(t1, r0) : K < 192 ? tiled(t1, r8) : tiled(t1, r16);
+        if (vec && tiles(M, N, 128) >= 256 && padded(M, N, 128) <= 1.14 * padded(M, N, 64) && (chain || K >= 192))
+            chain ? launch_tiled<2, kNT, true, kAdd, 0>(p) : launch_tiled<2, kNT, true, kAdd, 16>(p);
+        else if (chain) vec ? launch_tiled<1, kNT, true, kAdd, 0>(p) : launch_tiled<1, kNT, false, kAdd, 0>(p);
+        else if (K < 192) vec ? launch_tiled<1, kNT, true, kAdd, 8>(p) : launch_tiled<1, kNT, false, kAdd, 8>(p);
+        else vec ? launch_tiled<1, kNT, true, kAdd, 16>(p) : launch_tiled<1, kNT, false, kAdd, 16>(p);
     }
     return hipGetLastError();
 }
 }  // namespace
 
 bool gemm_f32_supported(long M, long N, long K) {
-    return M > 0 && N > 0 && K >= 64 && M * N >= ((1L << 18) + K - 1) / K && ((M + 15) / 16) * ((N + 15) / 16) <= 0x7fffffffL &&
-           (K <= 8192 || ((M + 63) / 64) * ((N + 63) / 64) >= 256);
+    return M > 0 && N > 0 && K >= 64 && M * N >= ((1L << 18) + K - 1) / K && tiles(M, N, 16) <= 0x7fffffffL &&
+           (K <= 8192 || tiles(M, N, 64) >= 256);
+}
+
+// Whole 64 x 64 tiles are a generated kernel of register tiles otherwise, whose work-items walk all of K, and lose to these
+// at every size (64 x 256 x 784: 36 us against 5).  Of the others the narrow ones are faster as reductions, the
+// more so the more K there is per output: 1000000 x 1 x 64 65 us against 128 in tiles of 32, 300 x 3 x 4096 4.2 / 13.7,
+// 64 x 10 x 784 3.1 / 4.9; but 65536 x 5 x 1024 91 / 68, 8192 x 10 x 784 69 / 9.  They go where the estimates are further apart
+// than they are off (1 us on the smallest), inside the sizes they were fitted to.  An addend is a kernel of its own (2.6 us) there.
+bool gemm_f32_preferred(long M, long N, long K, bool b_transposed, bool added) {
+    if (!gemm_f32_supported(M, N, K)) return false;
+    const int tile = tile_size(M, N, K, b_transposed);
+    if (tile == 64 || (M % 64 == 0 && N % 64 == 0) || ((M < N ? M : N) > 24 && K > 1024)) return true;
+    const double direct = direct_us((double)M, (double)N, (double)K, b_transposed, tile, padded(M, N, tile), tiles(M, N, tile));
+    const double reduction = reduction_us((double)M, (double)N, (double)K, b_transposed) + (added ? 2.6 : 0.0);
+    return direct < 1.05 * reduction || direct < reduction + 1.3;
 }
 
 int launch_gemm_f32(void* stream, const void* a, const void* b, void* c, const void* add, bool add_is_row, long M, long N, long K,
-                    bool b_transposed, int variant) {
-    if (M <= 0 || N <= 0 || K <= 0 || variant < 0 || variant > 4) return hipErrorInvalidValue;
-    auto misaligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
-    const bool vec = K % 4 == 0 && (b_transposed || N % 4 == 0) && !misaligned(a) && !misaligned(b);
-    const auto s = static_cast<hipStream_t>(stream);
-    const float *pa = static_cast<const float*>(a), *pb = static_cast<const float*>(b), *pr = static_cast<const float*>(add);
-    float* pc = static_cast<float*>(c);
-    auto with_add = [&](auto nt, auto v) {
-        if (!pr) return launch<decltype(nt)::value, decltype(v)::value, 0>(s, pa, pb, pc, pr, M, N, K, variant);
-        if (add_is_row) return launch<decltype(nt)::value, decltype(v)::value, 1>(s, pa, pb, pc, pr, M, N, K, variant);
-        return launch<decltype(nt)::value, decltype(v)::value, 2>(s, pa, pb, pc, pr, M, N, K, variant);
-    };
-    const std::true_type yes;
-    const std::false_type no;
-    if (b_transposed) return vec ? with_add(yes, yes) : with_add(yes, no);
-    return vec ? with_add(no, yes) : with_add(no, no);
+                    bool b_transposed) {
+    if (M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
+    const F32Call p{static_cast<hipStream_t>(stream), static_cast<const float*>(a), static_cast<const float*>(b), static_cast<const float*>(add),
+                    static_cast<float*>(c), M, N, K};
+    if (b_transposed) return !add ? launch<true, 0>(p) : add_is_row ? launch<true, 1>(p) : launch<true, 2>(p);
+    return !add ? launch<false, 0>(p) : add_is_row ? launch<false, 1>(p) : launch<false, 2>(p);
 }
 
 }  // namespace mrk

@@ -164,11 +164,13 @@ int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const 
 
 // C[M, N] = A[M, K] B in f32 on the f32 matrix instructions, B [K, N] or (b_transposed) [N, K]; any shape and alignment of
 // whole floats.  add (may be null): f32, one row [N] (add_is_row) or a matrix of C's shape, added to the sums: the bits
-// of the product followed by the add.  variant 0 = choose by shape, 1 / 4 = tiles of 32 / 16 with K split over a
-// workgroup's waves, 2 / 3 = tiles of 64 / 128 (128: 64 where rows are no whole 16-byte chunks).  gemm_f32_supported: the shapes a program's products are routed here for.
+// of the product followed by the add.  gemm_f32_supported: the shapes a builtin program takes; gemm_f32_preferred: those of
+// them that a tensor program's products run on (the others are faster as generated reductions); added: a row or a matrix is
+// added to the product and nothing else reads it.
 bool gemm_f32_supported(long M, long N, long K);
+bool gemm_f32_preferred(long M, long N, long K, bool b_transposed, bool added);
 int launch_gemm_f32(void* stream, const void* a, const void* b, void* c, const void* add, bool add_is_row, long M, long N, long K,
-                    bool b_transposed, int variant);
+                    bool b_transposed);
 
 // Synthetic benchmark inputs. dtype 0 = f32, 1 = bf16; mode 0 = uniform [a, b), 1 = normal(0, a).
 int launch_fill(void* stream, void* out, size_t n, int dtype, int mode, unsigned long long seed,

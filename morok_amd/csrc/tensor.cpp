@@ -1325,13 +1325,20 @@ struct Scheduler {
         }
     }
 
-    // An f32 product of two matrices that the hand-written f32 kernels take (any shape above a few thousand multiply-adds per
-    // output tile).  Under MOROK_BEAM products stay with the generated kernels, whose choices it searches.
+    // (a matter of the graph alone: which nodes have data by now changes while a plan is made)
+    static bool is_transpose(const TensorNode* w) {
+        return w->kind == TKind::Permute && w->shape.size() == 2 && w->arg.size() == 2 && w->arg[0] == 1 && w->arg[1] == 0;
+    }
+    // An f32 product of two matrices that runs on the hand-written f32 kernels.  Under MOROK_BEAM products stay with the
+    // generated kernels, whose choices it searches.
     bool matrix_f32(const TensorNode* mm) const {
         if (beam > 0 || mm->hint != HintKind::Matmul || mm->dtype != Scalar::Float32) return false;
         const TensorNode *a = mm->hint_inputs[0].get(), *w = mm->hint_inputs[1].get();
-        return a->dtype == Scalar::Float32 && w->dtype == Scalar::Float32 && a->shape.size() == 2 && w->shape.size() == 2 &&
-               gemm_f32_supported(a->shape[0], w->shape[1], a->shape[1]);
+        if (a->dtype != Scalar::Float32 || w->dtype != Scalar::Float32 || a->shape.size() != 2 || w->shape.size() != 2) return false;
+        const auto r = matmul_readers.find(mm);
+        const TensorNode* reader = r != matmul_readers.end() && r->second.size() == 1 ? r->second[0] : nullptr;
+        const bool added = reader && reader->kind == TKind::Binary && static_cast<BinaryOp>(reader->sub) == BinaryOp::Add;
+        return gemm_f32_preferred(a->shape[0], w->shape[1], a->shape[1], is_transpose(w), added);
     }
 
     // With the hand-written kernels switched off, a bf16 matmul whose shape fits still takes the
@@ -1512,10 +1519,7 @@ struct Scheduler {
     TensorNode* transposed_weight(const TensorNode* mm) const {
         if (!g_fusion) return nullptr;
         TensorNode* w = mm->hint_inputs[1].get();
-        if (w->buffer || w->kind != TKind::Permute || (w->dtype != Scalar::BFloat16 && w->dtype != Scalar::Float16 && !matrix_f32(mm)) ||
-            w->shape.size() != 2 || w->arg.size() != 2 ||
-            w->arg[0] != 1 || w->arg[1] != 0)
-            return nullptr;
+        if (w->buffer || !is_transpose(w) || (w->dtype != Scalar::BFloat16 && w->dtype != Scalar::Float16 && !matrix_f32(mm))) return nullptr;
         TensorNode* wt = w->src[0].get();
         const TensorNode* rb = wt;
         while (!rb->buffer && rb->kind == TKind::Reshape) rb = rb->src[0].get();

@@ -105,7 +105,8 @@ int launch_flash_fwd_bf16_ext(void* stream, const void*, const void*, const void
     return 0;
 }
 bool gemm_f32_supported(long M, long N, long K) { return M > 0 && N > 0 && K >= 64 && M * N * K >= (1L << 18); }
-int launch_gemm_f32(void* stream, const void*, const void*, void*, const void* add, bool add_is_row, long, long, long, bool b_transposed, int) {
+bool gemm_f32_preferred(long M, long N, long K, bool, bool) { return gemm_f32_supported(M, N, K); }
+int launch_gemm_f32(void* stream, const void*, const void*, void*, const void* add, bool add_is_row, long, long, long, bool b_transposed) {
     mrk_shim_note_launch(stream, add ? (add_is_row ? "gemm_f32_bias" : "gemm_f32_residual") : b_transposed ? "gemm_f32_nt" : "gemm_f32");
     return 0;
 }

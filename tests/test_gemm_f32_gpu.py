@@ -101,3 +101,19 @@ def test_ragged_products_are_no_less_exact_than_64_partial_sums(m, n, k, nt):
     ref = a.astype(np.float64) @ b.astype(np.float64)
     off = lambda y, r: np.linalg.norm(y - r) / np.linalg.norm(r)  # noqa: E731
     assert off(got, ref) <= 1.02 * off(_sums_of_64(a[:32], b), ref[:32])
+
+
+@pytest.mark.parametrize("m,n,k,nt,matrix", [(65536, 1, 200, True, False), (65536, 1, 200, False, False), (300, 3, 1024, False, False),
+                                             (1, 8192, 1024, True, False), (64, 10, 784, False, False), (65536, 12, 200, True, True),
+                                             (8192, 10, 784, False, True), (2, 65536, 200, False, True), (129, 64 * 65536 // 129, 64, False, True)])
+def test_narrow_products(m, n, k, nt, matrix):
+    """A side of a few: on the matrix kernels where tiles of 16 or 32 pay, a reduction where they do not; with a bias either way."""
+    rng = np.random.default_rng(m + n + k)
+    a, b, row = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n), (n,)))
+    x = T.Tensor.from_numpy(a)
+    w = T.Tensor.from_numpy(np.ascontiguousarray(b.T) if nt else b)
+    y = (x.linear(w) if nt else x.matmul(w)).realize()
+    assert (y.kernels() == [f"gemm_f32_nt_{m}_{n}_{k}" if nt else f"r_{m}_{n}_{k}"]) == matrix, y.kernels()
+    _check(y.to_numpy(), a, b)
+    z = (x.linear(w, T.Tensor.from_numpy(row)) if nt else x.matmul(w).try_add(T.Tensor.from_numpy(row))).to_numpy()
+    _check(z, a, b, row)
