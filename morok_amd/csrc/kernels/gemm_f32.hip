@@ -425,6 +425,7 @@ template <bool kNT, int kAdd>
 int launch(const F32Call& p) {
     const long M = p.M, N = p.N, K = p.K;
     if (tiles(M, N, 16) > 0x7fffffffL) return hipErrorInvalidValue;
+    (void)hipGetLastError();  // (an error that an earlier call left behind is not this launch's)
     auto aligned = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
     // whole aligned 16-byte chunks along the rows that a kernel reads in them (f32_direct reads columns of a [K, N] operand)
     const bool rows = K % 4 == 0 && aligned(p.a) && (!kNT || aligned(p.b)), vec = rows && (kNT || (N % 4 == 0 && aligned(p.b)));

@@ -117,3 +117,17 @@ def test_narrow_products(m, n, k, nt, matrix):
     _check(y.to_numpy(), a, b)
     z = (x.linear(w, T.Tensor.from_numpy(row)) if nt else x.matmul(w).try_add(T.Tensor.from_numpy(row))).to_numpy()
     _check(z, a, b, row)
+
+
+def test_an_error_left_by_an_earlier_call_is_not_the_products():
+    """The last error of a thread stays until it is read; a call that HIP refuses (a device that does not exist) leaves one."""
+    import ctypes
+
+    a = np.ones((640, 704), np.float32)
+    x, w = T.Tensor.from_numpy(a), T.Tensor.from_numpy(np.ones((704, 128), np.float32))
+    plan = x.matmul(w).prepare()
+    maps = open("/proc/self/maps").read().split()
+    hip = ctypes.CDLL(next(p for p in maps if "libamdhip64.so" in p))
+    assert hip.hipSetDevice(12345) != 0
+    plan.execute()
+    assert np.all(T.Tensor.from_numpy(a).matmul(w).to_numpy() == 704.0)
