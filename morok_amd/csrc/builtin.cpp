@@ -318,7 +318,8 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         for (int i = 26; i < 29; i++)
             if (p[i] < 0 || p[i] % 4) return fail(kInvalidArgument, "flash_fwd_bf16_ext: mask strides must be non-negative multiples of 4 elements");
         if (p[8] != 0 && (p[3] % 4 || p[13] % 4)) return fail(kInvalidArgument, "flash_fwd_bf16_ext: with a mask, Sk and the mask offset must be multiples of 4");
-        std::string name = std::string("flash_fwd_bf16_ext") + (p[8] == 1 ? "_bool" : p[8] == 2 ? "_add" : "") + (p[7] ? "_cap" : "") + "_" +
+        std::string name = std::string("flash_fwd_bf16_ext") + (p[8] == 1 ? "_bool" : p[8] == 2 ? "_add" : "") + (p[7] ? "_cap" : "") +
+                           (flash_fwd_row_mask(p[2], p[3], static_cast<int>(p[8]), p[28], p[7] != 0) ? "_row_" : "_") +
                            std::to_string(p[0] * p[1]) + "_" + std::to_string(p[2]) + "_" + std::to_string(p[3]) + (p[4] != 128 ? "_d" + std::to_string(p[4]) : "");
         const bool ws = p[29] > 0;
         out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), ws ? 6 : 5, p,

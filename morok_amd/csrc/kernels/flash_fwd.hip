@@ -834,6 +834,14 @@ int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, co
     return (int)hipGetLastError();
 }
 
+// One row of the mask for every query (its words are made once per workgroup), as long as the words fit their 8 KB.  Against the
+// general kernel, by where keys are hidden: behind the last visible one 1.2 to 2.5 times as fast, nowhere 1.1 to 1.4; in front or
+// all over up to 1.13 (32 x 12 heads, 384 x 384, D = 64), and 0.96 to 0.98 where few workgroups have long rows or D = 256
+// (32 heads, 64 x 4096, D = 128: 91.3 us, 93.5 here).  What a mask holds is not known before the launch.
+bool flash_fwd_row_mask(long Sq, long Sk, int mask_kind, long row_stride, bool cap) {
+    return mask_kind == 1 && !cap && (row_stride == 0 || Sq == 1) && Sk <= (long)mrk::dev::kMaxMaskTiles * mrk::dev::kKT;
+}
+
 int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk,
                               long D, float scale, int causal, const long* strides, const void* mask, int mask_kind,
                               const long* mask_strides, float softcap, void* workspace, size_t workspace_bytes) {
@@ -900,10 +908,7 @@ int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const 
         {{nullptr, flash_fwd_ext_d256_cap}, {flash_fwd_ext_d256_bool, flash_fwd_ext_d256_bool_cap}, {flash_fwd_ext_d256_add, flash_fwd_ext_d256_add_cap}}};
     static const Kernel row_table[3] = {flash_fwd_ext_d64_rowmask, flash_fwd_ext_d128_rowmask, flash_fwd_ext_d256_rowmask};
     const int dim = D == 64 ? 0 : D == 128 ? 1 : 2;
-    // one row of the mask for every query (its words are made once per workgroup; no query count was found at which the
-    // general kernel is ahead), as long as the words fit their 8 KB
-    const bool row_mask = mask_kind == 1 && !cap && (ext.row == 0 || Sq == 1) && Sk <= (long)kMaxMaskTiles * kKT;
-    const Kernel kernel = row_mask ? row_table[dim] : table[dim][mask_kind][cap ? 1 : 0];
+    const Kernel kernel = flash_fwd_row_mask(Sq, Sk, mask_kind, ext.row, cap) ? row_table[dim] : table[dim][mask_kind][cap ? 1 : 0];
     kernel<<<(unsigned)blocks, 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const __bf16*>(q), static_cast<const __bf16*>(k), static_cast<const __bf16*>(v), static_cast<__bf16*>(o), (int)BH,
         (int)Sq, (int)Sk, scale_log2e, causal_tiles, (int)q_tiles, (int)units, lay, ext);

@@ -158,6 +158,9 @@ int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, co
 // Without mask and softcap this is launch_flash_fwd_bf16_strided.
 // Without the causal rule a decode shape (see flash_decode_plan) takes the split kernel here as well, mask and
 // softcap inside it, with the same workspace.
+// Whether launch_flash_fwd_bf16_ext takes the kernel for a Bool mask that is one row of keys for every query (outside the
+// split kernel's shapes).
+bool flash_fwd_row_mask(long Sq, long Sk, int mask_kind, long row_stride, bool cap);
 int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk,
                               long D, float scale, int causal, const long* strides, const void* mask, int mask_kind,
                               const long* mask_strides, float softcap, void* workspace = nullptr, size_t workspace_bytes = 0);

@@ -99,6 +99,7 @@ int launch_flash_fwd_bf16_strided(void* stream, const void*, const void*, const 
     mrk_shim_note_launch(stream, ws ? "flash_fwd_bf16_strided_splitkv" : "flash_fwd_bf16_strided");
     return 0;
 }
+bool flash_fwd_row_mask(long, long, int, long, bool) { return false; }
 int launch_flash_fwd_bf16_ext(void* stream, const void*, const void*, const void*, void*, long, long, long, long, long, float, int,
                               const long*, const void*, int mask_kind, const long*, float softcap, void* ws, size_t) {
     mrk_shim_note_launch(stream, mask_kind == 0 && !(softcap > 0.0f) ? "flash_fwd_bf16_strided" : ws ? "flash_fwd_bf16_ext_splitkv" : "flash_fwd_bf16_ext");

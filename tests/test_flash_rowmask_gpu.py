@@ -14,7 +14,10 @@ def _attend(q, k, v, mask, causal):
     t = [T.Tensor.from_numpy(x, uop.BF16) for x in (q, k, v)]
     out = t[0].scaled_dot_product_attention(t[1], t[2], is_causal=causal, attn_mask=T.Tensor.from_numpy(mask))
     got = synth.from_bf16(out.to_numpy())
-    assert out.kernels()[0].startswith("flash_fwd_bf16_ext_bool"), out.kernels()
+    # (more than 65536 keys: the general kernel for any mask)
+    row = mask.shape[2] == 1 and k.shape[2] <= 65536
+    assert out.kernels()[0].startswith("flash_fwd_bf16_ext_bool" + ("_row_" if row else "_")), out.kernels()
+    assert row or "_row_" not in out.kernels()[0]
     return got
 
 
@@ -55,6 +58,18 @@ def test_row_mask_matches_the_general_kernel(d, causal, sq, sk):
     want = _attend(q, k, v, np.ascontiguousarray(np.broadcast_to(rows, (B, 1, sq, sk))), causal)
     # the two round probabilities to bf16 against reference points that may differ by up to 2^8, and the result once:
     # 2^-9 relative each on terms whose sum is at most max |v|
+    assert np.all(np.isfinite(got)) and np.abs(got - want).max() <= 2.0 ** -8 * np.abs(synth.from_bf16(v)).max()
+
+
+@pytest.mark.parametrize("sk", [65532, 65536, 65540])
+@pytest.mark.parametrize("pattern", ["end", "one", "random", "last"])
+def test_the_longest_rows(sk, pattern):
+    """The last tile whose words fit the local memory, and one key group more, which the general kernel takes."""
+    rng = np.random.default_rng(sk)
+    q, k, v = (synth.normal_bf16((1, 2, s, 64), 13, i) for i, s in enumerate((40, sk, sk)))
+    row = _row(pattern, sk, rng)[None, None, None, :]
+    got = _attend(q, k, v, row, False)
+    want = _attend(q, k, v, np.ascontiguousarray(np.broadcast_to(row, (1, 1, 40, sk))), False)
     assert np.all(np.isfinite(got)) and np.abs(got - want).max() <= 2.0 ** -8 * np.abs(synth.from_bf16(v)).max()
 
 

@@ -39,7 +39,7 @@ def test_layouts_and_addends(m, n, k):
     x, w, wt = T.Tensor.from_numpy(a), T.Tensor.from_numpy(b), T.Tensor.from_numpy(np.ascontiguousarray(b.T))
     plain = x.matmul(w)
     _check(plain.to_numpy(), a, b)
-    assert plain.kernels() == [f"r_{m}_{n}_{k}"]
+    assert plain.kernels() == [f"r_{m}_{n}_{k}"] and T.last_kernel_sources() == [""]  # (a generated kernel of that name has a source)
     lin = x.linear(wt)
     _check(lin.to_numpy(), a, b)
     assert lin.kernels() == [f"gemm_f32_nt_{m}_{n}_{k}"]
