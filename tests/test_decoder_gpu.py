@@ -218,3 +218,34 @@ def test_decode_step_over_cached_keys_is_the_last_row_of_a_causal_pass(dev, orac
     ka, va = k_all.to_numpy(), v_all.to_numpy()
     assert ka.shape == (B, cfg["heads"], S, cfg["hidden"] // cfg["heads"])
     assert np.array_equal(ka[:, :, :P], k.to_numpy()) and np.array_equal(va[:, :, :P], v.to_numpy())
+
+
+def test_decode_steps_rotate_with_the_blocks_theta(dev):
+    """Two consecutive steps, the second past the first table of 256 positions, the cache fed back: keys rotated as the causal
+    pass of a block with the same theta rotates them, and not as one with the default theta does.  Tolerance: a key and the
+    causal pass's are the same f32 rotation, rounded to bf16 once, of projections that differ by the order of their sums (a bf16 step)."""
+    from morok_amd import decoder, synth, tensor
+
+    B, S, P = 2, 257, 255
+    cfg = (256, 2, 512, 1e-6)
+    w = decoder.synthetic_weights(256, 512, 300, seed=3)
+    tok = synth.randint((B * S,), 3, 1, 300).reshape(B, S).astype(np.int32)
+
+    def ids(t):
+        return tensor.Tensor.from_numpy(np.ascontiguousarray(t).reshape(-1))
+
+    def causal(n, theta):
+        blk = decoder.DecoderBlock(w, B, n, *cfg, theta=theta, linear_layout=True)
+        return [t.realize() for t in blk.forward(ids(tok[:, :n]), with_cache=True)]
+
+    want, other = (synth.from_bf16(causal(S, t)[1].to_numpy()) for t in (500.0, 10000.0))
+    _, k, v = causal(P, 500.0)
+    step = decoder.DecoderBlock(w, B, 1, *cfg, theta=500.0, linear_layout=True)
+    for pos in (P, P + 1):
+        y, k, v = step.decode_step(ids(tok[:, pos]), k, v, pos)
+        y.realize()
+    got = synth.from_bf16(k.to_numpy())
+    for pos in (P, P + 1):
+        row = [x[:, :, pos] for x in (got, want, other)]
+        assert np.abs(row[0] - row[1]).max() <= 2.0 ** -7 * np.abs(row[1]).max()
+        assert np.abs(row[0] - row[2]).max() > 0.1 * np.abs(row[2]).max()
