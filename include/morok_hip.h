@@ -452,14 +452,16 @@ size_t mrk_hip_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_
  * of the result), the same bits on every run.  More than 64 rows with N not a multiple of 8, or K
  * not a multiple of 8: INVALID_ARGUMENT.  Builtin Program kind "gemm_bf16_nt"
  * ({M, N, K[, batch[, workspace bytes]]}; the workspace is used by split-K shapes of more than 64
- * rows, which without one run the plain tiled kernel). */
+ * rows, which without one run the plain tiled kernel, and by N and K of any other size, which this
+ * entry point refuses and the program takes given one). */
 int mrk_hip_gemm_bf16_nt(int device_id, const void* a, const void* bt, void* c, int64_t m, int64_t n, int64_t k);
 /* The same two products on IEEE half precision (f16) operands and result, f32 accumulate: the f16
  * 16x16x32 entry of the reference's CDNA4 tensor-core table
  * (schedule/src/optimizer/renderer.rs:724-733, listed ahead of the bf16 one) as a hand-written
  * kernel; what Tensor::matmul computes for f16 inputs (tensor/src/matmul.rs:82-110 with the
- * tensor-core rewrite).  Same shapes, fallbacks and argument rules as the bf16 entry points; the
- * fused residual / gated epilogues are bf16 only.  Builtin Program kinds "gemm_f16", "gemm_f16_nt". */
+ * tensor-core rewrite).  Same shapes, fallbacks and argument rules as the bf16 entry points.  Builtin
+ * Program kinds "gemm_f16", "gemm_f16_nt", and with a row or a matrix added in the epilogue "gemm_f16[_nt]_bias" and
+ * "gemm_f16[_nt]_residual"; the gated and rotary epilogues are bf16 only. */
 int mrk_hip_gemm_f16(int device_id, const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k);
 int mrk_hip_gemm_f16_nt(int device_id, const void* a, const void* bt, void* c, int64_t m, int64_t n, int64_t k);
 /* Same with an explicit kernel variant (0 choose by shape, 2 any-shape kernel, 3 / 4 tiled kernel
@@ -491,7 +493,8 @@ size_t mrk_hip_gemm_bf16_noalloc_capacity(void);
  * from the device allocator), the streaming kernels for a handful of rows.  INVALID_ARGUMENT for shapes
  * outside the tiled kernels' (N or K not a multiple of 8, K = 0).  Builtin Program kinds
  * "gemm_bf16_residual" / "gemm_bf16_nt_residual" / "gemm_bf16_bias" / "gemm_bf16_nt_bias" take
- * {M, N, K[, batch[, workspace bytes]]} and buffers {c, a, b, r[, scratch]}. */
+ * {M, N, K[, batch[, workspace bytes]]} and buffers {c, a, b, r[, scratch]}; given the scratch they take
+ * N and K of any size. */
 int mrk_hip_gemm_bf16_residual(int device_id, const void* a, const void* b, const void* r, void* c, int64_t m, int64_t n,
                                int64_t k);
 /* y[M, N] = x[M, K] * w[N, K]^T + bias[N]: a Linear layer's forward pass on its parameters as it stores them
