@@ -14,10 +14,10 @@ from .tensor import Tensor
 WEIGHT_NAMES = ("emb", "w_an", "Wq", "Wk", "Wv", "Wo", "w_fn", "W1", "W3", "W2")
 
 
-def rope_tables(seq, dim, theta=10000.0):
-    """cos/sin [seq, dim/2] in f32: angle(p, i) = p * theta^(-2i/dim)."""
+def rope_tables(seq, dim, theta=10000.0, first=0):
+    """cos/sin [seq, dim/2] in f32 of `seq` positions from `first` on: angle(p, i) = p * theta^(-2i/dim)."""
     inv = (theta ** (-np.arange(0, dim, 2, dtype=np.float64) / dim))
-    ang = np.arange(seq, dtype=np.float64)[:, None] * inv[None, :]
+    ang = np.arange(first, first + seq, dtype=np.float64)[:, None] * inv[None, :]
     return np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
 
 
@@ -53,7 +53,7 @@ class DecoderBlock:
         self.batch, self.seq, self.hidden, self.heads, self.ffn, self.eps = batch, seq, hidden, heads, ffn, eps
         self.dim = hidden // heads
         self.linear_layout = bool(linear_layout)
-        self.theta, self.device_id, self._rope = theta, device_id, None
+        self.theta, self.device_id, self._rope = theta, device_id, {}
         projections = ("Wq", "Wk", "Wv", "Wo", "W1", "W2", "W3")
         stored = {k: (np.ascontiguousarray(weights[k].T) if self.linear_layout and k in projections else np.ascontiguousarray(weights[k]))
                   for k in WEIGHT_NAMES}
@@ -119,17 +119,18 @@ class DecoderBlock:
         return (out, k.contiguous(), v.contiguous()) if with_cache else out
 
     def _rope_row(self, pos):
-        """cos and sin of one position as [1, 1, 1, dim/2] tensors: views of tables in device memory, made for the next
-        power of two of positions at a time (a step's own row costs no trigonometry, no upload and no wait)."""
+        """cos and sin of one position as [1, 1, 1, dim/2] tensors: views of tables in device memory, made for 64 consecutive
+        positions at a time (a step's own row costs no trigonometry, no upload and no wait, and a block that starts at a
+        late position does not pay for those before it)."""
         half = self.dim // 2
         pitch = -(-half // 16) * 16  # rows start on 64 bytes
-        tables = self._rope
-        if tables is None or pos >= tables[0]:
-            rows = max(256, 1 << pos.bit_length())
-            padded = np.zeros((2, rows, pitch), np.float32)
-            padded[0, :, :half], padded[1, :, :half] = rope_tables(rows, self.dim, self.theta)
-            tables = self._rope = (rows, Buffer.from_numpy(padded[0], self.device_id), Buffer.from_numpy(padded[1], self.device_id))
-        return [Tensor.from_buffer(t.view(pos * pitch * 4, half * 4), (1, 1, 1, half), uop.F32) for t in tables[1:]]
+        first, row = pos // 64 * 64, pos % 64
+        tables = self._rope.get(first)
+        if tables is None:
+            padded = np.zeros((2, 64, pitch), np.float32)
+            padded[0, :, :half], padded[1, :, :half] = rope_tables(64, self.dim, self.theta, first)
+            tables = self._rope[first] = [Buffer.from_numpy(t, self.device_id) for t in padded]
+        return [Tensor.from_buffer(t.view(row * pitch * 4, half * 4), (1, 1, 1, half), uop.F32) for t in tables]
 
     def decode_step(self, tokens, past_k, past_v, pos):
         """One new token per sequence against the keys and values of the `pos` tokens before it, the way the reference

@@ -221,7 +221,7 @@ def test_decode_step_over_cached_keys_is_the_last_row_of_a_causal_pass(dev, orac
 
 
 def test_decode_steps_rotate_with_the_blocks_theta(dev):
-    """Two consecutive steps, the second past the first table of 256 positions, the cache fed back: keys rotated as the causal
+    """Two consecutive steps, the second in the next table of rotary rows, the cache fed back: keys rotated as the causal
     pass of a block with the same theta rotates them, and not as one with the default theta does.  Tolerance: a key and the
     causal pass's are the same f32 rotation, rounded to bf16 once, of projections that differ by the order of their sums (a bf16 step)."""
     from morok_amd import decoder, synth, tensor

@@ -796,8 +796,8 @@ def test_kept_intermediates_are_realized_with_the_root(T, shim):
 
 
 def test_decode_step_is_one_realization(T, shim):
-    """The grown keys and values come with the output, and a step's rotary row is a view of tables that grow by powers of
-    two: equal to the row computed for that position alone, with no upload and no wait per step."""
+    """The grown keys and values come with the output, and a step's rotary row is a view of tables of 64
+    positions: equal to the row computed for that position alone, with no upload and no wait per step."""
     from morok_amd import decoder, uop
 
     blk = decoder.DecoderBlock(decoder.synthetic_weights(256, 512, 100, seed=1), 2, 1, 256, 2, 512, linear_layout=True)
@@ -812,6 +812,20 @@ def test_decode_step_is_one_realization(T, shim):
         out.realize()
         assert shim.mrk_shim_syncs() == syncs
         assert k.realize().kernels() == [] and v.realize().kernels() == [] and k.shape == (2, 2, pos + 1, 128)
+
+
+def test_a_late_first_step_makes_the_rotary_rows_around_its_position_alone(T, shim, monkeypatch):
+    """A block that starts at position 4000 does not pay for the rows before it, and two sequences of positions in turn keep both."""
+    from morok_amd import decoder
+
+    blk = decoder.DecoderBlock(decoder.synthetic_weights(256, 512, 100, seed=1), 2, 1, 256, 2, 512, theta=500.0, linear_layout=True)
+    made, whole = [], decoder.rope_tables
+    monkeypatch.setattr(decoder, "rope_tables", lambda seq, *args: made.append(seq) or whole(seq, *args))
+    for pos in (4000, 70, 4001, 71, 4031, 4032, 0):
+        cos, sin = whole(pos + 1, 128, 500.0)
+        got = blk._rope_row(pos)
+        assert np.array_equal(got[0].to_numpy().reshape(-1), cos[pos]) and np.array_equal(got[1].to_numpy().reshape(-1), sin[pos])
+    assert made == [64] * 4
 
 
 def test_failed_schedule_leaves_the_graph_lazy(T, shim):
