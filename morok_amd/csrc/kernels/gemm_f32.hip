@@ -459,6 +459,9 @@ bool gemm_f32_supported(long M, long N, long K) {
 // more so the more K there is per output: 1000000 x 1 x 64 65 us against 128 in tiles of 32, 300 x 3 x 4096 4.2 / 13.7,
 // 64 x 10 x 784 3.1 / 4.9; but 65536 x 5 x 1024 91 / 68, 8192 x 10 x 784 69 / 9.  They go where the estimates are further apart
 // than they are off (1 us on the smallest), inside the sizes they were fitted to.  An addend is a kernel of its own (2.6 us) there.
+// The smallest stay here although a reduction is 0.3 to 0.7 us shorter (up to some 0.9 M multiply-adds, 3 M against a [N, K]
+// operand: 65 x 192 x 64 3.5 us against 3.0, 100 x 29 x 192 3.5 / 2.9): with an addend, where these win, the sums would
+// come in another order than without.
 bool gemm_f32_preferred(long M, long N, long K, bool b_transposed, bool added) {
     if (!gemm_f32_supported(M, N, K)) return false;
     const int tile = tile_size(M, N, K, b_transposed);
