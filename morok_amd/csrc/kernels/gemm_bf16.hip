@@ -38,57 +38,24 @@
 // cannot be padded, is stored with 16-byte stores of 2-byte alignment.  A second instance of the
 // same body with a 128x256 workgroup tile serves shapes that would otherwise leave most compute
 // units idle; a leading batch dimension runs as grid.y.  The kernel at the end of this file, one
-// wave per 32x32 tile straight from global memory, is left for callers that bring no scratch for
-// the padded operands and for unaligned base pointers.
+// wave per 32x32 tile straight from global memory, is left for fewer than eight columns or a K below eight, and for sums in several
+// ranges of K without scratch.  Shapes of up to 256 tiles of 128x256 mostly run on smaller tiles (gemm_mid.hip, route_16bit).
 #include <hip/hip_runtime.h>
 #include <atomic>
 
 #include <cstdint>
 #include <type_traits>
 
+#include "gemm_elem.h"
+#include "gemm_mid.h"
 #include "kernels.h"
 
 namespace mrk::dev {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-// the same in memory where a row of 16-bit (of 32-bit) elements may start on any element
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-typedef f32x4 f32x4_any __attribute__((aligned(4)));
-
-#define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
 
 constexpr int kBM = 256, kBN = 256, kBK = 64;
 constexpr int kBStageSw = kBK * kBN * 2;       // 32768 B per B stage, row pitch 512 B, granule-swizzled
 // (an A stage is rows x 128 B, chunk-swizzled: 32768 B for the 256-row tile, which with two A
 // and three B stages fills all 160 KB of the LDS)
-
-// Maps the linear workgroup id to an output tile so that the workgroups that land on one
-// XCD (ids congruent mod 8 share an L2) cover a compact block of tiles: first regroup
-// ids by XCD, then walk tiles in column groups of 4 tile-rows.
-__device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int* tm, int* tn) {
-    const int total = tiles_m * tiles_n;
-    const int per = total >> 3, rem = total & 7;
-    const int xcd = bid & 7, idx = bid >> 3;
-    int id = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    if (total < 8) id = bid;
-    constexpr int kGroup = 4;
-    const int group_sz = kGroup * tiles_n;
-    const int g = id / group_sz;
-    const int first_m = g * kGroup;
-    const int gm = (tiles_m - first_m) < kGroup ? (tiles_m - first_m) : kGroup;
-    const int in = id - g * group_sz;
-    *tm = first_m + in % gm;
-    *tn = in / gm;
-}
-
-// Sixteen zero bytes in device memory: where the copies of a partial last K step point the
-// lanes whose k lies beyond K.
-__device__ __attribute__((aligned(16))) const unsigned g_zero16[4] = {0u, 0u, 0u, 0u};
 
 // kAny: K is not a multiple of 64, or N not of 8.  The copies of a partial last K step use
 // per-lane 64-bit addresses so that chunks beyond K can be redirected to g_zero16: zero
@@ -127,24 +94,6 @@ __device__ __attribute__((aligned(16))) const unsigned g_zero16[4] = {0u, 0u, 0u
 // schedule/src/optimizer/renderer.rs:724-733).  Both are 16-bit elements, so copies, LDS layout,
 // fragment reads and stores are the same bytes; only the matrix instruction and the conversion of
 // the f32 accumulators differ.  The element pointers stay typed as 16-bit carriers.
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-template <bool kF16>
-__device__ __forceinline__ bf16x4 round_to_elem(const f32x4& v) {
-    if constexpr (kF16) return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, f16x4));
-    else return __builtin_convertvector(v, bf16x4);
-}
-// the sum of two chunks of eight 16-bit elements, taken in f32 and rounded once
-template <bool kF16>
-__device__ __forceinline__ u32x4 add_elems(const u32x4& a, const u32x4& b) {
-    if constexpr (kF16) {
-        const f32x8 s = __builtin_convertvector(__builtin_bit_cast(f16x8, a), f32x8) + __builtin_convertvector(__builtin_bit_cast(f16x8, b), f32x8);
-        return __builtin_bit_cast(u32x4, __builtin_convertvector(s, f16x8));
-    } else {
-        const f32x8 s = __builtin_convertvector(__builtin_bit_cast(bf16x8, a), f32x8) + __builtin_convertvector(__builtin_bit_cast(bf16x8, b), f32x8);
-        return __builtin_bit_cast(u32x4, __builtin_convertvector(s, bf16x8));
-    }
-}
 //
 // kRope (256-row tile only): the product of a packed projection whose first `split` columns are
 // attention heads of 128 columns each (q | k of a fused QKV product).  The epilogue applies the
@@ -1040,11 +989,6 @@ SplitPlan plan_split_k(long M, long N, long K, long batch) {
     if (p.splits < 2) p.splits = 1;
     return p;
 }
-size_t split_k_bytes(long M, long N, long K, long batch) {
-    const SplitPlan p = plan_split_k(M, N, K, batch);
-    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
-}
-
 // shapes the tiled kernels address (32-bit offsets inside a tile, and from one tile of B to the next 64 rows on: the limits
 // hold for the row pitches, which round N and K up to 8); without scratch the operands' rows have to be whole
 // 16-byte chunks, see operand_padding
@@ -1066,9 +1010,8 @@ struct OperandPadding {
 };
 OperandPadding operand_padding(long M, long N, long K, long batch, bool b_transposed) {
     OperandPadding o;
-    // A small [K, N] product asks for no scratch: it is one launch of at most one wave per SIMD and a few steps of K on the
-    // kernel that needs no padding (6.4-6.9 us from 33 x 7 x 19 to 256 x 255 x 63), two or three launches here (12-13 us).
-    // Which of the others run there although there is scratch: unpadded_faster.
+    // A small [K, N] product asks for no scratch: it is one launch of a few steps of K on kernels that need no padding
+    // (4.6-6.9 us from 33 x 7 x 19 to 256 x 255 x 63), two or three launches here (12-13 us).
     if (!b_transposed && (K % 8 || N % 8) && K <= 128 && ((M + 31) / 32) * ((N + 31) / 32) * batch <= 1024) return o;
     const long row_b = b_transposed ? K : N, rows_b = batch * (b_transposed ? N : K);
     o.a = K % 8 != 0;
@@ -1079,20 +1022,75 @@ OperandPadding operand_padding(long M, long N, long K, long batch, bool b_transp
     if (o.b) o.b_bytes = ((size_t)rows_b * o.ldb * 2 + 255) / 256 * 256;
     return o;
 }
-// Whether a product that would have operands padded runs faster on the kernel that reads them as they are (also where there is
-// scratch): short K, or few rows against a wide weight.  Both times in us, from 445 shapes of 1 to 4096 rows, 9 to 50257
-// columns and K from 65 to 1032: one wave per 32 x 32 tile, four per CU at once (`rounds`; rows that are not there are not
-// loaded; tall products read B again; lanes along K of an [N, K] operand share fewer lines) against the tiles with their one
-// or two padding launches, whose traffic the last-level cache takes a part of.  On either side of the line the chosen kernel
-// was at most 20 % behind the other: 32 x 33 x 392 12.1 / 13.3, 256 x 255 x 257 11.0 / 15.2, 256 x 255 x 392 19.6 / 15.0,
-// 4 x 50257 x 769 29.4 / 40.9, 64 x 50257 x 513 74 / 33; [N, K] 256 x 255 x 129 9.6 / 13.8, 300 x 300 x 300 23.0 / 14.9.
-bool unpadded_faster(long M, long N, long K, long batch, const OperandPadding& pad, bool b_transposed) {
-    if (!pad.a && !pad.b) return false;
-    const double rounds = (double)(((M + 31) / 32) * ((N + 31) / 32) * batch) / 1024.0;
-    const double wait = rounds <= 1.0 ? 1.0 : M <= 4 ? 0.5 + 0.5 * rounds : M <= 128 && batch == 1 ? rounds : rounds + 1.25;
-    const double unpadded = 2.0 + K * wait * (M <= 4 ? 0.029 : M <= 16 ? 0.033 : 0.040) * (b_transposed ? 1.4 : 1.0);
-    const double padded = 8.5 + 3.5 * (pad.a + pad.b) + 6.0 * (double)batch * ((pad.a ? (double)M * K : 0.0) + (pad.b ? (double)K * N : 0.0)) / 8.5e6;
-    return unpadded < padded;
+// Which kernels a product of more rows than the streaming kernels take runs on: small tiles (gemm_mid.hip), several to a
+// compute unit and odd rows read as they are, or the 128- and 256-row tiles of this file.  A matter of the shape alone (not of the
+// layout of B, of scratch or of bases), and either way with the sums in ranges of kt_per_split steps of K: the same bits on every kernel.
+struct Route {
+    bool mid = false;
+    MidPlan plan;  // (mid: which tile)
+    long splits = 1, kt_per_split = 0;
+};
+// Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both,
+// fitted to 170 shapes (tiles of 128 x 256: 4.0 + 0.57 per step of K, 10 % off; split along K 7 %), decide, with a margin for their errors:
+// chosen so, no shape of the 300 timed lost more than 4 % where operands are whole chunks, and they gained 20 % on
+// average.  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
+Route choose_route(long M, long N, long K, long batch) {
+    Route r;
+    const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
+    r.splits = sp.splits, r.kt_per_split = sp.kt_per_split;
+    const long tiles = ((M + 127) / 128) * ((N + 255) / 256) * batch, kt = (K + 63) / 64;
+    if (tiles > 256) return r;
+    const bool whole = N % 8 == 0 && K % 8 == 0;
+    r.plan = plan_mid(M, N, K, batch, whole);
+    if (r.plan.tile < 0) return r;
+    const double operands = 2.0 * batch * ((double)M * K + (double)N * K + (double)M * N) * 1e-6;
+    double us = sp.splits > 1 ? 0.70 * sp.kt_per_split : 0.57 * kt;
+    if (operands / (sp.splits > 1 ? 8.3 : 7.0) > us) us = operands / (sp.splits > 1 ? 8.3 : 7.0);
+    us += sp.splits > 1 ? 8.2 + 0.34 * 4e-6 * sp.splits * batch * M * N : 4.0;
+    if (!whole) us += (K % 8 ? 7.0 : 3.5) + 0.7e-6 * batch * ((K % 8 ? (double)M * K : 0.0) + (double)K * N);
+    r.mid = r.plan.us < us * (!whole || sp.splits > 1 ? 0.85 : 0.95);
+    if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
+    return r;
+}
+// The estimates take about 2 us, a launch 3: each thread keeps the routes of the last shapes it ran (a pure function of the shape).
+Route route_16bit(long M, long N, long K, long batch) {
+    struct Entry {
+        long M = 0, N = 0, K = 0, batch = 0;
+        Route r;
+    };
+    static thread_local Entry kept[32];
+    const unsigned long long h = (unsigned long long)M * 0x9e3779b97f4a7c15ull ^ (unsigned long long)N * 0xc2b2ae3d27d4eb4full ^
+                                 (unsigned long long)K * 0x165667b19e3779f9ull ^ (unsigned long long)batch * 0x27d4eb2f165667c5ull;
+    Entry& e = kept[(h >> 40) % 32];
+    if (e.M != M || e.N != N || e.K != K || e.batch != batch) {
+        e.r = choose_route(M, N, K, batch);
+        e.M = M, e.N = N, e.K = K, e.batch = batch;
+    }
+    return e.r;
+}
+// One pass of 256-row tiles, in us (tiles of 256 x 256: fitted to 39 shapes, 8 % off)
+double tiles256_us(long M, long N, long K) {
+    const double rounds = (double)((((M + 255) / 256) * ((N + 255) / 256) + 255) / 256), mb = 2e-6 * ((double)M * K + (double)N * K + (double)M * N);
+    const double us = rounds * (1.02 * ((K + 63) / 64) + 5.8);
+    return 4.8 + (us > mb / 4.0 ? us : mb / 4.0);
+}
+// The gated (N = 2 F) and the rotary product: small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
+// two rounds of 256, against 860 of 128 x 128).
+MidPlan paired_plan(long M, long N, long K) {
+    MidPlan p = plan_mid(M, N, K, 1, true, false);
+    // (the kernel addresses B's columns from its first with 32-bit offsets)
+    if (p.tile >= 0 && ((double)N * K >= 1e9 || p.us >= 0.95 * tiles256_us(M, N, K))) p.tile = -1;
+    return p;
+}
+// f32 partial results of a product whose K is split
+size_t partial_bytes(const Route& r, long M, long N, long batch) { return r.splits > 1 ? (size_t)r.splits * batch * M * N * sizeof(float) : 0; }
+// Scratch a route takes: padded operands in front of the partial results (small tiles read odd operands as they are, but what a caller
+// has to bring for them is a matter of the shape: no less than the copies).
+size_t route_bytes(long M, long N, long K, long batch, bool b_transposed) {
+    const OperandPadding pad = operand_padding(M, N, K, batch, b_transposed);
+    const Route r = route_16bit(M, N, K, batch);
+    const size_t copies = pad.a_bytes + pad.b_bytes, partial = partial_bytes(r, M, N, batch);
+    return r.mid ? (copies > partial ? copies : partial) : copies + partial;
 }
 }  // namespace
 
@@ -1103,9 +1101,7 @@ size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch) {
     if (gemm_kn_skinny_plan(M, N, K, batch, &ks, &kr)) return (size_t)ks * M * N * sizeof(float);
     if (gemm_kn_rows_plan(M, N, K, batch, &ks, &kr)) return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
     if (!tile_addressable(M, N, K, batch)) return 0;
-    const OperandPadding pad = operand_padding(M, N, K, batch, false);
-    if (!pad.lda) return 0;
-    return pad.a_bytes + pad.b_bytes + split_k_bytes(M, N, K, batch);
+    return operand_padding(M, N, K, batch, false).lda ? route_bytes(M, N, K, batch, false) : 0;
 }
 
 int gemm_bf16_static_workspace_init(int device_id) {
@@ -1161,8 +1157,7 @@ size_t gemm_bf16_nt_workspace_bytes(long M, long N, long K, long batch) {
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
     if (gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch)) return 0;  // streamed in one launch
     if (!tile_addressable(M, N, K, batch)) return 0;
-    const OperandPadding pad = operand_padding(M, N, K, batch, true);
-    return pad.a_bytes + pad.b_bytes + split_k_bytes(M, N, K, batch);
+    return route_bytes(M, N, K, batch, true);
 }
 
 int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
@@ -1195,6 +1190,15 @@ bool gemm_bf16_swiglu_supported(long M, long F, long K, bool b_transposed) {
     return tm * tn <= 0x7fffffffL;
 }
 
+bool gemm_bf16_separate_preferred(long M, long N, long K) {
+    if (M <= 64 && K >= 512) return true;  // (the programs a block over a few tokens consists of stay as they are)
+    const Route r = route_16bit(M, N, K, 1);
+    if (!r.mid) return r.splits > 1;  // (as large tiles: the fused forms are theirs)
+    const MidPlan fused = plan_mid(M, N, K, 1, true, false);
+    const double large = tiles256_us(M, N, K), best = fused.tile >= 0 && fused.us < large ? fused.us : large;
+    return r.plan.us + 2.7 + 4e-6 * M * N / 5.0 < best;
+}
+
 int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C, long M, long F, long K, bool b_transposed) {
     using namespace mrk::dev;
     if (M <= 0 || F <= 0) return 0;
@@ -1204,6 +1208,8 @@ int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C,
     if (b_transposed && gemm_nt_swiglu_streamed(M, F, K)) return launch_gemm_nt_swiglu_streamed(stream, A, B, C, M, F, K);
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
+    const MidPlan mid = paired_plan(M, 2 * F, K);
+    if (mid.tile >= 0) return launch_gemm_mid_paired(s, mid, A, B, C, M, 2 * F, K, b_transposed, nullptr);
     const long tn = (F + 127) / 128, tm = (M + kBM - 1) / kBM;
     const dim3 grid((unsigned)(tm * tn), 1);
     const __bf16* a = static_cast<const __bf16*>(A);
@@ -1231,6 +1237,11 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
                           reinterpret_cast<uintptr_t>(C_rest) | reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin);
     if (all % 16 || reinterpret_cast<uintptr_t>(cos) % 32 || reinterpret_cast<uintptr_t>(sin) % 32) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
+    const MidPlan mid = paired_plan(M, N, K);
+    if (mid.tile >= 0) {
+        const MidRope angles{static_cast<const float*>(cos), static_cast<const float*>(sin), C_rest, (int)seq, (int)split};
+        return launch_gemm_mid_paired(static_cast<hipStream_t>(stream), mid, A, B, C_rot, M, N, K, b_transposed, &angles);
+    }
     const long tm = (M + kBM - 1) / kBM, tn = (N + kBN - 1) / kBN;
     RopeEpilogue rope{static_cast<const float*>(cos), static_cast<const float*>(sin), static_cast<__bf16*>(C_rest), (int)seq, (int)split};
     auto kernel = b_transposed ? gemm_bf16_nt_tile256_rope : gemm_bf16_tile256_rope;
@@ -1240,11 +1251,21 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
 }
 
 namespace {
+// C = the sums over `splits` partial results W[splits][batch][M][N], with the addend
+void reduce_partials(hipStream_t s, const float* w, __bf16* c, long M, long N, long batch, long splits, bool f16, const __bf16* add, bool add_is_row) {
+    using namespace mrk::dev;
+    const long total = batch * M * N;
+    const bool each = total % 8 != 0 || (add_is_row && N % 8 != 0) || (reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(add)) % 16;
+    auto reduce_kernel = f16 ? (each ? gemm_splitk_reduce<true, true> : gemm_splitk_reduce<true, false>)
+                             : (each ? gemm_splitk_reduce<false, true> : gemm_splitk_reduce<false, false>);
+    reduce_kernel<<<(unsigned)(((each ? total : total / 8) + 255) / 256), 256, 0, s>>>(w, c, total, (int)splits, add, add_is_row ? N : 0);
+}
+
 // Output tiles over the chip: the K loop spread over ranges when the shape has a split plan and the caller brought the
 // scratch for the partial results, else one pass of 256-row or 128-row tiles.  Operands aligned to 16 bytes; those whose
 // rows are no whole 16-byte chunks are padded into the scratch first.  False when the scratch for that is missing.
 bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
-                  size_t workspace_bytes, bool b_transposed, bool f16, const __bf16* add, bool add_is_row) {
+                  size_t workspace_bytes, bool b_transposed, bool f16, const __bf16* add, bool add_is_row, const Route& route) {
     using namespace mrk::dev;
     const OperandPadding pad = operand_padding(M, N, K, batch, b_transposed);
     const __bf16 *a = static_cast<const __bf16*>(A), *b = static_cast<const __bf16*>(B);
@@ -1269,16 +1290,12 @@ bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, 
     const long tn = (N + kBN - 1) / kBN, tm128 = (M + 127) / 128;
 #define MRK_PICK(stem) (f16 ? (b_transposed ? (any ? gemm_f16_nt_##stem##_any : gemm_f16_nt_##stem) : (any ? gemm_f16_##stem##_any : gemm_f16_##stem)) \
                             : (b_transposed ? (any ? gemm_bf16_nt_##stem##_any : gemm_bf16_nt_##stem) : (any ? gemm_bf16_##stem##_any : gemm_bf16_##stem)))
-    const SplitPlan sp = variant == 0 || variant == 5 ? plan_split_k(M, N, K, batch) : SplitPlan();
-    if (sp.splits > 1 && ws_left >= (size_t)sp.splits * batch * M * N * sizeof(float) && batch * sp.splits <= 65535) {
+    const size_t partial = variant == 0 || variant == 5 ? partial_bytes(route, M, N, batch) : 0;
+    if (partial && ws_left >= partial && batch * route.splits <= 65535) {
         float* w = reinterpret_cast<float*>(ws);
-        MRK_PICK(tile128_splitk)<<<dim3((unsigned)(tm128 * tn), (unsigned)batch, (unsigned)sp.splits), 256, 0, s>>>(
-            a, b, w, (int)M, (int)N, (int)K, (int)tm128, (int)tn, (int)sp.kt_per_split, pitch_a, pitch_b);
-        const long total = batch * M * N;
-        const bool each = total % 8 != 0 || (add_is_row && N % 8 != 0);
-        auto reduce_kernel = f16 ? (each ? gemm_splitk_reduce<true, true> : gemm_splitk_reduce<true, false>)
-                                 : (each ? gemm_splitk_reduce<false, true> : gemm_splitk_reduce<false, false>);
-        reduce_kernel<<<(unsigned)(((each ? total : total / 8) + 255) / 256), 256, 0, s>>>(w, c, total, (int)sp.splits, add, add_is_row ? N : 0);
+        MRK_PICK(tile128_splitk)<<<dim3((unsigned)(tm128 * tn), (unsigned)batch, (unsigned)route.splits), 256, 0, s>>>(
+            a, b, w, (int)M, (int)N, (int)K, (int)tm128, (int)tn, (int)route.kt_per_split, pitch_a, pitch_b);
+        reduce_partials(s, w, c, M, N, batch, route.splits, f16, add, add_is_row);
         return true;
     }
     // the 128-row tile when all its workgroups are resident at once (at most one per compute unit): twice the
@@ -1299,15 +1316,33 @@ bool launch_tiles(hipStream_t s, const void* A, const void* B, void* C, long M, 
 }  // namespace
 
 namespace {
-// The kernel that reads its operands as they are, whatever their rows and bases are aligned to.
-int launch_unpadded(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, long batch, bool b_transposed, bool f16,
-                    const __bf16* add, bool add_is_row) {
+// Small tiles, in the route's ranges of K: odd rows and bases are read as they are (`chunks`: rows of whole 16-byte chunks on 16-byte
+// bases, in this layout).  A negative answer: not covered (K or N below one chunk, or no scratch for the partial results).
+int launch_mid(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, long batch, void* workspace, size_t workspace_bytes,
+               bool b_transposed, bool f16, const __bf16* add, bool add_is_row, const Route& route, bool chunks) {
+    MidPlan p = route.mid ? route.plan : plan_mid(M, N, K, batch, false);
+    if (p.tile < 0) return -1;
+    if (!route.mid || (!chunks && N % 8 == 0 && K % 8 == 0)) p.tile = kMidUnaligned;
+    else if (chunks && p.tile == kMidUnaligned) p.tile = kMidSmallest;  // (odd rows of C alone)
+    p.splits = route.splits, p.kt_per_split = route.kt_per_split;
+    const size_t partial = partial_bytes(route, M, N, batch);
+    if (partial && (!workspace || workspace_bytes < partial || reinterpret_cast<uintptr_t>(workspace) % 16 || batch * p.splits > 65535)) return -1;
+    int rc = launch_gemm_mid(s, p, A, B, C, static_cast<float*>(workspace), add, add_is_row ? 0 : N, M, N, K, batch, b_transposed, f16);
+    if (rc == 0 && partial) {
+        reduce_partials(s, static_cast<float*>(workspace), static_cast<__bf16*>(C), M, N, batch, p.splits, f16, add, add_is_row);
+        rc = (int)hipGetLastError();
+    }
+    return rc;
+}
+
+// One wave per 32 x 32 tile, any shape, no scratch.
+int launch_generic(hipStream_t s, const void* A, const void* B, void* C, long M, long N, long K, long batch, bool b_transposed, bool f16,
+                   const __bf16* add, bool add_is_row, const Route& route) {
     using namespace mrk::dev;
     const long tn = (N + 31) / 32, total = ((M + 31) / 32) * tn, blocks = (total + 3) / 4;
     if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
-    // (the K ranges the tiled kernels would take: the result does not depend on whether there was scratch for them)
-    const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
-    const int k_range = sp.splits > 1 ? (int)sp.kt_per_split * kBK : 0x7fffffff;
+    // (the K ranges the other kernels take: the result does not depend on whether there was scratch for them)
+    const int k_range = route.splits > 1 ? (int)route.kt_per_split * kBK : 0x7fffffff;
     auto kernel = f16 ? (b_transposed ? gemm_bf16_generic<true, true> : gemm_bf16_generic<true, false>)
                       : (b_transposed ? gemm_bf16_generic<false, true> : gemm_bf16_generic<false, false>);
     kernel<<<dim3((unsigned)blocks, (unsigned)batch), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B),
@@ -1330,16 +1365,13 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
     const bool aligned = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16) == 0;
-    OperandPadding pad;
-    if (K > 0) pad = operand_padding(M, N, K, batch, b_transposed);
-    const bool unpadded = (variant == 0 || variant == 5) && aligned && unpadded_faster(M, N, K, batch, pad, b_transposed);
+    const bool choose = variant == 0 || variant == 5;  // (3 / 4 force a tile size, 2 the any-shape kernel)
     if (b_transposed) {
-        // B given as Bt[N, K]: the streaming or the tiled kernels, the unpadded one for small odd shapes, or nothing
-        // (variant 3 / 4 force a tile size)
+        // B given as Bt[N, K]: the streaming or the tiled kernels, or nothing
         if (!aligned || !gemm_bf16_nt_padded_supported(M, N, K, batch)) return (int)hipErrorInvalidValue;
         // up to 64 rows: one pass over the weight streams it faster than any tile (one or two rows on the
         // vector ALUs, more on the matrix pipes with 16-row blocks staged through LDS)
-        if (variant == 0 || variant == 5 || !tiled_shape(M, N, K, batch)) {
+        if (choose || !tiled_shape(M, N, K, batch)) {
             if (add) {
                 if (gemm_nt_bias_streamed(M, N, K, batch)) return launch_gemm_nt_bias_streamed(stream, A, B, add, C, M, N, K, f16, add_is_row);
             } else {
@@ -1348,29 +1380,54 @@ int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long 
             }
         }
         if (!tile_addressable(M, N, K, batch)) return (int)hipErrorInvalidValue;
-        if (!unpadded && !launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, true, f16, addp, add_is_row))
+        const OperandPadding pad = operand_padding(M, N, K, batch, true);
+        const Route route = route_16bit(M, N, K, batch);
+        // (odd operands want scratch for their copies, whichever kernel runs)
+        if (pad.a_bytes + pad.b_bytes > (workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 ? workspace_bytes : 0)) return (int)hipErrorInvalidValue;
+        if (choose && route.mid) {
+            const int rc = launch_mid(s, A, B, C, M, N, K, batch, workspace, workspace_bytes, true, f16, addp, add_is_row, route, K % 8 == 0);
+            if (rc >= 0) return rc;
+        }
+        if (!launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, true, f16, addp, add_is_row, route))
             return (int)hipErrorInvalidValue;
-        if (!unpadded) return (int)hipGetLastError();
-        return launch_unpadded(s, A, B, C, M, N, K, batch, true, f16, addp, add_is_row);
+        return (int)hipGetLastError();
     }
     // up to 16 rows: one streaming pass over the weight into f32 partial sums, then their sum
     {
         long ks = 0, kr = 0;
-        if ((variant == 0 || variant == 5) && aligned && gemm_kn_skinny_plan(M, N, K, batch, &ks, &kr) && workspace &&
+        if (choose && aligned && gemm_kn_skinny_plan(M, N, K, batch, &ks, &kr) && workspace &&
             workspace_bytes >= (size_t)ks * M * N * sizeof(float) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
             return launch_gemm_kn_skinny(stream, A, B, C, workspace, M, N, K, ks, kr, f16, add, add_is_row);
         }
-        if ((variant == 0 || variant == 5) && aligned && gemm_kn_rows_plan(M, N, K, batch, &ks, &kr) &&
+        if (choose && aligned && gemm_kn_rows_plan(M, N, K, batch, &ks, &kr) &&
             (ks == 1 || (workspace && workspace_bytes >= (size_t)ks * M * N * sizeof(float) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0))) {
             return launch_gemm_kn_rows(stream, A, B, C, workspace, M, N, K, ks, kr, f16, add, add_is_row);
         }
     }
-    if (variant != 2 && aligned && tile_addressable(M, N, K, batch) && !unpadded &&
-        launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, false, f16, addp, add_is_row))
-        return (int)hipGetLastError();
+    OperandPadding pad;
+    Route route;
+    if (K > 0) {
+        pad = operand_padding(M, N, K, batch, false);
+        route = route_16bit(M, N, K, batch);
+    }
     // (an addend is taken where there is scratch for the tiles, whichever kernel runs)
-    if (add && !(unpadded && pad.lda)) return (int)hipErrorInvalidValue;
-    return launch_unpadded(s, A, B, C, M, N, K, batch, false, f16, addp, add_is_row);
+    if (add && (!aligned || variant == 2 || !tile_addressable(M, N, K, batch) || !pad.lda ||
+                pad.a_bytes + pad.b_bytes > (workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 ? workspace_bytes : 0)))
+        return (int)hipErrorInvalidValue;
+    const bool whole = N % 8 == 0 && K % 8 == 0;
+    if (choose && K > 0 && route.mid) {
+        const int rc = launch_mid(s, A, B, C, M, N, K, batch, workspace, workspace_bytes, false, f16, addp, add_is_row, route, aligned && whole);
+        if (rc >= 0) return rc;
+    }
+    if (variant != 2 && aligned && tile_addressable(M, N, K, batch) &&
+        launch_tiles(s, A, B, C, M, N, K, variant, batch, workspace, workspace_bytes, false, f16, addp, add_is_row, route))
+        return (int)hipGetLastError();
+    // no scratch for padded operands, or unaligned bases
+    if (choose && K > 0) {
+        const int rc = launch_mid(s, A, B, C, M, N, K, batch, workspace, workspace_bytes, false, f16, addp, add_is_row, route, false);
+        if (rc >= 0) return rc;
+    }
+    return launch_generic(s, A, B, C, M, N, K, batch, false, f16, addp, add_is_row, route);
 }
 
 int launch_gemm_bf16(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,

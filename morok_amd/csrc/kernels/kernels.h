@@ -91,6 +91,9 @@ int launch_gemm_nt_bias_streamed(void* stream, const void* A, const void* Bt, co
 // epilogue, so that the [M, 2F] product never reaches memory.  F and K multiples of 8.
 // b_transposed: W is stored as [2F, K] (the rows of Wg^T, then the rows of Wu^T).
 bool gemm_bf16_swiglu_supported(long M, long F, long K, bool b_transposed = false);
+// Whether a product that could take the gated or the rotary epilogue (N all of its columns) runs faster as a product spread along K
+// and a kernel of its own for the rest: by estimates of both, and always with up to 64 rows from K = 512 on.
+bool gemm_bf16_separate_preferred(long M, long N, long K);
 int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c, long M, long F, long K, bool b_transposed = false);
 // A packed projection whose first `split` columns are attention heads of 128 columns (q | k of a
 // fused QKV product, split a multiple of 256) with the rotary embedding applied in the product

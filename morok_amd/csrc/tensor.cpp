@@ -1432,7 +1432,7 @@ struct Scheduler {
     // the gate: 70 us against 30 us for the streamed product plus an elementwise kernel), so they are not matched.
     bool spread_or_streamed(const TensorNode* mm, int64_t M, int64_t N, int64_t K, int64_t batch) const {
         long splits = 0, per = 0;
-        if (gemm_bf16_workspace_bytes(M, N, K, batch) || gemm_kn_rows_plan(M, N, K, batch, &splits, &per)) return true;
+        if (gemm_bf16_separate_preferred(M, N, K) || gemm_kn_rows_plan(M, N, K, batch, &splits, &per)) return true;
         return transposed_weight(mm) && (gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch));
     }
     // x + (a @ w) in bf16, f16 or f32 where nothing else reads the product: the product kernel adds x in its
