@@ -108,6 +108,34 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                       }));
         return kOk;
     }
+    if (k == "concat") {
+        // {outer0, outer1, then per part: pieces of 16 bytes a row, pieces a run, bytes from run to run, bytes per outer0, per outer1,
+        // byte offset}; buffers {out, a source per part}
+        if (nparams < 8 || (nparams - 2) % 6 || (nparams - 2) / 6 > static_cast<size_t>(kConcatParts))
+            return failf(kInvalidArgument, "concat: 2 parameters and 6 for each of up to %d parts, got %zu", kConcatParts, nparams);
+        const size_t parts = (nparams - 2) / 6;
+        int64_t row = 0;
+        bool ok = p[0] > 0 && p[1] > 0 && p[0] <= 0x7fffffff / p[1];
+        for (size_t i = 0; i < parts; i++) {
+            const int64_t* q = &p[2 + 6 * i];
+            ok = ok && q[0] > 0 && q[0] <= 0x7fffffff && q[1] > 0 && q[0] % q[1] == 0 && q[2] >= 0 && q[3] >= 0 && q[4] >= 0 && q[5] >= 0;
+            row += ok ? q[0] : 0;
+        }
+        if (!ok) return fail(kInvalidArgument, "concat: extents have to be positive, runs to divide their part, strides and offsets not negative");
+        const std::string name = "concat_" + std::to_string(p[0] * p[1]) + "x" + std::to_string(row * 16) + "_" + std::to_string(parts);
+        out->reset(new BuiltinProgram(device_id, stream, name, 1 + parts, p, [parts](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+            ConcatShape c{};
+            c.parts = static_cast<int>(parts);
+            c.outer0 = q[0], c.outer1 = q[1];
+            for (size_t i = 0; i < parts; i++) {
+                const int64_t* w = &q[2 + 6 * i];
+                c.part[i] = {static_cast<const char*>(b[1 + i]) + w[5], w[0], w[1], w[2], w[3], w[4]};
+                c.row_pieces += w[0];
+            }
+            return launch_concat(s, b[0], c);
+        }));
+        return kOk;
+    }
     if (k == "softmax_bf16" || k == "softmax_f16") {
         MRK_TRY(need(2));
         if (!softmax_half_supported(p[0], p[1])) return fail(kInvalidArgument, k + ": rows of 1 to 65536 elements");

@@ -184,6 +184,21 @@ int launch_fill(void* stream, void* out, size_t n, int dtype, int mode, unsigned
 int launch_fill_randint(void* stream, void* out, size_t n, unsigned long long seed, unsigned long long tensor_id,
                         int high);
 
+// out [outer0, outer1, row_pieces * 16 bytes] = the parts side by side in every row.  A part's row (o0, o1) starts at
+// src + o0 * stride0 + o1 * stride1 and is `pieces` of 16 bytes, in runs of `run` (which divides pieces) `stride` bytes apart;
+// any alignment.
+constexpr int kConcatParts = 4;
+struct ConcatPart {
+    const char* src;
+    long long pieces, run, stride, stride0, stride1;
+};
+struct ConcatShape {
+    int parts;
+    long long outer0, outer1, row_pieces;
+    ConcatPart part[kConcatParts];
+};
+int launch_concat(void* stream, void* out, const ConcatShape& shape);
+
 // Streaming device-to-device copy kernel (bytes % 16 == 0): traffic-counter calibration.
 int launch_copy(void* stream, const void* in, void* out, size_t bytes);
 

@@ -1760,6 +1760,11 @@ struct Scheduler {
             std::vector<int64_t> out_strides;
             if (TensorNode* att = attention_under(n, &out_strides)) return materialize_attention(att, n, out_strides);
         }
+        {
+            std::vector<int64_t> params;
+            std::vector<TensorNode*> bases;
+            if (concat_of_views(n, &params, &bases)) return materialize_concat(n, params, bases);
+        }
         if (generated_tc(n)) return materialize_generated_tc(n);
         // a reshape of materialised data is the same bytes, and so is making it contiguous
         if (n->kind == TKind::Reshape || n->kind == TKind::Contiguous) {
@@ -1841,6 +1846,84 @@ struct Scheduler {
             if (beam > 0 && !dry) return beam_generated(n, max_numel, beam);
         }
         return n->kind == TKind::Reduce ? gen_reduce(n, max_numel) : gen_elementwise(n, max_numel);
+    }
+
+    // A cat (made contiguous, or wanted in memory itself) of two to four tensors that are, or will be, in memory, or views of such:
+    // the parameters of the copy kernel, whose extents are launch arguments, and the tensors it reads.  Everything behind the
+    // cat axis has to be one run, a part's runs (or the part of a row that they make up) whole 16-byte pieces, the axes in front to
+    // fold into two, and an output row to fill a workgroup.  Other cats are index arithmetic in a generated kernel.
+    bool concat_of_views(TensorNode* n, std::vector<int64_t>* params, std::vector<TensorNode*>* bases) const {
+        const TensorNode* cat = n->kind == TKind::Contiguous && n->hint == HintKind::None ? n->src[0].get() : n;
+        if (!g_fusion || beam > 0 || cat->buffer || cat->kind != TKind::Cat || cat->hint != HintKind::None || cat->dtype != n->dtype) return false;
+        if (cat->src.size() < 2 || cat->src.size() > static_cast<size_t>(kConcatParts) || cat->numel() == 0) return false;
+        const size_t axis = static_cast<size_t>(cat->arg[0]), nd = cat->shape.size();
+        const int64_t es = static_cast<int64_t>(scalar_size(n->dtype));
+        int64_t inner = es, row = 0;  // bytes behind the cat axis
+        for (size_t a = axis + 1; a < nd; a++) inner *= cat->shape[a];
+        row = inner * cat->shape[axis];
+        if (row < 256 * 16) return false;
+        struct Part {
+            StridedView v;
+            std::vector<int64_t> st;  // of the axes in front, extents of 1 left out
+        };
+        std::vector<Part> parts(cat->src.size());
+        std::vector<int64_t> outer;
+        for (size_t a = 0; a < axis; a++)
+            if (cat->shape[a] != 1) outer.push_back(cat->shape[a]);
+        for (size_t i = 0; i < parts.size(); i++) {
+            TensorNode* s = cat->src[i].get();
+            StridedView& v = parts[i].v;
+            if (s->dtype != n->dtype || s->numel() == 0 || !strided_view(s, &v)) return false;
+            if (!v.base->buffer && !is_boundary_kind(v.base) && !fusable(v.base)) return false;
+            int64_t run = 1;
+            for (size_t a = nd; a-- > axis + 1;) {
+                if (s->shape[a] != 1 && v.strides[a] != run) return false;
+                run *= s->shape[a];
+            }
+            for (size_t a = 0; a <= axis; a++)
+                if (s->shape[a] != 1 && v.strides[a] < 0) return false;
+            for (size_t a = 0; a < axis; a++)
+                if (cat->shape[a] != 1) parts[i].st.push_back(v.strides[a]);
+        }
+        // neighbouring axes that are one axis in every part
+        for (size_t a = 0; a + 1 < outer.size();) {
+            bool one = true;
+            for (const Part& p : parts) one = one && p.st[a] == p.st[a + 1] * outer[a + 1];
+            if (!one) {
+                a++;
+                continue;
+            }
+            outer[a + 1] *= outer[a];
+            outer.erase(outer.begin() + a);
+            for (Part& p : parts) p.st.erase(p.st.begin() + a);
+        }
+        if (outer.size() > 2) return false;
+        while (outer.size() < 2) {
+            outer.insert(outer.begin(), 1);
+            for (Part& p : parts) p.st.insert(p.st.begin(), 0);
+        }
+        if (outer[0] * outer[1] > 0x7fffffff) return false;
+        params->assign(outer.begin(), outer.end());
+        for (size_t i = 0; i < parts.size(); i++) {
+            const TensorNode* s = cat->src[i].get();
+            const int64_t len = s->shape[axis], st = parts[i].v.strides[axis] * es;
+            const bool whole = len == 1 || st == inner;
+            if (len * inner % 16 || (!whole && inner % 16) || len * inner / 16 > 0x7fffffff) return false;
+            const int64_t pieces = len * inner / 16;
+            params->insert(params->end(), {pieces, whole ? pieces : inner / 16, whole ? 0 : st, parts[i].st[0] * es, parts[i].st[1] * es, parts[i].v.offset * es});
+            bases->push_back(parts[i].v.base);
+        }
+        return true;
+    }
+    int materialize_concat(TensorNode* n, const std::vector<int64_t>& params, const std::vector<TensorNode*>& bases) {
+        for (TensorNode* b : bases) MRK_TRY(materialize(b));
+        auto out = new_buffer(n);
+        std::vector<std::shared_ptr<Buffer>> bufs{out};
+        for (TensorNode* b : bases) bufs.push_back(b->buffer);
+        MRK_TRY(builtin("concat", params, bufs));
+        n->buffer = out;
+        produced.push_back(n);
+        return kOk;
     }
 
     // Beam search over the choices of one generated elementwise / reduce kernel
