@@ -65,7 +65,12 @@ void KernelCache::clear_all() {
     {
         std::lock_guard<std::mutex> lock(mu_);
         drained.swap(map_);
+        clears_++;
     }
+}
+uint64_t KernelCache::clears() {
+    std::lock_guard<std::mutex> lock(mu_);
+    return clears_;
 }
 
 // the cache key also covers the compiler backend (tensor/src/realize.rs:1052-1054)

@@ -40,9 +40,11 @@ class KernelCache {
     bool lookup(uint64_t ast_hash, const std::string& device, std::shared_ptr<CachedKernel>* out);
     size_t size();
     void clear_all();  // kernel_cache.rs:124-130
+    uint64_t clears();  // how often clear_all() has run: what refers to kernels of the cache by other means is stale when it changes
 
   private:
     std::mutex mu_;
+    uint64_t clears_ = 0;
     std::unordered_map<std::string, std::shared_ptr<CachedKernel>> map_;
 };
 

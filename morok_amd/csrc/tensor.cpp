@@ -1137,6 +1137,40 @@ static bool strided_view(TensorNode* n, StridedView* v) {
     }
 }
 
+// The nodes a walk has seen: open addressing over a power of two of slots, at most half of them taken (a walk is some tens of
+// nodes, a schedule makes hundreds of walks).
+class NodeSet {
+  public:
+    bool insert(const TensorNode* n) {  // whether it was new
+        if (slots_.empty() || (count_ + 1) * 2 > slots_.size()) grow();
+        const bool fresh = put(n);
+        count_ += fresh;
+        return fresh;
+    }
+    void clear() {
+        slots_.clear();
+        count_ = 0;
+    }
+
+  private:
+    bool put(const TensorNode* n) {
+        const size_t mask = slots_.size() - 1;
+        size_t i = (reinterpret_cast<uintptr_t>(n) >> 4) * 0x9e3779b97f4a7c15ull >> 32 & mask;
+        for (; slots_[i]; i = (i + 1) & mask)
+            if (slots_[i] == n) return false;
+        slots_[i] = n;
+        return true;
+    }
+    void grow() {
+        std::vector<const TensorNode*> old(slots_.empty() ? 128 : slots_.size() * 2, nullptr);
+        old.swap(slots_);
+        for (const TensorNode* n : old)
+            if (n) put(n);
+    }
+    std::vector<const TensorNode*> slots_;
+    size_t count_ = 0;
+};
+
 struct Scheduler {
     std::shared_ptr<Device> dev;
     std::unique_ptr<ExecutionPlan> plan;
@@ -1149,14 +1183,15 @@ struct Scheduler {
     std::unordered_map<const TensorNode*, std::vector<TensorNode*>> matmul_readers;  // who reads each product node
     void count_uses(const TensorNode* root) {
         std::vector<const TensorNode*> stack{root};
-        std::set<const TensorNode*> seen{root};
+        NodeSet seen;
+        seen.insert(root);
         while (!stack.empty()) {
             const TensorNode* n = stack.back();
             stack.pop_back();
             for (const TensorRef& c : n->src) {
                 uses[c.get()]++;
                 if (c->hint == HintKind::Matmul) matmul_readers[c.get()].push_back(const_cast<TensorNode*>(n));
-                if (seen.insert(c.get()).second) stack.push_back(c.get());
+                if (seen.insert(c.get())) stack.push_back(c.get());
             }
         }
     }
@@ -1221,9 +1256,9 @@ struct Scheduler {
     }
 
     // nodes that must exist in memory before the kernel rooted at `root` can read them
-    void boundaries(const TensorNode* n, const TensorNode* root, std::set<const TensorNode*>& seen,
+    void boundaries(const TensorNode* n, const TensorNode* root, NodeSet& seen,
                     std::vector<TensorNode*>& out, int64_t* max_numel) {
-        if (!seen.insert(n).second) return;
+        if (!seen.insert(n)) return;
         *max_numel = std::max(*max_numel, n->numel());
         if (n->buffer) return;
         TensorNode* other = nullptr;
@@ -1258,7 +1293,7 @@ struct Scheduler {
             if (rope_matmul(const_cast<TensorNode*>(d), &rest, &split, &seq) || attention_under(const_cast<TensorNode*>(d), &out_strides)) return false;
         }
         // no reduction of the row's own may hide under it (it would have to be fused as well)
-        std::set<const TensorNode*> seen;
+        NodeSet seen;
         std::vector<TensorNode*> deps;
         int64_t ignore = 0;
         boundaries(d, d, seen, deps, &ignore);
@@ -1605,7 +1640,8 @@ struct Scheduler {
             return fail(kUnsupportedDevice, "this backend computes on HIP devices only: the tensor lives on the CPU device; "
                                             "move its inputs with to(\"HIP:0\") first");
         std::vector<const TensorNode*> stack{root};
-        std::set<const TensorNode*> seen{root};
+        NodeSet seen;
+        seen.insert(root);
         while (!stack.empty()) {
             const TensorNode* n = stack.back();
             stack.pop_back();
@@ -1617,7 +1653,7 @@ struct Scheduler {
                 return fail(kUnsupportedDevice, "an operand lives on the CPU device: move it with to(\"HIP:0\") before computing "
                                                 "with it (this backend does not compute on the CPU)");
             for (const TensorRef& c : n->src)
-                if (seen.insert(c.get()).second) stack.push_back(c.get());
+                if (seen.insert(c.get())) stack.push_back(c.get());
         }
         return kOk;
     }
@@ -1782,7 +1818,7 @@ struct Scheduler {
             produced.push_back(n);
             return kOk;
         }
-        std::set<const TensorNode*> seen;
+        NodeSet seen;
         std::vector<TensorNode*> deps;
         int64_t max_numel = 0;
         boundaries(n, n, seen, deps, &max_numel);
@@ -1797,7 +1833,7 @@ struct Scheduler {
                     if (enabled && sides.size() < 2 && side_output_candidate(d, n)) sides.push_back(d);
                 for (TensorNode* R : Rs) {  // the reductions' expressions may read such a tensor as well
                     if (!enabled) break;
-                    std::set<const TensorNode*> seen_r;
+                    NodeSet seen_r;
                     std::vector<TensorNode*> deps_r;
                     int64_t ignore = 0;
                     boundaries(R, R, seen_r, deps_r, &ignore);
@@ -1828,7 +1864,7 @@ struct Scheduler {
             for (TensorNode* d : deps)
                 if (!fused(d)) MRK_TRY(input(d));
             for (TensorNode* R : Rs) {
-                std::set<const TensorNode*> seen_r;
+                NodeSet seen_r;
                 std::vector<TensorNode*> deps_r;
                 boundaries(R, R, seen_r, deps_r, &max_numel);
                 for (TensorNode* d : deps_r)
@@ -1838,14 +1874,155 @@ struct Scheduler {
                 const int beam = std::atoi(e);
                 if (beam > 0 && !dry) return beam_generated(n, max_numel, beam, &Rs, row_block, &sides);
             }
-            return gen_row_fused(n, Rs, row_block, max_numel, sides);
+            return generate(n, max_numel, &Rs, row_block, sides);
         }
         for (TensorNode* d : deps) MRK_TRY(materialize(d));
         if (const char* e = std::getenv("MOROK_BEAM")) {
             const int beam = std::atoi(e);
             if (beam > 0 && !dry) return beam_generated(n, max_numel, beam);
         }
-        return n->kind == TKind::Reduce ? gen_reduce(n, max_numel) : gen_elementwise(n, max_numel);
+        return generate(n, max_numel, nullptr, 0, {});
+    }
+
+    // The kernels generated for an expression, kept by its structure: building a kernel's program just to find, by its content, the
+    // compiled one took most of a realization's host time (a decode step of ten kernels 576 us, kept 218; a two-layer classifier 80, 42).  The key spells out everything the generators look at: the nodes down to
+    // the tensors in memory, with extents, arguments, constants and sharing, which of those tensors are the same buffer, the
+    // reductions and side outputs inside the kernel and the measurement switches.  Buffers are bound by their place in that walk,
+    // nothing is kept by identity.  At most kKeptPrograms, all dropped when that is reached; entries refer to the kernel cache's
+    // kernels weakly and are not used once it has been cleared.  Used under the graph lock only.
+    struct KeptProgram {
+        struct Launch {
+            std::weak_ptr<CachedKernel> kernel;
+            std::vector<int> args;  // 0: the result; 1 + i: tensor in memory i; -1 - i: own buffer i
+        };
+        std::vector<Launch> launches;
+        std::vector<std::pair<int, size_t>> own;  // own buffers: side output (its index) or scratch (-1) of that many bytes
+        uint64_t clears = 0;
+    };
+    static constexpr size_t kKeptPrograms = 1024;
+    static std::unordered_map<std::string, KeptProgram>& kept_programs() {
+        static std::unordered_map<std::string, KeptProgram> programs;
+        return programs;
+    }
+    struct Signature {
+        std::string key;
+        std::unordered_map<const TensorNode*, int> ids;
+        std::vector<std::shared_ptr<Buffer>> leaves;
+        void num(int64_t v) { key.append(reinterpret_cast<const char*>(&v), sizeof v); }
+        void walk(const TensorNode* n) {
+            const auto known = ids.emplace(n, static_cast<int>(ids.size()));
+            if (!known.second) {
+                key.push_back('=');
+                num(known.first->second);
+                return;
+            }
+            key.push_back(n->buffer ? 'b' : 'n');
+            num(static_cast<int64_t>(n->kind) | static_cast<int64_t>(n->dtype) << 8 | static_cast<int64_t>(n->hint) << 16 |
+                static_cast<int64_t>(n->sub) << 24 | static_cast<int64_t>(n->shape.size()) << 40);
+            key.append(reinterpret_cast<const char*>(n->shape.data()), n->shape.size() * sizeof(int64_t));
+            if (n->buffer) {
+                size_t i = 0;
+                while (i < leaves.size() && leaves[i].get() != n->buffer.get()) i++;
+                if (i == leaves.size()) leaves.push_back(n->buffer);
+                num(static_cast<int64_t>(i));
+                return;
+            }
+            num(static_cast<int64_t>(n->arg.size()));
+            key.append(reinterpret_cast<const char*>(n->arg.data()), n->arg.size() * sizeof(int64_t));
+            key.append(reinterpret_cast<const char*>(&n->cval), sizeof n->cval);
+            num(static_cast<int64_t>(n->src.size()));
+            for (const TensorRef& c : n->src) walk(c.get());
+        }
+    };
+    std::vector<std::pair<std::shared_ptr<CachedKernel>, std::vector<std::shared_ptr<Buffer>>>>* recorded = nullptr;  // what queue_kernel queues
+
+    int generate(TensorNode* n, int64_t max_numel, const std::vector<TensorNode*>* Rs, int64_t row_block, const std::vector<TensorNode*>& sides) {
+        auto run = [&]() -> int {
+            if (Rs) return gen_row_fused(n, *Rs, row_block, max_numel, sides);
+            return n->kind == TKind::Reduce ? gen_reduce(n, max_numel) : gen_elementwise(n, max_numel);
+        };
+        if (dry || beam > 0) return run();
+        Signature sig;
+        sig.num(dev->device_id);
+        auto on = [](const char* name) {
+            const char* e = std::getenv(name);
+            return e && e[0] && e[0] != '0';
+        };
+        sig.num((max_numel >= (1LL << 31) ? 1 : 0) | (Rs ? 2 : 0) | (on("MOROK_NO_FLAT_UPCAST") ? 4 : 0) | (on("MOROK_NO_GROUP_REDUCE") ? 8 : 0) | row_block << 8);
+        sig.walk(n);
+        if (Rs)
+            for (const TensorNode* R : *Rs) sig.walk(R);
+        sig.key.push_back('|');
+        for (const TensorNode* d : sides) sig.walk(d);
+        auto& programs = kept_programs();
+        const uint64_t clears = KernelCache::global().clears();
+        const auto found = programs.find(sig.key);
+        if (found != programs.end()) {
+            const KeptProgram& p = found->second;
+            std::vector<std::shared_ptr<CachedKernel>> kernels;
+            bool usable = p.clears == clears;
+            for (const KeptProgram::Launch& l : p.launches) {
+                kernels.push_back(l.kernel.lock());
+                usable = usable && kernels.back();
+            }
+            if (usable) {
+                auto out = new_buffer(n);
+                std::vector<std::shared_ptr<Buffer>> own;
+                for (const auto& o : p.own)
+                    own.push_back(o.first >= 0 ? new_buffer(sides[o.first]) : std::make_shared<Buffer>(dev->allocator, o.second, BufferOptions()));
+                for (size_t i = 0; i < p.launches.size(); i++) {
+                    std::vector<std::shared_ptr<Buffer>> bufs;
+                    for (int a : p.launches[i].args) bufs.push_back(a == 0 ? out : a > 0 ? sig.leaves[a - 1] : own[-1 - a]);
+                    MRK_TRY(add_kernel(kernels[i], bufs, true));
+                }
+                n->buffer = out;
+                produced.push_back(n);
+                for (size_t i = 0; i < p.own.size(); i++) {
+                    if (p.own[i].first < 0) continue;
+                    sides[p.own[i].first]->buffer = own[i];
+                    produced.push_back(sides[p.own[i].first]);
+                }
+                return kOk;
+            }
+            programs.erase(found);
+        }
+        const size_t waiting = deferred ? deferred->size() : 0;
+        std::vector<bool> had(sides.size());
+        for (size_t i = 0; i < sides.size(); i++) had[i] = sides[i]->buffer != nullptr;
+        std::vector<std::pair<std::shared_ptr<CachedKernel>, std::vector<std::shared_ptr<Buffer>>>> queued;
+        recorded = &queued;
+        const int rc = run();
+        recorded = nullptr;
+        if (rc != kOk) return rc;
+        if (deferred && deferred->size() != waiting) return kOk;  // (kernels still to be compiled: this schedule is thrown away)
+        KeptProgram p;
+        p.clears = clears;
+        std::vector<const Buffer*> own;
+        const int unbound = 1 << 30;
+        for (const auto& q : queued) {
+            KeptProgram::Launch l;
+            l.kernel = q.first;
+            for (const auto& buf : q.second) {
+                int arg = buf == n->buffer ? 0 : unbound;
+                for (size_t i = 0; arg == unbound && i < sig.leaves.size(); i++)
+                    if (sig.leaves[i] == buf) arg = static_cast<int>(i) + 1;
+                for (size_t i = 0; arg == unbound && i < own.size(); i++)
+                    if (own[i] == buf.get()) arg = -1 - static_cast<int>(i);
+                if (arg == unbound) {
+                    int side = -1;
+                    for (size_t i = 0; i < sides.size(); i++)
+                        if (!had[i] && sides[i]->buffer == buf) side = static_cast<int>(i);
+                    p.own.emplace_back(side, buf->size());
+                    own.push_back(buf.get());
+                    arg = -static_cast<int>(own.size());
+                }
+                l.args.push_back(arg);
+            }
+            p.launches.push_back(std::move(l));
+        }
+        if (programs.size() >= kKeptPrograms) programs.clear();
+        programs.emplace(std::move(sig.key), std::move(p));
+        return kOk;
     }
 
     // A cat (made contiguous, or wanted in memory itself) of two to four tensors that are, or will be, in memory, or views of such:
@@ -2349,6 +2526,7 @@ struct Scheduler {
         MRK_TRY(compile_kernel(k, name.c_str(), &ck, &cached));
         std::vector<std::shared_ptr<Buffer>> bufs{out};
         bufs.insert(bufs.end(), g.inputs.begin(), g.inputs.end());
+        if (recorded) recorded->emplace_back(ck, bufs);
         return add_kernel(ck, bufs, cached);
     }
     int finish_kernel(KernelGen& g, TensorNode* n, const std::shared_ptr<Buffer>& out, const std::string& name) {
@@ -2517,7 +2695,7 @@ struct Scheduler {
             }
             found.push_back(R);
             if (found.size() > 3) return {};
-            std::set<const TensorNode*> seen_r;
+            NodeSet seen_r;
             std::vector<TensorNode*> deps_r;
             int64_t ignore = 0;
             boundaries(R, R, seen_r, deps_r, &ignore);
@@ -3153,7 +3331,7 @@ int prepare_locked(const TensorRef& root, std::unique_ptr<ExecutionPlan>* out, s
     s.stats.memory_saved = s.plan->memory_plan().memory_saved;
     s.stats.intermediate_bytes = s.plan->memory_plan().memory_planned;
     s.stats.elapsed_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    g_stats = s.stats;
+    g_stats = std::move(s.stats);
     *out = std::move(s.plan);
     return kOk;
 }

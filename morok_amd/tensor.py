@@ -6,6 +6,7 @@ libmorok_hip.so; realize() / to_numpy() run it on the GPU.  bfloat16 data crosse
 boundary as uint16 bit patterns (numpy has no bfloat16).
 """
 import ctypes as C
+import math
 
 import numpy as np
 
@@ -16,15 +17,20 @@ from .device import Buffer, ExecutionPlan
 _NP_OF = {uop.F32: np.float32, uop.F64: np.float64, uop.F16: np.float16, uop.BF16: np.uint16, uop.I32: np.int32,
           uop.I64: np.int64, uop.U32: np.uint32, uop.U8: np.uint8, uop.I8: np.int8, uop.BOOL: np.bool_,
           uop.I16: np.int16, uop.U16: np.uint16, uop.U64: np.uint64}
+_ITEMSIZE = {tag: np.dtype(t).itemsize for tag, t in _NP_OF.items()}
 _TAG_OF = {np.dtype(np.float32): uop.F32, np.dtype(np.float64): uop.F64, np.dtype(np.float16): uop.F16,
            np.dtype(np.int32): uop.I32, np.dtype(np.int64): uop.I64, np.dtype(np.uint32): uop.U32,
            np.dtype(np.uint8): uop.U8, np.dtype(np.int8): uop.I8, np.dtype(np.bool_): uop.BOOL,
            np.dtype(np.int16): uop.I16, np.dtype(np.uint64): uop.U64}
 
 
+_I64 = [C.c_int64 * max(n, 1) for n in range(9)]
+
+
 def _i64(seq):
-    seq = [int(v) for v in seq]
-    return (C.c_int64 * max(len(seq), 1))(*seq), len(seq)
+    seq = tuple(map(int, seq))
+    n = len(seq)
+    return (_I64[n] if n < 9 else C.c_int64 * n)(*seq), n
 
 
 def set_fusion(enabled):
@@ -150,9 +156,9 @@ class Tensor:
     @property
     def shape(self):
         nd = lib.mrk_hip_tensor_ndim(self._h)
-        out = (C.c_int64 * max(nd, 1))()
+        out = (_I64[nd] if nd < 9 else C.c_int64 * nd)()
         check(lib.mrk_hip_tensor_shape(self._h, out, nd))
-        return tuple(out[i] for i in range(nd))
+        return tuple(out[:nd])
 
     @property
     def dtype(self):
@@ -359,5 +365,4 @@ class Tensor:
     def buffer(self):
         h = C.c_void_p()
         check(lib.mrk_hip_tensor_buffer(self._h, C.byref(h)))
-        n = int(np.prod(self.shape)) * np.dtype(_NP_OF[self.dtype]).itemsize
-        return Buffer(n, _handle=h)
+        return Buffer(math.prod(self.shape) * _ITEMSIZE[self.dtype], _handle=h)
