@@ -1312,7 +1312,7 @@ struct Scheduler {
                 if (n->dtype == Scalar::Float32) return true;
                 // half rows of whole waves of vectors are one row-resident generated kernel, which can take what is
                 // around the softmax in as well; all others would be three kernels
-                return is_half(n->dtype) && !row_fused_block(n) && softmax_half_supported(n->numel() / n->shape.back(), n->shape.back());
+                return is_half(n->dtype) && !row_fused_block(n, false) && softmax_half_supported(n->numel() / n->shape.back(), n->shape.back());
             case HintKind::Matmul: {
                 const TensorNode *a = n->hint_inputs[0].get(), *w = n->hint_inputs[1].get();
                 if (a->dtype != w->dtype) return false;
@@ -2642,8 +2642,9 @@ struct Scheduler {
         };
         return walk(root);
     }
-    // Work-items that share a row of `n` in a row-resident kernel; 0: rows of this shape are not kept in registers.
-    static int64_t row_fused_block(const TensorNode* n) {
+    // Work-items that share a row of `n` in a row-resident kernel; 0: rows of this shape are not kept in registers.  partial: also rows
+    // whose last vector per work-item only some of them have.
+    static int64_t row_fused_block(const TensorNode* n, bool partial = true) {
         const int64_t C = n->shape.back(), rows = n->numel() / C;
         int64_t width = 1;
         for (int64_t w = 16 / static_cast<int64_t>(scalar_size(n->dtype)); w > 1; w /= 2)
@@ -2662,7 +2663,24 @@ struct Scheduler {
         // handful of short rows (a decode step's activations: up to 1 MiB in all) is bound by launches, not by the
         // chip, and one kernel instead of a reduction and an elementwise kernel is the faster form there
         const bool tiny = n->numel() * static_cast<int64_t>(scalar_size(n->dtype)) <= (1 << 20);
-        return !block || V / block > 8 || (rows < 128 && !tiny) ? 0 : block;
+        if (rows < 128 && !tiny) return 0;
+        if (block && V / block <= 8) return block;
+        // Other rows: the workgroup that leaves the fewest places empty (the larger of two), with the registers of the whole form (64
+        // values of the row per work-item, at most 16 loads).  Against the reduction and the elementwise kernel, RMSNorm bf16:
+        // 909 x 6105 20.7 us, 6.3 here; 9196 x 3174 49.6 / 19.0; 57 x 1572 6.5 / 2.9; 11668 x 576 10.3 / 6.8; 13236 x 5952 67.0 / 53.3.
+        // Rows of at most half a wave of vectors would leave most lanes idle: they stay with those two kernels, unless there are so few (32 KB in
+        // all) that launches are what they cost (log_softmax over 64 x 10: three launches).  With the hand-written kernels
+        // switched off the kernels are divided as the reference divides them.
+        if (!partial || !g_fusion || (V <= 32 && n->numel() * static_cast<int64_t>(scalar_size(n->dtype)) > (32 << 10))) return 0;
+        block = 0;
+        int64_t least = 0;
+        for (int64_t c : {64, 128, 256, 512}) {
+            const int64_t items = (V + c - 1) / c, waste = items * c - V;
+            if (items > 16 || items * width > 64 || (block && waste > least)) continue;
+            block = c;
+            least = waste;
+        }
+        return block;
     }
     std::vector<TensorNode*> row_reduce_deps(const TensorNode* n, const std::vector<TensorNode*>& deps, int64_t* block_out) {
         const char* off = std::getenv("MOROK_NO_ROW_FUSION");
@@ -2797,16 +2815,25 @@ struct Scheduler {
             if (cand % 64 || cand > 1024 || Vt % cand || Vt / cand > 8) return fail(kInvalidArgument, "row-resident kernel: the row does not split over that many work-items");
             block = cand;
         }
-        const int64_t V = C / width, per_item = V / block, waves = block / 64;
+        const int64_t V = C / width, per_item = (V + block - 1) / block, waves = block / 64;
         uint32_t row = workgroup_index(b, g.idx_t, {rows});
         if (!row) return last_status();
         uint32_t lx = b.special("lidx0", block);
         if (g.idx_t != Scalar::Int32) lx = b.cast(lx, g.idx_t);
         // vector i of this work-item: lx + i * block, so that a wave reads consecutive 16-byte pieces
+        // (where the row ends among the last vectors, the work-items past it take the row's last one again: it is neither folded nor written)
         std::vector<uint32_t> base(per_item);
         std::vector<Coords> coords(per_item);
+        uint32_t inside = 0;  // whether this work-item has a last vector of its own (0: all have)
         for (int64_t i = 0; i < per_item; i++) {
-            base[i] = b.imul(b.iadd(b.iadd(b.imul(row, V), lx), g.ci(i * block)), width);
+            uint32_t at = b.iadd(lx, g.ci(i * block));
+            if ((i + 1) * block > V) {
+                inside = b.binary(BinaryOp::Lt, at, g.ci(V));
+                at = b.where(inside, at, g.ci(V - 1));
+                base[i] = b.imul(b.iadd(b.imul(row, V), at), width);
+            } else {
+                base[i] = b.imul(b.iadd(b.iadd(b.imul(row, V), lx), g.ci(i * block)), width);
+            }
             coords[i] = plain(unflatten(g, base[i], n->shape));
             if (width > 1) coords[i].back().aligned = true;
         }
@@ -2825,6 +2852,7 @@ struct Scheduler {
                     ce.back().off = e;
                     uint32_t v = emit(g, src, ce);
                     if (b.dtype(v).scalar != Scalar::Float32) v = b.cast(v, Scalar::Float32);
+                    if (inside && i + 1 == per_item) v = b.where(inside, v, b.cf(op == ReduceOp::Add ? 0.0 : -INFINITY, Scalar::Float32));
                     acc = acc ? b.binary(op == ReduceOp::Add ? BinaryOp::Add : BinaryOp::Max, acc, v) : v;
                 }
             uint32_t total = b.wave_reduce(op, acc);
@@ -2841,6 +2869,13 @@ struct Scheduler {
             }
             g.fixed[R] = R->dtype != Scalar::Float32 ? b.cast(total, compute_dtype(R->dtype)) : total;
         }
+        auto store_row = [&](uint32_t to, int64_t i, const std::vector<uint32_t>& vals) {
+            const uint32_t v = width > 1 ? b.vectorize(vals) : vals[0];
+            const bool some = inside && i + 1 == per_item;
+            if (some) b.if_(inside);
+            b.store(b.index(to, base[i]), v);
+            if (some) b.endif();
+        };
         // ---- the row's outputs, from the loads the reduction already made
         for (int64_t i = 0; i < per_item; i++) {
             std::vector<uint32_t> vals;
@@ -2851,8 +2886,7 @@ struct Scheduler {
                 if (b.dtype(v).scalar != n->dtype) v = b.cast(v, n->dtype);
                 vals.push_back(v);
             }
-            if (width > 1) b.store(b.index(po, base[i]), b.vectorize(vals));
-            else b.store(b.index(po, base[i]), vals[0]);
+            store_row(po, i, vals);
         }
         // ---- side outputs: inputs of the row that this kernel computed in passing (the values are
         // the ones the reductions and the outputs used: same memo entries), written where a kernel of
@@ -2871,8 +2905,7 @@ struct Scheduler {
                     if (b.dtype(v).scalar != d->dtype) v = b.cast(v, d->dtype);
                     vals.push_back(v);
                 }
-                if (width > 1) b.store(b.index(ps, base[i]), b.vectorize(vals));
-                else b.store(b.index(ps, base[i]), vals[0]);
+                store_row(ps, i, vals);
             }
         }
         MRK_TRY(finish_kernel(g, n, out, "rE_" + std::to_string(rows) + "_g" + std::to_string(C) + (width > 1 ? "_" + std::to_string(width) : "") +
