@@ -15,8 +15,7 @@
 //    go from memory straight to registers, a batch of loads ahead of the matrix instructions, and the waves' sums
 //    meet in local memory.  No barrier until then: a small product is one trip to memory.
 //
-// The order of the additions depends on the shape, the layout of B and whether rows are whole aligned 16-byte chunks, and
-// on nothing else.  How far a sum is off grows with the root of the longest chain of additions.  The kernels these
+// The order of the additions depends on the shape and the layout of B and on nothing else.  How far a sum is off grows with the root of the longest chain of additions.  The kernels these
 // took over from added 64 partial sums of K / 64 products for ragged sizes, and one chain of K for sizes of whole 64 x 64
 // tiles; neither loses precision here.  f32_direct chains 8 products, adds those sums up per wave, and the waves' in
 // 64 bits.  f32_tiled leaves whole tiles (and K < 128, where ragged sizes were one chain too) with a chain of K / 2 per
@@ -28,6 +27,8 @@
 // Bound by the f32 matrix rate (157 TFLOP/s nominal).  Measured: 1024^3 24.7 us (87 TFLOP/s; generated kernel on the vector
 // ALUs 55.3), [N, K] weight 22.3; 4096^3 1.11 ms (124 TFLOP/s); 1000^3 29.1 us (reduction 3500); 64 x 256 x 784 against
 // a [N, K] weight 4.3 us (36.8 and a transposing copy before).
+// Rows that are no whole groups of four are read in 16-byte loads of 4-byte alignment, the last group of a row where it ends with the
+// row; element by element before: 368 x 932 x 1342 59.9 -> 39.0 us, 602 x 640 x 1031 45.3 -> 31.0, 896 x 958 x 768 31.6 -> 24.4, same bits.
 // What is left at 1024^3, one workgroup per CU: the fill and drain of sixteen steps, and the barrier in each.
 #include <hip/hip_runtime.h>
 
@@ -39,22 +40,31 @@
 namespace mrk::dev {
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef f32x4v f32x4_any __attribute__((aligned(4)));  // (a row may start on any float)
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
-// Four elements k .. k + 3 of a row of n elements at p, zeros past the end.  kVec: rows are whole 16-byte chunks, so a
-// group is inside or outside as a whole.
+// v's elements `by` places further down (by 0 .. 3; what comes from behind the last is not used)
+__device__ __forceinline__ f32x4v move_down(const f32x4v& v, int by) {
+    f32x4v r = (by & 1) ? f32x4v{v[1], v[2], v[3], v[3]} : v;
+    return (by & 2) ? f32x4v{r[2], r[3], r[3], r[3]} : r;
+}
+
+// Four elements k .. k + 3 of a row of n >= 4 elements at p, zeros past the end: one load of 4-byte alignment, moved back where it would
+// reach past the row.  kVec: n is a multiple of four, so a group is inside or outside as a whole.
 template <bool kVec>
 __device__ __forceinline__ f32x4v load4(const float* p, long k, long n) {
     f32x4v v = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (kVec) {
-        if (k < n) v = *reinterpret_cast<const f32x4v*>(p + k);
+        if (k < n) v = *reinterpret_cast<const f32x4_any*>(p + k);
     } else {
+        const int left = n - k < 4 ? (int)(n - k) : 4;
+        if (left > 0) {
+            const f32x4v at = *reinterpret_cast<const f32x4_any*>(p + (left < 4 ? n - 4 : k));
+            v = move_down(at, 4 - left);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float x = p[k + i < n ? k + i : n - 1];
-            v[i] = k + i >= n ? 0.0f : x;
+            for (int x = 1; x < 4; x++) v[x] = x < left ? v[x] : 0.0f;
         }
     }
     return v;
@@ -122,10 +132,16 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     // around the loads: the compiler can only count how many are in flight in straight code.
     const bool transpose = !kNT && !moves_a;
     const long first = moves_a ? m0 : n0, end = moves_a ? M : N;
-    const char* base = reinterpret_cast<const char*>(transpose ? B + n0 : (moves_a ? A : B) + first * K);
+    // kVec: rows are whole groups of four.  Otherwise a group that reaches past the end of its row (of K, or of the columns of a
+    // [K, N] operand) is read where it ends with the row and moved down on the way to local memory.  The loads need no more than
+    // 4-byte alignment either way.
+    const int past = (int)(N - 1 - n0 < kBN ? N - 1 - n0 : kBN);
+    const int before = !kVec && past < 3 ? 3 - past : 0;  // columns in front of the tile that are read with its last group
+    const char* base = reinterpret_cast<const char*>(transpose ? B + n0 - before : (moves_a ? A : B) + first * K);
     const unsigned pitch = transpose ? (unsigned)N * 4u : 4u;
     unsigned fixed[4];
     int kr, to[4];  // a group's first k in the step (transpose: + i)
+    int moved = 0;  // transpose: columns the group was read too far in front
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         if (!transpose) {
@@ -134,10 +150,9 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
             kr = 4 * (tq % kSlots);
             to[i] = (moves_a ? 0 : kAF) + r * kBK + (((tq % kSlots) ^ swizzle(r)) << 2);
         } else {
-            // (i: column, for element-wise loads)
-            const int r = 4 * (tq % (kBN / 4)), past = (int)(N - 1 - n0);
-            if (kVec) fixed[i] = 4u * (unsigned)(r + 3 <= past ? r : past - 3);
-            else fixed[i] = 4u * (unsigned)(r + i <= past ? r + i : past);
+            const int r = 4 * (tq % (kBN / 4));
+            fixed[i] = 4u * (unsigned)((r + 3 <= past ? r : past - 3) + before);
+            moved = r + 3 <= past ? 0 : r - (past - 3);
             kr = 4 * (tq / (kBN / 4));
             to[i] = kAF + (r + i) * kBK + (((kr >> 2) ^ swizzle(r + i)) << 2);
         }
@@ -150,27 +165,27 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
         const int k = kr + (k_next - kb), last = (int)K - 1 - kb;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            if constexpr (kVec) {
-                const int ki = transpose ? (k + i < last ? k + i : last) : (k < last - 3 ? k : last - 3);
-                v[i] = *reinterpret_cast<const f32x4v*>(at + (fixed[i] + (unsigned)ki * pitch));
-            } else {
-#pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    const int kx = k + (transpose ? i : x);
-                    v[i][x] = *reinterpret_cast<const float*>(at + (fixed[transpose ? x : i] + (unsigned)(kx < last ? kx : last) * pitch));
-                }
-            }
+            const int ki = transpose ? (k + i < last ? k + i : last) : (k < last - 3 ? k : last - 3);
+            v[i] = *reinterpret_cast<const f32x4_any*>(at + (fixed[i] + (unsigned)ki * pitch));
         }
         k_next += kBK;
         __builtin_amdgcn_sched_barrier(0);  // the loads set out before the step's matrix instructions, not after them
     };
+    const bool columns_end = !kVec && transpose && past < kBN && (N & 3), rows_end = !kVec && !transpose && (K & 3);
     auto stash = [&](float* st, int k0, const f32x4v(&v)[4]) {
         const int left = (int)K - k0 - kr;
         f32x4v z[4];
 #pragma unroll
+        for (int i = 0; i < 4; i++) z[i] = v[i];
+        if (!kVec && (columns_end || (rows_end && k0 + kBK > (int)K))) {
+            const int by = transpose ? moved : left < 4 ? 4 - left : 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) z[i] = move_down(z[i], by);
+        }
+#pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int x = 0; x < 4; x++) z[i][x] = (transpose ? i : kVec ? 0 : x) < left ? v[i][x] : 0.0f;
+            for (int x = 0; x < 4; x++) z[i][x] = (transpose ? i : kVec ? 0 : x) < left ? z[i][x] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++)
             *reinterpret_cast<f32x4v*>(st + to[i]) = transpose ? f32x4v{z[0][i], z[1][i], z[2][i], z[3][i]} : z[i];
@@ -426,9 +441,7 @@ int launch(const F32Call& p) {
     const long M = p.M, N = p.N, K = p.K;
     if (tiles(M, N, 16) > 0x7fffffffL) return hipErrorInvalidValue;
     (void)hipGetLastError();  // (an error that an earlier call left behind is not this launch's)
-    auto aligned = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-    // whole aligned 16-byte chunks along the rows that a kernel reads in them (f32_direct reads columns of a [K, N] operand)
-    const bool rows = K % 4 == 0 && aligned(p.a) && (!kNT || aligned(p.b)), vec = rows && (kNT || (N % 4 == 0 && aligned(p.b)));
+    const bool rows = K % 4 == 0, vec = rows && (kNT || N % 4 == 0);  // rows of whole groups of four (f32_direct reads columns of a [K, N] operand)
     const int tile = tile_size(M, N, K, kNT);
     if (tile == 16) {
         rows ? launch_direct<16, kNT, true, kAdd>(p) : launch_direct<16, kNT, false, kAdd>(p);
@@ -436,7 +449,7 @@ int launch(const F32Call& p) {
         rows ? launch_direct<32, kNT, true, kAdd>(p) : launch_direct<32, kNT, false, kAdd>(p);
     } else {
         // 128 x 128 from one tile per CU (1536^3, 144 tiles: 118 us against 104; 2048^3, 256 tiles: 169 against 196) and where they
-        // pad no more than they gain.  Element-wise loads need too many registers for them.
+        // pad no more than they gain.
         // Products of whole 64 x 64 tiles, and short ones, keep one chain per wave, see the head of the file.
         const bool chain = (M % 64 == 0 && N % 64 == 0) || K < 128;
         if (vec && tiles(M, N, 128) >= 256 && padded(M, N, 128) <= 1.14 * padded(M, N, 64) && (chain || K >= 192))

@@ -1,0 +1,37 @@
+"""f32 products whose rows are no whole groups of four: the last group of a row is read where it ends with the row.  Whole-number operands
+(sums exact in f32, |sum| <= 9 K), NaNs right behind A and B, a pattern behind C."""
+import numpy as np
+import pytest
+
+import morok_amd
+from morok_amd import synth
+
+pytestmark = pytest.mark.gpu
+GUARD = 256
+
+
+def _whole(shape, tid):
+    return synth.randint(shape, 6, tid, 7).astype(np.float32) - 3.0
+
+
+def _guarded(x):
+    return morok_amd.Buffer.from_numpy(np.concatenate([x.reshape(-1), np.full(GUARD, np.nan, np.float32)]))
+
+
+# one, two and three columns / k past a group, tiles of 64 whose last one has less than a group of columns, less than a step and odd
+# numbers of steps; tiles of 32 and of 16
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", [(4200, 65, 67), (4200, 66, 129), (4200, 67, 190), (1300, 513, 258), (1300, 514, 131), (900, 961, 200), (700, 704, 77),
+                                   (300, 257, 253), (481, 500, 258), (40, 33, 255), (17, 4101, 66), (129, 70, 1021)])
+def test_rows_of_any_length_exact(dev, shape, nt):
+    M, N, K = shape
+    a, b, row = _whole((M, K), 0), _whole((K, N), 1), _whole((N,), 2)
+    want = (a.astype(np.float64) @ b).astype(np.float32)
+    ba, bb = _guarded(a), _guarded(np.ascontiguousarray(b.T) if nt else b)
+    for kind, add in (("", None), ("_bias", row)):
+        bc = morok_amd.Buffer.from_numpy(np.full(M * N + GUARD, 77.0, np.float32))
+        more = [_guarded(add)] if add is not None else []
+        morok_amd.Program.builtin("gemm_f32" + ("_nt" if nt else "") + kind, [M, N, K], dev.device_id).execute([bc, ba, bb, *more])
+        got = bc.copyout(np.float32)
+        assert np.array_equal(got[:M * N].reshape(M, N), want if add is None else want + add), kind
+        assert np.all(got[M * N:] == 77.0)
