@@ -182,7 +182,7 @@ __device__ __forceinline__ void flash_fwd_body(const __bf16* __restrict__ Q, con
         first_partial = __builtin_amdgcn_readfirstlane(first_partial);
     }
     const int first_qt = causal ? q_tiles - 1 - unit : unit;
-    const int npass = (causal && unit != first_qt) ? 2 : 1;
+    const int npass = (causal && units < q_tiles && unit != first_qt) ? 2 : 1;
     // key tiles a query tile visits
     auto tiles_of = [&](int qt) {
         int kend = Sk;
@@ -724,6 +724,16 @@ MRK_FLASH_EXT_KERNEL(flash_fwd_ext_d256_add_cap, 256, 1, 2, true)
 
 namespace mrk {
 
+// Work units of a (batch, head): query tiles, or under the causal rule pairs of a late and an early one, so that workgroups end together where
+// there are more tiles than run at once (one or two to a compute unit).  Where there are not, a pair is a longer chain and a second start and end:
+// 80 heads x 169, D = 128 12.2 us in pairs, 7.6 as tiles; 32 x 700 22.3 / 15.4, D = 256 41.4 / 28.5.  With two to a compute unit the
+// longest tiles share one, and short sequences alone gain (64 x 700, 384 tiles 23.3 / 20.2; 32 x 1500, as many 34.4 / 35.6).
+static long work_units(long BH, long q_tiles, long D, int causal) {
+    const long tiles = BH * q_tiles;
+    const bool pairs = causal && tiles > 256 && (D == 256 || tiles > 512 || q_tiles > 6);
+    return pairs ? (q_tiles + 1) / 2 : q_tiles;
+}
+
 // A handful of queries against a long key sequence: the kernel that splits the keys (flash_decode.hip), in as many
 // ranges as the workspace allows (one range needs none).
 static bool decode_route(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
@@ -773,7 +783,7 @@ int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void
         if (decode_route(stream, q, k, v, o, BH, 1, Sq, Sk, D, scale, causal, dense, workspace, workspace_bytes, &rc)) return rc;
     }
     const long q_tiles = (Sq + kQT - 1) / kQT;
-    const long units = causal ? (q_tiles + 1) / 2 : q_tiles;
+    const long units = work_units(BH, q_tiles, D, causal);
     const long blocks = BH * units;
     if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
@@ -814,7 +824,7 @@ int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, co
         if (decode_route(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, &rc)) return rc;
     }
     const long q_tiles = (Sq + kQT - 1) / kQT;
-    const long units = causal ? (q_tiles + 1) / 2 : q_tiles;
+    const long units = work_units(BH, q_tiles, D, causal);
     const long blocks = BH * units;
     if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
     FlashLayout lay;
@@ -887,7 +897,7 @@ int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const 
     // under a softcap a causally masked score becomes -cap and still counts: every key tile is visited
     const int causal_tiles = causal && !cap;
     const long q_tiles = (Sq + kQT - 1) / kQT;
-    const long units = causal_tiles ? (q_tiles + 1) / 2 : q_tiles;
+    const long units = work_units(BH, q_tiles, D, causal_tiles);
     const long blocks = BH * units;
     if (blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
     FlashLayout lay;
