@@ -7,7 +7,7 @@
 // adding the products of k = 8 c + i and 8 c + 4 + i.
 //
 // Two kernels:
-//  - f32_tiled: a workgroup of eight waves owns a 64 x 64 (128 x 128) tile of C; four waves (2 x 2) share the tile, and two
+//  - f32_tiled: a workgroup of eight waves owns a 64 x 64 (128 x 128) tile of C; four waves (2 x 2) share the tile (two of four: 64 x 32), and two
 //    such groups halve every K step and add their sums at the end: two waves per SIMD, so that one's reads of the
 //    local memory run under the other's matrix instructions, and two shorter chains of additions.  Global ->
 //    registers -> local memory, one step ahead, two stages, one barrier per step.
@@ -41,6 +41,7 @@ namespace mrk::dev {
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef f32x4v f32x4_any __attribute__((aligned(4)));  // (a row may start on any float)
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 namespace {
@@ -51,20 +52,30 @@ __device__ __forceinline__ f32x4v move_down(const f32x4v& v, int by) {
     return (by & 2) ? f32x4v{r[2], r[3], r[3], r[3]} : r;
 }
 
-// Four elements k .. k + 3 of a row of n >= 4 elements at p, zeros past the end: one load of 4-byte alignment, moved back where it would
-// reach past the row.  kVec: n is a multiple of four, so a group is inside or outside as a whole.
-template <bool kVec>
+// Four elements k .. k + 3 of a row of n >= 4 elements at p, zeros past the end.
+enum Rows {
+    kGroups4,   // n is a multiple of four: a group is inside or outside as a whole
+    kAnyLength,  // one load of 4-byte alignment, moved back where it would reach past the row
+    kShort,     // element by element: 0.2 us faster where K ends a few groups on (434 x 540 x 94 4.5 us against 4.8)
+};
+template <Rows kRows>
 __device__ __forceinline__ f32x4v load4(const float* p, long k, long n) {
     f32x4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-    if constexpr (kVec) {
+    if constexpr (kRows == kGroups4) {
         if (k < n) v = *reinterpret_cast<const f32x4_any*>(p + k);
-    } else {
+    } else if constexpr (kRows == kAnyLength) {
         const int left = n - k < 4 ? (int)(n - k) : 4;
         if (left > 0) {
             const f32x4v at = *reinterpret_cast<const f32x4_any*>(p + (left < 4 ? n - 4 : k));
             v = move_down(at, 4 - left);
 #pragma unroll
             for (int x = 1; x < 4; x++) v[x] = x < left ? v[x] : 0.0f;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float x = p[k + i < n ? k + i : n - 1];
+            v[i] = k + i >= n ? 0.0f : x;
         }
     }
     return v;
@@ -89,19 +100,19 @@ __device__ __forceinline__ int c_row(int e, int lane) { return 8 * (e >> 2) + 4 
 template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
 __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                                                const float* __restrict__ add, long M, long N, long K, int tiles_m, int tiles_n) {
-    constexpr int kBM = 64 * kT, kBN = 64 * kT;
+    constexpr int kBM = kT ? 64 * kT : 64, kBN = kT ? 64 * kT : 32;
     // Groups of four waves that share the tile and split every K step, and a wave's 32 x 32 blocks of C.  (The 128 tile with
     // 64-bit totals is shared out over all eight waves instead: 128 x 128 totals twice do not fit the registers.)
-    constexpr int kGroups = kT == 2 && kRun ? 1 : 2, kMi = kT, kNj = kT == 2 && kRun ? 1 : kT;
-    constexpr int kBK = kT == 1 ? 64 : 32;        // K step of the workgroup
+    constexpr int kGroups = kT == 2 && kRun ? 1 : 2, kMi = kT ? kT : 1, kNj = kT == 2 && kRun ? 1 : kMi;
+    constexpr int kBK = kT == 2 ? 32 : 64;        // K step of the workgroup
     constexpr int kChunks = kBK / (8 * kGroups);  // 8-deep chunks per step and wave
     constexpr int kSlots = kBK / 4;           // 16-byte slots of a row of either tile in local memory, k contiguous
     constexpr int kAF = kBM * kBK, kBF = kBN * kBK;
     constexpr int kStage = kAF + kBF;
     __shared__ __attribute__((aligned(16))) float smem[2 * kStage];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = kGroups == 2 ? wave >> 2 : 0;
-    const int wm = kGroups == 2 ? (wave >> 1) & 1 : wave >> 2, wn = kGroups == 2 ? wave & 1 : wave & 3;
+    const int group = kGroups == 1 ? 0 : kT ? wave >> 2 : wave >> 1;
+    const int wm = kGroups == 1 ? wave >> 2 : kT ? (wave >> 1) & 1 : wave & 1, wn = kGroups == 1 ? wave & 3 : kT ? wave & 1 : 0;
     const int lr = lane & 31, lg = lane >> 5;
     // Workgroups congruent mod 8 share an L2: each such set takes a run of consecutive tiles, walked in bands of four
     // rows of tiles, so that it reads a few rows of A and of B many times instead of all of both.
@@ -121,7 +132,7 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     // Slot c of row r lies at c ^ swizzle(r).  The local memory serves 16 lanes of 16 bytes from its 64 banks at a time: 16
     // consecutive rows (a fragment read) and 16 rows four apart (the stores of a transposed block) fall into
     // different banks (rows of 128 bytes: two of the latter share one).
-    auto swizzle = [](int r) { return kT == 1 ? ((r >> 2) & 3) | (((r ^ (r >> 4)) & 3) << 2) : ((r >> 1) & 7) ^ ((r >> 4) & 1); };
+    auto swizzle = [](int r) { return kT != 2 ? ((r >> 2) & 3) | (((r ^ (r >> 4)) & 3) << 2) : ((r >> 1) & 7) ^ ((r >> 4) & 1); };
     // staging: waves 4-7 move A, waves 0-3 move B, four 16-byte groups per thread and step; of a [K, N] matrix a block of
     // four rows by four columns, which goes to local memory transposed, so that both fragments are read alike
     const bool moves_a = wave >= 4;
@@ -157,8 +168,58 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
             to[i] = kAF + (r + i) * kBK + (((kr >> 2) ^ swizzle(r + i)) << 2);
         }
     }
+    // Tiles of 64 x 32 are staged by four waves that all move both operands: per work-item four groups of A, and of B two groups or (transposed)
+    // two k-rows by four columns.
+    unsigned a_fixed[4], b_fixed[2];
+    int a_to[4], b_to[4], b_kr = 0;
+    const char *a_base = nullptr, *b_base = nullptr;
+    constexpr bool kFlip = !kNT;
+    if constexpr (kT == 0) {
+        kr = 4 * (tq % kSlots);
+        a_base = reinterpret_cast<const char*>(A + m0 * K);
+        b_base = reinterpret_cast<const char*>(kFlip ? B + n0 - before : B + n0 * K);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = tq / kSlots + i * 16;
+            a_fixed[i] = (unsigned)(m0 + r < M ? r : M - 1 - m0) * (unsigned)K * 4u;
+            a_to[i] = r * kBK + (((tq % kSlots) ^ swizzle(r)) << 2);
+        }
+        if constexpr (kFlip) {
+            const int r = 4 * (tq % 8);
+            b_kr = 2 * (tq / 8);
+            b_fixed[0] = b_fixed[1] = 4u * (unsigned)((r + 3 <= past ? r : past - 3) + before);
+            moved = r + 3 <= past ? 0 : r - (past - 3);
+#pragma unroll
+            for (int x = 0; x < 4; x++) b_to[x] = kAF + (r + x) * kBK + (((b_kr >> 2) ^ swizzle(r + x)) << 2) + (b_kr & 3);
+        } else {
+            b_kr = kr;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int r = tq / kSlots + i * 16;
+                b_fixed[i] = (unsigned)(n0 + r < N ? r : N - 1 - n0) * (unsigned)K * 4u;
+                b_to[i] = kAF + r * kBK + (((tq % kSlots) ^ swizzle(r)) << 2);
+            }
+        }
+    }
+    constexpr int kLoads = kT ? 4 : 6;
     int k_next = 0;  // first k of the step to be fetched
-    auto fetch = [&](f32x4v(&v)[4]) {
+    auto fetch = [&](f32x4v(&v)[kLoads]) {
+        if constexpr (kT == 0) {
+            const int kb = k_next <= (int)K - kBK ? k_next : (int)K > kBK ? (int)K - kBK : 0;
+            const int k = kr + (k_next - kb), bk = b_kr + (k_next - kb), last = (int)K - 1 - kb;
+            const char* aa = a_base + (long)kb * 4;
+            const char* bb = b_base + (long)kb * (kFlip ? (long)N * 4 : 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const f32x4_any*>(aa + (a_fixed[i] + (unsigned)(k < last - 3 ? k : last - 3) * 4u));
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int ki = kFlip ? (bk + i < last ? bk + i : last) : (bk < last - 3 ? bk : last - 3);
+                v[4 + i] = *reinterpret_cast<const f32x4_any*>(bb + (b_fixed[i] + (unsigned)ki * (kFlip ? (unsigned)N * 4u : 4u)));
+            }
+            k_next += kBK;
+            __builtin_amdgcn_sched_barrier(0);
+            return;
+        }
         // (the base stays inside K: the steps fetched past the end read the last one again)
         const int kb = k_next <= (int)K - kBK ? k_next : (int)K > kBK ? (int)K - kBK : 0;
         const char* at = base + (long)kb * pitch;
@@ -172,8 +233,40 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
         __builtin_amdgcn_sched_barrier(0);  // the loads set out before the step's matrix instructions, not after them
     };
     const bool columns_end = !kVec && transpose && past < kBN && (N & 3), rows_end = !kVec && !transpose && (K & 3);
-    auto stash = [&](float* st, int k0, const f32x4v(&v)[4]) {
+    auto stash = [&](float* st, int k0, const f32x4v(&v)[kLoads]) {
         const int left = (int)K - k0 - kr;
+        if constexpr (kT == 0) {
+            f32x4v z[6];
+#pragma unroll
+            for (int i = 0; i < 6; i++) z[i] = v[i];
+            if constexpr (!kVec) {
+                if ((K & 3) && k0 + kBK > (int)K) {
+                    const int by = left < 4 ? 4 - left : 0;
+#pragma unroll
+                    for (int i = 0; i < (kFlip ? 4 : 6); i++) z[i] = move_down(z[i], by);
+                }
+                if (kFlip && past < kBN && (N & 3)) {
+                    z[4] = move_down(z[4], moved);
+                    z[5] = move_down(z[5], moved);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < (kFlip ? 4 : 6); i++)
+#pragma unroll
+                for (int x = 0; x < 4; x++) z[i][x] = (kVec ? 0 : x) < left ? z[i][x] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4v*>(st + a_to[i]) = z[i];
+            if constexpr (kFlip) {
+                const int b_left = (int)K - k0 - b_kr;
+#pragma unroll
+                for (int x = 0; x < 4; x++)
+                    *reinterpret_cast<f32x2*>(st + b_to[x]) = f32x2{0 < b_left ? z[4][x] : 0.0f, 1 < b_left ? z[5][x] : 0.0f};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; i++) *reinterpret_cast<f32x4v*>(st + b_to[i]) = z[4 + i];
+            }
+            return;
+        }
         f32x4v z[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) z[i] = v[i];
@@ -210,8 +303,8 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     const int steps = (int)((K + kBK - 1) / kBK);
     // Step s multiplies stage s & 1 while step s + 1's operands are on their way to registers since step s - 1 (an L2 miss
     // takes longer than a step) and step s + 2's set out.
-    f32x4v in0[4], in1[4];
-    auto step = [&](int s, f32x4v(&arriving)[4], f32x4v(&leaving)[4]) {
+    f32x4v in0[kLoads], in1[kLoads];
+    auto step = [&](int s, f32x4v(&arriving)[kLoads], f32x4v(&leaving)[kLoads]) {
         const float* st = smem + (s & 1) * kStage;
         fetch(leaving);
         const int slot = group * (kSlots / kGroups) + lg;
@@ -243,10 +336,10 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
             if constexpr (kRun == 0) {
                 // (a chunk's fragments are read under the matrix instructions of the chunk before)
                 if (c + 1 < kChunks) {
-                    if (c == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kT, 0);
+                    if (c == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2 * kMi, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kMi, 0);
                 }
-                __builtin_amdgcn_sched_group_barrier(0x8, 4 * kT * kT, 0);
+                __builtin_amdgcn_sched_group_barrier(0x8, 4 * kMi * kMi, 0);
             } else if (closes) {
                 each([&](int i, int j, int e) { total[i][j][e] += (double)acc[i][j][e]; });
                 __builtin_amdgcn_sched_barrier(0);  // (one set of accumulators at a time: there are no registers for two)
@@ -275,8 +368,9 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     if constexpr (kGroups == 2) {
         // the second group hands its sums over through local memory (all reads of the stages are behind the last barrier)
         constexpr int kWave = kMi * kNj * 16 * 64;
-        static_assert(4 * kWave * sizeof(Total) <= sizeof smem, "the second group's sums fit into the stages");
-        Total* x = reinterpret_cast<Total*>(smem) + (wave & 3) * kWave + lane;
+        constexpr int kShare = kT ? 4 : 2;  // waves of a group
+        static_assert(kShare * kWave * sizeof(Total) <= sizeof smem, "the second group's sums fit into the stages");
+        Total* x = reinterpret_cast<Total*>(smem) + (wave & (kShare - 1)) * kWave + lane;
         if (group == 1) each([&](int i, int j, int e) { x[((i * kNj + j) * 16 + e) * 64] = sum(i, j, e); });
         __syncthreads();
         if (group == 0) each([&](int i, int j, int e) { store(i, j, e, x[((i * kNj + j) * 16 + e) * 64]); });
@@ -286,14 +380,14 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
 }
 
 template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
-__global__ void __launch_bounds__(512, kT == 1 && kVec ? 4 : 2) f32_tiled(const float* A, const float* B, float* C, const float* add, long M, long N, long K, int tiles_m,
+__global__ void __launch_bounds__(kT ? 512 : 256, kT == 1 && kVec ? 4 : 2) f32_tiled(const float* A, const float* B, float* C, const float* add, long M, long N, long K, int tiles_m,
                                                  int tiles_n) {
     f32_tiled_body<kT, kNT, kVec, kAdd, kRun>(A, B, C, add, M, N, K, tiles_m, tiles_n);
 }
 
 // kWaves waves split K into runs of whole chunks (of eight for tiles of 32, of sixteen for tiles of 16, whose lane groups
 // are four)
-template <int kTile, int kWaves, bool kNT, bool kVec, int kAdd>
+template <int kTile, int kWaves, bool kNT, Rows kRows, int kAdd>
 __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                                                           const float* __restrict__ add, long M, long N, long K, int tiles_n) {
     constexpr int kBatch = 4;  // chunks whose loads are in flight together
@@ -319,9 +413,9 @@ __global__ void __launch_bounds__(kWaves * 64) f32_direct(const float* __restric
         for (int i = 0; i < kBatch; i++) {
             // chunks past this wave's run multiply zeros
             const long k = c + i < c1 ? (c + i) * kDeep + 4 * lg : K;
-            a[i] = load4<kVec>(pa, k, K);
+            a[i] = load4<kRows>(pa, k, K);
             if constexpr (kNT) {
-                b[i] = load4<kVec>(pb, k, K);
+                b[i] = load4<kRows>(pb, k, K);
             } else {
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
@@ -397,8 +491,12 @@ double padded(long M, long N, long t) { return (double)tiles(M, N, t) * t * t; }
 int tile_size(long M, long N, long K, bool b_transposed) {
     const bool narrow = padded(M, N, 64) > 1.4 * padded(M, N, 32), far = K > (1L << 22) || (!b_transposed && N > (1L << 22));
     if (tiles(M, N, 16) <= 512 || far || (narrow && K >= 768 && padded(M, N, 32) > 1.4 * padded(M, N, 16))) return 16;
-    return tiles(M, N, 32) <= 384 || narrow ? 32 : 64;
+    return tiles(M, N, 32) <= (K > 256 ? 256 : 384) || narrow ? 32 : 64;
 }
+// Products that tiles of 32 would take in two rounds (257 to 384 of them) run on tiles of 64 x 32 in one, from K = 256 on: 602 x 640 x 1031
+// 31.0 us there, 22.2 here, 700 x 500 x 777 30.9 / 18.0, 1472 x 256 x 704 20.7 / 15.8, 576 x 640 x 256 7.6 / 7.9.  They keep sums of eight
+// products: 0.59e-7 off (2-norm) at every K measured, f32_direct 0.69 to 0.90.
+bool two_rounds_of_32(long M, long N, long K) { return K > 256 && tiles(M, N, 32) > 256 && tiles(M, N, 32) <= 384; }
 
 // Times in us of f32_direct, and of the generated reduction that a product is without these kernels (K >= 128: one wave
 // per output; below: one work-item), fitted to 890 products with a side of 1 to 24 against 300 to 10^6, and of 17 to 600,
@@ -421,19 +519,34 @@ double reduction_us(double M, double N, double K, bool b_transposed) {
     return N * K < (1 << 18) ? 1.8 + 1.5e-3 * K + 1.5e-6 * x : 1.8 + 1.5e-3 * K + 3.5e-6 * x + 2.5e-6 * edges;
 }
 
-template <int kTile, bool kNT, bool kVec, int kAdd>
-void launch_direct(const F32Call& p) {
+// Tiles of 64 x 32 instead of 64 x 64: half the work each, where they come out in fewer rounds of one workgroup per CU (us, 64 x 64 / 64 x 32:
+// 512 x 1024 x 1024, 128 tiles 23.7 / 16.2; 1100^3, 324 tiles 55.0 / 45.8; 1536^3 87 / 76; but 1280^3, 400 tiles 50 / 54, 768^3, 144
+// tiles 18.9 / 19.0).
+bool half_tiles(long M, long N) {
+    const long whole = (tiles(M, N, 64) + 255) / 256, half = ((M + 63) / 64 * ((N + 31) / 32) + 255) / 256;
+    return half * 0.53 < (double)whole;
+}
+
+template <int kTile, bool kNT, dev::Rows kRows, int kAdd>
+void launch_direct_rows(const F32Call& p) {
     const int tn = (int)((p.N + kTile - 1) / kTile);
     const dim3 grid((unsigned)((p.M + kTile - 1) / kTile * tn));
-    if (p.K <= 256) dev::f32_direct<kTile, 4, kNT, kVec, kAdd><<<grid, 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
-    else dev::f32_direct<kTile, 16, kNT, kVec, kAdd><<<grid, 1024, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+    if (p.K <= 256) dev::f32_direct<kTile, 4, kNT, kRows, kAdd><<<grid, 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+    else dev::f32_direct<kTile, 16, kNT, kRows, kAdd><<<grid, 1024, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+}
+
+template <int kTile, bool kNT, int kAdd>
+void launch_direct(const F32Call& p) {
+    if (p.K % 4 == 0) launch_direct_rows<kTile, kNT, dev::kGroups4, kAdd>(p);
+    else if (p.K >= 128) launch_direct_rows<kTile, kNT, dev::kAnyLength, kAdd>(p);
+    else launch_direct_rows<kTile, kNT, dev::kShort, kAdd>(p);
 }
 
 template <int kT, bool kNT, bool kVec, int kAdd, int kRun>
 void launch_tiled(const F32Call& p) {
-    constexpr int kB = 64 * kT;
-    const long tm = (p.M + kB - 1) / kB, tn = (p.N + kB - 1) / kB;
-    dev::f32_tiled<kT, kNT, kVec, kAdd, kRun><<<dim3((unsigned)(tm * tn)), 512, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, (int)tm, (int)tn);
+    constexpr int kBM = kT ? 64 * kT : 64, kBN = kT ? 64 * kT : 32;
+    const long tm = (p.M + kBM - 1) / kBM, tn = (p.N + kBN - 1) / kBN;
+    dev::f32_tiled<kT, kNT, kVec, kAdd, kRun><<<dim3((unsigned)(tm * tn)), kT ? 512 : 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, (int)tm, (int)tn);
 }
 
 template <bool kNT, int kAdd>
@@ -441,12 +554,12 @@ int launch(const F32Call& p) {
     const long M = p.M, N = p.N, K = p.K;
     if (tiles(M, N, 16) > 0x7fffffffL) return hipErrorInvalidValue;
     (void)hipGetLastError();  // (an error that an earlier call left behind is not this launch's)
-    const bool rows = K % 4 == 0, vec = rows && (kNT || N % 4 == 0);  // rows of whole groups of four (f32_direct reads columns of a [K, N] operand)
+    const bool vec = K % 4 == 0 && (kNT || N % 4 == 0);  // rows of whole groups of four
     const int tile = tile_size(M, N, K, kNT);
     if (tile == 16) {
-        rows ? launch_direct<16, kNT, true, kAdd>(p) : launch_direct<16, kNT, false, kAdd>(p);
+        launch_direct<16, kNT, kAdd>(p);
     } else if (tile == 32) {
-        rows ? launch_direct<32, kNT, true, kAdd>(p) : launch_direct<32, kNT, false, kAdd>(p);
+        launch_direct<32, kNT, kAdd>(p);
     } else {
         // 128 x 128 from one tile per CU (1536^3, 144 tiles: 118 us against 104; 2048^3, 256 tiles: 169 against 196) and where they
         // pad no more than they gain.
@@ -454,7 +567,12 @@ int launch(const F32Call& p) {
         const bool chain = (M % 64 == 0 && N % 64 == 0) || K < 128;
         if (vec && tiles(M, N, 128) >= 256 && padded(M, N, 128) <= 1.14 * padded(M, N, 64) && (chain || K >= 192))
             chain ? launch_tiled<2, kNT, true, kAdd, 0>(p) : launch_tiled<2, kNT, true, kAdd, 16>(p);
-        else if (chain) vec ? launch_tiled<1, kNT, true, kAdd, 0>(p) : launch_tiled<1, kNT, false, kAdd, 0>(p);
+        else if (two_rounds_of_32(M, N, K)) vec ? launch_tiled<0, kNT, true, kAdd, 8>(p) : launch_tiled<0, kNT, false, kAdd, 8>(p);
+        else if (half_tiles(M, N)) {
+            if (chain) vec ? launch_tiled<0, kNT, true, kAdd, 0>(p) : launch_tiled<0, kNT, false, kAdd, 0>(p);
+            else if (K < 192) vec ? launch_tiled<0, kNT, true, kAdd, 8>(p) : launch_tiled<0, kNT, false, kAdd, 8>(p);
+            else vec ? launch_tiled<0, kNT, true, kAdd, 16>(p) : launch_tiled<0, kNT, false, kAdd, 16>(p);
+        } else if (chain) vec ? launch_tiled<1, kNT, true, kAdd, 0>(p) : launch_tiled<1, kNT, false, kAdd, 0>(p);
         else if (K < 192) vec ? launch_tiled<1, kNT, true, kAdd, 8>(p) : launch_tiled<1, kNT, false, kAdd, 8>(p);
         else vec ? launch_tiled<1, kNT, true, kAdd, 16>(p) : launch_tiled<1, kNT, false, kAdd, 16>(p);
     }
