@@ -210,6 +210,12 @@ void mrk_hip_program_destroy(mrk_program* p);
  *                     q k v o (12)}                                  buffers = {o, q, k, v}
  *                     (both: optionally one more parameter, the bytes of a scratch buffer that follows v:
  *                     mrk_hip_flash_attn_workspace_bytes, for a key sequence split over workgroups)
+ *   "flash_decode_append"  one query per head over a bf16 cache grown by one key (B*H <= 65535, Sk >= 256 with the new key):
+ *                     params = {B, H, Sk, D, f32 bits of scale, element offsets of q, the new key and the new value into their
+ *                     buffers (3), (batch, head) element strides of q, the new key, the new value and o (8), workspace bytes}
+ *                     buffers = {o, grown k, grown v, q, past k, past v, new k, new v[, workspace]}, caches [B, H, keys, D]
+ *   "concat"          params = {outer0, outer1, then per part: 16-byte pieces a row, pieces a run, bytes from run to run, per
+ *                     outer0, per outer1, byte offset}             buffers = {out, a source per part}
  * Buffer order follows the reference's PARAM numbering: outputs first. */
 int mrk_hip_program_builtin(int device_id, const char* kind, const int64_t* params, size_t nparams, mrk_program** out);
 

@@ -108,6 +108,27 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                       }));
         return kOk;
     }
+    if (k == "flash_decode_append") {
+        // {B, H, Sk, D, scale bits, offset of q, of the new key, of the new value, strides: q batch, head, new key batch, head, new value batch,
+        // head, o batch, head (all in elements), workspace bytes}; buffers {o, grown k, grown v, q, past k, past v, new k, new v[, scratch]}
+        MRK_TRY(need(17));
+        if (!flash_decode_append_supported(p[0], p[1], p[2], p[3])) return fail(kInvalidArgument, "flash_decode_append: shape not covered (256 keys and more, D = 64, 128, 256)");
+        for (size_t i = 5; i < 16; i++)
+            if (p[i] < 0 || p[i] % 8) return fail(kInvalidArgument, "flash_decode_append: offsets and strides are multiples of 8");
+        if (p[16] < 0) return fail(kInvalidArgument, "flash_decode_append: negative workspace size");
+        const std::string name = "flash_fwd_bf16_append_" + std::to_string(p[0] * p[1]) + "_1_" + std::to_string(p[2]) + (p[3] != 128 ? "_d" + std::to_string(p[3]) : "");
+        out->reset(new BuiltinProgram(device_id, stream, name, p[16] > 0 ? 9 : 8, p, [](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+            float scale;
+            const uint32_t bits = static_cast<uint32_t>(q[4]);
+            std::memcpy(&scale, &bits, 4);
+            long st[8];
+            for (int i = 0; i < 8; i++) st[i] = q[8 + i];
+            auto at = [](void* p, int64_t off) { return static_cast<const char*>(p) + off * 2; };
+            return launch_flash_decode_append(s, at(b[3], q[5]), b[4], b[5], at(b[6], q[6]), at(b[7], q[7]), b[0], b[1], b[2], q[0], q[1], q[2], q[3], scale, st,
+                                              q[16] > 0 ? b[8] : nullptr, static_cast<size_t>(q[16]));
+        }));
+        return kOk;
+    }
     if (k == "concat") {
         // {outer0, outer1, then per part: pieces of 16 bytes a row, pieces a run, bytes from run to run, bytes per outer0, per outer1,
         // byte offset}; buffers {out, a source per part}

@@ -141,6 +141,13 @@ size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal);
 int launch_flash_decode(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
                         float scale, const long* strides, long splits, long keys_per_split, void* W, const void* mask = nullptr,
                         int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f, long group = 1);
+// One query per (batch, head) over past_k / past_v [B, H, Sk - 1, D] and one new key and value each (all bf16), which also writes the grown
+// caches k_out / v_out [B, H, Sk, D]: the bits of the copies followed by the attention over them.  strides (elements, multiples of
+// 8): q batch, head; new key batch, head; new value batch, head; o batch, head.  Workspace as flash_fwd_workspace_bytes says.
+bool flash_decode_append_supported(long B, long H, long Sk, long D);
+int launch_flash_decode_append(void* stream, const void* q, const void* past_k, const void* past_v, const void* new_k, const void* new_v, void* o,
+                               void* k_out, void* v_out, long B, long H, long Sk, long D, float scale, const long* strides, void* workspace,
+                               size_t workspace_bytes);
 int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* o, long BH, long Sq, long Sk,
                           long D, float scale, int causal, void* workspace = nullptr, size_t workspace_bytes = 0);
 // The same kernel over operands given as views: strides holds (batch, head, row) element

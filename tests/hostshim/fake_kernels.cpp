@@ -120,6 +120,12 @@ int launch_fill_randint(void* stream, void*, size_t, unsigned long long, unsigne
     mrk_shim_note_launch(stream, "fill_randint");
     return 0;
 }
+bool flash_decode_append_supported(long, long, long Sk, long) { return Sk >= 256; }
+int launch_flash_decode_append(void* stream, const void*, const void*, const void*, const void*, const void*, void*, void*, void*, long, long, long, long,
+                               float, const long*, void*, size_t) {
+    mrk_shim_note_launch(stream, "flash_decode_append");
+    return 0;
+}
 int launch_concat(void* stream, void*, const ConcatShape&) {
     mrk_shim_note_launch(stream, "concat");
     return 0;
