@@ -5,7 +5,11 @@
 // grid = (splits, pairs), a workgroup owns a contiguous range of keys, its waves take the range's 32-key
 // chunks in turn.  A wave copies its chunk of K and of V (32 rows each) with direct global -> LDS loads into a
 // region of its own (1 KB per instruction, non-temporal: every byte is read once), so the loop has no barrier,
-// and what streams is bounded by the bytes in flight per CU, i.e. by what the LDS holds.
+// and what streams is bounded by the bytes in flight per CU, i.e. by what the LDS holds: the next chunk's keys are
+// requested as soon as this one's are in registers, its values likewise, so that half of a wave's region is always
+// under way (32 pairs of 4096 keys, D = 128: 16.9 us with the merge, 18.1 where both were requested after the
+// products; 5 x 8 pairs of 3703, D = 256: 29.1 and 32.1).  Under a mask, and where the caches grow, a lane has other
+// loads or stores in the queue that the waits count: there a chunk is requested and awaited as a whole.
 // S^T = K Q^T on v_mfma_f32_16x16x32_bf16 (operand A: 16 keys x 32 d read back from LDS, rows swizzled by the key
 // so that the 16 rows of a read fall into different banks; operand B: the queries, 16 columns, loaded once;
 // queries beyond Sq repeat the last one and are not written; from 17 on a second block of 16 takes the same K and V
@@ -106,25 +110,6 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
     const char* k_head = reinterpret_cast<const char*>(K + b * lay.k_batch + h * lay.k_head);
     const char* v_head = reinterpret_cast<const char*>(V + b * lay.v_batch + h * lay.v_head);
 
-    // the queries: operand B, query slot 16 qb + jl (the last one again beyond the pair's slots), eight d at 32 s + 8 blk
-    // (query slots: head g of a folded run, row r of its Sq rows, slot g * Sq + r)
-    u32x4 qf[kQB][kSteps];
-    const int nq = Sq * lay.group;
-    // the mask row of a lane's query: a lane needs the mask of its eight keys per chunk, two groups of four
-    // consecutive ones (the key count is a multiple of 4 under a mask, so a group is inside the sequence or outside)
-    const char* mrow[kQB];
-#pragma unroll
-    for (int qb = 0; qb < kQB; qb++) {
-        const int want = 16 * qb + jl;
-        const int slot = want < nq ? want : nq - 1;
-        const int qg = slot / Sq, qi = slot - qg * Sq;
-        mrow[qb] = nullptr;
-        if constexpr (kMask != 0)
-            mrow[qb] = static_cast<const char*>(dm.mask) + (b * dm.batch + (h + qg) * dm.head + qi * dm.row) * (kMask == 2 ? 2 : 1);
-        const char* qrow = reinterpret_cast<const char*>(Q + b * lay.q_batch + (h + qg) * lay.q_head) + (size_t)qi * lay.q_row;
-#pragma unroll
-        for (int s = 0; s < kSteps; s++) qf[qb][s] = *reinterpret_cast<const u32x4*>(qrow + 64 * s + 16 * blk);
-    }
     // copy side: copy i covers rows i * kRowsPerCopy ..; lane -> row rsub of them, position pos of the row in LDS.
     // K: position p holds piece p ^ key(row), key = row & 15 (rows of 256 bytes and more) or (row >> 1) & 7
     // (128-byte rows, two to a bank period).  V: 32-byte granule G at granule G ^ key(row), key = row & 7
@@ -167,13 +152,57 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
     }
 
     const int chunks = (k_end - k_begin + kChunkKeys - 1) / kChunkKeys;
+    // (rows past the end repeat the last one, masked below)
+    auto copy = [&](int ci, unsigned lds, const char* head, unsigned row, const unsigned* piece) {
+        const int k0 = k_begin + ci * kChunkKeys, last = k_end - 1 - k0;
+        const char* base = head + (size_t)k0 * row;
+#pragma unroll
+        for (int i = 0; i < kCopies; i++) {
+            int r = i * kRowsPerCopy + rsub;
+            r = r < last ? r : last;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                         :
+                         : "s"(lds + i * 1024), "v"((unsigned)r * row + piece[i]), "s"(base)
+                         : "m0", "memory");
+        }
+    };
+    constexpr bool kPipe = kMask == 0 && !kAppend;
+    if (kPipe && wave < chunks) {
+        copy(wave, lds_k, k_head, lay.k_row, k_piece);
+        copy(wave, lds_v, v_head, lay.v_row, v_piece);
+    }
+    // the queries: operand B, query slot 16 qb + jl (the last one again beyond the pair's slots), eight d at 32 s + 8 blk
+    // (query slots: head g of a folded run, row r of its Sq rows, slot g * Sq + r)
+    u32x4 qf[kQB][kSteps];
+    const int nq = Sq * lay.group;
+    // the mask row of a lane's query: a lane needs the mask of its eight keys per chunk, two groups of four
+    // consecutive ones (the key count is a multiple of 4 under a mask, so a group is inside the sequence or outside)
+    const char* mrow[kQB];
+#pragma unroll
+    for (int qb = 0; qb < kQB; qb++) {
+        const int want = 16 * qb + jl;
+        const int slot = want < nq ? want : nq - 1;
+        const int qg = slot / Sq, qi = slot - qg * Sq;
+        mrow[qb] = nullptr;
+        if constexpr (kMask != 0)
+            mrow[qb] = static_cast<const char*>(dm.mask) + (b * dm.batch + (h + qg) * dm.head + qi * dm.row) * (kMask == 2 ? 2 : 1);
+        const char* qrow = reinterpret_cast<const char*>(Q + b * lay.q_batch + (h + qg) * lay.q_head) + (size_t)qi * lay.q_row;
+#pragma unroll
+        for (int s = 0; s < kSteps; s++) qf[qb][s] = *reinterpret_cast<const u32x4*>(qrow + 64 * s + 16 * blk);
+    }
+    if constexpr (kPipe) {  // here, so that the loop's waits are those for the copies alone
+#pragma unroll
+        for (int qb = 0; qb < kQB; qb++)
+#pragma unroll
+            for (int st = 0; st < kSteps; st++) asm volatile("" : "+v"(qf[qb][st]));
+    }
     for (int ci = wave; ci < chunks; ci += kWaves) {
         const int k0 = k_begin + ci * kChunkKeys;
         const bool full = k0 + kChunkKeys <= k_end;
         const int last = k_end - 1 - k0;  // the chunk's last valid row
         const char* kb = k_head + (size_t)k0 * lay.k_row;
         const char* vb = v_head + (size_t)k0 * lay.v_row;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous chunk's fragment reads are done
+        if (!kPipe) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous chunk's fragment reads are done
         const bool newest = kAppend && k0 + kChunkKeys >= Sk;  // the chunk with the key that is not in the cache yet, its row Sk - 1 - k0
         if (newest) {
 #pragma unroll
@@ -185,25 +214,9 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_k + i * 1024), "v"(ka) : "m0", "memory");
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_v + i * 1024), "v"(va) : "m0", "memory");
             }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kCopies; i++) {
-                int r = i * kRowsPerCopy + rsub;
-                if (!full) r = r < last ? r : last;  // a row past the end repeats the last one (masked below)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                             :
-                             : "s"(lds_k + i * 1024), "v"((unsigned)r * lay.k_row + k_piece[i]), "s"(kb)
-                             : "m0", "memory");
-            }
-#pragma unroll
-            for (int i = 0; i < kCopies; i++) {
-                int r = i * kRowsPerCopy + rsub;
-                if (!full) r = r < last ? r : last;
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                             :
-                             : "s"(lds_v + i * 1024), "v"((unsigned)r * lay.v_row + v_piece[i]), "s"(vb)
-                             : "m0", "memory");
-            }
+        } else if (!kPipe) {
+            copy(ci, lds_k, k_head, lay.k_row, k_piece);
+            copy(ci, lds_v, v_head, lay.v_row, v_piece);
         }
         // the mask of this lane's keys, requested together with the copies
         unsigned mb0[kQB], mb1[kQB];  // Bool: four bytes per group
@@ -223,7 +236,11 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
                 }
             }
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const bool more = ci + kWaves < chunks;
+        if constexpr (kPipe)
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies) : "memory");  // the keys; the values may still be on their way
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if constexpr (kAppend) {
             // what this lane copied, to its place in the grown cache
 #pragma unroll
@@ -250,6 +267,10 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
                 s0[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f0), __builtin_bit_cast(bf16x8, qf[qb][s]), s0[qb], 0, 0, 0);
                 s1[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f1), __builtin_bit_cast(bf16x8, qf[qb][s]), s1[qb], 0, 0, 0);
             }
+        }
+        if (kPipe && more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this chunk's keys are in registers
+            copy(ci + kWaves, lds_k, k_head, lay.k_row, k_piece);
         }
         bf16x8 pb[kQB];
         float alpha[kQB];
@@ -314,6 +335,10 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
             l_run[qb] = l_run[qb] * alpha[qb] + psum;
             pb[qb] = __builtin_convertvector(p, bf16x8);
         }
+        if constexpr (kPipe) {  // the values
+            if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
 #pragma unroll
         for (int c = 0; c < kColBlocks; c++) {
             const unsigned off = rd_v + (((unsigned)c ^ vx) << 5);
@@ -331,6 +356,10 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
             const bf16x8 vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
             for (int qb = 0; qb < kQB; qb++) acc[qb][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pb[qb], acc[qb][c] * alpha[qb], 0, 0, 0);
+        }
+        if (kPipe && more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // its values too
+            copy(ci + kWaves, lds_v, v_head, lay.v_row, v_piece);
         }
     }
     // a query's sum over the four lanes that share it
