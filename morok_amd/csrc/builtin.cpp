@@ -143,6 +143,7 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
             row += ok ? q[0] : 0;
         }
         if (!ok) return fail(kInvalidArgument, "concat: extents have to be positive, runs to divide their part, strides and offsets not negative");
+        if (row > kConcatRowPieces) return fail(kInvalidArgument, "concat: a row has fewer than 2^32 pieces (the launch's limit on work-items)");
         const std::string name = "concat_" + std::to_string(p[0] * p[1]) + "x" + std::to_string(row * 16) + "_" + std::to_string(parts);
         out->reset(new BuiltinProgram(device_id, stream, name, 1 + parts, p, [parts](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
             ConcatShape c{};

@@ -63,11 +63,10 @@ int launch_concat(void* stream, void* out, const ConcatShape& s) {
         if (!c.src || c.pieces <= 0 || c.run <= 0 || c.pieces % c.run || c.pieces > 0x7fffffffLL) return (int)hipErrorInvalidValue;
         pieces += c.pieces;
     }
-    if (pieces != s.row_pieces) return (int)hipErrorInvalidValue;
+    if (pieces != s.row_pieces || pieces > kConcatRowPieces) return (int)hipErrorInvalidValue;
     if (s.outer0 > 0x7fffffffLL || s.outer1 > 0x7fffffffLL || s.outer0 * s.outer1 > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const long long rows = s.outer0 * s.outer1, groups = (s.row_pieces + 256 * mrk::dev::kPieces - 1) / (256 * mrk::dev::kPieces);
     if (rows == 0) return 0;
-    if (groups > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
     mrk::dev::concat_copy<<<dim3((unsigned)groups, (unsigned)(rows < 65535 ? rows : 65535)), 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<char*>(out), s);

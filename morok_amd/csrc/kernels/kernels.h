@@ -195,6 +195,7 @@ int launch_fill_randint(void* stream, void* out, size_t n, unsigned long long se
 // src + o0 * stride0 + o1 * stride1 and is `pieces` of 16 bytes, in runs of `run` (which divides pieces) `stride` bytes apart;
 // any alignment.
 constexpr int kConcatParts = 4;
+constexpr long long kConcatRowPieces = 0xffffff00LL;  // a work-item each: a grid dimension holds fewer than 2^32, here in workgroups of 256
 struct ConcatPart {
     const char* src;
     long long pieces, run, stride, stride0, stride1;

@@ -2028,7 +2028,7 @@ struct Scheduler {
     // A cat (made contiguous, or wanted in memory itself) of two to four tensors that are, or will be, in memory, or views of such:
     // the parameters of the copy kernel, whose extents are launch arguments, and the tensors it reads.  Everything behind the
     // cat axis has to be one run, a part's runs (or the part of a row that they make up) whole 16-byte pieces, the axes in front to
-    // fold into two, and an output row to fill a workgroup.  Other cats are index arithmetic in a generated kernel.
+    // fold into two, and an output row to fill a workgroup and to be no wider than a launch.  Other cats are index arithmetic in a generated kernel.
     bool concat_of_views(TensorNode* n, std::vector<int64_t>* params, std::vector<TensorNode*>* bases) const {
         const TensorNode* cat = n->kind == TKind::Contiguous && n->hint == HintKind::None ? n->src[0].get() : n;
         if (!g_fusion || beam > 0 || cat->buffer || cat->kind != TKind::Cat || cat->hint != HintKind::None || cat->dtype != n->dtype) return false;
@@ -2038,7 +2038,7 @@ struct Scheduler {
         int64_t inner = es, row = 0;  // bytes behind the cat axis
         for (size_t a = axis + 1; a < nd; a++) inner *= cat->shape[a];
         row = inner * cat->shape[axis];
-        if (row < 256 * 16) return false;
+        if (row < 256 * 16 || row / 16 > kConcatRowPieces) return false;
         struct Part {
             StridedView v;
             std::vector<int64_t> st;  // of the axes in front, extents of 1 left out

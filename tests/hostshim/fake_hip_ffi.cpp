@@ -2,6 +2,8 @@
 // the product's host sources into libmorok_hostshim.so so that allocator, buffer, kernel
 // cache, renderer/compiler plumbing, scheduling and error paths can be exercised on a machine
 // without a GPU.  "Device" memory is host memory, launches are recorded and compute nothing.
+#include <sys/mman.h>
+
 #include <atomic>
 #include <chrono>
 #include <cstdlib>
@@ -122,13 +124,16 @@ int device_count(int* out) {
 }
 int set_device(int device_id) { return device_id >= 0 && device_id < g_devices ? 0 : kInvalidDevice; }
 
+constexpr size_t kReservedOnly = size_t(8) << 30;
 int malloc_device(void** out, size_t bytes) {
     std::lock_guard<std::mutex> l(g_mu);
     g_alloc_calls++;
     if (g_in_use + bytes > g_limit) return kOutOfMemory;
-    void* p = std::malloc(bytes ? bytes : 1);
-    if (!p) return kOutOfMemory;
-    std::memset(p, 0xCD, bytes);  // fresh device memory is not zero
+    // (what is larger than this machine's memory may be is address space alone: nothing in the shim writes it)
+    void* p = bytes >= kReservedOnly ? mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0)
+                                     : std::malloc(bytes ? bytes : 1);
+    if (!p || p == MAP_FAILED) return kOutOfMemory;
+    if (bytes < kReservedOnly) std::memset(p, 0xCD, bytes);  // fresh device memory is not zero
     g_allocs[p] = bytes;
     g_in_use += bytes;
     *out = p;
@@ -141,8 +146,9 @@ int free_device(void* ptr) {
     if (it == g_allocs.end()) return kInvalidValue;
     g_free_calls++;
     g_in_use -= it->second;
+    if (it->second >= kReservedOnly) munmap(ptr, it->second);
+    else std::free(ptr);
     g_allocs.erase(it);
-    std::free(ptr);
     return 0;
 }
 int mem_info(size_t* free_bytes, size_t* total_bytes) {

@@ -1099,3 +1099,28 @@ def test_folds_are_read_in_groups_where_that_is_one_request(T, shim):
     assert steps(zeros(T, (65536, 136)).sum(1)) == 3                                          # two steps of 128 would be half empty
     assert steps(zeros(T, (65536, 264)).sum(1)) == 5
     assert steps(zeros(T, (4096, 1000)).sum(1)) == 4                                          # 250 groups of four in steps of 64
+
+
+def test_cats_of_rows_past_the_launch_limit_stay_generated(T, dev, shim):
+    """A grid dimension holds fewer than 2^32 work-items, and the copy kernel gives every 16-byte piece of a row one: rows of 64 GiB
+    and more run as index arithmetic in a generated kernel, whose grid has a second dimension."""
+    cols, pieces = 1 << 19, 1 << 17                                       # of a row of the parts
+
+    def cat(rows):
+        x = zeros(T, (1, cols))
+        plan = T.Tensor.cat([x.try_expand([r, cols]) for r in rows], 0).contiguous().prepare()
+        names = T.last_kernels()
+        plan.execute()                                                    # (recorded, nothing is written)
+        if not names[0].startswith("concat_"):
+            grid, block = hostshim_lib.last_dims(shim)
+            assert all(g * b < 1 << 32 for g, b in zip(grid, block)), (grid, block)
+        return names
+
+    most = (1 << 14) - 1                                                  # just below 2^31 pieces a part
+    assert cat([most, most]) == [f"concat_1x{2 * most * pieces * 16}_2"]
+    names = cat([most, most, 2])                                          # 2^32
+    assert len(names) == 1 and not names[0].startswith("concat_"), names
+    part = lambda r: [r * pieces, pieces, 0, 0, 0, 0]  # noqa: E731
+    morok_amd.Program.builtin("concat", [1, 1, *part(most), *part(most)], dev.device_id)
+    with pytest.raises(MorokHipError):
+        morok_amd.Program.builtin("concat", [1, 1, *part(most), *part(most), *part(2)], dev.device_id)
