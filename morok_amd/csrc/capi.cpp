@@ -408,7 +408,7 @@ int mrk_hip_kernel_builtin(int device_id, const char* kind, const int64_t* param
             *fresh = std::move(k);
             return kOk;
         },
-        &ck));
+        &ck, nullptr, true));
     *out = new mrk_kernel{ck};
     return kOk;
 }

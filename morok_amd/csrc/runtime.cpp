@@ -25,12 +25,13 @@ KernelCache& KernelCache::global() {
 }
 
 int KernelCache::get_or_compile(uint64_t ast_hash, const std::string& device, const CompileFn& compile_fn,
-                                std::shared_ptr<CachedKernel>* out, bool* was_cached) {
+                                std::shared_ptr<CachedKernel>* out, bool* was_cached, bool builtin) {
     const std::string key = std::to_string(ast_hash) + "@" + device;
+    Map& map = builtin ? builtins_ : map_;
     {
         std::lock_guard<std::mutex> lock(mu_);
-        auto it = map_.find(key);
-        if (it != map_.end()) {
+        auto it = map.find(key);
+        if (it != map.end()) {
             *out = it->second;
             if (was_cached) *was_cached = true;
             return kOk;
@@ -39,8 +40,10 @@ int KernelCache::get_or_compile(uint64_t ast_hash, const std::string& device, co
     // compile outside the lock (expensive); a racing thread may compile the same kernel
     std::shared_ptr<CachedKernel> fresh;
     MRK_TRY(compile_fn(&fresh));
+    Map dropped;  // (destroyed once the lock is released)
     std::lock_guard<std::mutex> lock(mu_);
-    auto ins = map_.emplace(key, fresh);
+    if (builtin && map.size() >= kBuiltins && !map.count(key)) dropped.swap(map);
+    auto ins = map.emplace(key, fresh);
     *out = ins.first->second;  // first insert wins
     if (was_cached) *was_cached = false;
     return kOk;
@@ -57,14 +60,15 @@ bool KernelCache::lookup(uint64_t ast_hash, const std::string& device, std::shar
 
 size_t KernelCache::size() {
     std::lock_guard<std::mutex> lock(mu_);
-    return map_.size();
+    return map_.size() + builtins_.size();
 }
 
 void KernelCache::clear_all() {
-    std::unordered_map<std::string, std::shared_ptr<CachedKernel>> drained;
+    Map drained, drained_builtins;
     {
         std::lock_guard<std::mutex> lock(mu_);
         drained.swap(map_);
+        drained_builtins.swap(builtins_);
         clears_++;
     }
 }

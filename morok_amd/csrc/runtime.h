@@ -29,13 +29,15 @@ struct CachedKernel {
 
 // Global dedup cache keyed by (AST content hash, device string)
 // (kernel_cache.rs:52-56,87-118).  Two threads racing on one key may both compile; the
-// first insert wins and both receive the winner.
+// first insert wins and both receive the winner.  Programs around hand-written kernels (builtin) hold their extents, strides and
+// offsets, so that a cache that grows by a token is a new one on every step; they cost a few allocations to make again, and
+// at most kBuiltins of them stay: all are dropped when that is reached (plans keep those they use).
 class KernelCache {
   public:
     static KernelCache& global();
     using CompileFn = std::function<int(std::shared_ptr<CachedKernel>*)>;
     int get_or_compile(uint64_t ast_hash, const std::string& device, const CompileFn& compile_fn,
-                       std::shared_ptr<CachedKernel>* out, bool* was_cached = nullptr);
+                       std::shared_ptr<CachedKernel>* out, bool* was_cached = nullptr, bool builtin = false);
     // the cached kernel, if there is one (no compile)
     bool lookup(uint64_t ast_hash, const std::string& device, std::shared_ptr<CachedKernel>* out);
     size_t size();
@@ -43,9 +45,11 @@ class KernelCache {
     uint64_t clears();  // how often clear_all() has run: what refers to kernels of the cache by other means is stale when it changes
 
   private:
+    using Map = std::unordered_map<std::string, std::shared_ptr<CachedKernel>>;
+    static constexpr size_t kBuiltins = 1024;
     std::mutex mu_;
     uint64_t clears_ = 0;
-    std::unordered_map<std::string, std::shared_ptr<CachedKernel>> map_;
+    Map map_, builtins_;
 };
 
 // Render -> compile -> load through the three hooks of a Device, memoised in the cache:

@@ -1251,7 +1251,7 @@ struct Scheduler {
                 *fresh = std::move(k);
                 return kOk;
             },
-            &ck, &cached));
+            &ck, &cached, true));
         return add_kernel(ck, bufs, cached);
     }
 

@@ -1124,3 +1124,26 @@ def test_cats_of_rows_past_the_launch_limit_stay_generated(T, dev, shim):
     morok_amd.Program.builtin("concat", [1, 1, *part(most), *part(most)], dev.device_id)
     with pytest.raises(MorokHipError):
         morok_amd.Program.builtin("concat", [1, 1, *part(most), *part(most), *part(2)], dev.device_id)
+
+
+def test_programs_of_every_position_do_not_pile_up(T, shim):
+    """A cache that grows by a token takes a copy program of its own on every step.  They are bounded; a plan keeps the one it uses
+    and the generated kernels stay."""
+    morok_amd.kernel_cache_clear()
+    grow = lambda n: T.Tensor.cat([zeros(T, (n, 8)), zeros(T, (1, 8))], 0).contiguous()  # noqa: E731
+    plan = grow(200).prepare()
+    assert T.last_kernels()[0].startswith("concat_")
+    zeros(T, (1000,)).try_mul(3.0).realize()
+    sizes = []
+    for n in range(201, 201 + 2500):
+        grow(n).realize()
+        assert T.last_kernels()[0].startswith("concat_")
+        sizes.append(morok_amd.kernel_cache_size())
+    assert max(sizes) <= 1025, max(sizes)
+    zeros(T, (1000,)).try_mul(3.0).realize()
+    assert T.last_cached_count() == 1
+    n = shim.mrk_shim_launches()
+    plan.execute()
+    assert shim.mrk_shim_launches() == n + 1 and shim.mrk_shim_last_kernel() == b"concat"
+    morok_amd.kernel_cache_clear()
+    assert morok_amd.kernel_cache_size() == 0
