@@ -1052,22 +1052,6 @@ Route choose_route(long M, long N, long K, long batch) {
     if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
     return r;
 }
-// The estimates take about 2 us, a launch 3: each thread keeps the routes of the last shapes it ran (a pure function of the shape).
-Route route_16bit(long M, long N, long K, long batch) {
-    struct Entry {
-        long M = 0, N = 0, K = 0, batch = 0;
-        Route r;
-    };
-    static thread_local Entry kept[32];
-    const unsigned long long h = (unsigned long long)M * 0x9e3779b97f4a7c15ull ^ (unsigned long long)N * 0xc2b2ae3d27d4eb4full ^
-                                 (unsigned long long)K * 0x165667b19e3779f9ull ^ (unsigned long long)batch * 0x27d4eb2f165667c5ull;
-    Entry& e = kept[(h >> 40) % 32];
-    if (e.M != M || e.N != N || e.K != K || e.batch != batch) {
-        e.r = choose_route(M, N, K, batch);
-        e.M = M, e.N = N, e.K = K, e.batch = batch;
-    }
-    return e.r;
-}
 // One pass of 256-row tiles, in us (tiles of 256 x 256: fitted to 39 shapes, 8 % off)
 double tiles256_us(long M, long N, long K) {
     const double rounds = (double)((((M + 255) / 256) * ((N + 255) / 256) + 255) / 256), mb = 2e-6 * ((double)M * K + (double)N * K + (double)M * N);
@@ -1075,12 +1059,42 @@ double tiles256_us(long M, long N, long K) {
     return 4.8 + (us > mb / 4.0 ? us : mb / 4.0);
 }
 // The gated (N = 2 F) and the rotary product: small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
-// two rounds of 256, against 860 of 128 x 128).
-MidPlan paired_plan(long M, long N, long K) {
-    MidPlan p = plan_mid(M, N, K, 1, true, false);
+// two rounds of 256, against 860 of 128 x 128).  A negative answer: tiles of 256 x 256.
+int choose_paired_tile(long M, long N, long K) {
+    const MidPlan p = plan_mid(M, N, K, 1, true, false);
     // (the kernel addresses B's columns from its first with 32-bit offsets)
-    if (p.tile >= 0 && ((double)N * K >= 1e9 || p.us >= 0.95 * tiles256_us(M, N, K))) p.tile = -1;
-    return p;
+    return p.tile >= 0 && (double)N * K < 1e9 && p.us < 0.95 * tiles256_us(M, N, K) ? p.tile : -1;
+}
+// Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form
+bool choose_separate(const Route& r, long M, long N, long K) {
+    if (!r.mid) return r.splits > 1;  // (as large tiles: the fused forms are theirs)
+    const MidPlan fused = plan_mid(M, N, K, 1, true, false);
+    const double large = tiles256_us(M, N, K), best = fused.tile >= 0 && fused.us < large ? fused.us : large;
+    return r.plan.us + 2.7 + 4e-6 * M * N / 5.0 < best;
+}
+// The estimates take about 2 us, a launch 3, and a realization matches a product several times: each thread keeps what it chose for the
+// last shapes it met (pure functions of the shape).
+struct Chosen {
+    long M = 0, N = 0, K = 0, batch = 0;
+    bool has_route = false, has_paired = false, has_separate = false, separate = false;
+    Route route;
+    int paired = -1;
+};
+Chosen& chosen(long M, long N, long K, long batch) {
+    static thread_local Chosen kept[32];
+    const unsigned long long h = (unsigned long long)M * 0x9e3779b97f4a7c15ull ^ (unsigned long long)N * 0xc2b2ae3d27d4eb4full ^
+                                 (unsigned long long)K * 0x165667b19e3779f9ull ^ (unsigned long long)batch * 0x27d4eb2f165667c5ull;
+    Chosen& e = kept[(h >> 40) % 32];
+    if (e.M != M || e.N != N || e.K != K || e.batch != batch) {
+        e = Chosen();
+        e.M = M, e.N = N, e.K = K, e.batch = batch;
+    }
+    return e;
+}
+Route route_16bit(long M, long N, long K, long batch) {
+    Chosen& e = chosen(M, N, K, batch);
+    if (!e.has_route) e.route = choose_route(M, N, K, batch), e.has_route = true;
+    return e.route;
 }
 // f32 partial results of a product whose K is split
 size_t partial_bytes(const Route& r, long M, long N, long batch) { return r.splits > 1 ? (size_t)r.splits * batch * M * N * sizeof(float) : 0; }
@@ -1193,13 +1207,19 @@ bool gemm_bf16_swiglu_supported(long M, long F, long K, bool b_transposed) {
 bool gemm_bf16_separate_preferred(long M, long N, long K) {
     if (M <= 64 && K >= 512) return true;  // (the programs a block over a few tokens consists of stay as they are)
     const Route r = route_16bit(M, N, K, 1);
-    if (!r.mid) return r.splits > 1;  // (as large tiles: the fused forms are theirs)
-    const MidPlan fused = plan_mid(M, N, K, 1, true, false);
-    const double large = tiles256_us(M, N, K), best = fused.tile >= 0 && fused.us < large ? fused.us : large;
-    return r.plan.us + 2.7 + 4e-6 * M * N / 5.0 < best;
+    Chosen& e = chosen(M, N, K, 1);
+    if (!e.has_separate) e.separate = choose_separate(r, M, N, K), e.has_separate = true;
+    return e.separate;
 }
 
-int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C, long M, long F, long K, bool b_transposed) {
+int gemm_bf16_paired_tile(long M, long N, long K) {
+    if (M <= 0 || N <= 0 || K <= 0) return -1;
+    Chosen& e = chosen(M, N, K, 1);
+    if (!e.has_paired) e.paired = choose_paired_tile(M, N, K), e.has_paired = true;
+    return e.paired;
+}
+
+int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C, long M, long F, long K, bool b_transposed, int tile) {
     using namespace mrk::dev;
     if (M <= 0 || F <= 0) return 0;
     if (!gemm_bf16_swiglu_supported(M, F, K, b_transposed)) return (int)hipErrorInvalidValue;
@@ -1208,8 +1228,8 @@ int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C,
     if (b_transposed && gemm_nt_swiglu_streamed(M, F, K)) return launch_gemm_nt_swiglu_streamed(stream, A, B, C, M, F, K);
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
-    const MidPlan mid = paired_plan(M, 2 * F, K);
-    if (mid.tile >= 0) return launch_gemm_mid_paired(s, mid, A, B, C, M, 2 * F, K, b_transposed, nullptr);
+    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, 2 * F, K);
+    if (tile >= 0) return launch_gemm_mid_paired(s, tile, A, B, C, M, 2 * F, K, b_transposed, nullptr);
     const long tn = (F + 127) / 128, tm = (M + kBM - 1) / kBM;
     const dim3 grid((unsigned)(tm * tn), 1);
     const __bf16* a = static_cast<const __bf16*>(A);
@@ -1229,7 +1249,7 @@ bool gemm_bf16_rope_supported(long M, long N, long K, long split, long seq) {
 }
 
 int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_rot, void* C_rest, long M, long N, long K, long split,
-                          const void* cos, const void* sin, long seq, bool b_transposed) {
+                          const void* cos, const void* sin, long seq, bool b_transposed, int tile) {
     using namespace mrk::dev;
     if (!gemm_bf16_rope_supported(M, N, K, split, seq) || !A || !B || !C_rot || !cos || !sin || (split < N && !C_rest))
         return (int)hipErrorInvalidValue;
@@ -1237,10 +1257,10 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
                           reinterpret_cast<uintptr_t>(C_rest) | reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin);
     if (all % 16 || reinterpret_cast<uintptr_t>(cos) % 32 || reinterpret_cast<uintptr_t>(sin) % 32) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
-    const MidPlan mid = paired_plan(M, N, K);
-    if (mid.tile >= 0) {
+    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, N, K);
+    if (tile >= 0) {
         const MidRope angles{static_cast<const float*>(cos), static_cast<const float*>(sin), C_rest, (int)seq, (int)split};
-        return launch_gemm_mid_paired(static_cast<hipStream_t>(stream), mid, A, B, C_rot, M, N, K, b_transposed, &angles);
+        return launch_gemm_mid_paired(static_cast<hipStream_t>(stream), tile, A, B, C_rot, M, N, K, b_transposed, &angles);
     }
     const long tm = (M + kBM - 1) / kBM, tn = (N + kBN - 1) / kBN;
     RopeEpilogue rope{static_cast<const float*>(cos), static_cast<const float*>(sin), static_cast<__bf16*>(C_rest), (int)seq, (int)split};

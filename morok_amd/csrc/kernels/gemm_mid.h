@@ -27,8 +27,8 @@ struct MidRope {
     int seq = 1, split = 0;
 };
 // bf16 products of whole chunks with an epilogue that pairs columns: the gated one (rope null; B holds F = N / 2 gate columns, then F up
-// columns: C [M, F]) and the rotary one (C [M, rope->split]).  p unsplit.
-int launch_gemm_mid_paired(hipStream_t s, const MidPlan& p, const void* A, const void* B, void* C, long M, long N, long K, bool b_transposed,
+// columns: C [M, F]) and the rotary one (C [M, rope->split]).  K in one range.
+int launch_gemm_mid_paired(hipStream_t s, int tile, const void* A, const void* B, void* C, long M, long N, long K, bool b_transposed,
                            const MidRope* rope);
 
 }  // namespace mrk

@@ -503,13 +503,13 @@ MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool spl
 }
 
 namespace {
-// f(tile rows, tile columns, stages) of plan p's tile as constants
+// f(tile rows, tile columns, stages) of a tile as constants
 template <class F>
-void with_tile(const MidPlan& p, F&& f) {
+void with_tile(int tile, F&& f) {
     using std::integral_constant;
     using I64 = integral_constant<int, 64>;
     using I128 = integral_constant<int, 128>;
-    switch (p.tile) {
+    switch (tile) {
         case 0: f(I128{}, I128{}, integral_constant<int, 2>{}); break;
         case 1: f(I128{}, I128{}, integral_constant<int, 3>{}); break;
         case 2: f(I128{}, I64{}, integral_constant<int, 3>{}); break;
@@ -542,19 +542,19 @@ int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* 
         else f16 ? pick(F{}, T{}) : pick(F{}, F{});
     };
     if (p.tile == kMidUnaligned) go(std::integral_constant<int, 64>{}, std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{}, std::false_type{});
-    else with_tile(p, [&](auto tile_m, auto tile_n, auto stages) { go(tile_m, tile_n, stages, std::true_type{}); });
+    else with_tile(p.tile, [&](auto tile_m, auto tile_n, auto stages) { go(tile_m, tile_n, stages, std::true_type{}); });
     return (int)hipGetLastError();
 }
 
 // The gated product C[M, N / 2] (rope null) or the rotated one C[M, rope->split].
-int launch_gemm_mid_paired(hipStream_t s, const MidPlan& p, const void* A, const void* B, void* C, long M, long N, long K, bool b_transposed,
+int launch_gemm_mid_paired(hipStream_t s, int tile, const void* A, const void* B, void* C, long M, long N, long K, bool b_transposed,
                            const MidRope* rope) {
     using namespace mrk::dev;
-    if (p.tile < 0 || p.tile == kMidUnaligned || p.splits != 1 || (rope && (rope->split % 128 || rope->seq <= 0))) return (int)hipErrorInvalidValue;
-    const long tm = (M + kTiles[p.tile].tm - 1) / kTiles[p.tile].tm;
+    if (tile < 0 || tile >= kMidUnaligned || (rope && (rope->split % 128 || rope->seq <= 0))) return (int)hipErrorInvalidValue;
+    const long tm = (M + kTiles[tile].tm - 1) / kTiles[tile].tm;
     // (a tile of 64 columns takes half of a head's pairs: the last head is covered whole)
-    const long cols = rope ? (N + 127) / 128 * 128 : N, tn = (cols + kTiles[p.tile].tn - 1) / kTiles[p.tile].tn;
-    with_tile(p, [&](auto tile_m, auto tile_n, auto stages) {
+    const long cols = rope ? (N + 127) / 128 * 128 : N, tn = (cols + kTiles[tile].tn - 1) / kTiles[tile].tn;
+    with_tile(tile, [&](auto tile_m, auto tile_n, auto stages) {
         constexpr int kTM = decltype(tile_m)::value, kTN = decltype(tile_n)::value, kStages = decltype(stages)::value;
         auto kernel = rope ? (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kRotate> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kRotate>)
                            : (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kGate> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kGate>);

@@ -94,7 +94,12 @@ bool gemm_bf16_swiglu_supported(long M, long F, long K, bool b_transposed = fals
 // Whether a product that could take the gated or the rotary epilogue (N all of its columns) runs faster as a product spread along K
 // and a kernel of its own for the rest: by estimates of both, and always with up to 64 rows from K = 512 on.
 bool gemm_bf16_separate_preferred(long M, long N, long K);
-int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c, long M, long F, long K, bool b_transposed = false);
+// The tile the gated and the rotary product (N all of their columns) run on, for their last argument: a matter of the shape alone, so
+// a program asks once, when it is created; kChooseTile asks at the launch.
+constexpr int kChooseTile = -2;
+int gemm_bf16_paired_tile(long M, long N, long K);
+int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c, long M, long F, long K, bool b_transposed = false,
+                            int tile = kChooseTile);
 // A packed projection whose first `split` columns are attention heads of 128 columns (q | k of a
 // fused QKV product, split a multiple of 256) with the rotary embedding applied in the product
 // kernel's epilogue: c_rot [M, split] = rope(bf16(a b)[:, :split]) (non-interleaved halves, cos /
@@ -103,7 +108,7 @@ int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c,
 // K a multiple of 64, N of 8.
 bool gemm_bf16_rope_supported(long M, long N, long K, long split, long seq);
 int launch_gemm_bf16_rope(void* stream, const void* a, const void* b, void* c_rot, void* c_rest, long M, long N, long K, long split,
-                          const void* cos, const void* sin, long seq, bool b_transposed = false);
+                          const void* cos, const void* sin, long seq, bool b_transposed = false, int tile = kChooseTile);
 // Bytes of scratch launch_gemm_bf16 wants for this shape: padded copies of operands whose rows are
 // no whole 16-byte chunks (K, or N, no multiple of 8), and f32 partial results with which the K
 // loop is spread over the chip (split-K: partial products per K range, added up in a fixed order by a

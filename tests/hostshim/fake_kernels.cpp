@@ -2,6 +2,8 @@
 // (morok_amd/csrc/kernels/kernels.h).  TEST INFRASTRUCTURE ONLY: they compute nothing.
 #include "kernels/kernels.h"
 
+#include <atomic>
+
 extern "C" void mrk_shim_note_launch(void* stream, const char* name);
 
 namespace mrk {
@@ -76,14 +78,22 @@ int launch_gemm_bf16_residual(void* stream, const void*, const void*, const void
     return 0;
 }
 bool gemm_bf16_swiglu_supported(long M, long F, long K, bool) { return M > 0 && F > 0 && K > 0 && F % 8 == 0 && K % 8 == 0; }
-int launch_gemm_bf16_swiglu(void* stream, const void*, const void*, void*, long, long, long, bool b_transposed) {
+static std::atomic<size_t> g_tile_choices{0};
+extern "C" size_t mrk_shim_tile_choices() { return g_tile_choices; }
+int gemm_bf16_paired_tile(long, long, long) {
+    g_tile_choices++;
+    return -1;
+}
+int launch_gemm_bf16_swiglu(void* stream, const void*, const void*, void*, long M, long F, long K, bool b_transposed, int tile) {
+    if (tile == kChooseTile) gemm_bf16_paired_tile(M, 2 * F, K);
     mrk_shim_note_launch(stream, b_transposed ? "gemm_bf16_nt_swiglu" : "gemm_bf16_swiglu");
     return 0;
 }
 bool gemm_bf16_rope_supported(long M, long N, long K, long split, long seq) {
     return M > 0 && N > 0 && K > 0 && seq > 0 && K % 64 == 0 && N % 8 == 0 && split > 0 && split <= N && split % 256 == 0;
 }
-int launch_gemm_bf16_rope(void* stream, const void*, const void*, void*, void*, long, long, long, long, const void*, const void*, long, bool b_transposed) {
+int launch_gemm_bf16_rope(void* stream, const void*, const void*, void*, void*, long M, long N, long K, long, const void*, const void*, long, bool b_transposed, int tile) {
+    if (tile == kChooseTile) gemm_bf16_paired_tile(M, N, K);
     mrk_shim_note_launch(stream, b_transposed ? "gemm_bf16_nt_rope" : "gemm_bf16_rope");
     return 0;
 }

@@ -1147,3 +1147,17 @@ def test_programs_of_every_position_do_not_pile_up(T, shim):
     assert shim.mrk_shim_launches() == n + 1 and shim.mrk_shim_last_kernel() == b"concat"
     morok_amd.kernel_cache_clear()
     assert morok_amd.kernel_cache_size() == 0
+
+
+def test_gated_and_rotary_programs_choose_their_tile_once(dev, shim):
+    """Which tile such a product runs on is estimated when its program is created, not on every launch."""
+    buffers = [dev.buffer(1 << 16) for _ in range(6)]
+    for kind, params, n in (("gemm_bf16_swiglu", [96, 64, 64], 3), ("gemm_bf16_nt_swiglu", [96, 64, 64], 3),
+                            ("gemm_bf16_rope", [64, 384, 64, 256, 64], 6), ("gemm_bf16_nt_rope", [64, 384, 64, 256, 64], 6)):
+        before = shim.mrk_shim_tile_choices()
+        program = morok_amd.Program.builtin(kind, params, dev.device_id)
+        assert shim.mrk_shim_tile_choices() == before + 1
+        for _ in range(3):
+            program.execute(buffers[:n])
+            assert shim.mrk_shim_last_kernel() == kind.encode()
+        assert shim.mrk_shim_tile_choices() == before + 1
