@@ -493,7 +493,7 @@ int tile_size(long M, long N, long K, bool b_transposed) {
     if (tiles(M, N, 16) <= 512 || far || (narrow && K >= 768 && padded(M, N, 32) > 1.4 * padded(M, N, 16))) return 16;
     return tiles(M, N, 32) <= (K > 256 ? 256 : 384) || narrow ? 32 : 64;
 }
-// Products that tiles of 32 would take in two rounds (257 to 384 of them) run on tiles of 64 x 32 in one, from K = 256 on: 602 x 640 x 1031
+// Products that tiles of 32 would take in two rounds (257 to 384 of them) run on tiles of 64 x 32 in one, above K = 256: 602 x 640 x 1031
 // 31.0 us there, 22.2 here, 700 x 500 x 777 30.9 / 18.0, 1472 x 256 x 704 20.7 / 15.8, 576 x 640 x 256 7.6 / 7.9.  They keep sums of eight
 // products: 0.59e-7 off (2-norm) at every K measured, f32_direct 0.69 to 0.90.
 bool two_rounds_of_32(long M, long N, long K) { return K > 256 && tiles(M, N, 32) > 256 && tiles(M, N, 32) <= 384; }
@@ -531,8 +531,8 @@ template <int kTile, bool kNT, dev::Rows kRows, int kAdd>
 void launch_direct_rows(const F32Call& p) {
     const int tn = (int)((p.N + kTile - 1) / kTile);
     const dim3 grid((unsigned)((p.M + kTile - 1) / kTile * tn));
-    if (p.K <= 256) dev::f32_direct<kTile, 4, kNT, kRows, kAdd><<<grid, 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
-    else dev::f32_direct<kTile, 16, kNT, kRows, kAdd><<<grid, 1024, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+    if (kRows == dev::kShort || p.K <= 256) dev::f32_direct<kTile, 4, kNT, kRows, kAdd><<<grid, 256, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
+    else if constexpr (kRows != dev::kShort) dev::f32_direct<kTile, 16, kNT, kRows, kAdd><<<grid, 1024, 0, p.s>>>(p.a, p.b, p.c, p.add, p.M, p.N, p.K, tn);
 }
 
 template <int kTile, bool kNT, int kAdd>
