@@ -16,38 +16,30 @@ namespace mrk::dev {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_any __attribute__((aligned(1)));  // (a view may start on any byte)
 
-constexpr int kPieces = 1;  // per work-item
-
 __device__ __forceinline__ u32x4 piece_at(const char* p) { return *reinterpret_cast<const u32x4_any*>(p); }
 
 __global__ __launch_bounds__(256) void concat_copy(char* __restrict__ out, ConcatShape s) {
-    const long long start = (long long)blockIdx.x * (kPieces * 256), first = start + threadIdx.x;
+    const long long start = (long long)blockIdx.x * 256, first = start + threadIdx.x;
     for (long long row = blockIdx.y; row < s.outer0 * s.outer1; row += gridDim.y) {
         const unsigned o0 = s.outer0 == 1 ? 0 : (unsigned)row / (unsigned)s.outer1, o1 = (unsigned)row - o0 * (unsigned)s.outer1;
         char* o = out + (row * s.row_pieces + first) * 16;
         // workgroups inside the first part, one run per row: all but the few at the seams
-        if (s.part[0].run == s.part[0].pieces && start + kPieces * 256 <= s.part[0].pieces) {
-            const char* at = s.part[0].src + o0 * s.part[0].stride0 + o1 * s.part[0].stride1 + first * 16;
-            u32x4 v[kPieces];
-#pragma unroll
-            for (int i = 0; i < kPieces; i++) v[i] = piece_at(at + i * 4096);
-#pragma unroll
-            for (int i = 0; i < kPieces; i++) *reinterpret_cast<u32x4_any*>(o + i * 4096) = v[i];
+        if (s.part[0].run == s.part[0].pieces && start + 256 <= s.part[0].pieces) {
+            *reinterpret_cast<u32x4_any*>(o) = piece_at(s.part[0].src + o0 * s.part[0].stride0 + o1 * s.part[0].stride1 + first * 16);
             continue;
         }
-        for (int i = 0; i < kPieces && first + i * 256 < s.row_pieces; i++) {
-            long long c = first + i * 256;
-            int p = 0;
-            while (p + 1 < s.parts && c >= s.part[p].pieces) c -= s.part[p++].pieces;
-            const ConcatPart& part = s.part[p];
-            const char* at = part.src + o0 * part.stride0 + o1 * part.stride1;
-            if (part.run == part.pieces) at += c * 16;
-            else {
-                const unsigned l = (unsigned)c / (unsigned)part.run;
-                at += l * part.stride + (c - (long long)l * part.run) * 16;
-            }
-            *reinterpret_cast<u32x4_any*>(o + i * 4096) = piece_at(at);
+        if (first >= s.row_pieces) continue;
+        long long c = first;
+        int p = 0;
+        while (p + 1 < s.parts && c >= s.part[p].pieces) c -= s.part[p++].pieces;
+        const ConcatPart& part = s.part[p];
+        const char* at = part.src + o0 * part.stride0 + o1 * part.stride1;
+        if (part.run == part.pieces) at += c * 16;
+        else {
+            const unsigned l = (unsigned)c / (unsigned)part.run;
+            at += l * part.stride + (c - (long long)l * part.run) * 16;
         }
+        *reinterpret_cast<u32x4_any*>(o) = piece_at(at);
     }
 }
 
@@ -65,7 +57,7 @@ int launch_concat(void* stream, void* out, const ConcatShape& s) {
     }
     if (pieces != s.row_pieces || pieces > kConcatRowPieces) return (int)hipErrorInvalidValue;
     if (s.outer0 > 0x7fffffffLL || s.outer1 > 0x7fffffffLL || s.outer0 * s.outer1 > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    const long long rows = s.outer0 * s.outer1, groups = (s.row_pieces + 256 * mrk::dev::kPieces - 1) / (256 * mrk::dev::kPieces);
+    const long long rows = s.outer0 * s.outer1, groups = (s.row_pieces + 255) / 256;
     if (rows == 0) return 0;
     (void)hipGetLastError();
     mrk::dev::concat_copy<<<dim3((unsigned)groups, (unsigned)(rows < 65535 ? rows : 65535)), 256, 0, static_cast<hipStream_t>(stream)>>>(
