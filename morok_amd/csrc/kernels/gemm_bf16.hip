@@ -1174,6 +1174,36 @@ size_t gemm_bf16_nt_workspace_bytes(long M, long N, long K, long batch) {
     return route_bytes(M, N, K, batch, true);
 }
 
+ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, bool paired) {
+    using namespace mrk::dev;
+    ProductTile t;
+    if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return t;
+    if (paired) {
+        const int tile = gemm_bf16_paired_tile(M, N, K);
+        t.rows = kBM, t.cols = kBN;
+        if (tile >= 0) mid_tile_shape(tile, &t.rows, &t.cols, &t.stages);
+        return t;
+    }
+    long splits = 0, per = 0;
+    if (b_transposed ? gemm_nt_skinny_supported(M, N, K, batch) || gemm_nt_rows_supported(M, N, K, batch)
+                     : gemm_kn_skinny_plan(M, N, K, batch, &splits, &per) || gemm_kn_rows_plan(M, N, K, batch, &splits, &per))
+        return t;
+    const Route r = route_16bit(M, N, K, batch);
+    const bool large = tile_addressable(M, N, K, batch) && operand_padding(M, N, K, batch, b_transposed).lda;
+    const MidPlan p = r.mid ? r.plan : plan_mid(M, N, K, batch, false);
+    t.k_ranges = r.splits;
+    if (r.mid || (!large && p.tile >= 0)) {
+        // (launch_mid's choice between the two tiles of 64 x 64)
+        const bool chunks = K % 8 == 0 && (b_transposed || N % 8 == 0);
+        const int tile = !r.mid ? kMidUnaligned : chunks && p.tile == kMidUnaligned ? kMidSmallest : p.tile;
+        mid_tile_shape(tile, &t.rows, &t.cols, &t.stages);
+    } else {
+        t.rows = !large ? 32 : r.splits > 1 || ((M + 127) / 128) * ((N + kBN - 1) / kBN) * batch <= 256 ? 128 : kBM;
+        t.cols = large ? kBN : 32;
+    }
+    return t;
+}
+
 int launch_gemm_16bit(void* stream, const void* A, const void* B, void* C, long M, long N, long K, int variant, long batch, void* workspace,
                       size_t workspace_bytes, bool b_transposed, bool f16, const void* add, bool add_is_row);
 

@@ -518,6 +518,11 @@ void with_tile(int tile, F&& f) {
 }
 }  // namespace
 
+void mid_tile_shape(int tile, int* rows, int* cols, int* stages) {
+    *rows = kTiles[tile].tm, *cols = kTiles[tile].tn;
+    *stages = tile == kMidUnaligned || tile == 0 ? 2 : 3;
+}
+
 int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* B, void* C, float* W, const void* add, long add_pitch, long M, long N, long K,
                     long batch, bool b_transposed, bool f16) {
     using namespace mrk::dev;

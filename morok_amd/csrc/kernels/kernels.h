@@ -115,6 +115,15 @@ int launch_gemm_bf16_rope(void* stream, const void* a, const void* b, void* c_ro
 // second kernel); 0 for whole chunks and enough output tiles.  Without the workspace the same shape
 // runs unsplit, and one with odd rows on a kernel that reads them element by element.
 size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch);
+// The tile of C that a workgroup of the product owns, given aligned operands and the scratch asked for above: rows, columns, ranges of K and
+// the stages of the small-tile kernel (0: the kernels of large tiles).  rows = 0: a streaming kernel (up to 64 rows).  paired: with the
+// gated or the rotary epilogue, N all of its columns (the [N, K] gated form streams up to 64 rows).
+struct ProductTile {
+    int rows = 0, cols = 0;
+    long k_ranges = 1;
+    int stages = 0;
+};
+ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, bool paired);
 // The same product with the split-K partials in a file-scope device array instead of a
 // caller's workspace, for callers that must not allocate.  gemm_bf16_static_workspace_init
 // resolves the array's address on one device (that device current; once per device, at

@@ -17,6 +17,7 @@ int launch_softmax_half(void* stream, const void*, void*, long, long, bool f16) 
     return 0;
 }
 size_t gemm_bf16_workspace_bytes(long, long, long, long) { return 0; }
+ProductTile gemm_16bit_tile(long, long, long, long, bool, bool) { return ProductTile(); }
 size_t gemm_bf16_nt_workspace_bytes(long, long, long, long) { return 0; }
 bool gemm_bf16_separate_preferred(long, long, long) { return false; }
 int launch_gemm_bf16(void* stream, const void*, const void*, void*, long, long, long, int, long, void*, size_t, bool b_transposed, bool f16) {

@@ -5,8 +5,8 @@ import pytest
 
 import morok_amd
 from morok_amd import synth
+from tests.test_gemm_f32_gpu import test_ragged_products_are_no_less_exact_than_64_partial_sums as ragged_accuracy
 
-pytestmark = pytest.mark.gpu
 GUARD = 256
 
 
@@ -20,6 +20,7 @@ def _guarded(x):
 
 # one, two and three columns / k past a group, tiles of 64 whose last one has less than a group of columns, less than a step and odd
 # numbers of steps; tiles of 32 and of 16
+@pytest.mark.gpu
 @pytest.mark.parametrize("nt", [False, True])
 @pytest.mark.parametrize("shape", [(4200, 65, 67), (4200, 66, 129), (4200, 67, 190), (1300, 513, 258), (1300, 514, 131), (900, 961, 200), (700, 704, 77),
                                    (300, 257, 253), (481, 500, 258), (40, 33, 255), (17, 4101, 66), (129, 70, 1021)])
@@ -35,3 +36,35 @@ def test_rows_of_any_length_exact(dev, shape, nt):
         got = bc.copyout(np.float32)
         assert np.array_equal(got[:M * N].reshape(M, N), want if add is None else want + add), kind
         assert np.all(got[M * N:] == 77.0)
+
+
+# 257 to 384 tiles of 32 x 32 above K = 256, which run on tiles of 64 x 32 with sums of eight products: K and N in no groups of four, whole
+# groups and whole tiles, whole groups and ragged rows, a partial last tile of columns; odd and even numbers of steps
+TWO_ROUNDS = [(602, 640, 1031), (700, 500, 777), (576, 640, 704), (570, 636, 704), (481, 530, 260)]
+
+
+def test_two_rounds_of_tiles_of_32():
+    for m, n, k in TWO_ROUNDS:
+        assert 256 < -(-m // 32) * -(-n // 32) <= 384 and k > 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", TWO_ROUNDS)
+def test_tiles_of_64_by_32_exact(dev, shape, nt):
+    test_rows_of_any_length_exact(dev, shape, nt)
+    M, N, K = shape
+    a, b, mat = _whole((M, K), 0), _whole((K, N), 1), _whole((M, N), 2)
+    bc = morok_amd.Buffer.from_numpy(np.full(M * N + GUARD, 77.0, np.float32))
+    kind = "gemm_f32" + ("_nt" if nt else "") + "_residual"
+    morok_amd.Program.builtin(kind, [M, N, K], dev.device_id).execute([bc, _guarded(a), _guarded(np.ascontiguousarray(b.T) if nt else b), _guarded(mat)])
+    got = bc.copyout(np.float32)
+    assert np.array_equal(got[:M * N].reshape(M, N), (a.astype(np.float64) @ b).astype(np.float32) + mat)
+    assert np.all(got[M * N:] == 77.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", TWO_ROUNDS)
+def test_tiles_of_64_by_32_are_no_less_exact_than_64_partial_sums(dev, shape, nt):
+    ragged_accuracy(*shape, nt)
