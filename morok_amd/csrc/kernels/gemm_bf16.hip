@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 #include <atomic>
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -1030,10 +1031,19 @@ struct Route {
     MidPlan plan;  // (mid: which tile)
     long splits = 1, kt_per_split = 0;
 };
-// Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both,
-// fitted to 170 shapes (tiles of 128 x 256: 4.0 + 0.57 per step of K, 10 % off; split along K 7 %), decide, with a margin for their errors:
-// chosen so, no shape of the 300 timed lost more than 4 % where operands are whole chunks, and they gained 20 % on
-// average.  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
+// One pass of 128-row tiles, up to 256 of them, or one split along K, in us (fitted to 2000 products, 15 % off).
+double large_tiles_us(long M, long N, long K, long batch, long splits, long kt_per_split) {
+    const double deep = K <= 2048 ? 0.0 : K >= 11585 ? 2.5 : std::log2(K / 2048.0);
+    const double operands = 2e-6 * batch * ((double)M * K + (double)N * K + (double)M * N);
+    const double staged = 1e-6 * ((M + 127) / 128) * ((N + 255) / 256) * batch * splits * kt_per_split * (128 + 256) * 128;
+    double us = 0.67 * kt_per_split * (1.0 + 0.05 * deep);
+    if (operands / 6.5 > us) us = operands / 6.5;
+    if (staged / 13.3 > us) us = staged / 13.3;
+    return us + 6.5 + (splits > 1 ? 4.2 + 0.25 * splits + 0.06 * 4e-6 * splits * batch * M * N : 0.0);
+}
+// Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both
+// decide, with a margin for their errors: against the large tiles alone 0.71 of the time over 1400 shapes (geometric mean), 2 of them
+// slower by more than 5 % (8 at most).  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
 Route choose_route(long M, long N, long K, long batch) {
     Route r;
     const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
@@ -1043,12 +1053,11 @@ Route choose_route(long M, long N, long K, long batch) {
     const bool whole = N % 8 == 0 && K % 8 == 0;
     r.plan = plan_mid(M, N, K, batch, whole);
     if (r.plan.tile < 0) return r;
-    const double operands = 2.0 * batch * ((double)M * K + (double)N * K + (double)M * N) * 1e-6;
-    double us = sp.splits > 1 ? 0.70 * sp.kt_per_split : 0.57 * kt;
-    if (operands / (sp.splits > 1 ? 8.3 : 7.0) > us) us = operands / (sp.splits > 1 ? 8.3 : 7.0);
-    us += sp.splits > 1 ? 8.2 + 0.34 * 4e-6 * sp.splits * batch * M * N : 4.0;
-    if (!whole) us += (K % 8 ? 7.0 : 3.5) + 0.7e-6 * batch * ((K % 8 ? (double)M * K : 0.0) + (double)K * N);
-    r.mid = r.plan.us < us * (!whole || sp.splits > 1 ? 0.85 : 0.95);
+    const double us = large_tiles_us(M, N, K, batch, sp.splits, sp.splits > 1 ? sp.kt_per_split : kt);
+    const double copies = (K % 8 ? 7.0 : 3.5) + 0.7e-6 * batch * ((K % 8 ? (double)M * K : 0.0) + (double)K * N);
+    // (where N alone is odd an [N, K] operand needs no copy: the small tiles have to win there as well)
+    if (whole) r.mid = r.plan.us < 0.95 * us;
+    else r.mid = r.plan.us < 0.85 * (us + copies) && (K % 8 || r.plan.us < us);
     if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
     return r;
 }
@@ -1061,14 +1070,14 @@ double tiles256_us(long M, long N, long K) {
 // The gated (N = 2 F) and the rotary product: small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
 // two rounds of 256, against 860 of 128 x 128).  A negative answer: tiles of 256 x 256.
 int choose_paired_tile(long M, long N, long K) {
-    const MidPlan p = plan_mid(M, N, K, 1, true, false);
+    const MidPlan p = plan_mid(M, N, K, 1, true, true);
     // (the kernel addresses B's columns from its first with 32-bit offsets)
     return p.tile >= 0 && (double)N * K < 1e9 && p.us < 0.95 * tiles256_us(M, N, K) ? p.tile : -1;
 }
 // Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form
 bool choose_separate(const Route& r, long M, long N, long K) {
     if (!r.mid) return r.splits > 1;  // (as large tiles: the fused forms are theirs)
-    const MidPlan fused = plan_mid(M, N, K, 1, true, false);
+    const MidPlan fused = plan_mid(M, N, K, 1, true, true);
     const double large = tiles256_us(M, N, K), best = fused.tile >= 0 && fused.us < large ? fused.us : large;
     return r.plan.us + 2.7 + 4e-6 * M * N / 5.0 < best;
 }

@@ -12,8 +12,8 @@ struct MidPlan {
 };
 constexpr int kMidSmallest = 3, kMidUnaligned = 4;  // tiles of 64 x 64: rows of whole chunks; rows that start on any element
 // The fastest by estimate.  whole_chunks: rows of both operands are whole 16-byte chunks on 16-byte bases, whichever way B is stored; else
-// (N and K at least 8) they are read element-aligned.
-MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool splittable = true);
+// (N and K at least 8) they are read element-aligned.  paired: for the gated or the rotary epilogue, K in one range.
+MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool paired = false);
 // rows, columns and stages of a tile
 void mid_tile_shape(int tile, int* rows, int* cols, int* stages);
 // C = A B (B [K, N] or, b_transposed, [N, K]); with p.splits > 1 the partial sums W[splits][batch][M][N] instead, without

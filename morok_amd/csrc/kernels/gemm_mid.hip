@@ -8,10 +8,11 @@
 // workgroups where even those are few, and the choice by an estimate of the time (plan_mid).
 //
 // us before (128 x 256 tiles, split along K where that paid, padded copies of odd operands) and now: 1024 x 1024 x 1024 12.3 / 7.3,
-// 198 x 3072 x 1024 12.2 / 7.5, [N, K] weights: 219 x 4288 x 3232 42.4 / 19.2, 700 x 700 x 4096 52.1 / 14.3,
-// 75 x 1536 x 4576 18.6 / 11.7, 1000 x 3000 x 2048 23.7 / 19.6; odd: 300 x 3001 x 777 23.4 / 8.5, 5 x 7152 x 1638 27.8 / 9.0.
+// 198 x 3072 x 1024 12.2 / 7.5, [N, K] weights: 219 x 4288 x 3232 43.1 / 19.1, 700 x 700 x 4096 53.1 / 15.6,
+// 75 x 1536 x 4576 18.7 / 11.5, 1000 x 3000 x 2048 22.9 / 19.8, 2791 x 96 x 13584 30.0 / 25.0, 487 x 4920 x 13416 171 / 98; odd: 300 x 3001 x 777 23.4 / 8.5, 5 x 7152 x 1638 27.8 / 9.0.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -449,53 +450,66 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
 namespace mrk {
 
 namespace {
-// The tiles and, fitted to 7000 timings over 300 shapes (1 to 4096 rows; 8 to 12 % off, root mean square), what one costs in us:
-// start of a launch, step of K that waits for its data (any number of workgroups resident at once), step when a compute unit's
-// bandwidth is shared, start and end of a workgroup, the second launch of a split and its MB of partial sums, TB/s of the operands.
+// The tiles and what one costs in us, fitted to 25000 timings of every tile and number of ranges over 950 shapes (10 to 12 % off,
+// root mean square): start of a launch, step of K that waits for its data (any number of workgroups resident at
+// once), step of one workgroup more on the same compute unit, start and end of a workgroup, TB/s of the operands, TB/s of what all
+// tiles bring into the LDS.
 struct Tile {
     int tm, tn, resident;  // resident: workgroups a compute unit holds
-    double start, wait, step, edge, reduce, reduce_mb, tbps;
+    double start, wait, step, edge, tbps, staged;
 };
 constexpr Tile kTiles[] = {
-    {128, 128, 2, 2.7, 0.71, 0.50, 1.6, 4.1, 0.33, 5.7},  // two stages: two workgroups share a compute unit
-    {128, 128, 1, 2.7, 0.31, 0.46, 1.6, 3.1, 0.38, 6.1},  // three stages
-    {128, 64, 2, 3.0, 0.33, 0.29, 1.0, 2.8, 0.35, 6.0},
-    {64, 64, 3, 3.3, 0.26, 0.19, 0.4, 2.8, 0.39, 7.0},
-    {64, 64, 4, 2.8, 0.37, 0.21, 0.75, 2.8, 0.39, 6.3},  // through registers
+    {128, 128, 2, 0.63, 0.69, 0.45, 4.3, 4.9, 15.1},  // two stages: two workgroups share a compute unit
+    {128, 128, 1, 1.3, 0.40, 0.41, 4.75, 5.0, 13.0},  // three stages
+    {128, 64, 2, 2.7, 0.0, 0.31, 1.6, 5.5, 64.0},
+    {64, 64, 3, 3.0, 0.24, 0.20, 0.64, 5.6, 21.5},
+    {64, 64, 4, 2.4, 0.40, 0.27, 1.27, 50.0, 11.5},  // through registers
 };
+// The same with the gated or the rotary epilogue, where neither the depth nor the unevenness below is told apart: the choice against tiles of
+// 256 x 256 (tiles256_us) is as good without (over the widths of decoder blocks; 0.46 of the time of those tiles alone, none
+// slower by more than 12 % of 320).
+constexpr Tile kPairedTiles[] = {
+    {128, 128, 2, 2.7, 0.71, 0.50, 1.6, 5.7, 1e3},
+    {128, 128, 1, 2.7, 0.31, 0.46, 1.6, 6.1, 1e3},
+    {128, 64, 2, 3.0, 0.33, 0.29, 1.0, 6.0, 1e3},
+    {64, 64, 3, 3.3, 0.26, 0.19, 0.4, 7.0, 1e3},
+};
+// The second launch of a split, in us: its start, per range, per MB of partial sums.  A split has to promise 4 % to be taken.
+constexpr double kReduce = 2.5, kReduceRange = 0.25, kReduceMb = 0.06, kSplitGain = 1.04;
 }  // namespace
 
-MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool splittable) {
+MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool paired) {
     MidPlan best;
     if (M <= 0 || N < 8 || K < 8 || batch <= 0 || batch > 65535 || M > 0x7fffffffL || K > (1L << 23) || N > (1L << 24)) return best;
     const long kt = (K + 63) / 64;
     const double operands = 2.0 * batch * ((double)M * K + (double)N * K + (double)M * N) * 1e-6;
-    for (int i = 0; i < 5; i++) {
+    // Long rows: each of a tile's is a page of its own, and workgroups that share an operand drift apart over many steps.  A step takes 10 %
+    // longer per doubling of K, and the compute unit that holds the most workgroups ends last instead of the chip evening out
+    // (376 tiles of 128 x 64: 1000 x 3000 x 2048 0.47 us a step; 308: 487 x 4920 x 13416 0.88).
+    const double deep = paired || K <= 2048 ? 0.0 : K >= 11585 ? 2.5 : std::log2(K / 2048.0);
+    for (int i = 0; i < (paired ? 4 : 5); i++) {
         if ((i == kMidUnaligned) == whole_chunks) continue;
-        const Tile& t = kTiles[i];
+        const Tile& t = paired ? kPairedTiles[i] : kTiles[i];
         const long tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
         if ((double)tm * tn > 0x7fffffff) continue;
         for (long want : {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L}) {
-            if (want > 1 && (!splittable || kt < 10)) break;  // few steps are not split
+            if (want > 1 && (paired || kt < 10)) break;  // few steps are not split
             const long per = (kt + want - 1) / want, splits = (kt + per - 1) / per, groups = tm * tn * batch * splits;
             const double partial = 4.0 * splits * batch * M * N;
             // at least two steps a range; partial sums within the scratch of a call that must not allocate
             if (want > 1 && (splits != want || per < 2 || groups > 1024 || partial > (32 << 20))) continue;
             const long rounds = (groups + 255) / 256, waits = (groups + 256 * t.resident - 1) / (256 * t.resident);
-            const double share = t.resident == 1 ? (double)rounds : groups > 256 ? groups / 256.0 : 1.0;
-            double us = t.wait * per * waits;
-            if (t.step * per * share > us) us = t.step * per * share;
-            us += t.edge * rounds;
+            const double even = groups > 256 ? groups / 256.0 : 1.0, uneven = t.resident == 1 || deep > 2.16 ? 1.0 : paired ? 0.0 : 0.35 + 0.3 * deep;
+            const double share = even + uneven * (rounds - even);
+            double us = (t.wait * waits > t.step * share ? t.wait * waits : t.step * share) * per * (1.0 + 0.1 * deep) + t.edge * rounds;
             if (operands / t.tbps > us) us = operands / t.tbps;
-            // odd rows: a chunk may lie on two lines, the tiles' reads arrive at 7 TB/s at most (2187 x 300 x 10615 62 us); operands that
-            // come from memory rather than from the L2s keep the two register sets waiting for longer (2 x 22088 x 3134 33 us in one
-            // range of K, 26 in two)
-            if (i == kMidUnaligned) {
-                const double reads = 1e-6 * groups * per * (t.tm + t.tn) * 128 / 7.0, fetch = operands > 32.0 ? 0.6 * per * waits : 0.0;
-                if (reads > us) us = reads;
-                if (fetch > us) us = fetch;
-            }
-            us += t.start + (splits > 1 ? t.reduce + t.reduce_mb * partial * 1e-6 : 0.0);
+            const double staged = 1e-6 * groups * per * (t.tm + t.tn) * 128;
+            if (staged / t.staged > us) us = staged / t.staged;
+            // operands that come from memory rather than from the L2s keep the two register sets waiting for longer (2 x 22088 x 3134 33 us
+            // in one range of K, 26 in two)
+            if (i == kMidUnaligned && operands > 32.0 && 0.49 * per * waits > us) us = 0.49 * per * waits;
+            us += t.start;
+            if (splits > 1) us = (us + kReduce + kReduceRange * splits + kReduceMb * partial * 1e-6) * kSplitGain;
             if (best.tile < 0 || us < best.us) best = MidPlan{i, splits, per, us};
         }
     }

@@ -23,8 +23,8 @@ def _guarded(dev, bits):
     return morok_amd.Buffer.from_numpy(np.concatenate([bits.reshape(-1), np.full(GUARD, 0x7FFF, np.uint16)]), dev.device_id)
 
 
-# one short of, at and past a tile in rows and columns; one K step, one chunk more, fewer steps than stages; several ranges of K with
-# a partial last step; shapes for tiles of 128 x 128 (both stage counts) and 128 x 64; a batch
+# one short of, at and past a tile of 64 in rows and columns; one K step, one chunk more, fewer steps than stages; several ranges of K with
+# a partial last step; a batch (the other tiles: test_gemm_routes_gpu.py)
 SHAPES = [(65, 64, 64, 1), (127, 72, 72, 1), (129, 136, 136, 1), (128, 248, 200, 1), (66, 1408, 512, 1), (100, 264, 4000, 1), (200, 1000, 1096, 1),
           (2106, 1024, 264, 1), (250, 4104, 1032, 1), (600, 3704, 1544, 1), (70, 72, 1000, 3), (130, 65, 129, 2)]
 

@@ -13,17 +13,18 @@ from tests.test_gemm_mid_gpu import test_small_tiles_exact as _exact
 
 # (M, N, K): each tile with ragged rows and columns, whole and partial last steps of K, and K in ranges
 PLAIN = {
+    (1164, 2744, 64): (128, 128, 1, 2),
+    (201, 8200, 3976): (128, 128, 3, 2),
     (676, 4872, 488): (128, 128, 1, 3),
     (452, 6632, 600): (128, 128, 1, 3),
     (415, 1848, 5944): (128, 128, 4, 3),
     (2131, 856, 9936): (128, 128, 2, 3),
     (2297, 688, 72): (128, 64, 1, 3),
-    (1034, 96, 7368): (128, 64, 12, 3),
-    (337, 1200, 7352): (128, 64, 4, 3),
-    (100, 264, 4000): (64, 64, 16, 3),
-    (347, 5744, 128): (128, 256, 1, 0),
-    (3251, 824, 72): (128, 256, 1, 0),
-    (78, 8, 6328): (128, 256, 33, 0),
+    (900, 160, 9712): (128, 64, 8, 3),
+    (100, 264, 4000): (64, 64, 8, 3),
+    (972, 5592, 64): (128, 256, 1, 0),
+    (1314, 4976, 72): (128, 256, 1, 0),
+    (136, 4424, 6088): (128, 256, 7, 0),
     (2169, 4400, 64): (256, 256, 1, 0),
     (1322, 6672, 72): (256, 256, 1, 0),
     (2169, 4401, 136): (256, 256, 1, 0),
