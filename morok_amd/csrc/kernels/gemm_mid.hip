@@ -491,7 +491,8 @@ MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool pai
         if ((i == kMidUnaligned) == whole_chunks) continue;
         const Tile& t = paired ? kPairedTiles[i] : kTiles[i];
         const long tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
-        if ((double)tm * tn > 0x7fffffff) continue;
+        // fewer than 2^32 work-items, 256 a tile, in the grid's first dimension (rotary: whole heads)
+        if ((double)tm * (paired ? ((N + 127) / 128 * 128 + t.tn - 1) / t.tn : tn) > 0xffffff) continue;
         for (long want : {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L}) {
             if (want > 1 && (paired || kt < 10)) break;  // few steps are not split
             const long per = (kt + want - 1) / want, splits = (kt + per - 1) / per, groups = tm * tn * batch * splits;

@@ -54,6 +54,15 @@ def test_shapes_reach_the_tiles_they_stand_for():
     assert _tile(8, 4096, 4096, True)[0] == 0                  # streamed
 
 
+@pytest.mark.parametrize("m,n,k", [(1 << 30, 16, 8), (1 << 30, 256, 8), (1 << 28, 264, 64)])
+def test_tiles_stay_within_the_launch_limit(m, n, k):
+    """A grid dimension holds fewer than 2^32 work-items: products of that many small tiles stay on tiles of 256 x 256."""
+    for nt in (False, True):
+        rows, cols, _, stages = _tile(m, n, k, nt, True)
+        groups = -(-m // rows) * -(-(-(-n // 128) * 128) // cols)
+        assert groups * (256 if stages else 512) < 1 << 32, (rows, cols)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("nt", [False, True])
