@@ -2721,7 +2721,8 @@ struct Scheduler {
         // chip, and one kernel instead of a reduction and an elementwise kernel is the faster form there
         const bool tiny = n->numel() * static_cast<int64_t>(scalar_size(n->dtype)) <= (1 << 20);
         if (rows < 128 && !tiny) return 0;
-        if (block && V / block <= 8) return block;
+        const auto launchable = [rows](int64_t b) { return rows <= 0xffffffffLL / b; };  // (fewer than 2^32 work-items in a grid dimension)
+        if (block && V / block <= 8) return launchable(block) ? block : 0;
         // Other rows: the workgroup that leaves the fewest places empty (the larger of two), with the registers of the whole form (64
         // values of the row per work-item, at most 16 loads).  Against the reduction and the elementwise kernel, RMSNorm bf16:
         // 909 x 6105 20.7 us, 6.3 here; 9196 x 3174 49.6 / 19.0; 57 x 1572 6.5 / 2.9; 11668 x 576 10.3 / 6.8; 13236 x 5952 67.0 / 53.3.
@@ -2733,7 +2734,7 @@ struct Scheduler {
         int64_t least = 0;
         for (int64_t c : {64, 128, 256, 512}) {
             const int64_t items = (V + c - 1) / c, waste = items * c - V;
-            if (items > 16 || items * width > 64 || (block && waste > least)) continue;
+            if (items > 16 || items * width > 64 || !launchable(c) || (block && waste > least)) continue;
             block = c;
             least = waste;
         }

@@ -1161,3 +1161,14 @@ def test_gated_and_rotary_programs_choose_their_tile_once(dev, shim):
             program.execute(buffers[:n])
             assert shim.mrk_shim_last_kernel() == kind.encode()
         assert shim.mrk_shim_tile_choices() == before + 1
+
+
+@pytest.mark.parametrize("rows", [(1 << 26) - 1, 1 << 26])
+def test_rows_past_the_launch_limit_are_no_row_kernel(T, shim, rows):
+    """A grid dimension holds fewer than 2^32 work-items, and a row-resident kernel gives every row a workgroup: 2^26 rows of 33
+    vectors, a wave each, are a reduction and an elementwise kernel, whose lanes are no more than there are vectors."""
+    T.Tensor.rms_norm(zeros(T, (1, 132)).try_expand([rows, 132])).prepare().execute()
+    names = T.last_kernels()
+    assert names[0].startswith("rE_") == (rows < 1 << 26) and len(names) == (1 if rows < 1 << 26 else 2), names
+    grid, block = hostshim_lib.last_dims(shim)
+    assert all(g * b < 1 << 32 for g, b in zip(grid, block)), (names, grid, block)
