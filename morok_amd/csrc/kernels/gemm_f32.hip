@@ -19,7 +19,8 @@
 // took over from added 64 partial sums of K / 64 products for ragged sizes, and one chain of K for sizes of whole 64 x 64
 // tiles; neither loses precision here.  f32_direct chains 8 products, adds those sums up per wave, and the waves' in
 // 64 bits.  f32_tiled leaves whole tiles (and K < 128, where ragged sizes were one chain too) with a chain of K / 2 per
-// group; for ragged sizes a chain ends after 16 products (8 up to K of 192) and goes on in 64 bits, in registers: the vector
+// group; for ragged sizes a chain ends after 16 products (8 up to K of 192, and in 64 x 32 tiles that stand in for two rounds of 32 x 32,
+// whole ones too) and goes on in 64 bits, in registers: the vector
 // instructions for that do not run under f32 matrix instructions and cost 10 to 18 %.  (f32 totals cost as much:
 // short of the old error they need two levels of them.)  Error against 64 bits, 2-norm, uniform operands, in 1e-7, before and
 // now: 1000 x 1000 x K 0.77 / 0.59 at K = 130, 0.82 / 0.78 at 257, 1.04 / 0.78 at 1000, 1.62 / 0.78 at 4000; 130 x 200 x K

@@ -1,10 +1,10 @@
 // 16-bit products on output tiles of 64 and 128 rows and columns: shapes whose 128 x 256 tiles (gemm_bf16.hip) would leave
 // compute units without work, and operands whose rows start on any element, read as they are.
 //
-// What bounds it: the path from the caches into the LDS.  A K step of a 128 x 128 tile brings 32 KB and takes 0.46 us
-// with one workgroup per compute unit (70 GB/s), one of a 64 x 64 tile 16 KB and 0.19 us with three (84 GB/s; 20 TB/s over the
-// chip), where the matrix instructions of either would take half of that; a 128 x 256 tile does twice the work of the former
-// in 0.57 us, so it stays where enough such tiles exist.  Hence smaller tiles for fewer rows and columns, K split over
+// What bounds it: the path from the caches into the LDS.  A K step of a 128 x 128 tile brings 32 KB and takes 0.50 us
+// with one workgroup per compute unit (66 GB/s), one of a 64 x 64 tile 16 KB and 0.18 us with two or three (93 GB/s; 24 TB/s over the
+// chip, as 128 x 64 tiles reach with two), where the matrix instructions of either would take half of that; a 128 x 256 tile does
+// twice the work of the former in 0.68 us (73 GB/s), so it stays where enough such tiles exist (profiles/gemm_mid_steps.txt).  Hence smaller tiles for fewer rows and columns, K split over
 // workgroups where even those are few, and the choice by an estimate of the time (plan_mid).
 //
 // us before (128 x 256 tiles, split along K where that paid, padded copies of odd operands) and now: 1024 x 1024 x 1024 12.3 / 7.3,

@@ -23,8 +23,8 @@ def _guarded(dev, bits):
     return morok_amd.Buffer.from_numpy(np.concatenate([bits.reshape(-1), np.full(GUARD, 0x7FFF, np.uint16)]), dev.device_id)
 
 
-# one row / column past and short of a tile and of a chunk, K of one element, a partial and a whole last K step, split-K plans
-# (few tiles, long K), more than one 256-row tile
+# one row / column past and short of a tile and of a chunk, K of one element, a partial and a whole last K step, K in ranges
+# (few tiles, long K), more than 256 rows
 SHAPES = [(1, 1, 1), (2, 7, 9), (65, 9, 63), (129, 255, 65), (100, 257, 127), (257, 513, 64), (300, 1001, 320), (70, 129, 1003), (17, 999, 2050),
           (520, 3001, 72), (128, 256, 1023)]
 

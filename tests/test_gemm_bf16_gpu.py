@@ -92,7 +92,7 @@ def test_gemm_does_not_read_past_the_operands(dev, oracle, shape, variant):
     assert np.all(out[M * N:] == 0x7FC0)   # and nothing is written behind C
 
 
-# The 128-row tile (chosen by itself when the shape has few tiles) and the 256-row tile are the
+# The 128-row tile (chosen by itself for up to 256 tiles, where smaller ones are not faster) and the 256-row tile are the
 # same pipeline: forced either way they agree bit for bit with each other and with the oracle
 # within tolerance, on full, ragged-M/N and ragged-K shapes and on a batch.
 @pytest.mark.parametrize("shape", [(128, 256, 64), (512, 512, 256), (1000, 776, 320), (100, 264, 200), (384, 1024, 1000),
@@ -179,7 +179,8 @@ def test_gemm_random_shapes(dev, oracle, seed):
 @pytest.mark.parametrize("shape", [(1, 4096, 4096), (16, 1024, 2048), (100, 264, 4000), (16, 512, 2056), (37, 2048, 4096)])
 def test_gemm_split_k(dev, oracle, shape):
     """Few output tiles against a long K: the K loop is spread over the chip, f32 partials go to
-    scratch from the device allocator and are added in a fixed order.  Against the oracle, the
+    scratch from the device allocator and are added in a fixed order, by the streaming kernels for a handful of
+    rows and by small tiles for (100, 264, 4000); ranges of larger tiles: test_gemm_routes_gpu.py.  Against the oracle, the
     unsplit kernel (which it may differ from by the rounding of one more f32 addition chain)
     and itself (the same bits on every run)."""
     from morok_amd._ffi import lib
@@ -333,8 +334,8 @@ def test_gemm_swiglu_epilogue_parity(dev, oracle, shape):
                                    (100, 264, 200), (256, 256, 72), (129, 8, 72), (2048, 512, 136), (137, 4096, 64)])
 def test_gemm_transposed_second_operand(dev, oracle, shape):
     """a @ bt.T with bt [N, K] read in place: the same products in the same order as the
-    [K, N] form, so the same bits, on full, ragged-M/N and ragged-K shapes and with either tile
-    size; NaNs right behind a, bt and c show that no edge reads or writes past them."""
+    [K, N] form, so the same bits, on full, ragged-M/N and ragged-K shapes (mostly small tiles; the others:
+    test_gemm_routes_gpu.py); NaNs right behind a, bt and c show that no edge reads or writes past them."""
     M, N, K = shape
     a = synth.normal_bf16((M, K), 3, 20)
     b = synth.normal_bf16((K, N), 3, 21)
