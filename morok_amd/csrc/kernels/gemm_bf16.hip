@@ -681,7 +681,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         const f32x8 x = __builtin_convertvector(__builtin_bit_cast(bf16x8, v[t]), f32x8);
                         const f32x8 y = __builtin_convertvector(__builtin_bit_cast(bf16x8, pv[t]), f32x8);
                         const f32x8 sn = lc < 8 ? -sn_cur[t] : sn_cur[t];  // first half: x1 cos - x2 sin; second half: x2 cos + x1 sin
-                        const f32x8 o = x * cs_cur[t] + y * sn;
+                        const f32x8 o = __builtin_elementwise_fma(y, sn, x * cs_cur[t]);
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
@@ -1041,6 +1041,13 @@ double large_tiles_us(long M, long N, long K, long batch, long splits, long kt_p
     if (staged / 13.3 > us) us = staged / 13.3;
     return us + 6.5 + (splits > 1 ? 4.2 + 0.25 * splits + 0.06 * 4e-6 * splits * batch * M * N : 0.0);
 }
+// One pass of 256-row tiles, in us (tiles of 256 x 256: fitted to 39 shapes, 8 % off)
+double tiles256_us(long M, long N, long K) {
+    if (mid_pipelined(N, K) && mid_many_tiles(M, N, 1)) return large_pass_us(M, N, K, 1);
+    const double rounds = (double)((((M + 255) / 256) * ((N + 255) / 256) + 255) / 256), mb = 2e-6 * ((double)M * K + (double)N * K + (double)M * N);
+    const double us = rounds * (1.02 * ((K + 63) / 64) + 5.8);
+    return 4.8 + (us > mb / 4.0 ? us : mb / 4.0);
+}
 // Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both
 // decide, with a margin for their errors: against the large tiles alone 0.71 of the time over 1400 shapes (geometric mean), 2 of them
 // slower by more than 5 % (8 at most).  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
@@ -1049,23 +1056,24 @@ Route choose_route(long M, long N, long K, long batch) {
     const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
     r.splits = sp.splits, r.kt_per_split = sp.kt_per_split;
     const long tiles = ((M + 127) / 128) * ((N + 255) / 256) * batch, kt = (K + 63) / 64;
-    if (tiles > 256) return r;
+    const bool pipelined = sp.splits == 1 && mid_pipelined(N, K);
+    if (tiles > 256 && !pipelined) return r;
     const bool whole = N % 8 == 0 && K % 8 == 0;
     r.plan = plan_mid(M, N, K, batch, whole);
     if (r.plan.tile < 0) return r;
+    if (pipelined && r.plan.splits == 1) {
+        r.mid = r.plan.us < 0.97 * large_pass_us(M, N, K, batch);
+        if (r.mid) r.splits = 1, r.kt_per_split = r.plan.kt_per_split;
+        return r;
+    }
+    if (tiles > 256) return r;
     const double us = large_tiles_us(M, N, K, batch, sp.splits, sp.splits > 1 ? sp.kt_per_split : kt);
     const double copies = (K % 8 ? 7.0 : 3.5) + 0.7e-6 * batch * ((K % 8 ? (double)M * K : 0.0) + (double)K * N);
     // (where N alone is odd an [N, K] operand needs no copy: the small tiles have to win there as well)
-    if (whole) r.mid = r.plan.us < 0.95 * us;
-    else r.mid = r.plan.us < 0.85 * (us + copies) && (K % 8 || r.plan.us < us);
+    if (whole) r.mid = r.plan.ranges_us < 0.95 * us;
+    else r.mid = r.plan.ranges_us < 0.85 * (us + copies) && (K % 8 || r.plan.ranges_us < us);
     if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
     return r;
-}
-// One pass of 256-row tiles, in us (tiles of 256 x 256: fitted to 39 shapes, 8 % off)
-double tiles256_us(long M, long N, long K) {
-    const double rounds = (double)((((M + 255) / 256) * ((N + 255) / 256) + 255) / 256), mb = 2e-6 * ((double)M * K + (double)N * K + (double)M * N);
-    const double us = rounds * (1.02 * ((K + 63) / 64) + 5.8);
-    return 4.8 + (us > mb / 4.0 ? us : mb / 4.0);
 }
 // The gated (N = 2 F) and the rotary product: small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
 // two rounds of 256, against 860 of 128 x 128).  A negative answer: tiles of 256 x 256.
@@ -1297,6 +1305,9 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
     if (all % 16 || reinterpret_cast<uintptr_t>(cos) % 32 || reinterpret_cast<uintptr_t>(sin) % 32) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
     if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, N, K);
+    // In several rounds of small tiles each waits for its rows' angles anew (8000 x 3072 x 1024: 64.3 us on 256 x 128, 61.0 on 256 x 256; gated
+    // products of such sizes gain, 4096 x 5632 x 1024 55.0 -> 48.9)
+    if (mid_many_tiles(M, N, 1)) tile = -1;
     if (tile >= 0) {
         const MidRope angles{static_cast<const float*>(cos), static_cast<const float*>(sin), C_rest, (int)seq, (int)split};
         return launch_gemm_mid_paired(static_cast<hipStream_t>(stream), tile, A, B, C_rot, M, N, K, b_transposed, &angles);

@@ -9,11 +9,18 @@ struct MidPlan {
     int tile = -1;
     long splits = 1, kt_per_split = 0;
     double us = 0.0;
+    double ranges_us = 0.0;  // what the number of ranges follows from (us, where that is more than one)
 };
 constexpr int kMidSmallest = 3, kMidUnaligned = 4;  // tiles of 64 x 64: rows of whole chunks; rows that start on any element
+constexpr int kMidTall = 5;                         // tiles of 256 x 128
 // The fastest by estimate.  whole_chunks: rows of both operands are whole 16-byte chunks on 16-byte bases, whichever way B is stored; else
 // (N and K at least 8) they are read element-aligned.  paired: for the gated or the rotary epilogue, K in one range.
 MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool paired = false);
+// Whether a product of these extents in one range of K is a matter of the estimates below: long enough for a pipeline, whole chunks.
+inline bool mid_pipelined(long N, long K) { return N % 8 == 0 && K % 8 == 0 && K > 256; }
+inline bool mid_many_tiles(long M, long N, long batch) { return ((M + 127) / 128) * ((N + 255) / 256) * batch > 256; }
+// One pass of the tiles of gemm_bf16.hip (256 x 256, up to 256 tiles of 128 x 256 those) over such a product, in us
+double large_pass_us(long M, long N, long K, long batch);
 // rows, columns and stages of a tile
 void mid_tile_shape(int tile, int* rows, int* cols, int* stages);
 // C = A B (B [K, N] or, b_transposed, [N, K]); with p.splits > 1 the partial sums W[splits][batch][M][N] instead, without

@@ -1,15 +1,21 @@
 // 16-bit products on output tiles of 64 and 128 rows and columns: shapes whose 128 x 256 tiles (gemm_bf16.hip) would leave
 // compute units without work, and operands whose rows start on any element, read as they are.
 //
-// What bounds it: the path from the caches into the LDS.  A K step of a 128 x 128 tile brings 32 KB and takes 0.50 us
-// with one workgroup per compute unit (66 GB/s), one of a 64 x 64 tile 16 KB and 0.18 us with two or three (93 GB/s; 24 TB/s over the
-// chip, as 128 x 64 tiles reach with two), where the matrix instructions of either would take half of that; a 128 x 256 tile does
-// twice the work of the former in 0.68 us (73 GB/s), so it stays where enough such tiles exist (profiles/gemm_mid_steps.txt).  Hence smaller tiles for fewer rows and columns, K split over
-// workgroups where even those are few, and the choice by an estimate of the time (plan_mid).
+// What bounds it: with one workgroup on a compute unit, the instruction stream of its four waves.  A copy of 1 KB into the LDS waits for its
+// turn on the vector-memory path (one takes 16 cycles, four waves ask at once), and the matrix instructions behind it wait as well: a K step
+// of a 128 x 128 tile, 512 cycles of matrix instructions, 512 of copies and 512 of LDS reads, took 0.49 us (1170 cycles).  Above four steps of
+// K, four more waves make the copies, two waves to a SIMD, and the four that multiply issue nothing else but their LDS reads: 0.38 to 0.41 us, and a
+// launch starts 1 to 2 us sooner.  A ring of four or five stages changes neither (0.49 / 0.46 without such waves, 0.38 to 0.41 with them).  With several
+// workgroups on a compute unit the path from the caches into the LDS bounds it (94 GB/s, 24 TB/s over the chip; profiles/gemm_mid_steps.txt), with
+// or without them.  Tiles of 128 x 128 and more leave room for one workgroup: it takes its tiles in turn, and the next one's copies run under the stores
+// of the last (3076 x 3072 x 1024 28.1 -> 25.4 us, 512 x 50257 x 768 65 -> 54 against a workgroup to each).
+// Hence smaller tiles for fewer rows and columns, K split over workgroups where even those are few, and the choice by an estimate of the
+// time (plan_mid).
 //
-// us before (128 x 256 tiles, split along K where that paid, padded copies of odd operands) and now: 1024 x 1024 x 1024 12.3 / 7.3,
-// 198 x 3072 x 1024 12.2 / 7.5, [N, K] weights: 219 x 4288 x 3232 43.1 / 19.1, 700 x 700 x 4096 53.1 / 15.6,
-// 75 x 1536 x 4576 18.7 / 11.5, 1000 x 3000 x 2048 22.9 / 19.8, 2791 x 96 x 13584 30.0 / 25.0, 487 x 4920 x 13416 171 / 98; odd: 300 x 3001 x 777 23.4 / 8.5, 5 x 7152 x 1638 27.8 / 9.0.
+// us on 128 x 256 tiles (split along K where that paid, padded copies of odd operands), on these tiles without and with copying waves:
+// 1024 x 1024 x 1024 12.3 / 7.0 / 5.5, 1000 x 3000 x 2048 [N, K] 22.9 / 20.3 / 16.7, 3076 x 1024 x 1024 20.3 / 15.1 / 9.8, 512 x 8192 x 8192 92 / 74 / 56;
+// [N, K] weights: 219 x 4288 x 3232 43.1 / 19.1, 700 x 700 x 4096 53.1 / 15.6, 75 x 1536 x 4576 18.7 / 11.5; odd: 300 x 3001 x 777 23.4 / 8.5,
+// 5 x 7152 x 1638 27.8 / 9.0.  500 random products: 1.05 of the speed without copying waves (geometric mean), one slower by more than 4 %.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -37,6 +43,7 @@ __device__ __forceinline__ u32x4 shift_elems(u32x4 v, int by) {
 }
 
 // kTM x kTN output tile per workgroup of 4 waves (2 x 2), K step 64.  B is [K, N] or (kBT) [N, K].
+// kCopyWaves: eight waves, of which the last four make all copies; workgroups take tiles blockIdx.x, + gridDim.x, ... in turn (else one each).
 // kDirect: operand rows are whole 16-byte chunks (K, and N of a [K, N] operand, multiples of 8) on 16-byte bases: tiles go
 // global -> LDS directly, a ring of kAhead stages.  Otherwise (rows that start on any element, K and N at least 8) they pass
 // through registers: kAhead register sets in flight and two stages.
@@ -47,8 +54,8 @@ __device__ __forceinline__ u32x4 shift_elems(u32x4 v, int by) {
 // The products, their order per accumulator and the roundings are those of the tiled kernels of gemm_bf16.hip: the same bits.
 // The columns of a pair of 16-column matrix tiles are dealt to the two so that a lane ends up with eight consecutive ones.
 enum MidEpilogue { kPlain, kGate, kRotate };
-template <int kTM, int kTN, int kAhead, bool kBT, bool kF16, bool kDirect, bool kSplit, MidEpilogue kEpilogue = kPlain>
-__global__ __launch_bounds__(256, 2) void gemm_mid(
+template <int kTM, int kTN, int kAhead, bool kBT, bool kF16, bool kDirect, bool kSplit, MidEpilogue kEpilogue = kPlain, bool kCopyWaves = false>
+__global__ __launch_bounds__(kCopyWaves ? 512 : 256, !kCopyWaves || kTM * kTN >= 128 * 128 ? 2 : kTM * kTN == 128 * 64 ? 4 : 6) void gemm_mid(
     const __bf16* __restrict__ A, const __bf16* __restrict__ B, __bf16* __restrict__ C, float* __restrict__ W, const __bf16* __restrict__ R,
     int r_pitch, int M, int N, int K, int tiles_m, int tiles_n, int kt_per_split, MidRope rope) {
     static_assert(kEpilogue == kPlain || (kDirect && !kSplit && !kF16), "the gated and the rotary epilogue: bf16, whole chunks, one range of K");
@@ -57,14 +64,11 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
     constexpr int kAStage = kTM * 128, kBStage = kTN * 128, kStage = kAStage + kBStage;
     constexpr int kStages = kDirect ? kAhead : 2;
     __shared__ __attribute__((aligned(1024))) char smem[kStages * kStage];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave_of_8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = kCopyWaves ? wave_of_8 & 3 : wave_of_8;
     const int wm = wave >> 1, wn = wave & 1;
     A += (size_t)blockIdx.y * M * K;
     B += (size_t)blockIdx.y * N * K;
-    int tile_m, tile_n;
-    tile_of_block(blockIdx.x, tiles_m, tiles_n, &tile_m, &tile_n);
-    const int m0 = tile_m * kTM;
-    const int n0 = tile_n * (kEpilogue == kGate ? kTN / 2 : kTN);  // (gated: of the F columns; rotary: the first in the order below)
+    int m0, n0;  // (gated: n0 of the F columns; rotary: the first in the order below)
     // Where column `c` of half `h` of the tile's column pair `p` lies: gated, F = N / 2 between gate and up; rotary, heads of 128
     auto paired_col = [&](int p, int h, int c) {
         if constexpr (kEpilogue == kGate) {
@@ -82,13 +86,16 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
     // the last step of the range is the partial last one of K
     const bool ragged = (K & 63) && kt0 + KT == KT_all;
 
+    auto at_tile = [&](int t) {
+        int tile_m, tile_n;
+        tile_of_block(t, tiles_m, tiles_n, &tile_m, &tile_n);
+        m0 = tile_m * kTM;
+        n0 = tile_n * (kEpilogue == kGate ? kTN / 2 : kTN);
+    };
+
     // Sources.  A and B^T chunk q of a wave: eight rows of 128 bytes, LDS chunk lane % 8 of row lane / 8 holds the logical chunk of
     // the row's swizzle.  Rows beyond the edge are the last valid one (their products are not stored).
-    const char* a_base = reinterpret_cast<const char*>(A + (size_t)m0 * K + (size_t)kt0 * 64);
-    // (paired columns are addressed from the first of B)
-    const int b_first = kEpilogue == kPlain ? n0 : 0;
-    const char* b_base = kBT ? reinterpret_cast<const char*>(B + (size_t)b_first * K + (size_t)kt0 * 64)
-                             : reinterpret_cast<const char*>(B + (size_t)kt0 * 64 * N + b_first);
+    const char *a_base, *b_base;
     const size_t b_step = kBT ? 128 : (size_t)N * 128;
     // first k of a lane's chunk q of A and of B inside a step (its k-row, [K, N] form)
     auto a_chunk = [&](int l, int q) { return ((l & 7) ^ (((wave * (kTM / 4) + q * 8 + (l >> 3)) >> 1) & 7)) * 8; };
@@ -98,28 +105,35 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
     };
     unsigned a_off[kAq], b_off[kBq];  // byte offsets of the chunks from the bases of a step
     int b_back[kBq];                  // [K, N] form at the edge of N: elements by which a chunk was moved back to end at N
+    auto sources = [&]() {
+        a_base = reinterpret_cast<const char*>(A + (size_t)m0 * K + (size_t)kt0 * 64);
+        // (paired columns are addressed from the first of B)
+        const int b_first = kEpilogue == kPlain ? n0 : 0;
+        b_base = kBT ? reinterpret_cast<const char*>(B + (size_t)b_first * K + (size_t)kt0 * 64)
+                     : reinterpret_cast<const char*>(B + (size_t)kt0 * 64 * N + b_first);
 #pragma unroll
-    for (int q = 0; q < kAq; q++) {
-        const int r = wave * (kTM / 4) + q * 8 + (lane >> 3), row = m0 + r < M ? r : M - 1 - m0;
-        a_off[q] = (unsigned)row * (unsigned)K * 2u + (kDirect ? a_chunk(lane, q) * 2 : 0);
-    }
-#pragma unroll
-    for (int q = 0; q < kBq; q++) {
-        b_back[q] = 0;
-        if constexpr (kBT) {
-            const int r = wave * (kTN / 4) + q * 8 + (lane >> 3);
-            const int row = kEpilogue != kPlain ? paired_col(r >> 5, (r >> 2) & 1, 4 * ((r & 31) >> 3) + (r & 3)) : n0 + r < N ? r : N - 1 - n0;
-            b_off[q] = (unsigned)row * (unsigned)K * 2u + (kDirect ? b_chunk(lane, q) * 2 : 0);
-        } else {
-            // k-rows of kTN * 2 bytes, 64-byte granules swizzled by the k-row
-            const int kr = b_chunk(lane, q), ch = lane % (kTN / 8), f = kTN == 128 ? kr & 3 : (kr >> 1) & 1;
-            const int col = (((ch >> 2) ^ f) * 4 + (ch & 3)) * 8;
-            // (paired: a granule holds 16 columns of one half, then the 16 of the other)
-            const int c = kEpilogue != kPlain ? paired_col((ch >> 2) ^ f, (ch >> 1) & 1, (ch & 1) * 8) / 8 * 8 : n0 + col + 8 <= N ? col : N - 8 - n0;
-            b_off[q] = (unsigned)(kr * N + c) * 2u;
-            b_back[q] = col - c;
+        for (int q = 0; q < kAq; q++) {
+            const int r = wave * (kTM / 4) + q * 8 + (lane >> 3), row = m0 + r < M ? r : M - 1 - m0;
+            a_off[q] = (unsigned)row * (unsigned)K * 2u + (kDirect ? a_chunk(lane, q) * 2 : 0);
         }
-    }
+#pragma unroll
+        for (int q = 0; q < kBq; q++) {
+            b_back[q] = 0;
+            if constexpr (kBT) {
+                const int r = wave * (kTN / 4) + q * 8 + (lane >> 3);
+                const int row = kEpilogue != kPlain ? paired_col(r >> 5, (r >> 2) & 1, 4 * ((r & 31) >> 3) + (r & 3)) : n0 + r < N ? r : N - 1 - n0;
+                b_off[q] = (unsigned)row * (unsigned)K * 2u + (kDirect ? b_chunk(lane, q) * 2 : 0);
+            } else {
+                // k-rows of kTN * 2 bytes, 64-byte granules swizzled by the k-row
+                const int kr = b_chunk(lane, q), ch = lane % (kTN / 8), f = kTN == 128 ? kr & 3 : (kr >> 1) & 1;
+                const int col = (((ch >> 2) ^ f) * 4 + (ch & 3)) * 8;
+                // (paired: a granule holds 16 columns of one half, then the 16 of the other)
+                const int c = kEpilogue != kPlain ? paired_col((ch >> 2) ^ f, (ch >> 1) & 1, (ch & 1) * 8) / 8 * 8 : n0 + col + 8 <= N ? col : N - 8 - n0;
+                b_off[q] = (unsigned)(kr * N + c) * 2u;
+                b_back[q] = col - c;
+            }
+        }
+    };
     const int lds_w = wave * (kAq * 1024);
     const int lds_wb = kAStage + wave * (kBq * 1024);
 
@@ -136,12 +150,6 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
         }
     }
     f32x4 acc[kI][kP][2];
-#pragma unroll
-    for (int i = 0; i < kI; i++)
-#pragma unroll
-        for (int p = 0; p < kP; p++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) acc[i][p][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     // Fragments are read a 32-deep sub-step ahead of their matrix instructions, into two register slots.
     bf16x8 fa[2][kI], fb[2][kP][2];
@@ -170,6 +178,14 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
     auto mfma = [&](f32x4& c, const bf16x8& a, const bf16x8& b) {
         if constexpr (kF16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
         else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    };
+    auto clear_acc = [&]() {
+#pragma unroll
+        for (int i = 0; i < kI; i++)
+#pragma unroll
+            for (int p = 0; p < kP; p++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) acc[i][p][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     };
     auto touch_acc = [&]() {
 #pragma unroll
@@ -203,9 +219,116 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
     using K0 = std::integral_constant<int, 0>;
     using K1 = std::integral_constant<int, 1>;
     auto none = [](int) {};
-    touch_acc();
-    asm volatile("s_nop 7" ::: "memory");
+    auto start_acc = [&]() {
+        clear_acc();
+        touch_acc();
+        asm volatile("s_nop 7" ::: "memory");
+    };
+    // stores the tile at m0, n0
+    auto finish = [&]() {
+        // the last matrix instructions' results have to have left the matrix pipe before the vector unit reads them
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        touch_acc();
 
+        if constexpr (kEpilogue != kPlain) {
+            // lane l: C[m = i * 16 + l % 16], columns 4 * (l / 16) + 0..3 of either half of a pair
+            const int row_p = wm * kWM + (lane & 15), c4 = 4 * (lane >> 4);
+            const bool rotated = kEpilogue == kRotate && n0 < rope.split;
+#pragma unroll
+            for (int i = 0; i < kI; i++) {
+                const int row = m0 + row_p + i * 16;
+                if (row >= M) continue;
+                const size_t pos = rotated ? (size_t)(row % rope.seq) * 64 : 0;
+#pragma unroll
+                for (int p = 0; p < kP; p++) {
+                    const int pair = wn * kP + p;
+                    const f32x4 x = __builtin_convertvector(round_to_elem<false>(acc[i][p][0]), f32x4);
+                    const f32x4 y = __builtin_convertvector(round_to_elem<false>(acc[i][p][1]), f32x4);
+                    if constexpr (kEpilogue == kGate) {
+                        const int F = N >> 1, col = n0 + pair * 16 + c4;
+                        f32x4 o;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            // x * sigmoid(x) * y with sigmoid(x) = 1 / (1 + exp2(x * (-1 / ln 2)))
+                            const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x[e] * -1.4426950408889634f));
+                            o[e] = x[e] * sg * y[e];
+                        }
+                        if (col < F) *reinterpret_cast<bf16x4*>(C + (size_t)row * F + col) = __builtin_convertvector(o, bf16x4);
+                    } else {
+                        const int in_head = ((n0 & 127) >> 1) + pair * 16 + c4, col = (n0 & ~127) + in_head;
+                        f32x4 first = x, second = y;
+                        if (rotated) {
+                            const f32x4 cs = *reinterpret_cast<const f32x4*>(rope.cos + pos + in_head), sn = *reinterpret_cast<const f32x4*>(rope.sin + pos + in_head);
+                            // (the product that is rounded is the cosine's, as in the tiles of 256 x 256: left to the compiler it was the sine's here,
+                            // and 386 of 25 million results an ulp from theirs)
+                            first = __builtin_elementwise_fma(y, -sn, x * cs);
+                            second = __builtin_elementwise_fma(x, sn, y * cs);
+                        }
+                        // rotated columns: row pitch `split`; those behind: a matrix of their own
+                        const size_t ldc = rotated ? (size_t)rope.split : (size_t)(N - rope.split);
+                        __bf16* at = (rotated ? C : static_cast<__bf16*>(rope.rest) - rope.split) + (size_t)row * ldc + col;
+                        if (col < N) *reinterpret_cast<bf16x4*>(at) = __builtin_convertvector(first, bf16x4);
+                        if (col + 64 < N) *reinterpret_cast<bf16x4*>(at + 64) = __builtin_convertvector(second, bf16x4);
+                    }
+                }
+            }
+            return;
+        }
+        // With swapped operands lane l holds, in the eight registers of a pair, C[m = i * 16 + l % 16][n = pair * 32 + 8 * (l / 16) + 0..7].
+        const int row_l = wm * kWM + (lane & 15), col_l = wn * kWN + 8 * (lane >> 4);
+        if constexpr (kSplit) {
+            float* Wt = W + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * (size_t)M * N;
+#pragma unroll
+            for (int i = 0; i < kI; i++)
+#pragma unroll
+                for (int p = 0; p < kP; p++) {
+                    const int row = m0 + row_l + i * 16, col = n0 + col_l + p * 32;
+                    if (row >= M) continue;
+                    float* at = Wt + (size_t)row * N + col;
+                    if (col + 8 <= N) {
+                        *reinterpret_cast<f32x4_any*>(at) = acc[i][p][0];
+                        *reinterpret_cast<f32x4_any*>(at + 4) = acc[i][p][1];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 7; e++)
+                            if (col + e < N) at[e] = acc[i][p][e >> 2][e & 3];
+                    }
+                }
+            return;
+        }
+        __bf16* Cb = C + (size_t)blockIdx.y * M * N;
+        const __bf16* Rb = R + (size_t)blockIdx.y * M * r_pitch;
+#pragma unroll
+        for (int i = 0; i < kI; i++)
+#pragma unroll
+            for (int p = 0; p < kP; p++) {
+                const int row = m0 + row_l + i * 16, col = n0 + col_l + p * 32;
+                if (row >= M) continue;
+                const bf16x4 lo = round_to_elem<kF16>(acc[i][p][0]), hi = round_to_elem<kF16>(acc[i][p][1]);
+                u32x4 v = __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                __bf16* at = Cb + (size_t)row * N + col;
+                const __bf16* r = Rb + (size_t)row * r_pitch + col;
+                if (col + 8 <= N) {
+                    if (R) {
+                        const u32x4 add = *reinterpret_cast<const u32x4_any*>(r);
+                        v = add_elems<kF16>(v, add);
+                    }
+                    *reinterpret_cast<u32x4_any*>(at) = v;
+                } else if (col < N) {
+                    if (R) {
+                        bf16x8 e8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+                        for (int e = 0; e < 7; e++)
+                            if (col + e < N) e8[e] = r[e];
+                        v = add_elems<kF16>(v, __builtin_bit_cast(u32x4, e8));
+                    }
+                    const bf16x8 e8 = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+                    for (int e = 0; e < 7; e++)
+                        if (col + e < N) at[e] = e8[e];
+                }
+            }
+    };
     if constexpr (kDirect) {
         const unsigned lds0 = (unsigned)(uintptr_t)LDS_PTR(char, smem);
         const char* zero16 = reinterpret_cast<const char*>(g_zero16);
@@ -238,6 +361,71 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(stage + lds_wb + q * 1024), "v"(at) : "m0");
             }
         };
+        if constexpr (kCopyWaves) {
+            const int tiles = tiles_m * tiles_n;
+            const int rounds = ((tiles - (int)blockIdx.x - 1) / (int)gridDim.x) + 1;
+            if (wave_of_8 >= 4) {
+                // The copying waves: one sequence of steps over all of the workgroup's tiles, up to kStages ahead of the multiplying waves.  Both
+                // meet at one barrier a step.  (A copy that waits for an issue slot holds up all waves one step on: priority.)
+                __builtin_amdgcn_s_setprio(1);
+                const int total = rounds * KT;
+                int t = blockIdx.x, kt = 0, slot = 0;
+                const char *as, *bs;
+                auto aim = [&]() {
+                    at_tile(t);
+                    sources();
+                    as = a_base;
+                    bs = b_base;
+                };
+                auto copy_step = [&]() {  // the step at (t, kt) into `slot`
+                    if (ragged && kt == KT - 1) copy_ragged(kt, lds0 + slot * kStage);
+                    else {
+#pragma unroll
+                        for (int c = 0; c < kCopies; c++) copy_at(c, lds0 + slot * kStage, as, bs, 1);
+                    }
+                    as += 128;
+                    bs += b_step;
+                    slot = slot == kStages - 1 ? 0 : slot + 1;
+                    if (++kt == KT) {
+                        kt = 0;
+                        t += gridDim.x;
+                        if (t < tiles) aim();
+                    }
+                };
+                aim();
+#pragma clang loop unroll(disable)
+                for (int g = 0; g < kStages && g < total; g++) copy_step();
+                if (total >= kStages) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((kStages - 1) * kCopies) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+                for (int g = 0; g + 1 < total; g++) {
+                    // step g + 1 has landed (those behind it may be in flight), and everyone has read step g
+                    if (g + kStages <= total) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((kStages - 2) * kCopies) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+                    if (g + kStages < total) copy_step();
+                }
+                return;
+            }
+            asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+            for (int n = 0; n < kReads; n++) read_one(K0{}, n, smem);
+            int slot = 0, left = rounds * KT;
+            for (int r = 0; r < rounds; r++) {
+                at_tile(blockIdx.x + r * gridDim.x);
+                start_acc();
+                for (int kt = 0; kt < KT; kt++) {
+                    half(K0{}, std::true_type{}, smem + slot * kStage, none, std::integral_constant<int, 0>{});
+                    // everyone has read this step, and the next one has landed (there is none behind the last: what is read then is not used)
+                    if (--left) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    slot = slot == kStages - 1 ? 0 : slot + 1;
+                    half(K1{}, std::true_type{}, smem + slot * kStage, none, std::integral_constant<int, 0>{});
+                }
+                finish();
+            }
+            return;
+        }
+        at_tile(blockIdx.x);
+        sources();
+        start_acc();
 #pragma unroll
         for (int t = 0; t < kStages; t++)
             if (t < KT) {
@@ -253,19 +441,19 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
         for (int n = 0; n < kReads; n++) read_one(K0{}, n, smem);
         // Step kt: its first half carries the second half of the copies of tile kt - 1 + kStages, which the barrier in the
         // middle of step kt - 1 made room for, its second half the first of those of tile kt + kStages.
+        int steps = KT;
+        asm volatile("" : "+s"(steps));  // (kept from being tied to the tests above: the loop would be split up and its accumulators copied)
         int slot = 0, prev = 0;
         int live = 0;  // > 0: there is such a tile
         const char *as = a_base + (size_t)kStages * 128, *bs = b_base + (size_t)kStages * b_step;  // tile kt + kStages
         const char *as_p = as, *bs_p = bs;                                                        // the one whose copies are under way
-        for (int kt = 0; kt < KT; kt++) {
-            const char* st = smem + slot * kStage;
-            half(K0{}, std::true_type{}, st, [&](int c) { copy_at(kCopies / 2 + c, lds0 + prev * kStage, as_p, bs_p, live); }, std::integral_constant<int, kCopies / 2>{});
-            if (kt + 1 == KT) break;
+        for (int kt = 0; kt + 1 < steps; kt++) {
+            half(K0{}, std::true_type{}, smem + slot * kStage, [&](int c) { copy_at(kCopies / 2 + c, lds0 + prev * kStage, as_p, bs_p, live); }, std::integral_constant<int, kCopies / 2>{});
             // stage kt + 1 has landed (the copies of the kStages - 2 behind it may be in flight), and everyone has read stage kt
-            if (kt + kStages <= KT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((kStages - 2) * kCopies) : "memory");
+            if (kt + kStages <= steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((kStages - 2) * kCopies) : "memory");
             else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            live = __builtin_amdgcn_readfirstlane(KT - kStages - kt);
-            if (ragged && kt + kStages == KT - 1) {
+            live = __builtin_amdgcn_readfirstlane(steps - kStages - kt);
+            if (ragged && kt + kStages == steps - 1) {
                 copy_ragged(kt + kStages, lds0 + slot * kStage);
                 live = 0;
             }
@@ -277,10 +465,14 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
             as += 128;
             bs += b_step;
         }
+        half(K0{}, std::true_type{}, smem + slot * kStage, none, std::integral_constant<int, 0>{});
         half(K1{}, std::false_type{}, nullptr, none, std::integral_constant<int, 0>{});
     } else {
         // Through registers: chunks of 2-byte alignment.  In the partial last step a chunk that reaches past K is read where it ends at
         // K and moved down, so nothing behind a row is read; likewise the column chunks of a [K, N] operand at the edge of N.
+        at_tile(blockIdx.x);
+        sources();
+        start_acc();
         u32x4 ra[kAhead][kAq], rb[kAhead][kBq];
         auto load = [&](int set, int kt) {
             const char* as = a_base + (size_t)kt * 128;
@@ -343,106 +535,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
             }
         }
     }
-    // the last matrix instructions' results have to have left the matrix pipe before the vector unit reads them
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-    touch_acc();
-
-    if constexpr (kEpilogue != kPlain) {
-        // lane l: C[m = i * 16 + l % 16], columns 4 * (l / 16) + 0..3 of either half of a pair
-        const int row_p = wm * kWM + (lane & 15), c4 = 4 * (lane >> 4);
-        const bool rotated = kEpilogue == kRotate && n0 < rope.split;
-#pragma unroll
-        for (int i = 0; i < kI; i++) {
-            const int row = m0 + row_p + i * 16;
-            if (row >= M) continue;
-            const size_t pos = rotated ? (size_t)(row % rope.seq) * 64 : 0;
-#pragma unroll
-            for (int p = 0; p < kP; p++) {
-                const int pair = wn * kP + p;
-                const f32x4 x = __builtin_convertvector(round_to_elem<false>(acc[i][p][0]), f32x4);
-                const f32x4 y = __builtin_convertvector(round_to_elem<false>(acc[i][p][1]), f32x4);
-                if constexpr (kEpilogue == kGate) {
-                    const int F = N >> 1, col = n0 + pair * 16 + c4;
-                    f32x4 o;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        // x * sigmoid(x) * y with sigmoid(x) = 1 / (1 + exp2(x * (-1 / ln 2)))
-                        const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x[e] * -1.4426950408889634f));
-                        o[e] = x[e] * sg * y[e];
-                    }
-                    if (col < F) *reinterpret_cast<bf16x4*>(C + (size_t)row * F + col) = __builtin_convertvector(o, bf16x4);
-                } else {
-                    const int in_head = ((n0 & 127) >> 1) + pair * 16 + c4, col = (n0 & ~127) + in_head;
-                    f32x4 first = x, second = y;
-                    if (rotated) {
-                        const f32x4 cs = *reinterpret_cast<const f32x4*>(rope.cos + pos + in_head), sn = *reinterpret_cast<const f32x4*>(rope.sin + pos + in_head);
-                        first = x * cs + y * -sn;
-                        second = y * cs + x * sn;
-                    }
-                    // rotated columns: row pitch `split`; those behind: a matrix of their own
-                    const size_t ldc = rotated ? (size_t)rope.split : (size_t)(N - rope.split);
-                    __bf16* at = (rotated ? C : static_cast<__bf16*>(rope.rest) - rope.split) + (size_t)row * ldc + col;
-                    if (col < N) *reinterpret_cast<bf16x4*>(at) = __builtin_convertvector(first, bf16x4);
-                    if (col + 64 < N) *reinterpret_cast<bf16x4*>(at + 64) = __builtin_convertvector(second, bf16x4);
-                }
-            }
-        }
-        return;
-    }
-    // With swapped operands lane l holds, in the eight registers of a pair, C[m = i * 16 + l % 16][n = pair * 32 + 8 * (l / 16) + 0..7].
-    const int row_l = wm * kWM + (lane & 15), col_l = wn * kWN + 8 * (lane >> 4);
-    if constexpr (kSplit) {
-        float* Wt = W + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * (size_t)M * N;
-#pragma unroll
-        for (int i = 0; i < kI; i++)
-#pragma unroll
-            for (int p = 0; p < kP; p++) {
-                const int row = m0 + row_l + i * 16, col = n0 + col_l + p * 32;
-                if (row >= M) continue;
-                float* at = Wt + (size_t)row * N + col;
-                if (col + 8 <= N) {
-                    *reinterpret_cast<f32x4_any*>(at) = acc[i][p][0];
-                    *reinterpret_cast<f32x4_any*>(at + 4) = acc[i][p][1];
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 7; e++)
-                        if (col + e < N) at[e] = acc[i][p][e >> 2][e & 3];
-                }
-            }
-        return;
-    }
-    C += (size_t)blockIdx.y * M * N;
-    if (R) R += (size_t)blockIdx.y * M * r_pitch;
-#pragma unroll
-    for (int i = 0; i < kI; i++)
-#pragma unroll
-        for (int p = 0; p < kP; p++) {
-            const int row = m0 + row_l + i * 16, col = n0 + col_l + p * 32;
-            if (row >= M) continue;
-            const bf16x4 lo = round_to_elem<kF16>(acc[i][p][0]), hi = round_to_elem<kF16>(acc[i][p][1]);
-            u32x4 v = __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            __bf16* at = C + (size_t)row * N + col;
-            const __bf16* r = R + (size_t)row * r_pitch + col;
-            if (col + 8 <= N) {
-                if (R) {
-                    const u32x4 add = *reinterpret_cast<const u32x4_any*>(r);
-                    v = add_elems<kF16>(v, add);
-                }
-                *reinterpret_cast<u32x4_any*>(at) = v;
-            } else if (col < N) {
-                if (R) {
-                    bf16x8 e8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-#pragma unroll
-                    for (int e = 0; e < 7; e++)
-                        if (col + e < N) e8[e] = r[e];
-                    v = add_elems<kF16>(v, __builtin_bit_cast(u32x4, e8));
-                }
-                const bf16x8 e8 = __builtin_bit_cast(bf16x8, v);
-#pragma unroll
-                for (int e = 0; e < 7; e++)
-                    if (col + e < N) at[e] = e8[e];
-            }
-        }
+    if constexpr (!kCopyWaves) finish();
 }
 
 }  // namespace mrk::dev
@@ -450,6 +543,9 @@ __global__ __launch_bounds__(256, 2) void gemm_mid(
 namespace mrk {
 
 namespace {
+// Up to four steps of K the multiplying waves copy as well: 1.5 to 2.5 us of copies in flight hide nothing, and starting four more waves costs 0.15 to
+// 0.25 us (541 x 1216 x 192 3.47 us / 3.73 with them, 567 x 512 x 256 3.65 / 3.81; 384 deep and more is faster with them).
+constexpr long kFewSteps = 4;
 // The tiles and what one costs in us, fitted to 25000 timings of every tile and number of ranges over 950 shapes (10 to 12 % off,
 // root mean square): start of a launch, step of K that waits for its data (any number of workgroups resident at
 // once), step of one workgroup more on the same compute unit, start and end of a workgroup, TB/s of the operands, TB/s of what all
@@ -476,13 +572,58 @@ constexpr Tile kPairedTiles[] = {
 };
 // The second launch of a split, in us: its start, per range, per MB of partial sums.  A split has to promise 4 % to be taken.
 constexpr double kReduce = 2.5, kReduceRange = 0.25, kReduceMb = 0.06, kSplitGain = 1.04;
+
+// Products in one range of K of more than four steps, whole chunks: what a pass of tiles takes, in us, fitted to 2800 timings over 1400 shapes
+// of 17 to 8192 rows and 256 to 52000 columns (11 % off, root mean square; the tile chosen by it costs 0.5 % over the best of them, and 0.55
+// of tiles of 128 x 256 alone).
+// Start of a launch; a step of K on an empty chip, what a chip with a workgroup on each compute unit adds, and one more on
+// the same compute unit (that one in parts: `whole` of it as soon as any compute unit has one); start and end of one more; the share a step
+// grows by per doubling of K beyond 2048; TB/s of the operands behind the first 64 MB (40 x 33792 x 2112 on 64 x 64: 30.4 us, 25.7 on 128 x 256).
+struct Timed {
+    int tile, tm, tn;
+    double start, step, full, layer, whole, edge, deep, tbps;
+};
+constexpr Timed kTimed[] = {
+    {1, 128, 128, 4.0, 0.265, 0.178, 0.334, 0.7, 3.3, 0.055, 4.7},
+    {2, 128, 64, 3.2, 0.202, 0.123, 0.259, 0.51, 1.0, 0.078, 4.7},
+    {kMidSmallest, 64, 64, 2.9, 0.167, 0.070, 0.176, 0.35, 0.46, 0.092, 4.7},
+    {kMidTall, 256, 128, 5.5, 0.449, 0.241, 0.0, 0.0, 0.0, 0.009, 4.7},  // (in one round)
+};
+constexpr Timed kTimed128x256 = {-1, 128, 256, 4.6, 0.508, 0.203, 0.0, 0.0, 0.0, 0.019, 7.0};  // (in one round)
+double timed_us(const Timed& t, double groups, double kt, double K, double operands) {
+    const double x = groups / 256, layers = std::ceil(x) - 1;
+    const double step = t.step + t.full * (x < 1.0 ? x : 1.0) + t.layer * (layers * t.whole + (x > 1.0 ? x - 1.0 : 0.0) * (1.0 - t.whole));
+    const double multiply = step * kt * (K > 2048 ? 1.0 + t.deep * std::log2(K / 2048) : 1.0), read = operands < 64.0 ? operands / 7.0 : 64.0 / 7.0 + (operands - 64.0) / t.tbps;
+    return t.start + t.edge * layers + (multiply > read ? multiply : read);
+}
+// The same where more than 256 tiles of 128 x 256 exist: start of a launch, per round of 256 tiles its start and end and a step of K, what a
+// step of the last round is shorter by where that is not full; TB/s of the operands.  Fitted to the 262 of those timings (10 % off): 0.967
+// of the time of tiles of 256 x 256 alone (1639 x 10368 x 416 34.4 / 23.5 us), which win where K is long.
+struct Rounds {
+    int tile, tm, tn;
+    double start, round, step, spare, tbps;
+};
+constexpr Rounds kRounds[] = {{1, 128, 128, 2.5, 1.6, 0.462, 0.276, 19.0}, {kMidTall, 256, 128, 2.3, 3.6, 0.721, 0.264, 14.9}};
+constexpr Rounds kRounds256 = {-1, 256, 256, 0.0, 8.4, 1.268, 0.558, 6.2};
+double rounds_us(const Rounds& t, double groups, double kt, double operands) {
+    const double layers = std::ceil(groups / 256);
+    const double us = t.start + layers * (t.round + kt * t.step) - t.spare * kt * (layers - groups / 256);
+    return us > t.start + operands / t.tbps ? us : t.start + operands / t.tbps;
+}
+double operand_mb(long M, long N, long K, long batch) { return 2e-6 * batch * ((double)M * K + (double)N * K + (double)M * N); }
 }  // namespace
+
+double large_pass_us(long M, long N, long K, long batch) {
+    if (mid_many_tiles(M, N, batch))
+        return rounds_us(kRounds256, (double)(((M + 255) / 256) * ((N + 255) / 256) * batch), (double)((K + 63) / 64), operand_mb(M, N, K, batch));
+    return timed_us(kTimed128x256, (double)(((M + 127) / 128) * ((N + 255) / 256) * batch), (double)((K + 63) / 64), (double)K, operand_mb(M, N, K, batch));
+}
 
 MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool paired) {
     MidPlan best;
     if (M <= 0 || N < 8 || K < 8 || batch <= 0 || batch > 65535 || M > 0x7fffffffL || K > (1L << 23) || N > (1L << 24)) return best;
     const long kt = (K + 63) / 64;
-    const double operands = 2.0 * batch * ((double)M * K + (double)N * K + (double)M * N) * 1e-6;
+    const double operands = operand_mb(M, N, K, batch);
     // Long rows: each of a tile's is a page of its own, and workgroups that share an operand drift apart over many steps.  A step takes 10 %
     // longer per doubling of K, and the compute unit that holds the most workgroups ends last instead of the chip evening out
     // (376 tiles of 128 x 64: 1000 x 3000 x 2048 0.47 us a step; 308: 487 x 4920 x 13416 0.88).
@@ -491,8 +632,8 @@ MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool pai
         if ((i == kMidUnaligned) == whole_chunks) continue;
         const Tile& t = paired ? kPairedTiles[i] : kTiles[i];
         const long tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
-        // fewer than 2^32 work-items, 256 a tile, in the grid's first dimension (rotary: whole heads)
-        if ((double)tm * (paired ? ((N + 127) / 128 * 128 + t.tn - 1) / t.tn : tn) > 0xffffff) continue;
+        // fewer than 2^32 work-items, up to 512 a tile, in the grid's first dimension (rotary: whole heads)
+        if ((double)tm * (paired ? ((N + 127) / 128 * 128 + t.tn - 1) / t.tn : tn) > 0x7fffff) continue;
         for (long want : {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L}) {
             if (want > 1 && (paired || kt < 10)) break;  // few steps are not split
             const long per = (kt + want - 1) / want, splits = (kt + per - 1) / per, groups = tm * tn * batch * splits;
@@ -511,9 +652,22 @@ MidPlan plan_mid(long M, long N, long K, long batch, bool whole_chunks, bool pai
             if (i == kMidUnaligned && operands > 32.0 && 0.49 * per * waits > us) us = 0.49 * per * waits;
             us += t.start;
             if (splits > 1) us = (us + kReduce + kReduceRange * splits + kReduceMb * partial * 1e-6) * kSplitGain;
-            if (best.tile < 0 || us < best.us) best = MidPlan{i, splits, per, us};
+            if (best.tile < 0 || us < best.us) best = MidPlan{i, splits, per, us, us};
         }
     }
+    // How many ranges K is summed in is a matter of the estimates above alone: it decides the bits.
+    if (best.tile < 0 || best.splits > 1 || !whole_chunks || !mid_pipelined(N, K)) return best;
+    const double ranges_us = best.us;
+    best = MidPlan();
+    const bool many = mid_many_tiles(M, N, batch);
+    auto consider = [&](const auto& t, auto&& estimate) {
+        const long cols = paired ? (N + 127) / 128 * 128 : N, groups = ((M + t.tm - 1) / t.tm) * ((cols + t.tn - 1) / t.tn);
+        if ((double)groups > 0x7fffff || (!many && t.tile == kMidTall && (!paired || groups * batch > 256))) return;  // (the plain product has tiles of 128 x 256)
+        const double us = estimate(t, (double)groups * batch);
+        if (best.tile < 0 || us < best.us) best = MidPlan{t.tile, 1, kt, us, ranges_us};
+    };
+    if (many) for (const Rounds& t : kRounds) consider(t, [&](const Rounds& r, double groups) { return rounds_us(r, groups, (double)kt, operands); });
+    else for (const Timed& t : kTimed) consider(t, [&](const Timed& r, double groups) { return timed_us(r, groups, (double)kt, (double)K, operands); });
     return best;
 }
 
@@ -528,12 +682,17 @@ void with_tile(int tile, F&& f) {
         case 0: f(I128{}, I128{}, integral_constant<int, 2>{}); break;
         case 1: f(I128{}, I128{}, integral_constant<int, 3>{}); break;
         case 2: f(I128{}, I64{}, integral_constant<int, 3>{}); break;
+        case kMidTall: f(integral_constant<int, 256>{}, I128{}, integral_constant<int, 3>{}); break;
         default: f(I64{}, I64{}, integral_constant<int, 3>{}); break;
     }
 }
 }  // namespace
 
 void mid_tile_shape(int tile, int* rows, int* cols, int* stages) {
+    if (tile == kMidTall) {
+        *rows = 256, *cols = 128, *stages = 3;
+        return;
+    }
     *rows = kTiles[tile].tm, *cols = kTiles[tile].tn;
     *stages = tile == kMidUnaligned || tile == 0 ? 2 : 3;
 }
@@ -541,18 +700,28 @@ void mid_tile_shape(int tile, int* rows, int* cols, int* stages) {
 int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* B, void* C, float* W, const void* add, long add_pitch, long M, long N, long K,
                     long batch, bool b_transposed, bool f16) {
     using namespace mrk::dev;
-    if (p.tile < 0 || p.tile >= 5) return (int)hipErrorInvalidValue;
+    if (p.tile < 0 || p.tile > kMidTall) return (int)hipErrorInvalidValue;
     const bool split = p.splits > 1;
     if (split && (!W || batch * p.splits > 65535)) return (int)hipErrorInvalidValue;
-    const long tm = (M + kTiles[p.tile].tm - 1) / kTiles[p.tile].tm, tn = (N + kTiles[p.tile].tn - 1) / kTiles[p.tile].tn;
+    int rows = 0, cols = 0, stages = 0;
+    mid_tile_shape(p.tile, &rows, &cols, &stages);
+    const long tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols;
     const dim3 grid((unsigned)(tm * tn), (unsigned)batch, (unsigned)(split ? p.splits : 1));
     auto go = [&](auto tile_m, auto tile_n, auto ahead, auto direct) {
         constexpr int kTM = decltype(tile_m)::value, kTN = decltype(tile_n)::value, kAhead = decltype(ahead)::value;
         constexpr bool kDirect = decltype(direct)::value;
         auto pick = [&](auto bt, auto half) {
             constexpr bool kBT = decltype(bt)::value, kF16 = decltype(half)::value;
-            auto kernel = split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true> : gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, false>;
-            kernel<<<grid, 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B), static_cast<__bf16*>(C), W,
+            // waves of their own copy in more than four steps; tiles of 128 x 128 and more, one workgroup to a compute unit, are taken in turn
+            constexpr bool kMay = kDirect && kAhead == 3, kAlways = kTM == 256;
+            const bool copy_waves = kMay && (kAlways || (split ? p.kt_per_split : (K + 63) / 64) > kFewSteps);
+            auto of = [&](auto waves) {
+                constexpr bool kWaves = decltype(waves)::value;
+                return split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true, kPlain, kWaves> : gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, false, kPlain, kWaves>;
+            };
+            auto kernel = copy_waves ? of(std::integral_constant<bool, kMay>{}) : of(std::integral_constant<bool, kAlways>{});
+            const bool in_turn = copy_waves && kTM * kTN >= 128 * 128 && !split && batch == 1 && tm * tn > 256;
+            kernel<<<in_turn ? dim3(256) : grid, copy_waves ? 512 : 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B), static_cast<__bf16*>(C), W,
                                         static_cast<const __bf16*>(add), (int)add_pitch, (int)M, (int)N, (int)K, (int)tm, (int)tn, (int)p.kt_per_split,
                                         MidRope{});
         };
@@ -570,15 +739,23 @@ int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* 
 int launch_gemm_mid_paired(hipStream_t s, int tile, const void* A, const void* B, void* C, long M, long N, long K, bool b_transposed,
                            const MidRope* rope) {
     using namespace mrk::dev;
-    if (tile < 0 || tile >= kMidUnaligned || (rope && (rope->split % 128 || rope->seq <= 0))) return (int)hipErrorInvalidValue;
-    const long tm = (M + kTiles[tile].tm - 1) / kTiles[tile].tm;
+    if (tile < 0 || tile > kMidTall || tile == kMidUnaligned || (rope && (rope->split % 128 || rope->seq <= 0))) return (int)hipErrorInvalidValue;
+    int rows = 0, width = 0, stages = 0;
+    mid_tile_shape(tile, &rows, &width, &stages);
+    const long tm = (M + rows - 1) / rows;
     // (a tile of 64 columns takes half of a head's pairs: the last head is covered whole)
-    const long cols = rope ? (N + 127) / 128 * 128 : N, tn = (cols + kTiles[tile].tn - 1) / kTiles[tile].tn;
+    const long cols = rope ? (N + 127) / 128 * 128 : N, tn = (cols + width - 1) / width;
     with_tile(tile, [&](auto tile_m, auto tile_n, auto stages) {
         constexpr int kTM = decltype(tile_m)::value, kTN = decltype(tile_n)::value, kStages = decltype(stages)::value;
-        auto kernel = rope ? (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kRotate> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kRotate>)
-                           : (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kGate> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kGate>);
-        kernel<<<dim3((unsigned)(tm * tn)), 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B), static_cast<__bf16*>(C), nullptr, nullptr, 0,
+        constexpr bool kMay = kStages == 3, kAlways = kTM == 256;
+        const bool copy_waves = kMay && (kAlways || K > 64 * kFewSteps), in_turn = copy_waves && kTM * kTN >= 128 * 128 && tm * tn > 256;
+        auto of = [&](auto waves) {
+            constexpr bool kWaves = decltype(waves)::value;
+            return rope ? (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kRotate, kWaves> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kRotate, kWaves>)
+                        : (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kGate, kWaves> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kGate, kWaves>);
+        };
+        auto kernel = copy_waves ? of(std::integral_constant<bool, kMay>{}) : of(std::integral_constant<bool, kAlways>{});
+        kernel<<<dim3(in_turn ? 256u : (unsigned)(tm * tn)), copy_waves ? 512 : 256, 0, s>>>(static_cast<const __bf16*>(A), static_cast<const __bf16*>(B), static_cast<__bf16*>(C), nullptr, nullptr, 0,
                                                          (int)M, (int)N, (int)K, (int)tm, (int)tn, 0, rope ? *rope : MidRope{});
     });
     return (int)hipGetLastError();

@@ -1,0 +1,86 @@
+"""16-bit products whose copies are made by waves of their own, in one range of K long enough for the pipeline (more than four steps): every
+tile such a product can be sent to, with ragged rows and columns, whole and partial last steps of K.  As in test_gemm_routes_gpu.py each
+shape states its tile, checked on the CPU; the checks themselves are those of the tests imported here."""
+import numpy as np
+import pytest
+
+import morok_amd
+from morok_amd import synth
+from tests.test_gemm_bf16_gpu import (test_gemm_rotary_epilogue as _rotary, test_gemm_swiglu_epilogue_parity as _gated,
+                                      test_gemm_transposed_second_operand as _transposed,
+                                      test_gemm_transposed_second_operand_epilogues as _transposed_epilogues)
+from tests.test_gemm_mid_gpu import test_small_tiles_exact as _exact
+from tests.test_gemm_routes_gpu import _tile
+
+PLAIN = {
+    (65, 72, 328): (64, 64, 1, 3),        # one row and one chunk of columns past a tile
+    (256, 2048, 512): (64, 64, 1, 3),     # whole tiles
+    (129, 5592, 360): (128, 64, 1, 3),
+    (384, 3072, 1024): (128, 64, 1, 3),
+    (341, 5464, 328): (128, 128, 1, 3),
+    (1541, 4968, 328): (128, 128, 1, 3),  # more than 256 tiles of 128 x 256
+    (2492, 3144, 328): (256, 128, 1, 3),
+}
+GATED = {(68, 144, 392): (64, 64, 1, 3), (147, 5456, 360): (128, 64, 1, 3), (2055, 912, 328): (128, 128, 1, 3), (2124, 2880, 328): (256, 128, 1, 3)}
+ROTARY = {(67, 264, 384, 256, 50): (64, 64, 1, 3), (147, 5384, 384, 5120, 147): (128, 64, 1, 3), (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
+          (2124, 2888, 384, 2816, 531): (256, 128, 1, 3)}
+
+
+def test_shapes_reach_the_tiles_they_stand_for():
+    for nt in (False, True):
+        for shape, tile in PLAIN.items():
+            assert _tile(*shape, nt) == tile, shape
+        for shape, tile in GATED.items():
+            assert _tile(*shape, nt, True) == tile, shape
+        for (m, n, k, _, _), tile in ROTARY.items():
+            assert _tile(m, n, k, nt, True) == tile, (m, n, k)
+        for m, tile in ((1830, (256, 128)), (732, (128, 128)), (61, (64, 64))):  # (of the last test)
+            assert _tile(m, 3112, 384, nt, True)[:2] == tile, m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", list(PLAIN))
+def test_plain_bias_and_residual_exact(dev, shape, nt, f16):
+    _exact(dev, (*shape, 1), nt, f16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", list(PLAIN))
+def test_both_layouts_give_the_same_bits(dev, oracle, shape):
+    _transposed(dev, oracle, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", list(GATED))
+def test_gated_epilogue(dev, oracle, shape):
+    m, n, k = shape
+    _gated(dev, oracle, (m, n // 2, k))
+    _transposed_epilogues(dev, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", list(ROTARY))
+def test_rotary_epilogue(dev, oracle, shape):
+    _rotary(dev, oracle, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [False, True])
+def test_rotation_gives_the_same_bits_on_every_tile(dev, nt):
+    """The same rows in a product of each tile: 256 x 256 (2440 rows) rounds the products of a rotation as the small tiles do."""
+    n, k, split, seq = 3112, 384, 3072, 61
+    rows = (2440, 1830, 732, 61)
+    a, b = synth.normal_bf16((2440, k), 31, 0), synth.normal_bf16((k, n), 31, 1, sigma=k ** -0.5)
+    angle = synth.uniform((seq, 64), 31, 2).astype(np.float64) * 3.0
+    cos, sin = (morok_amd.Buffer.from_numpy(f(angle).astype(np.float32), dev.device_id) for f in (np.cos, np.sin))
+    bb = morok_amd.Buffer.from_numpy(np.ascontiguousarray(b.T) if nt else b, dev.device_id)
+    got = []
+    for m in rows:
+        ba = morok_amd.Buffer.from_numpy(np.ascontiguousarray(a[:m]), dev.device_id)
+        rot, rest = dev.buffer(m * split * 2), dev.buffer(m * (n - split) * 2)
+        morok_amd.Program.builtin("gemm_bf16_nt_rope" if nt else "gemm_bf16_rope", [m, n, k, split, seq], dev.device_id).execute([rot, ba, bb, rest, cos, sin])
+        got.append((rot.copyout(np.uint16, (m, split)), rest.copyout(np.uint16, (m, n - split))))
+    for rot, rest in got[1:]:
+        assert np.array_equal(rot, got[0][0][:len(rot)]) and np.array_equal(rest, got[0][1][:len(rest)])
