@@ -393,7 +393,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     // without delaying the next one: the reads take the first slots of a phase one by one, every
     // copy (M0, the wait state, the load) a later slot of its own, its source address the slot
     // before, and the carried scalars the tail of the last phase.
-    auto phase = [&](auto p_c, auto cur_c, const char* sAn, const char* sBn) {
+    auto phase = [&](auto p_c, auto cur_c, auto last_c, const char* sAn, const char* sBn) {
         constexpr int p = decltype(p_c)::value, cur = decltype(cur_c)::value;
         constexpr int slot = p >> 1, nslot = slot ^ 1, h = p & 1;
         constexpr int kHalfJ = kJ16 / 2;  // tile columns per half
@@ -404,7 +404,8 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         constexpr int kEvery = (kSlots - kFirst - kTail) / kCopies;  // slots per copy (address, then copy)
         static_assert(kEvery >= 2, "a copy needs two slots");
         const unsigned lds_dst = p < 2 ? lds_b + ls.sb_fill : lds_a + cur * kAStageT;
-        const bool ragged_now = kAny && has_last && ls.kt2 == KT - 1;  // this step copies the partial last tile
+        constexpr bool kMaybe = kAny && decltype(last_c)::value;         // one of the last steps, which copy the last tile
+        const bool ragged_now = kMaybe && has_last && ls.kt2 == KT - 1;  // this step copies the partial last tile
         const char* src = p < 2 ? ls.b_src : ls.a_src;
         if (p == 1 && !kBT) src += 4 * b_row2;
 #pragma unroll
@@ -420,7 +421,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             const int c = copy_range ? (n - kFirst) / kEvery : 0, part = copy_range ? (n - kFirst) % kEvery : -1;
             const int q = (p & 1) * kCopies + c;  // chunk of the tile
             // a copy slot: the MFMA and the copy as one statement; where a step may have to copy
-            // the partial last tile instead (kAny) the choice is made at run time, and the MFMA
+            // the partial last tile instead (kMaybe) the choice is made at run time, and the MFMA
             // stays outside that branch: an accumulator that flows through a branch would be moved
             // by the compiler, which does not know that it has to wait for the matrix pipe first
             auto with_q = [&](auto&& f) {
@@ -439,7 +440,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                 constexpr int qq = decltype(q_c)::value;
                 return p >= 2 ? a_voff[qq < kAq ? qq : 0] : kBT ? bt_voff[kBT ? qq : 0] : b_voff[qq & 1];
             };
-            if (part == 1 && !kAny) {
+            if (part == 1 && !kMaybe) {
                 with_q([&](auto q_c) { mfma_dma(acc[mi][mj], fb[slot][mj], fa[slot][mi], lds_dst, q_c, voff_of(q_c), src); });
             } else {
                 mfma(acc[mi][mj], fb[slot][mj], fa[slot][mi]);
@@ -503,7 +504,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     using C2 = std::integral_constant<int, 2>;
     using C3 = std::integral_constant<int, 3>;
     // tile kt: A in stage cur = kt & 1, B in the stage at ls.sb_cur (next tile's B at ls.sb_nxt, the one after goes to ls.sb_fill)
-    auto iteration = [&](auto cur_c) {
+    auto iteration = [&](auto cur_c, auto last_c) {
         constexpr int cur = decltype(cur_c)::value;
         using C = std::integral_constant<int, cur>;
         const char* sAc = sA0 + cur * kAStageT + a_base_l;
@@ -512,12 +513,12 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         const char* sBx = sB0 + ls.sb_nxt + (kBT ? bt_base_l : 0);
         // sub-step ks of a B stage: 32 k-rows of 512 B further, or (kBT) the same chunk offset as A's
         auto b_ks = [&](int ks) { return kBT ? a_xo[ks] : ks * 32 * 512; };
-        phase(C0{}, C{}, sAc + a_xo[1], sBc + b_ks(1));
-        phase(C1{}, C{}, sAc + a_xo[1], sBc + b_ks(1));
+        phase(C0{}, C{}, last_c, sAc + a_xo[1], sBc + b_ks(1));
+        phase(C1{}, C{}, last_c, sAc + a_xo[1], sBc + b_ks(1));
         // tile kt+1 has landed; nobody reads A stage cur any more
         tile_barrier();
-        phase(C2{}, C{}, sAx + a_xo[0], sBx + b_ks(0));
-        phase(C3{}, C{}, sAx + a_xo[0], sBx + b_ks(0));
+        phase(C2{}, C{}, last_c, sAx + a_xo[0], sBx + b_ks(0));
+        phase(C3{}, C{}, last_c, sAx + a_xo[0], sBx + b_ks(0));
     };
     // What the epilogue of the plain and the residual product needs, ahead of the loop's end: lane l
     // stores (and fetches from R) 16-byte chunk l % kChunks of row it * kRowsPerIt + l / kChunks of
@@ -531,6 +532,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     const bool col_ok = col0 + lc * 8 + 8 <= (size_t)N;
     // columns of this lane's chunk inside C when the chunk is the partial last one of a row (kAny: N % 8 of them), else 0
     const int col_tail = kAny && !col_ok && col0 + lc * 8 < (size_t)N ? (int)((size_t)N - (col0 + lc * 8)) : 0;
+    const bool inside = rows_here == 128 && col0 + kJ * 32 <= (size_t)N;  // the whole wave's tile
     auto store_any = [&](__bf16* dst, const u32x4& v, bool row_ok) {
         if (col_ok && row_ok) *reinterpret_cast<u32x4_any*>(dst) = v;
         else if (row_ok) {
@@ -549,7 +551,8 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             const __bf16* src = Rl + (size_t)(it * kRowsPerIt) * r_pitch;
             if constexpr (kAny) {
                 const bool row_ok = it * kRowsPerIt + lr < rows_here;
-                if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
+                if (inside) res[it] = *reinterpret_cast<const u32x4_any*>(src);
+                else if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
                 else if (row_ok) {
                     bf16x8 e8 = __builtin_bit_cast(bf16x8, res[it]);
 #pragma unroll
@@ -563,12 +566,22 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
         }
     };
     {
+        using Last = std::true_type;
         int kt = 0;
-        for (; kt + 1 < KT; kt += 2) {
-            iteration(C0{});
-            iteration(C1{});
+        // (512 x 50264 x 776 with the choice of the source in every step 52.6 us, 49.6 so; 4096 x 4096 x 4088 107.6 / 94.4; odd columns, which
+        // have no partial step, 512 x 50257 x 768 47.1 / 43.7 with whole tiles stored without a test, 1000 x 30001 x 2048 103.7 / 90.0)
+        if constexpr (kAny) {
+            const int whole = has_last ? KT - 3 : KT;  // the first step that copies tile KT - 1, clamped to which those behind it do as well
+            for (; kt + 1 < whole; kt += 2) {
+                iteration(C0{}, std::false_type{});
+                iteration(C1{}, std::false_type{});
+            }
         }
-        if (kt < KT) iteration(C0{});
+        for (; kt + 1 < KT; kt += 2) {
+            iteration(C0{}, Last{});
+            iteration(C1{}, Last{});
+        }
+        if (kt < KT) iteration(C0{}, Last{});
     }
     // The residual rows are on their way while the accumulators are converted and staged: the
     // fragment registers of the loop are free from here on.  (Fetching half of them before the
@@ -685,7 +698,10 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
-                if constexpr (kAny) store_any(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
+                if constexpr (kAny) {
+                    if (inside) *reinterpret_cast<u32x4_any*>(Cl + (size_t)r * ldc) = v[t];
+                    else store_any(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
+                }
                 else if (col_ok && r + lr < rows_here) *reinterpret_cast<u32x4*>(Cl + (size_t)r * ldc) = v[t];
             }
         }
