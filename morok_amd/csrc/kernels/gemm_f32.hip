@@ -25,12 +25,13 @@
 // short of the old error they need two levels of them.)  Error against 64 bits, 2-norm, uniform operands, in 1e-7, before and
 // now: 1000 x 1000 x K 0.77 / 0.59 at K = 130, 0.82 / 0.78 at 257, 1.04 / 0.78 at 1000, 1.62 / 0.78 at 4000; 130 x 200 x K
 // 0.77 / 0.74, 0.82 / 0.71, 1.04 / 0.77, 1.60 / 1.00; 1024 x 1024 x K 2.05 / 1.48, 2.88 / 2.06, 5.67 / 4.02, 11.3 / 8.0.
-// Bound by the f32 matrix rate (157 TFLOP/s nominal).  Measured: 1024^3 24.7 us (87 TFLOP/s; generated kernel on the vector
-// ALUs 55.3), [N, K] weight 22.3; 4096^3 1.11 ms (124 TFLOP/s); 1000^3 29.1 us (reduction 3500); 64 x 256 x 784 against
+// Bound by the f32 matrix rate (157 TFLOP/s nominal).  Measured: 1024^3 22.7 us (95 TFLOP/s; generated kernel on the vector
+// ALUs 55.3); 4096^3 1.06 ms (129 TFLOP/s); 1000^3 28.7 us (reduction 3500); 64 x 256 x 784 against
 // a [N, K] weight 4.3 us (36.8 and a transposing copy before).
 // Rows that are no whole groups of four are read in 16-byte loads of 4-byte alignment, the last group of a row where it ends with the
-// row; element by element before: 368 x 932 x 1342 59.9 -> 39.0 us, 602 x 640 x 1031 45.3 -> 31.0, 896 x 958 x 768 31.6 -> 24.4, same bits.
-// What is left at 1024^3, one workgroup per CU: the fill and drain of sixteen steps, and the barrier in each.
+// row; element by element before: 368 x 932 x 1342 59.9 -> 39.0 us, 602 x 640 x 1031 45.3 -> 31.0, 896 x 958 x 768 31.6 -> 24.4 (22.5 now), same bits.
+// What is left at 1024^3, one workgroup per CU: the launch and the fill and drain of sixteen steps.  Not the barrier in each: a third stage, with
+// the next step's fragments read before this step's last matrix instructions, measured 23.1 us against 22.7.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -204,7 +205,27 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
     }
     constexpr int kLoads = kT ? 4 : 6;
     int k_next = 0;  // first k of the step to be fetched
-    auto fetch = [&](f32x4v(&v)[kLoads]) {
+    // Steps that end before K does (`inside`) need neither a clamped k nor zeros: their offsets are worked out here, once.
+    unsigned inside_at[kLoads];
+    if constexpr (kT == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) inside_at[i] = a_fixed[i] + (unsigned)kr * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) inside_at[4 + i] = b_fixed[i] + (kFlip ? (unsigned)(b_kr + i) * (unsigned)N * 4u : (unsigned)b_kr * 4u);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) inside_at[i] = fixed[i] + (unsigned)(transpose ? kr + i : kr) * pitch;
+    }
+    auto fetch = [&](auto inside, f32x4v(&v)[kLoads]) {
+        if constexpr (decltype(inside)::value) {
+            const char* a_at = (kT ? base : a_base) + (long)k_next * (kT ? pitch : 4u);
+            const char* b_at = kT ? a_at : b_base + (long)k_next * (kFlip ? (long)N * 4 : 4);
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) v[i] = *reinterpret_cast<const f32x4_any*>((i < 4 ? a_at : b_at) + inside_at[i]);
+            k_next += kBK;
+            __builtin_amdgcn_sched_barrier(0);
+            return;
+        }
         if constexpr (kT == 0) {
             const int kb = k_next <= (int)K - kBK ? k_next : (int)K > kBK ? (int)K - kBK : 0;
             const int k = kr + (k_next - kb), bk = b_kr + (k_next - kb), last = (int)K - 1 - kb;
@@ -234,14 +255,15 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
         __builtin_amdgcn_sched_barrier(0);  // the loads set out before the step's matrix instructions, not after them
     };
     const bool columns_end = !kVec && transpose && past < kBN && (N & 3), rows_end = !kVec && !transpose && (K & 3);
-    auto stash = [&](float* st, int k0, const f32x4v(&v)[kLoads]) {
+    auto stash = [&](auto inside, float* st, int k0, const f32x4v(&v)[kLoads]) {
+        constexpr bool kInside = decltype(inside)::value;
         const int left = (int)K - k0 - kr;
         if constexpr (kT == 0) {
             f32x4v z[6];
 #pragma unroll
             for (int i = 0; i < 6; i++) z[i] = v[i];
             if constexpr (!kVec) {
-                if ((K & 3) && k0 + kBK > (int)K) {
+                if (!kInside && (K & 3) && k0 + kBK > (int)K) {
                     const int by = left < 4 ? 4 - left : 0;
 #pragma unroll
                     for (int i = 0; i < (kFlip ? 4 : 6); i++) z[i] = move_down(z[i], by);
@@ -254,14 +276,14 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
 #pragma unroll
             for (int i = 0; i < (kFlip ? 4 : 6); i++)
 #pragma unroll
-                for (int x = 0; x < 4; x++) z[i][x] = (kVec ? 0 : x) < left ? z[i][x] : 0.0f;
+                for (int x = 0; x < 4; x++) z[i][x] = kInside || (kVec ? 0 : x) < left ? z[i][x] : 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4v*>(st + a_to[i]) = z[i];
             if constexpr (kFlip) {
                 const int b_left = (int)K - k0 - b_kr;
 #pragma unroll
                 for (int x = 0; x < 4; x++)
-                    *reinterpret_cast<f32x2*>(st + b_to[x]) = f32x2{0 < b_left ? z[4][x] : 0.0f, 1 < b_left ? z[5][x] : 0.0f};
+                    *reinterpret_cast<f32x2*>(st + b_to[x]) = f32x2{kInside || 0 < b_left ? z[4][x] : 0.0f, kInside || 1 < b_left ? z[5][x] : 0.0f};
             } else {
 #pragma unroll
                 for (int i = 0; i < 2; i++) *reinterpret_cast<f32x4v*>(st + b_to[i]) = z[4 + i];
@@ -271,7 +293,7 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
         f32x4v z[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) z[i] = v[i];
-        if (!kVec && (columns_end || (rows_end && k0 + kBK > (int)K))) {
+        if (!kVec && (columns_end || (!kInside && rows_end && k0 + kBK > (int)K))) {
             const int by = transpose ? moved : left < 4 ? 4 - left : 0;
 #pragma unroll
             for (int i = 0; i < 4; i++) z[i] = move_down(z[i], by);
@@ -279,7 +301,7 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int x = 0; x < 4; x++) z[i][x] = (transpose ? i : kVec ? 0 : x) < left ? z[i][x] : 0.0f;
+            for (int x = 0; x < 4; x++) z[i][x] = kInside || (transpose ? i : kVec ? 0 : x) < left ? z[i][x] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++)
             *reinterpret_cast<f32x4v*>(st + to[i]) = transpose ? f32x4v{z[0][i], z[1][i], z[2][i], z[3][i]} : z[i];
@@ -303,11 +325,16 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
 
     const int steps = (int)((K + kBK - 1) / kBK);
     // Step s multiplies stage s & 1 while step s + 1's operands are on their way to registers since step s - 1 (an L2 miss
-    // takes longer than a step) and step s + 2's set out.
+    // takes longer than a step) and step s + 2's set out.  `inside`: step s + 2 ends before K does.  Those steps' offsets and zeros
+    // are not worked out again and again: f32 matrix instructions leave the vector ALUs no time of their own (us before / now: 1024^3
+    // 24.0 / 22.7, 512 x 1024 x 1024 16.1 / 14.4, 1408 x 320 x 1408 20.7 / 18.4, 896 x 958 x 768 24.1 / 22.5, 4096^3 1084 / 1062).
+    // A second form of the step spills where 64-bit totals fill the registers (700 x 500 x 777 17.7 / 23.1): not there.
+    constexpr bool kTwoForms = kRun == 0 || (kT == 1 && !kVec);
     f32x4v in0[kLoads], in1[kLoads];
-    auto step = [&](int s, f32x4v(&arriving)[kLoads], f32x4v(&leaving)[kLoads]) {
+    auto step = [&](auto inside, int s, f32x4v(&arriving)[kLoads], f32x4v(&leaving)[kLoads]) {
+        constexpr bool kAll = decltype(inside)::value || !kTwoForms;  // nothing is left out of the last steps
         const float* st = smem + (s & 1) * kStage;
-        fetch(leaving);
+        if (kAll || s + 2 < steps) fetch(inside, leaving);
         const int slot = group * (kSlots / kGroups) + lg;
         f32x4v fa[2][kMi], fb[2][kNj];
         auto fragments = [&](int c) {
@@ -347,18 +374,28 @@ __device__ __forceinline__ void f32_tiled_body(const float* __restrict__ A, cons
             }
         }
         // (the other stage was last read in step s - 1, which every wave has left at the barrier before this step)
-        stash(smem + ((s + 1) & 1) * kStage, (s + 1) * kBK, arriving);
+        if (kAll || s + 1 < steps) stash(inside, smem + ((s + 1) & 1) * kStage, (s + 1) * kBK, arriving);
         __syncthreads();
     };
-    fetch(in0);
-    fetch(in1);
-    stash(smem, 0, in0);
+    constexpr std::true_type kInside{};
+    constexpr std::false_type kEdge{};
+    fetch(kEdge, in0);
+    fetch(kEdge, in1);
+    stash(kEdge, smem, 0, in0);
     __syncthreads();
-    for (int s = 0; s + 1 < steps; s += 2) {
-        step(s, in1, in0);
-        step(s + 1, in0, in1);
+    int s = 0;
+    if constexpr (kTwoForms) {
+        const int full = (int)(K / kBK);
+        for (; s + 3 < full; s += 2) {
+            step(kInside, s, in1, in0);
+            step(kInside, s + 1, in0, in1);
+        }
     }
-    if (steps & 1) step(steps - 1, in1, in0);
+    for (; s + 1 < steps; s += 2) {
+        step(kEdge, s, in1, in0);
+        step(kEdge, s + 1, in0, in1);
+    }
+    if (s < steps) step(kEdge, s, in1, in0);
     auto sum = [&](int i, int j, int e) -> Total {
         if constexpr (kRun == 0) return acc[i][j][e];
         else return total[i][j][e];

@@ -68,3 +68,14 @@ def test_tiles_of_64_by_32_exact(dev, shape, nt):
 @pytest.mark.parametrize("shape", TWO_ROUNDS)
 def test_tiles_of_64_by_32_are_no_less_exact_than_64_partial_sums(dev, shape, nt):
     ragged_accuracy(*shape, nt)
+
+
+# Steps that end before K does run a loop of their own, two at a time, up to the three that meet the end of K: every count of whole steps around
+# it, with a partial one behind and without.  Whole tiles of 64 x 64 (steps of 64), of 64 x 32 and of 128 x 128 (steps of 32), rows in no
+# groups of four
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("k", [64, 96, 100, 128, 132, 160, 192, 200, 256, 260, 320, 323, 384, 448, 516])
+def test_steps_inside_of_k_exact(dev, k, nt):
+    for M, N in ((640, 640), (512, 1024), (2048, 2048), (901, 963)):
+        test_rows_of_any_length_exact(dev, (M, N, k), nt)
