@@ -2764,9 +2764,10 @@ struct Scheduler {
             todo.pop_back();
             if (std::find(found.begin(), found.end(), R) != found.end()) continue;
             if (!qualifies(R)) {
-                // a reduction of another shape directly under n rules the fusion out; further down it is
-                // simply computed first, like any other input
-                if (std::find(deps.begin(), deps.end(), R) != deps.end()) return {};
+                // Computed first, like any other input.  Directly under n only what reduces another tensor (a product whose rows are
+                // normalised: log_softmax of a classifier's 64 x 10 logits 3 launches, 1 now): a reduction of the row itself that has to be
+                // in memory anyway leaves this kernel less to keep.
+                if (R->src.size() == 1 && R->src[0]->shape == n->shape && std::find(deps.begin(), deps.end(), R) != deps.end()) return {};
                 continue;
             }
             found.push_back(R);

@@ -652,6 +652,11 @@ def test_row_resident_fusion_needs_a_path_that_keeps_the_row(T):
     chain = x.try_sub(m.try_transpose(0, 1).try_expand([256, 256])).try_exp()
     bad_chain = chain.try_div(chain.sum(1, keepdim=True).try_expand([256, 256]))
     assert not any(k.endswith("_x2") for k in names(bad_chain))
+    # a reduction of another tensor is an input like any other; one of the row's tensor along another axis keeps the separate kernels
+    logits = zeros(T, (64, 256)).linear(zeros(T, (10, 256)), zeros(T, (10,))).log_softmax(-1)
+    assert len(names(logits)) == 2 and T.last_kernels()[-1].startswith("rE_64_g10")
+    centred = x.try_sub(x.sum(0, keepdim=True).try_expand([256, 256]))
+    assert len(names(centred.try_sub(centred.max(1, keepdim=True).try_expand([256, 256])))) >= 2
     good = names(zeros(T, (256, 1024), np.uint16, uop.BF16).softmax(-1))
     assert len(good) == 1 and good[0].startswith("rE_") and good[0].endswith("_x2")
 

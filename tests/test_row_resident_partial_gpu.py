@@ -71,3 +71,40 @@ def test_side_output(dev):
     x = synth.from_bf16(table[ids])
     want = x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + 1e-6) * synth.from_bf16(w)
     assert np.abs(synth.from_bf16(y.to_numpy()) - want).max() <= 2.0 ** -8 * np.abs(want).max()
+
+
+# Rows that a product or another reduction leaves: that is computed first, the row's reductions and its elementwise part are one kernel
+@pytest.mark.parametrize("shape", [(64, 256, 10), (1, 33, 2), (3, 700, 257), (512, 32, 1000), (17, 64, 65)])
+@pytest.mark.parametrize("activation", [False, True])
+def test_log_softmax_of_a_product(dev, shape, activation):
+    b, k, c = shape
+    x, w, bias = synth.normal((b, k), 6, 0), synth.normal((c, k), 6, 1, sigma=k ** -0.5), synth.normal((c,), 6, 2)
+
+    def build():
+        t = T.Tensor.from_numpy(x)
+        if activation:
+            t = t.maximum(0.0)
+        return t.linear(T.Tensor.from_numpy(w), T.Tensor.from_numpy(bias)).log_softmax(-1)
+
+    y = build().realize()
+    assert y.kernels()[-1].startswith("rE_") and sum(n.startswith(("rE_", "r_")) for n in y.kernels()) <= 2, y.kernels()
+    z = (np.maximum(x, 0) if activation else x).astype(np.float64) @ w.T.astype(np.float64) + bias
+    m = z.max(-1, keepdims=True)
+    # (products of K terms in f32, up to |z| of about 10)
+    np.testing.assert_allclose(y.to_numpy(), z - (m + np.log(np.exp(z - m).sum(-1, keepdims=True))), rtol=1e-5, atol=2e-5)
+    np.testing.assert_allclose(y.to_numpy(), _separate(build), rtol=1e-5, atol=1e-5)
+
+
+def test_statistics_of_other_rows_and_columns_come_first(dev):
+    x, o = synth.normal((130, 520), 7, 0), synth.normal((520, 130, 3), 7, 1)
+    t, u = T.Tensor.from_numpy(x), T.Tensor.from_numpy(o)
+    columns = u.sum([1, 2]).try_reshape([1, 520]).try_expand([130, 520])  # a reduction of another tensor
+    build = lambda: t.try_add(columns).softmax(-1)  # noqa: E731
+    z = x.astype(np.float64) + o.astype(np.float64).sum((1, 2))
+    want = np.exp(z - z.max(-1, keepdims=True))
+    want /= want.sum(-1, keepdims=True)
+    np.testing.assert_allclose(build().to_numpy(), want, rtol=1e-4, atol=1e-7)  # (sums of 390 terms in f32 under an exponential)
+    y = t.try_sub(t.sum(0, keepdim=True).try_expand([130, 520])).log_softmax(-1).to_numpy()  # one of the row's own tensor along columns
+    z = x.astype(np.float64) - x.astype(np.float64).sum(0)
+    m = z.max(-1, keepdims=True)
+    np.testing.assert_allclose(y, z - (m + np.log(np.exp(z - m).sum(-1, keepdims=True))), rtol=1e-5, atol=1e-4)
