@@ -686,6 +686,14 @@ int mrk_hip_tensor_contiguous(const mrk_tensor* t, mrk_tensor** out);           
  * keys and values beside its output).  Plans from mrk_hip_tensor_prepare keep their root alone. */
 int mrk_hip_tensor_keep(const mrk_tensor* t);
 int mrk_hip_tensor_cat(const mrk_tensor* const* parts, size_t nparts, int64_t axis, mrk_tensor** out);
+/* The graph of one decode step of a pre-norm decoder block (RMSNorm, packed QKV, rotary, attention over the grown cache, output projection
+ * and residual, RMSNorm, gated MLP and residual), in one call: weights[7] = embedding, first gain, Wqkv, Wo, second gain, W1|W3, W2 in bf16
+ * ([in, out], or [out, in] with linear_layout), tokens int32 [batch], past keys and values [batch, heads, pos, dim] with the keys rotated, the
+ * position's row of cos and sin (dim / 2 floats) at byte offset row_offset of either table.  out[3] = output [batch, hidden], grown keys and
+ * values, which a realization of the output leaves realized (mrk_hip_tensor_keep).  On an error nothing is written to out. */
+int mrk_hip_tensor_decode_step(const mrk_tensor* const* weights, int linear_layout, const mrk_tensor* tokens, const mrk_tensor* past_k,
+                               const mrk_tensor* past_v, const mrk_buffer* cos_table, const mrk_buffer* sin_table, size_t row_offset,
+                               int64_t batch, int64_t hidden, int64_t heads, int64_t ffn, double eps, mrk_tensor** out);
 /* elementwise, with broadcasting and dtype promotion (dtype/src/cast.rs:88) */
 int mrk_hip_tensor_cast(const mrk_tensor* t, int dtype, mrk_tensor** out);                    /* lib.rs:495 */
 int mrk_hip_tensor_unary(const mrk_tensor* t, int unary_op, mrk_tensor** out);

@@ -214,6 +214,8 @@ _SIGS = {
     "mrk_hip_tensor_keep": (C.c_int, [C.c_void_p]),
     "mrk_hip_tensor_contiguous": (C.c_int, [C.c_void_p, c_void_pp]),
     "mrk_hip_tensor_cat": (C.c_int, [c_void_pp, C.c_size_t, C.c_int64, c_void_pp]),
+    "mrk_hip_tensor_decode_step": (C.c_int, [c_void_pp, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t,
+                                             C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_double, c_void_pp]),
     "mrk_hip_tensor_cast": (C.c_int, [C.c_void_p, C.c_int, c_void_pp]),
     "mrk_hip_tensor_unary": (C.c_int, [C.c_void_p, C.c_int, c_void_pp]),
     "mrk_hip_tensor_binary": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, c_void_pp]),

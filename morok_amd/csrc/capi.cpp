@@ -1366,6 +1366,34 @@ int mrk_hip_tensor_cat(const mrk_tensor* const* parts, size_t nparts, int64_t ax
     }
     return wrap_tensor(Tensor::cat(ts, axis), out);
 }
+int mrk_hip_tensor_decode_step(const mrk_tensor* const* weights, int linear_layout, const mrk_tensor* tokens, const mrk_tensor* past_k,
+                               const mrk_tensor* past_v, const mrk_buffer* cos_table, const mrk_buffer* sin_table, size_t row_offset,
+                               int64_t batch, int64_t hidden, int64_t heads, int64_t ffn, double eps, mrk_tensor** out) {
+    MRK_NONNULL(weights);
+    for (int i = 0; i < 7; i++) MRK_NONNULL(weights[i]);
+    MRK_NONNULL(tokens);
+    MRK_NONNULL(past_k);
+    MRK_NONNULL(past_v);
+    MRK_NONNULL(cos_table);
+    MRK_NONNULL(sin_table);
+    MRK_NONNULL(out);
+    clear_error();
+    if (heads <= 0 || hidden <= 0 || hidden % heads || hidden / heads % 2) return fail(kInvalidArgument, "decode step: hidden is no whole even heads");
+    const int64_t half = hidden / heads / 2;
+    std::unique_ptr<Buffer> cos, sin;
+    MRK_TRY(cos_table->b->view(row_offset, half * sizeof(float), &cos));
+    MRK_TRY(sin_table->b->view(row_offset, half * sizeof(float), &sin));
+    const Tensor c = Tensor::from_buffer(std::move(cos), {1, 1, 1, half}, Scalar::Float32), s = Tensor::from_buffer(std::move(sin), {1, 1, 1, half}, Scalar::Float32);
+    if (!c.valid() || !s.valid()) return last_status();
+    const DecodeStep step{weights[0]->t, weights[1]->t, weights[2]->t, weights[3]->t, weights[4]->t, weights[5]->t, weights[6]->t,
+                          linear_layout != 0, batch, hidden, heads, ffn, eps};
+    Tensor y, k, v;
+    MRK_TRY(step.build(tokens->t, past_k->t, past_v->t, c, s, &y, &k, &v));
+    out[0] = new mrk_tensor{std::move(y)};
+    out[1] = new mrk_tensor{std::move(k)};
+    out[2] = new mrk_tensor{std::move(v)};
+    return kOk;
+}
 int mrk_hip_tensor_cast(const mrk_tensor* t, int dtype, mrk_tensor** out) {
     MRK_T1(t);
     MRK_DTYPE(dtype);

@@ -521,6 +521,56 @@ Tensor Tensor::softmax(int64_t axis) const {
     return res;
 }
 
+int DecodeStep::build(const Tensor& tokens, const Tensor& past_k, const Tensor& past_v, const Tensor& cos, const Tensor& sin, Tensor* out,
+                      Tensor* keys, Tensor* values) const {
+    if (batch <= 0 || hidden <= 0 || heads <= 0 || ffn <= 0 || hidden % heads) return fail(kInvalidArgument, "decode step: sizes");
+    const int64_t B = batch, H = heads, D = hidden / heads;
+    Tensor t;
+    const auto ok = [&t](Tensor r) {
+        t = std::move(r);
+        return t.valid();
+    };
+    const auto project = [&](const Tensor& x, const Tensor& w) { return linear_layout ? x.linear(w, nullptr) : x.matmul(w); };
+    const auto normalize = [&](const Tensor& x, const Tensor& gain) {
+        return ok(x.rms_norm(-1, eps)) && ok(t.try_mul(gain)) && ok(t.cast(Scalar::BFloat16));
+    };
+    const auto columns = [&](const Tensor& x, int64_t from, int64_t to) { return x.try_shrink({0, from}, {B, to}); };
+    const auto heads_first = [&]() { return ok(t.try_permute({0, 2, 1, 3})); };
+    const auto failed = []() { return last_status() != kOk ? last_status() : fail(kInvalidArgument, "decode step: invalid operand"); };
+    if (!ok(emb.embedding(tokens)) || !ok(t.contiguous())) return failed();
+    const Tensor h = t;
+    if (!normalize(h, attn_gain) || !ok(project(t, Wqkv))) return failed();
+    const Tensor qkv = t;
+    if (!ok(columns(qkv, 0, 2 * hidden)) || !ok(t.try_reshape({B, 1, 2 * H, D})) || !ok(t.apply_rotary_emb(cos, sin, false)) ||
+        !ok(t.cast(Scalar::BFloat16)) || !ok(t.contiguous()))
+        return failed();
+    const Tensor qk = t;
+    if (!ok(qk.try_shrink({0, 0, 0, 0}, {B, 1, H, D})) || !heads_first()) return failed();
+    const Tensor q = t;
+    if (!ok(qk.try_shrink({0, 0, H, 0}, {B, 1, 2 * H, D})) || !heads_first() || !ok(Tensor::cat({past_k, t}, 2)) || !ok(t.contiguous())) return failed();
+    const Tensor k_all = t;
+    if (!ok(columns(qkv, 2 * hidden, 3 * hidden)) || !ok(t.try_reshape({B, 1, H, D})) || !heads_first() || !ok(Tensor::cat({past_v, t}, 2)) ||
+        !ok(t.contiguous()))
+        return failed();
+    const Tensor v_all = t;
+    // (kept: whoever realizes the output has the grown cache with it, and realizing those finds them done)
+    MRK_TRY(k_all.keep());
+    MRK_TRY(v_all.keep());
+    if (!ok(q.scaled_dot_product_attention(k_all, v_all, 0.0, false)) || !heads_first() || !ok(t.try_reshape({B, hidden})) || !ok(project(t, Wo)) ||
+        !ok(h.try_add(t)) || !ok(t.contiguous()))
+        return failed();
+    const Tensor h2 = t;
+    if (!normalize(h2, ffn_gain) || !ok(project(t, W13))) return failed();
+    const Tensor gate_up = t;
+    if (!ok(columns(gate_up, ffn, 2 * ffn))) return failed();
+    const Tensor up = t;
+    if (!ok(columns(gate_up, 0, ffn)) || !ok(t.silu()) || !ok(t.try_mul(up)) || !ok(project(t, W2)) || !ok(h2.try_add(t))) return failed();
+    *out = t;
+    *keys = k_all;
+    *values = v_all;
+    return kOk;
+}
+
 Tensor Tensor::log_softmax(int64_t axis) const {
     // x - max(x) - log(sum(exp(x - max(x))))  (activation.rs:117-128)
     if (!n_) return Tensor();

@@ -182,6 +182,19 @@ class Tensor {
     TensorRef n_;
 };
 
+// One decode step of a pre-norm decoder block, as a graph: the ops and their order are a caller's own (rms_norm, linear / matmul, rotary,
+// cat, attention, ...).  Built here because some forty calls across the C boundary and as many short-lived handles took longer than the kernels
+// of a small block (batch 1, hidden 1024, 300 keys: 162 us a step of which the graph 90).
+struct DecodeStep {
+    Tensor emb, attn_gain, Wqkv, Wo, ffn_gain, W13, W2;  // projections [in, out], linear_layout: [out, in]
+    bool linear_layout = false;
+    int64_t batch = 0, hidden = 0, heads = 0, ffn = 0;
+    double eps = 0.0;
+    // tokens int32 [batch]; past [batch, heads, pos, dim], keys rotated; cos / sin [1, 1, 1, dim / 2] of the new position
+    int build(const Tensor& tokens, const Tensor& past_k, const Tensor& past_v, const Tensor& cos, const Tensor& sin, Tensor* out, Tensor* keys,
+              Tensor* values) const;
+};
+
 // Per-thread switch: hand-written fused kernels on (default) or off (every op goes through
 // generated kernels) - the counterpart of choosing a backend through PrepareConfig
 // (tensor/src/config.rs:17-89).

@@ -9,7 +9,7 @@ import numpy as np
 
 from . import synth, uop
 from .device import Buffer
-from .tensor import Tensor
+from .tensor import Tensor, decode_step
 
 WEIGHT_NAMES = ("emb", "w_an", "Wq", "Wk", "Wv", "Wo", "w_fn", "W1", "W3", "W2")
 
@@ -118,8 +118,8 @@ class DecoderBlock:
         out = h2.try_add(self._proj(g, "W2"))
         return (out, k.contiguous(), v.contiguous()) if with_cache else out
 
-    def _rope_row(self, pos):
-        """cos and sin of one position as [1, 1, 1, dim/2] tensors: views of tables in device memory, made for 64 consecutive
+    def _rope_at(self, pos):
+        """The tables in device memory that hold cos and sin of position `pos`, and the byte offset of its row: made for 64 consecutive
         positions at a time (a step's own row costs no trigonometry, no upload and no wait, and a block that starts at a
         late position does not pay for those before it)."""
         half = self.dim // 2
@@ -130,7 +130,13 @@ class DecoderBlock:
             padded = np.zeros((2, 64, pitch), np.float32)
             padded[0, :, :half], padded[1, :, :half] = rope_tables(64, self.dim, self.theta, first)
             tables = self._rope[first] = [Buffer.from_numpy(t, self.device_id) for t in padded]
-        return [Tensor.from_buffer(t.view(row * pitch * 4, half * 4), (1, 1, 1, half), uop.F32) for t in tables]
+        return tables, row * pitch * 4
+
+    def _rope_row(self, pos):
+        """cos and sin of one position as [1, 1, 1, dim/2] tensors: views of those tables."""
+        tables, offset = self._rope_at(pos)
+        half = self.dim // 2
+        return [Tensor.from_buffer(t.view(offset, half * 4), (1, 1, 1, half), uop.F32) for t in tables]
 
     def decode_step(self, tokens, past_k, past_v, pos):
         """One new token per sequence against the keys and values of the `pos` tokens before it, the way the reference
@@ -141,24 +147,5 @@ class DecoderBlock:
         pos + 1 tokens would give for the last token.  With Linear-layout weights the projections stream their weights
         once, and the attention is one query per head over pos + 1 keys."""
         assert self.fused, "decode_step uses the packed projections"
-        w, B, H, D = self.w, self.batch, self.heads, self.dim
-        cos_p, sin_p = self._rope_row(pos)
-        h = w["emb"].embedding(tokens).contiguous()
-        xn = self._norm(h, w["w_an"])
-        qkv = self._proj(xn, "Wqkv")
-        xv = qkv.try_shrink([(0, B), (2 * self.hidden, 3 * self.hidden)])
-        qk = qkv.try_shrink([(0, B), (0, 2 * self.hidden)]).try_reshape([B, 1, 2 * H, D])
-        qk = qk.apply_rotary_emb(cos_p, sin_p, False).cast(uop.BF16).contiguous()
-        q = qk.try_shrink([(0, B), (0, 1), (0, H), (0, D)]).try_permute([0, 2, 1, 3])
-        k_new = qk.try_shrink([(0, B), (0, 1), (H, 2 * H), (0, D)]).try_permute([0, 2, 1, 3])
-        v_new = xv.try_reshape([B, 1, H, D]).try_permute([0, 2, 1, 3])
-        # kept: whoever realizes the output has the grown cache with it, and realizing those finds them done
-        k_all = Tensor.cat([past_k, k_new], 2).contiguous().keep()
-        v_all = Tensor.cat([past_v, v_new], 2).contiguous().keep()
-        a = q.scaled_dot_product_attention(k_all, v_all)
-        a = a.try_permute([0, 2, 1, 3]).try_reshape([B, self.hidden])
-        h2 = h.try_add(self._proj(a, "Wo")).contiguous()
-        xn2 = self._norm(h2, w["w_fn"])
-        gu = self._proj(xn2, "W13")
-        g = gu.try_shrink([(0, B), (0, self.ffn)]).silu().try_mul(gu.try_shrink([(0, B), (self.ffn, 2 * self.ffn)]))
-        return h2.try_add(self._proj(g, "W2")), k_all, v_all
+        weights = [self.w[k] for k in ("emb", "w_an", "Wqkv", "Wo", "w_fn", "W13", "W2")]
+        return decode_step(weights, self.linear_layout, tokens, past_k, past_v, *self._rope_at(pos), self.batch, self.hidden, self.heads, self.ffn, self.eps)

@@ -366,3 +366,12 @@ class Tensor:
         h = C.c_void_p()
         check(lib.mrk_hip_tensor_buffer(self._h, C.byref(h)))
         return Buffer(math.prod(self.shape) * _ITEMSIZE[self.dtype], _handle=h)
+
+
+def decode_step(weights, linear_layout, tokens, past_k, past_v, rope_tables, row_offset, batch, hidden, heads, ffn, eps):
+    """The graph of one decode step of a decoder block, in one call: see mrk_hip_tensor_decode_step.  The forty ops it is made of took 90 us of a
+    162 us step (batch 1, hidden 1024, 300 keys) when each was a call of its own."""
+    out = (C.c_void_p * 3)()
+    check(lib.mrk_hip_tensor_decode_step((C.c_void_p * 7)(*[w._h for w in weights]), int(linear_layout), tokens._h, past_k._h, past_v._h,
+                                         rope_tables[0]._h, rope_tables[1]._h, row_offset, batch, hidden, heads, ffn, float(eps), out))
+    return tuple(Tensor(C.c_void_p(h)) for h in out)

@@ -819,6 +819,45 @@ def test_decode_step_is_one_realization(T, shim):
         assert k.realize().kernels() == [] and v.realize().kernels() == [] and k.shape == (2, 2, pos + 1, 128)
 
 
+def composed_decode_step(T, blk, ids, past_k, past_v, pos):
+    """The decode step as tensor ops, one call each."""
+    from morok_amd import uop
+
+    w, B, H, D, hidden, ffn = blk.w, blk.batch, blk.heads, blk.dim, blk.hidden, blk.ffn
+    cos, sin = blk._rope_row(pos)
+    h = w["emb"].embedding(ids).contiguous()
+    qkv = blk._proj(blk._norm(h, w["w_an"]), "Wqkv")
+    qk = qkv.try_shrink([(0, B), (0, 2 * hidden)]).try_reshape([B, 1, 2 * H, D]).apply_rotary_emb(cos, sin, False).cast(uop.BF16).contiguous()
+    q = qk.try_shrink([(0, B), (0, 1), (0, H), (0, D)]).try_permute([0, 2, 1, 3])
+    k = qk.try_shrink([(0, B), (0, 1), (H, 2 * H), (0, D)]).try_permute([0, 2, 1, 3])
+    v = qkv.try_shrink([(0, B), (2 * hidden, 3 * hidden)]).try_reshape([B, 1, H, D]).try_permute([0, 2, 1, 3])
+    k, v = (T.Tensor.cat([past, new], 2).contiguous().keep() for past, new in ((past_k, k), (past_v, v)))
+    a = q.scaled_dot_product_attention(k, v).try_permute([0, 2, 1, 3]).try_reshape([B, hidden])
+    h2 = h.try_add(blk._proj(a, "Wo")).contiguous()
+    gu = blk._proj(blk._norm(h2, w["w_fn"]), "W13")
+    g = gu.try_shrink([(0, B), (0, ffn)]).silu().try_mul(gu.try_shrink([(0, B), (ffn, 2 * ffn)]))
+    return h2.try_add(blk._proj(g, "W2")), k, v
+
+
+@pytest.mark.parametrize("linear_layout", [False, True])
+@pytest.mark.parametrize("batch,pos", [(1, 0), (2, 300), (3, 31)])
+def test_decode_step_is_the_graph_of_its_ops(T, batch, pos, linear_layout):
+    from morok_amd import decoder, uop
+
+    blk = decoder.DecoderBlock(decoder.synthetic_weights(256, 512, 100, seed=1), batch, 1, 256, 2, 512, linear_layout=linear_layout)
+    ids = T.Tensor.from_numpy(np.zeros(batch, np.int32))
+    past = T.Tensor.from_numpy(np.zeros((batch, 2, pos, 128), np.uint16), uop.BF16)
+    names = []
+    for step in (blk.decode_step, lambda *args: composed_decode_step(T, blk, *args)):
+        out, k, v = step(ids, past, past, pos)
+        assert out.shape == (batch, 256) and k.shape == v.shape == (batch, 2, pos + 1, 128)
+        names.append(out.realize().kernels())
+        assert k.realize().kernels() == [] and v.realize().kernels() == []
+    assert names[0] == names[1] and len(names[0]) > 5
+    with pytest.raises(MorokHipError):  # one head too many
+        blk.decode_step(ids, T.Tensor.from_numpy(np.zeros((batch, 3, pos, 128), np.uint16), uop.BF16), past, pos)
+
+
 def test_a_late_first_step_makes_the_rotary_rows_around_its_position_alone(T, shim, monkeypatch):
     """A block that starts at position 4000 does not pay for the rows before it, and two sequences of positions in turn keep both."""
     from morok_amd import decoder
@@ -1071,6 +1110,8 @@ def test_null_arguments_are_errors_not_crashes(T, dev, shim):
         lambda: shim.mrk_hip_tensor_linear(x._h, null, null, -1, C.byref(out)),
         lambda: shim.mrk_hip_tensor_linear(x._h, x._h, null, 99, C.byref(out)),
         lambda: shim.mrk_hip_tensor_log_softmax(null, -1, C.byref(out)),
+        lambda: shim.mrk_hip_tensor_decode_step(null, 0, x._h, x._h, x._h, null, null, 0, 1, 256, 2, 512, 1e-6, C.byref(out)),
+        lambda: shim.mrk_hip_tensor_decode_step((C.c_void_p * 7)(*[x._h] * 7), 0, x._h, x._h, x._h, null, null, 0, 1, 256, 2, 512, 1e-6, C.byref(out)),
         lambda: shim.mrk_hip_tensor_logsumexp(x._h, -1, null),
         lambda: shim.mrk_hip_gemm_bf16_residual(0, null, 1, 1, 1, 8, 8, 8),
         lambda: shim.mrk_hip_flash_attn_fwd_bf16_strided(0, 1, 1, 1, 1, 1, 1, 8, 8, 128, 1.0, 0, null),
