@@ -302,42 +302,47 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                       }));
         return kOk;
     }
-    if (k == "flash_fwd_bf16") {  // {BH, Sq, Sk, D, causal, scale bits[, workspace bytes]}; buffers {o, q, k, v[, scratch]}
-        if (nparams != 6 && nparams != 7)
-            return failf(kInvalidArgument, "builtin '%s' takes 6 or 7 parameters, got %zu", k.c_str(), nparams);
-        if (p.size() < 7) p.push_back(0);
+    if (k == "flash_fwd_bf16") {  // {BH, Sq, Sk, D, causal, scale bits[, workspace bytes[, counted]]}; buffers {o, q, k, v[, scratch[, arrivals]]}
+        if (nparams < 6 || nparams > 8)
+            return failf(kInvalidArgument, "builtin '%s' takes 6 to 8 parameters, got %zu", k.c_str(), nparams);
+        p.resize(8, 0);
         if (p[6] < 0) return fail(kInvalidArgument, "flash_fwd_bf16: negative workspace size");
+        if (p[7] < 0 || p[7] > 1 || (p[7] && p[6] == 0)) return fail(kInvalidArgument, "flash_fwd_bf16: arrivals are counted (1) beside a workspace, or not (0)");
         if (p[0] < 0 || p[1] < 0 || p[2] <= 0 || (p[3] != 256 && p[3] != 128 && p[3] != 64))
             return fail(kInvalidArgument, "flash_fwd_bf16: bad shape (params BH, Sq, Sk, D = 256, 128 or 64, causal, scale bits)");
         std::string name = "flash_fwd_bf16_" + std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]) + (p[3] != 128 ? "_d" + std::to_string(p[3]) : "");
         // a fifth buffer of p[6] bytes: scratch for the partial results of a key sequence split over workgroups
-        const bool ws = p[6] > 0;
-        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), ws ? 5 : 4, p,
-                                      [ws](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+        // counted: and a sixth of BH zeros (a word each), which one plan's launches keep to themselves: no second launch for the merge
+        const bool ws = p[6] > 0, counted = p[7] != 0;
+        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), counted ? 6 : ws ? 5 : 4, p,
+                                      [ws, counted](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                           uint32_t bits = static_cast<uint32_t>(q[5]);
                                           float scale;
                                           std::memcpy(&scale, &bits, 4);
                                           return launch_flash_fwd_bf16(s, b[1], b[2], b[3], b[0], q[0], q[1], q[2], q[3],
-                                                                       scale, q[4] != 0, ws ? b[4] : nullptr, ws ? static_cast<size_t>(q[6]) : 0);
+                                                                       scale, q[4] != 0, ws ? b[4] : nullptr, ws ? static_cast<size_t>(q[6]) : 0,
+                                                                       counted ? static_cast<unsigned*>(b[5]) : nullptr);
                                       }));
         return kOk;
     }
     if (k == "flash_fwd_bf16_strided") {
         // params: B, H, Sq, Sk, D, causal, scale bits, element offsets of q k v o into their
         // buffers (4), then (batch, head, row) element strides of q k v o (12)
-        // optionally a 24th: workspace bytes, with a fifth buffer of that size (scratch for a split key sequence)
-        if (nparams != 23 && nparams != 24)
-            return failf(kInvalidArgument, "builtin '%s' takes 23 or 24 parameters, got %zu", k.c_str(), nparams);
-        if (p.size() < 24) p.push_back(0);
+        // optionally a 24th: workspace bytes, with a fifth buffer of that size (scratch for a split key sequence); and a 25th, 1: counted, with a
+        // sixth of B H zeros as above
+        if (nparams < 23 || nparams > 25)
+            return failf(kInvalidArgument, "builtin '%s' takes 23 to 25 parameters, got %zu", k.c_str(), nparams);
+        p.resize(25, 0);
         if (p[23] < 0) return fail(kInvalidArgument, "flash_fwd_bf16_strided: negative workspace size");
+        if (p[24] < 0 || p[24] > 1 || (p[24] && p[23] == 0)) return fail(kInvalidArgument, "flash_fwd_bf16_strided: arrivals are counted (1) beside a workspace, or not (0)");
         if (p[0] < 0 || p[1] < 0 || p[2] < 0 || p[3] <= 0 || (p[4] != 256 && p[4] != 128 && p[4] != 64))
             return fail(kInvalidArgument, "flash_fwd_bf16_strided: bad shape (params B, H, Sq, Sk, D = 256, 128 or 64, causal, scale bits, 4 offsets, 12 strides)");
         for (int i = 7; i < 23; i++)
             if (p[i] < 0 || p[i] % 8) return fail(kInvalidArgument, "flash_fwd_bf16_strided: offsets and strides must be non-negative multiples of 8 elements");
         std::string name = "flash_fwd_bf16_strided_" + std::to_string(p[0] * p[1]) + "_" + std::to_string(p[2]) + "_" + std::to_string(p[3]) + (p[4] != 128 ? "_d" + std::to_string(p[4]) : "");
-        const bool ws = p[23] > 0;
-        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), ws ? 5 : 4, p,
-                                      [ws](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+        const bool ws = p[23] > 0, counted = p[24] != 0;
+        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), counted ? 6 : ws ? 5 : 4, p,
+                                      [ws, counted](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                           uint32_t bits = static_cast<uint32_t>(q[6]);
                                           float scale;
                                           std::memcpy(&scale, &bits, 4);
@@ -348,7 +353,8 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                           };
                                           return launch_flash_fwd_bf16_strided(s, at(1, 0), at(2, 1), at(3, 2), at(0, 3), q[0], q[1],
                                                                                q[2], q[3], q[4], scale, q[5] != 0, strides, ws ? b[4] : nullptr,
-                                                                               ws ? static_cast<size_t>(q[23]) : 0);
+                                                                               ws ? static_cast<size_t>(q[23]) : 0,
+                                                                               counted ? static_cast<unsigned*>(b[5]) : nullptr);
                                       }));
         return kOk;
     }
@@ -357,11 +363,13 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         // softcap bits (0 = none), mask kind (0 none, 1 Bool bytes, 2 additive bf16), element offsets of
         // q k v o mask into their buffers (5), (batch, head, row) element strides of q k v o (12) and of
         // the mask (3).  buffers {o, q, k, v, mask}; without a mask the fifth buffer is not read.
-        // optionally a 30th: workspace bytes, with a sixth buffer of that size (scratch for a split key sequence)
-        if (nparams != 29 && nparams != 30)
-            return failf(kInvalidArgument, "builtin '%s' takes 29 or 30 parameters, got %zu", k.c_str(), nparams);
-        if (p.size() < 30) p.push_back(0);
+        // optionally a 30th: workspace bytes, with a sixth buffer of that size (scratch for a split key sequence); and a 31st, 1: counted, with a
+        // seventh of B H zeros as above
+        if (nparams < 29 || nparams > 31)
+            return failf(kInvalidArgument, "builtin '%s' takes 29 to 31 parameters, got %zu", k.c_str(), nparams);
+        p.resize(31, 0);
         if (p[29] < 0) return fail(kInvalidArgument, "flash_fwd_bf16_ext: negative workspace size");
+        if (p[30] < 0 || p[30] > 1 || (p[30] && p[29] == 0)) return fail(kInvalidArgument, "flash_fwd_bf16_ext: arrivals are counted (1) beside a workspace, or not (0)");
         if (p[0] < 0 || p[1] < 0 || p[2] < 0 || p[3] <= 0 || (p[4] != 256 && p[4] != 128 && p[4] != 64) || p[8] < 0 || p[8] > 2)
             return fail(kInvalidArgument, "flash_fwd_bf16_ext: bad shape (params B, H, Sq, Sk, D = 256, 128 or 64, causal, scale bits, "
                                           "softcap bits, mask kind 0..2, 5 offsets, 12 strides, 3 mask strides)");
@@ -373,9 +381,9 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         std::string name = std::string("flash_fwd_bf16_ext") + (p[8] == 1 ? "_bool" : p[8] == 2 ? "_add" : "") + (p[7] ? "_cap" : "") +
                            (flash_fwd_row_mask(p[2], p[3], static_cast<int>(p[8]), p[28], p[7] != 0) ? "_row_" : "_") +
                            std::to_string(p[0] * p[1]) + "_" + std::to_string(p[2]) + "_" + std::to_string(p[3]) + (p[4] != 128 ? "_d" + std::to_string(p[4]) : "");
-        const bool ws = p[29] > 0;
-        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), ws ? 6 : 5, p,
-                                      [ws](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
+        const bool ws = p[29] > 0, counted = p[30] != 0;
+        out->reset(new BuiltinProgram(device_id, stream, name + (ws ? "_splitkv" : ""), counted ? 7 : ws ? 6 : 5, p,
+                                      [ws, counted](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                           uint32_t bits = static_cast<uint32_t>(q[6]), cbits = static_cast<uint32_t>(q[7]);
                                           float scale, cap;
                                           std::memcpy(&scale, &bits, 4);
@@ -388,7 +396,8 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
                                           const void* mask = kind ? static_cast<char*>(b[4]) + q[13] * (kind == 2 ? 2 : 1) : nullptr;
                                           return launch_flash_fwd_bf16_ext(s, at(1, 0), at(2, 1), at(3, 2), at(0, 3), q[0], q[1], q[2], q[3], q[4],
                                                                            scale, q[5] != 0, strides, mask, kind, mstrides, cap, ws ? b[5] : nullptr,
-                                                                           ws ? static_cast<size_t>(q[29]) : 0);
+                                                                           ws ? static_cast<size_t>(q[29]) : 0,
+                                                                           counted ? static_cast<unsigned*>(b[6]) : nullptr);
                                       }));
         return kOk;
     }

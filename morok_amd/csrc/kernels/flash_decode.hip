@@ -7,7 +7,7 @@
 // region of its own (1 KB per instruction, non-temporal: every byte is read once), so the loop has no barrier,
 // and what streams is bounded by the bytes in flight per CU, i.e. by what the LDS holds: the next chunk's keys are
 // requested as soon as this one's are in registers, its values likewise, so that half of a wave's region is always
-// under way (32 pairs of 4096 keys, D = 128: 16.9 us with the merge, 18.1 where both were requested after the
+// under way (32 pairs of 4096 keys, D = 128: 16.9 us with a launch for the merge, 18.1 where both were requested after the
 // products; 5 x 8 pairs of 3703, D = 256: 29.1 and 32.1).  Under a mask, and where the caches grow, a lane has other
 // loads or stores in the queue that the waits count: there a chunk is requested and awaited as a whole.
 // S^T = K Q^T on v_mfma_f32_16x16x32_bf16 (operand A: 16 keys x 32 d read back from LDS, rows swizzled by the key
@@ -22,7 +22,7 @@
 // softmax; a query's maximum sits in four lanes (l % 16 equal), two exchanges per chunk.
 // At the end the waves' (maximum, sum, O) meet in LDS and are merged in a fixed order; with one split the
 // workgroup writes O, otherwise f32 partial results W[split][pair][16][D + 2] (the unnormalised O, then
-// maximum and sum), which flash_decode_merge folds the same way.  Results do not depend on scheduling.
+// maximum and sum), which the pair's last workgroup to arrive or, without counters for that, flash_decode_merge folds the same way.  Results do not depend on scheduling.
 // A pair is a (batch, head), or a (batch, run of consecutive heads) when those heads share their K and V (zero
 // head strides: multi-query / grouped-query attention): the run's heads then occupy the query slots together
 // and K and V are read once for all of them.  attn_mask (Bool bytes or additive bf16, any broadcast layout) and
@@ -74,6 +74,30 @@ struct DecodeAppend {
     unsigned short *k_out, *v_out;
 };
 
+// The fold of a query's key ranges in their order, four columns at d: part(s) points at range s's unnormalised O [kD], maximum and sum.
+template <int kD, class Part>
+__device__ __forceinline__ void fold_ranges(Part part, int splits, unsigned short* __restrict__ O, int bh, int q, int d, int Sq, const DecodeLayout& lay) {
+    // (both loops unrolled by four: the loads of four ranges are in flight together, the sums keep their order)
+    float m_tot = -INFINITY;
+#pragma unroll 4
+    for (int s = 0; s < splits; s++) m_tot = fmaxf(m_tot, part(s)[kD]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float l_tot = 0.0f;
+#pragma unroll 4
+    for (int s = 0; s < splits; s++) {
+        const float* p = part(s);
+        const float wgt = __builtin_amdgcn_exp2f(p[kD] - m_tot);
+        const float2 a = *reinterpret_cast<const float2*>(p + d), c = *reinterpret_cast<const float2*>(p + d + 2);
+        o += f32x4{a.x, a.y, c.x, c.y} * wgt;
+        l_tot += p[kD + 1] * wgt;
+    }
+    const float inv = 1.0f / l_tot;
+    const f32x4 v = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+    const int b = bh / lay.heads, h = (bh % lay.heads) * lay.group, og = q / Sq, orw = q - og * Sq;
+    char* orow = reinterpret_cast<char*>(O + b * lay.o_batch + (h + og) * lay.o_head) + (size_t)orw * lay.o_row;
+    *reinterpret_cast<bf16x4*>(orow + d * 2) = __builtin_convertvector(v, bf16x4);
+}
+
 template <int kD>
 constexpr int decode_waves() {
     return kD == 256 ? 4 : 8;  // a wave's region is 4 * 32 * kD bytes: 128 KB of LDS for 128 and 256, 64 KB for 64
@@ -81,11 +105,12 @@ constexpr int decode_waves() {
 
 // kQB: 16-slot query blocks a workgroup carries (1 or 2: up to 32 query slots per pair); the K and V fragments a wave
 // reads from LDS serve every block.
-template <int kD, int kMask, bool kCap, int kQB, bool kAppend = false>
+// kCounted: the pair's last workgroup to arrive folds its ranges.
+template <int kD, int kMask, bool kCap, int kQB, bool kAppend = false, bool kCounted = false>
 __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
     const unsigned short* __restrict__ Q, const unsigned short* __restrict__ K, const unsigned short* __restrict__ V,
     unsigned short* __restrict__ O, float* __restrict__ W, int Sq, int Sk, int keys_per_split, float scale_log2e, DecodeLayout lay,
-    DecodeMask dm, DecodeAppend ap) {
+    DecodeMask dm, DecodeAppend ap, unsigned* __restrict__ arrivals) {
     constexpr int kWaves = decode_waves<kD>();
     constexpr int kRowBytes = kD * 2;
     constexpr int kPieces = kD / 8;                      // 16-byte pieces of a row
@@ -385,6 +410,12 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
         }
     }
     __syncthreads();
+    // (to be read by a workgroup that another XCD may run: written through, past this one's L2)
+    auto put = [&](float* to, float x, float y) {
+        const float2 v = make_float2(x, y);
+        if constexpr (kCounted) __hip_atomic_store(reinterpret_cast<unsigned long long*>(to), __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *reinterpret_cast<float2*>(to) = v;
+    };
     // element e: query block, column block c, lane l of it: slot 16 qb + l % 16, columns 16 c + 4 (l / 16) + 0..3
     for (int e = threadIdx.x; e < kQB * kColBlocks * 64; e += kWaves * 64) {
         const int qb = e / (kColBlocks * 64), c = (e >> 6) % kColBlocks, l = e & 63, ql = l & 15, q = 16 * qb + ql;
@@ -408,12 +439,9 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
         const int d = 16 * c + 4 * (l >> 4);
         if (W) {
             float* dst = W + (((size_t)blockIdx.x * gridDim.y + bh) * kSlots + q) * (kD + 2);
-            *reinterpret_cast<float2*>(dst + d) = make_float2(o[0], o[1]);
-            *reinterpret_cast<float2*>(dst + d + 2) = make_float2(o[2], o[3]);
-            if (d == 0) {
-                dst[kD] = m_tot;
-                dst[kD + 1] = l_tot;
-            }
+            put(dst + d, o[0], o[1]);
+            put(dst + d + 2, o[2], o[3]);
+            if (d == 0) put(dst + kD, m_tot, l_tot);
         } else {
             const float inv = 1.0f / l_tot;
             const f32x4 v = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
@@ -421,6 +449,42 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
             char* orow = reinterpret_cast<char*>(O + b * lay.o_batch + (h + og) * lay.o_head) + (size_t)orw * lay.o_row;
             *reinterpret_cast<bf16x4*>(orow + d * 2) = __builtin_convertvector(v, bf16x4);
         }
+    }
+    if constexpr (!kCounted) return;
+    // The pair's workgroup that arrives last folds its ranges: all partial results of the others have left their compute units (each wave waits
+    // for its own before the barrier, one work-item counts the workgroup behind it).  The counter wraps to zero with the last arrival, ready
+    // for the next launch.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned* told = reinterpret_cast<unsigned*>(smem);
+    if (threadIdx.x == 0) *told = atomicInc(arrivals + bh, gridDim.x - 1);
+    __syncthreads();
+    const bool last_in = *told == gridDim.x - 1;
+    __syncthreads();
+    if (!last_in) return;
+    // (all of them into LDS first: one trip to memory instead of one per four ranges)
+    const int row = nq * (kD + 2), splits = (int)gridDim.x;
+    float* all = reinterpret_cast<float*>(smem);
+    constexpr int kInFlight = 8;
+    const int pieces = splits * (row / 2);
+    for (int i = threadIdx.x; i < pieces; i += kInFlight * kWaves * 64) {
+        unsigned long long v[kInFlight];
+#pragma unroll
+        for (int u = 0; u < kInFlight; u++) {
+            const int at = i + u * kWaves * 64;
+            if (at >= pieces) break;
+            const int s = at / (row / 2), x = 2 * (at - s * (row / 2));
+            const float* src = W + ((size_t)s * gridDim.y + bh) * kSlots * (kD + 2) + x;
+            v[u] = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int u = 0; u < kInFlight; u++)
+            if (i + u * kWaves * 64 < pieces) *reinterpret_cast<unsigned long long*>(all + 2 * (i + u * kWaves * 64)) = v[u];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nq * (kD / 4); e += kWaves * 64) {
+        const int q = e / (kD / 4), d = 4 * (e % (kD / 4));
+        fold_ranges<kD>([&](int s) { return all + s * row + q * (kD + 2); }, splits, O, bh, q, d, Sq, lay);
     }
 }
 
@@ -438,25 +502,7 @@ __global__ __launch_bounds__(256) void flash_decode_merge(const float* __restric
     const int bh = (int)(e / ((long)kQuads * nq));
     const size_t slice = (size_t)BH * slot_cap * (kD + 2);  // slot_cap: 16 or 32 slots per pair, as the split kernel laid them out
     const float* src = W + ((size_t)bh * slot_cap + q) * (kD + 2);
-    // (both loops unrolled by four: the loads of four ranges are in flight together, the sums keep their order)
-    float m_tot = -INFINITY;
-#pragma unroll 4
-    for (int s = 0; s < splits; s++) m_tot = fmaxf(m_tot, src[s * slice + kD]);
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    float l_tot = 0.0f;
-#pragma unroll 4
-    for (int s = 0; s < splits; s++) {
-        const float* p = src + s * slice;
-        const float wgt = __builtin_amdgcn_exp2f(p[kD] - m_tot);
-        const float2 a = *reinterpret_cast<const float2*>(p + d), c = *reinterpret_cast<const float2*>(p + d + 2);
-        o += f32x4{a.x, a.y, c.x, c.y} * wgt;
-        l_tot += p[kD + 1] * wgt;
-    }
-    const float inv = 1.0f / l_tot;
-    const f32x4 v = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
-    const int b = bh / lay.heads, h = (bh % lay.heads) * lay.group, og = q / Sq, orw = q - og * Sq;
-    char* orow = reinterpret_cast<char*>(O + b * lay.o_batch + (h + og) * lay.o_head) + (size_t)orw * lay.o_row;
-    *reinterpret_cast<bf16x4*>(orow + d * 2) = __builtin_convertvector(v, bf16x4);
+    fold_ranges<kD>([&](int s) { return src + s * slice; }, splits, O, bh, q, d, Sq, lay);
 }
 
 }  // namespace mrk::dev
@@ -508,11 +554,13 @@ size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal) 
 // strides: (batch, head, row) element strides of q, k, v and o (validated by the caller: multiples of 8, rows
 // addressable in 32 bits, pointers 16-byte aligned); W: splits * pairs * flash_decode_slot_capacity(group * Sq) * (D + 2)
 // floats, needed with several splits (pairs = B * H / group).
+// arrivals (may be null): one counter per pair, zero before the first launch that uses them and after every one, for launches that follow each other
+// (one plan's): the ranges are folded by the split kernel itself, without a second launch.
 // mask_kind 0: none; 1: Bool bytes, 2: additive bf16, with (batch, head, query row) element strides that are multiples
 // of 4, a mask pointer aligned to four elements and Sk a multiple of 4 (validated by the caller as well).  softcap 0: none.
 int launch_flash_decode(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
                         float scale, const long* strides, long splits, long keys_per_split, void* W, const void* mask, int mask_kind,
-                        const long* mask_strides, float softcap, long group) {
+                        const long* mask_strides, float softcap, long group, unsigned* arrivals) {
     // group > 1: runs of `group` consecutive heads share K and V (zero head strides) and become query slots of one pair
     if (B <= 0 || H <= 0 || group < 1 || H % group || !strides || !q || !k || !v || !o) return (int)hipErrorInvalidValue;
     const long pairs = B * (H / group), slots = group * Sq;
@@ -548,8 +596,14 @@ int launch_flash_decode(void* stream, const void* q, const void* k, const void* 
     const long quads = pairs * slots * (D / 4);
     const unsigned merge_blocks = (unsigned)((quads + 255) / 256);
     const int slot_cap = (int)flash_decode_slot_capacity(slots);
+    // The last workgroup of a pair folds its ranges where they fit the local memory a workgroup has anyway.  Its three trips to memory in a row
+    // (results out, the count, results in) take less than a second launch (us with it / without: 32 pairs of 4096 keys 17.2 / 15.3, D = 64:
+    // 16 x 4000 11.4 / 9.4, 4 x 30000 18.5 / 13.6; 8 slots of 32 x 2243 17.8 / 16.5), but for rows of 256 from five slots on, which four waves
+    // fold (4 slots of 16 x 2000 17.6 / 16.7, 8 of 8 x 1500 15.3 / 17.0).
+    const bool fold = splits * slots * (D + 2) * (long)sizeof(float) <= (D == 64 ? 64 : 128) * 1024 && (D != 256 || slots <= 4);
+    unsigned* counted = w && fold ? arrivals : nullptr;
 #define MRK_DECODE_QB(DIM, MASK, CAP, QB) \
-    flash_decode_split<DIM, MASK, CAP, QB><<<grid, decode_waves<DIM>() * 64, 0, s>>>(qp, kp, vp, op, w, (int)Sq, (int)Sk, (int)keys_per_split, scale_log2e, lay, dm, DecodeAppend{})
+    (counted ? flash_decode_split<DIM, MASK, CAP, QB, false, true> : flash_decode_split<DIM, MASK, CAP, QB>)<<<grid, decode_waves<DIM>() * 64, 0, s>>>(qp, kp, vp, op, w, (int)Sq, (int)Sk, (int)keys_per_split, scale_log2e, lay, dm, DecodeAppend{}, counted)
 #define MRK_DECODE(DIM, MASK)                              \
     do {                                                   \
         if (cap) {                                         \
@@ -565,7 +619,7 @@ int launch_flash_decode(void* stream, const void* q, const void* k, const void* 
         if (mask_kind == 0) MRK_DECODE(DIM, 0);                                                                     \
         else if (mask_kind == 1) MRK_DECODE(DIM, 1);                                                                \
         else MRK_DECODE(DIM, 2);                                                                                    \
-        if (w) flash_decode_merge<DIM><<<merge_blocks, 256, 0, s>>>(w, op, (int)pairs, (int)Sq, (int)splits, slot_cap, lay); \
+        if (w && !counted) flash_decode_merge<DIM><<<merge_blocks, 256, 0, s>>>(w, op, (int)pairs, (int)Sq, (int)splits, slot_cap, lay); \
     } while (0)
     if (D == 128) MRK_DECODE_DIM(128);
     else if (D == 64) MRK_DECODE_DIM(64);
@@ -619,7 +673,7 @@ int launch_flash_decode_append(void* stream, const void* q, const void* past_k, 
     auto go = [&](auto dim) {
         constexpr int kD = decltype(dim)::value;
         flash_decode_split<kD, 0, false, 1, true><<<grid, decode_waves<kD>() * 64, 0, s>>>(
-            as(q), as(past_k), as(past_v), static_cast<unsigned short*>(o), w, 1, (int)Sk, (int)per, scale * 1.4426950408889634f, lay, DecodeMask{}, ap);
+            as(q), as(past_k), as(past_v), static_cast<unsigned short*>(o), w, 1, (int)Sk, (int)per, scale * 1.4426950408889634f, lay, DecodeMask{}, ap, nullptr);
         if (w) flash_decode_merge<kD><<<merge_blocks, 256, 0, s>>>(w, static_cast<unsigned short*>(o), (int)(B * H), 1, (int)splits, 16, lay);
     };
     if (D == 128) go(std::integral_constant<int, 128>{});

@@ -737,7 +737,7 @@ static long work_units(long BH, long q_tiles, long D, int causal) {
 // A handful of queries against a long key sequence: the kernel that splits the keys (flash_decode.hip), in as many
 // ranges as the workspace allows (one range needs none).
 static bool decode_route(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
-                         float scale, int causal, const long* strides, void* workspace, size_t workspace_bytes, int* rc,
+                         float scale, int causal, const long* strides, void* workspace, size_t workspace_bytes, unsigned* arrivals, int* rc,
                          const void* mask = nullptr, int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f) {
     using namespace mrk::dev;
     // heads that share K and V (zero head strides) become query slots of one pair: K and V are read once per batch
@@ -765,12 +765,12 @@ static bool decode_route(void* stream, const void* q, const void* k, const void*
         }
     }
     *rc = launch_flash_decode(stream, q, k, v, o, B, H, Sq, Sk, D, scale, strides, splits, per, workspace, mask, mask_kind, mask_strides,
-                              softcap, group);
+                              softcap, group, arrivals);
     return true;
 }
 
 int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* o, long BH, long Sq, long Sk,
-                          long D, float scale, int causal, void* workspace, size_t workspace_bytes) {
+                          long D, float scale, int causal, void* workspace, size_t workspace_bytes, unsigned* arrivals) {
     using namespace mrk::dev;
     if (BH <= 0 || Sq <= 0) return 0;
     if ((D != 256 && D != 128 && D != 64) || Sk <= 0 || !(scale > 0.0f)) return (int)hipErrorInvalidValue;
@@ -780,7 +780,7 @@ int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void
     {
         const long dense[12] = {Sq * D, 0, D, Sk * D, 0, D, Sk * D, 0, D, Sq * D, 0, D};  // (batch * head, -, row) per operand
         int rc = 0;
-        if (decode_route(stream, q, k, v, o, BH, 1, Sq, Sk, D, scale, causal, dense, workspace, workspace_bytes, &rc)) return rc;
+        if (decode_route(stream, q, k, v, o, BH, 1, Sq, Sk, D, scale, causal, dense, workspace, workspace_bytes, arrivals, &rc)) return rc;
     }
     const long q_tiles = (Sq + kQT - 1) / kQT;
     const long units = work_units(BH, q_tiles, D, causal);
@@ -796,7 +796,7 @@ int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void
 }
 
 int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq,
-                                  long Sk, long D, float scale, int causal, const long* strides, void* workspace, size_t workspace_bytes) {
+                                  long Sk, long D, float scale, int causal, const long* strides, void* workspace, size_t workspace_bytes, unsigned* arrivals) {
     using namespace mrk::dev;
     if (B < 0 || H < 0 || !strides) return (int)hipErrorInvalidValue;
     const long BH = B * H;
@@ -818,10 +818,10 @@ int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, co
         if (t == 3 && ((Sq > 1 && sr < D) || (H > 1 && sh == 0) || (B > 1 && sb == 0))) return (int)hipErrorInvalidValue;
         dense = dense && sr == D && sh == rows[t] * D && sb == H * rows[t] * D;
     }
-    if (dense) return launch_flash_fwd_bf16(stream, q, k, v, o, BH, Sq, Sk, D, scale, causal, workspace, workspace_bytes);
+    if (dense) return launch_flash_fwd_bf16(stream, q, k, v, o, BH, Sq, Sk, D, scale, causal, workspace, workspace_bytes, arrivals);
     {
         int rc = 0;
-        if (decode_route(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, &rc)) return rc;
+        if (decode_route(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, arrivals, &rc)) return rc;
     }
     const long q_tiles = (Sq + kQT - 1) / kQT;
     const long units = work_units(BH, q_tiles, D, causal);
@@ -854,12 +854,12 @@ bool flash_fwd_row_mask(long Sq, long Sk, int mask_kind, long row_stride, bool c
 
 int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk,
                               long D, float scale, int causal, const long* strides, const void* mask, int mask_kind,
-                              const long* mask_strides, float softcap, void* workspace, size_t workspace_bytes) {
+                              const long* mask_strides, float softcap, void* workspace, size_t workspace_bytes, unsigned* arrivals) {
     using namespace mrk::dev;
     if (B < 0 || H < 0 || !strides) return (int)hipErrorInvalidValue;
     if (mask_kind < 0 || mask_kind > 2 || (mask_kind != 0 && (!mask || !mask_strides)) || !(softcap >= 0.0f)) return (int)hipErrorInvalidValue;
     if (mask_kind == 0 && !(softcap > 0.0f))
-        return launch_flash_fwd_bf16_strided(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes);
+        return launch_flash_fwd_bf16_strided(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, arrivals);
     const long BH = B * H;
     if (BH == 0 || Sq <= 0) return 0;
     if ((D != 256 && D != 128 && D != 64) || Sk <= 0 || !(scale > 0.0f)) return (int)hipErrorInvalidValue;
@@ -888,7 +888,7 @@ int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const 
     const bool cap = softcap > 0.0f;
     {  // a handful of queries without the causal rule: the kernel that splits the keys
         int rc = 0;
-        if (decode_route(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, &rc, mask, mask_kind, mask_strides,
+        if (decode_route(stream, q, k, v, o, B, H, Sq, Sk, D, scale, causal, strides, workspace, workspace_bytes, arrivals, &rc, mask, mask_kind, mask_strides,
                          softcap))
             return rc;
     }

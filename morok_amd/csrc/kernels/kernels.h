@@ -146,6 +146,8 @@ inline bool flash_fwd_rows_addressable(long rows, long row_bytes, long D) {
 // a kernel that also splits the key sequence over workgroups (flash_decode_plan tells how); with several key
 // ranges their f32 partial results go through `workspace` (flash_fwd_workspace_bytes; 0 = one range), which a
 // second kernel merges.  Without a workspace of that size such a shape runs in as many ranges as the workspace holds.
+// `arrivals` (may be null): a counter per (batch, head), zero, for launches that follow each other (a plan's own): the split kernel then
+// merges by itself.
 // Heads that share their keys and values (zero head strides of k and v: multi-query attention, or grouped-query
 // attention with the groups as batches) are folded into one pair's query slots, as many consecutive heads as give at
 // most 32 slots (a divisor of the head count), so that K and V are read once per such run instead of once per head.
@@ -154,7 +156,8 @@ long flash_decode_slot_capacity(long slots);
 size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal);
 int launch_flash_decode(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
                         float scale, const long* strides, long splits, long keys_per_split, void* W, const void* mask = nullptr,
-                        int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f, long group = 1);
+                        int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f, long group = 1,
+                        unsigned* arrivals = nullptr);
 // One query per (batch, head) over past_k / past_v [B, H, Sk - 1, D] and one new key and value each (all bf16), which also writes the grown
 // caches k_out / v_out [B, H, Sk, D]: the bits of the copies followed by the attention over them.  strides (elements, multiples of
 // 8): q batch, head; new key batch, head; new value batch, head; o batch, head.  Workspace as flash_fwd_workspace_bytes says.
@@ -163,14 +166,14 @@ int launch_flash_decode_append(void* stream, const void* q, const void* past_k, 
                                void* k_out, void* v_out, long B, long H, long Sk, long D, float scale, const long* strides, void* workspace,
                                size_t workspace_bytes);
 int launch_flash_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* o, long BH, long Sq, long Sk,
-                          long D, float scale, int causal, void* workspace = nullptr, size_t workspace_bytes = 0);
+                          long D, float scale, int causal, void* workspace = nullptr, size_t workspace_bytes = 0, unsigned* arrivals = nullptr);
 // The same kernel over operands given as views: strides holds (batch, head, row) element
 // strides of q, k, v and o, in that order (12 values); the 128 elements of a row are
 // contiguous.  Strides must be multiples of 8 elements and the pointers 16-byte aligned;
 // zero batch / head strides broadcast an input.  Dense strides take the kernel above.
 int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq,
                                   long Sk, long D, float scale, int causal, const long* strides, void* workspace = nullptr,
-                                  size_t workspace_bytes = 0);
+                                  size_t workspace_bytes = 0, unsigned* arrivals = nullptr);
 
 // The same attention with an attn_mask and / or a softcap (transformer.rs:112-132), operands as
 // views like the strided launcher.  mask_kind 0: none; 1: Bool, one byte per element, nonzero =
@@ -187,7 +190,8 @@ int launch_flash_fwd_bf16_strided(void* stream, const void* q, const void* k, co
 bool flash_fwd_row_mask(long Sq, long Sk, int mask_kind, long row_stride, bool cap);
 int launch_flash_fwd_bf16_ext(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk,
                               long D, float scale, int causal, const long* strides, const void* mask, int mask_kind,
-                              const long* mask_strides, float softcap, void* workspace = nullptr, size_t workspace_bytes = 0);
+                              const long* mask_strides, float softcap, void* workspace = nullptr, size_t workspace_bytes = 0,
+                              unsigned* arrivals = nullptr);
 
 // C[M, N] = A[M, K] B in f32 on the f32 matrix instructions, B [K, N] or (b_transposed) [N, K]; any shape and alignment of
 // whole floats.  add (may be null): f32, one row [N] (add_is_row) or a matrix of C's shape, added to the sums: the bits

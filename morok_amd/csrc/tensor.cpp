@@ -2408,6 +2408,22 @@ struct Scheduler {
         return kOk;
     }
 
+    // A plan that outlives this call keeps a counter per pair for the attention that splits its keys, which spares it the launch that merges
+    // the ranges (one query against 32 pairs of 4096 keys 16.9 -> 15.0 us).  They have to be zero at a launch and are again after it: memory of
+    // the plan's own, not an intermediate that shares a block.  A realization would have to clear them first, as long a launch as the one
+    // it saves.
+    bool outlives = false;
+    int count_arrivals(int64_t pairs, std::vector<int64_t>* params, std::vector<std::shared_ptr<Buffer>>* bufs) {
+        if (!outlives || dry) return kOk;
+        BufferOptions zeros;
+        zeros.zero_init = true;
+        auto arrivals = std::make_shared<Buffer>(dev->allocator, static_cast<size_t>(pairs) * sizeof(unsigned), zeros);
+        MRK_TRY(arrivals->ensure_allocated());
+        bufs->push_back(arrivals);
+        params->push_back(1);
+        return kOk;
+    }
+
     // The attention kernel over whatever views its operands are: an operand that is a strided
     // view of data in memory (rows of head-dim contiguous elements, 16-byte aligned) is read in
     // place, anything else is materialised first.  `dst` is the node that receives the buffer,
@@ -2502,6 +2518,7 @@ struct Scheduler {
             if (ws) {
                 bufs.push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
                 params.push_back(static_cast<int64_t>(ws));
+                MRK_TRY(count_arrivals(B * H, &params, &bufs));
             }
             MRK_TRY(builtin("flash_fwd_bf16_ext", params, bufs));
         } else {
@@ -2515,7 +2532,10 @@ struct Scheduler {
                 params = {B, H, Sq, Sk, D, att->hint_causal ? 1 : 0, static_cast<int64_t>(bits), offsets[0], offsets[1], offsets[2], 0};
                 params.insert(params.end(), strides.begin(), strides.end());
             }
-            if (ws) params.push_back(static_cast<int64_t>(ws));
+            if (ws) {
+                params.push_back(static_cast<int64_t>(ws));
+                MRK_TRY(count_arrivals(B * H, &params, &bufs));
+            }
             MRK_TRY(builtin(dense ? "flash_fwd_bf16" : "flash_fwd_bf16_strided", params, bufs));
         }
         dst->buffer = out;
@@ -3427,6 +3447,7 @@ int prepare_locked(const TensorRef& root, std::unique_ptr<ExecutionPlan>* out, s
     Scheduler s;
     s.deferred = deferred;
     s.fresh = fresh;
+    s.outlives = kept == nullptr;
     // every exit that is not the successful one returns the touched nodes to their lazy state
     struct Rollback {
         Scheduler& s;

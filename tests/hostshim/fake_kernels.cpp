@@ -102,18 +102,18 @@ int launch_gemm_bf16_rope(void* stream, const void*, const void*, void*, void*, 
 size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal) {
     return !causal && Sq >= 1 && Sq <= 16 && Sk >= 1024 && BH >= 1 && BH <= 96 ? (size_t)2 * BH * 16 * (D + 2) * 4 : 0;
 }
-int launch_flash_fwd_bf16(void* stream, const void*, const void*, const void*, void*, long, long, long, long, float, int, void* ws, size_t) {
+int launch_flash_fwd_bf16(void* stream, const void*, const void*, const void*, void*, long, long, long, long, float, int, void* ws, size_t, unsigned*) {
     mrk_shim_note_launch(stream, ws ? "flash_fwd_bf16_splitkv" : "flash_fwd_bf16");
     return 0;
 }
 int launch_flash_fwd_bf16_strided(void* stream, const void*, const void*, const void*, void*, long, long, long, long, long, float,
-                                  int, const long*, void* ws, size_t) {
+                                  int, const long*, void* ws, size_t, unsigned*) {
     mrk_shim_note_launch(stream, ws ? "flash_fwd_bf16_strided_splitkv" : "flash_fwd_bf16_strided");
     return 0;
 }
 bool flash_fwd_row_mask(long, long, int, long, bool) { return false; }
 int launch_flash_fwd_bf16_ext(void* stream, const void*, const void*, const void*, void*, long, long, long, long, long, float, int,
-                              const long*, const void*, int mask_kind, const long*, float softcap, void* ws, size_t) {
+                              const long*, const void*, int mask_kind, const long*, float softcap, void* ws, size_t, unsigned*) {
     mrk_shim_note_launch(stream, mask_kind == 0 && !(softcap > 0.0f) ? "flash_fwd_bf16_strided" : ws ? "flash_fwd_bf16_ext_splitkv" : "flash_fwd_bf16_ext");
     return 0;
 }

@@ -1,0 +1,72 @@
+"""Attention of a few queries in a prepared plan: the last workgroup of a pair folds the pair's key ranges.  Against the same graph realized, whose
+ranges a second kernel folds in the same order: the same bits, on every execution and every replay."""
+import numpy as np
+import pytest
+
+import morok_amd
+from morok_amd import synth
+from morok_amd import tensor as T, uop
+from morok_amd._ffi import lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _build(B, H, group, Sq, Sk, d, mask, cap, seed):
+    """group > 1: heads that share their keys."""
+    q, k, v = (T.Tensor.from_numpy(synth.normal_bf16(s, seed, i), uop.BF16) for i, s in
+               enumerate([(B, H, Sq, d), (B, 1 if group else H, Sk, d), (B, 1 if group else H, Sk, d)]))
+    if group:
+        k, v = k.try_expand([B, H, Sk, d]), v.try_expand([B, H, Sk, d])
+    m = None
+    if mask:
+        keep = np.arange(Sk)[None, :] < np.maximum(1, synth.randint((B, 1), seed, 7, Sk))
+        m = T.Tensor.from_numpy(np.ascontiguousarray(keep.reshape(B, 1, 1, Sk)))
+    return lambda: q.scaled_dot_product_attention(k, v, attn_mask=m, softcap=cap)
+
+
+# two ranges and the most there are; one, several and 32 query slots; more partial results than a workgroup's local memory holds (the
+# second kernel folds those); heads that share their keys; masks that leave ranges empty
+CASES = [(1, 32, False, 1, 4096, 128, False, None), (2, 3, False, 1, 1030, 64, False, None), (1, 1, False, 1, 70000, 128, False, None),
+         (1, 4, False, 3, 5000, 256, False, None), (1, 2, False, 32, 16384, 128, False, None), (1, 1, False, 17, 2000, 64, False, None),
+         (4, 8, True, 1, 9000, 128, False, None), (3, 12, True, 2, 3000, 256, False, None), (2, 4, True, 1, 5000, 256, False, None), (3, 4, False, 1, 4100, 128, True, None),
+         (2, 4, False, 2, 2048, 64, True, 20.0), (40, 4, False, 1, 513, 128, False, None), (1, 2, False, 1, 300, 128, False, None)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(x) for x in c))
+def test_a_plans_executions_match_a_realization(dev, case):
+    B, H, group, Sq, Sk, d, mask, cap = case
+    build = _build(B, H, group, Sq, Sk, d, mask, cap, seed=31)
+    want = build().realize().to_numpy()
+    root = build()
+    plan = root.prepare()
+    other = T.Tensor.from_numpy(np.ones((64, 512), np.float32))
+    for i in range(4):
+        root.buffer().copyin(np.full(want.shape, 0x7FC0, np.uint16))
+        if i < 2:
+            plan.execute()
+        else:
+            plan.execute_graph()
+        got = root.buffer().copyout(np.uint16, want.shape)
+        assert np.array_equal(got, want), i
+        assert np.all(other.try_mul(float(i)).sum(1).to_numpy() == 512.0 * i)  # (work of others in between)
+
+
+def test_executions_that_follow_each_other_without_a_wait(dev):
+    build = _build(2, 4, False, 1, 6000, 128, False, None, seed=32)
+    want = build().realize().to_numpy()
+    roots = [build() for _ in range(3)]
+    plans = [r.prepare() for r in roots]
+    for _ in range(50):
+        for p in plans:
+            p.execute()
+    for r in roots:
+        assert np.array_equal(r.buffer().copyout(np.uint16, want.shape), want)
+
+
+def test_counters_come_with_a_workspace(dev):
+    bits = int(np.float32(0.1).view(np.uint32))
+    for params in ([8, 1, 2048, 128, 0, bits, 0, 1], [8, 1, 2048, 128, 0, bits, 1 << 20, 2]):
+        with pytest.raises(morok_amd.MorokHipError):
+            morok_amd.Program.builtin("flash_fwd_bf16", params, dev.device_id)
+    ws = lib.mrk_hip_flash_attn_workspace_bytes(8, 1, 1, 2048, 128, 0)
+    assert morok_amd.Program.builtin("flash_fwd_bf16", [8, 1, 2048, 128, 0, bits, ws, 1], dev.device_id).name.endswith("_splitkv")
