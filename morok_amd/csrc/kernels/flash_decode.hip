@@ -524,7 +524,12 @@ bool flash_decode_plan(long BH, long Sq, long Sk, long D, int causal, long* spli
     // workgroups, one per CU, measured best at one per CU: 21 against 24 us at [1, 16, 1, 4096], 30 against 33 with 32 pairs)
     const long min_keys = D == 256 ? 256 : 512, target = D == 256 ? 256 : 192;
     const long max_splits = Sk / min_keys > 0 ? Sk / min_keys : 1;
-    long want = (target + BH / 2) / BH;
+    // Rows of 256: no more workgroups than compute units, each of which holds one (rounded to the nearest count of ranges, us before / now: 96 pairs of
+    // 1500 40.7 / 28.4, 72 x 2500 47.2 / 34.3, 160 x 700 33.4 / 23.5, 20 x 4000 30.4 / 23.0).
+    long want = D == 256 ? target / BH : (target + BH / 2) / BH;
+    // A few pairs more than compute units, each of which holds one workgroup of these: three shorter ranges a pair instead of a second round for
+    // those few (us in one / three: 288 x 4000 114 / 98, x 2000 60 / 57, x 1000 level; 272 x 2500, D = 256 144 / 125; 384 x 2500 78 / 82).
+    if (D != 64 && Sq <= 16 && BH > 256 && BH <= 320 && Sk >= 1500) want = 3;
     want = want < max_splits ? want : max_splits;
     want = want < 1 ? 1 : want;
     const long per = ((Sk + want - 1) / want + kChunkKeys - 1) / kChunkKeys * kChunkKeys;

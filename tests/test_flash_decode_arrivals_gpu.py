@@ -7,6 +7,7 @@ import morok_amd
 from morok_amd import synth
 from morok_amd import tensor as T, uop
 from morok_amd._ffi import lib
+from tests.test_flash_decode_gpu import _attn, _check, _inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,17 @@ def test_executions_that_follow_each_other_without_a_wait(dev):
             p.execute()
     for r in roots:
         assert np.array_equal(r.buffer().copyout(np.uint16, want.shape), want)
+
+
+# rows of 256 in as many workgroups as there are compute units, or one more pair than that; three ranges a pair just above, first and last count
+@pytest.mark.parametrize("shape", [(6, 16, 1, 1231, 256), (1, 129, 1, 900, 256), (1, 257, 1, 1500, 128), (10, 32, 1, 1501, 128), (1, 321, 1, 1500, 128),
+                                   (1, 260, 16, 1530, 256), (1, 260, 17, 1500, 128)])
+def test_ranges_that_follow_the_count_of_compute_units(dev, oracle, shape):
+    B, H, Sq, Sk, d = shape
+    q, k, v = _inputs(B, H, Sq, Sk, d, seed=33)
+    want = oracle.sdpa_bf16(q, k, v, float(d) ** -0.5, causal=False)
+    for mode in ("abi", "program"):
+        _check(_attn(dev, q, k, v, float(d) ** -0.5, mode=mode), want)
 
 
 def test_counters_come_with_a_workspace(dev):
