@@ -728,9 +728,17 @@ namespace mrk {
 // there are more tiles than run at once (one or two to a compute unit).  Where there are not, a pair is a longer chain and a second start and end:
 // 80 heads x 169, D = 128 12.2 us in pairs, 7.6 as tiles; 32 x 700 22.3 / 15.4, D = 256 41.4 / 28.5.  With two to a compute unit the
 // longest tiles share one, and short sequences alone gain (64 x 700, 384 tiles 23.3 / 20.2; 32 x 1500, as many 34.4 / 35.6).
+// Rows of 256, one workgroup to a compute unit: tiles take about half a round of pairs longer than evenly spread work would, the more the more rounds
+// there are; pairs take the rest of their last round.  Tiles below three rounds where the last is filled to half or less (us in pairs / as
+// tiles: 32 x 3000, 1.5 rounds 213 / 187; 24 x 6437, 2.44 626 / 562; 160 x 378, 1.25 62 / 41; but 72 x 1500, 1.69 128 / 137; 128 x 1000, 2 107 / 132;
+// 208 x 952, 3.25 206 / 219), unless all that is left for it are the unpaired middle tiles of an odd count (88 x 628, 1.03 41.5 / 50.4).
 static long work_units(long BH, long q_tiles, long D, int causal) {
     const long tiles = BH * q_tiles;
-    const bool pairs = causal && tiles > 256 && (D == 256 || tiles > 512 || q_tiles > 6);
+    bool pairs = causal && tiles > 256 && (D == 256 || tiles > 512 || q_tiles > 6);
+    if (D == 256 && pairs) {
+        const long count = BH * ((q_tiles + 1) / 2), last = count % 256;
+        pairs = count >= 3 * 256 || last == 0 || last > 136 || (q_tiles % 2 && last <= 8);
+    }
     return pairs ? (q_tiles + 1) / 2 : q_tiles;
 }
 

@@ -29,3 +29,10 @@ def test_units_do_not_change_the_bits(dev, heads, s, d, mask):
     p = np.exp(sc - sc.max(-1, keepdims=True))
     want = p @ vf / p.sum(-1, keepdims=True)
     assert np.abs(synth.from_bf16(many[0, -1]) - want).max() <= 2e-2 * np.abs(want).max()
+
+
+# rows of 256: pairs and single tiles by how far the last round of pairs is filled; an even and an odd count of tiles, few and many rounds
+@pytest.mark.parametrize("heads,s", [(160, 378), (200, 500), (88, 628), (144, 250), (416, 300)])
+def test_units_of_rows_of_256(dev, heads, s):
+    test_units_do_not_change_the_bits(dev, heads, s, 256, False)
+    test_units_do_not_change_the_bits(dev, heads, s, 256, True)
