@@ -732,12 +732,19 @@ namespace mrk {
 // there are; pairs take the rest of their last round.  Tiles below three rounds where the last is filled to half or less (us in pairs / as
 // tiles: 32 x 3000, 1.5 rounds 213 / 187; 24 x 6437, 2.44 626 / 562; 160 x 378, 1.25 62 / 41; but 72 x 1500, 1.69 128 / 137; 128 x 1000, 2 107 / 132;
 // 208 x 952, 3.25 206 / 219), unless all that is left for it are the unpaired middle tiles of an odd count (88 x 628, 1.03 41.5 / 50.4).
+// Rows of 64 and 128, two workgroups to a compute unit, which have the longer of them to themselves at the end: tiles where pairs fill a quarter of their
+// last round, or put a second workgroup on up to a third of the compute units (us in pairs / as tiles: 88 x 1516, 1.03 rounds 99.1 / 85.7; 128 x 1046, 1.25
+// 77.3 / 70.5; 72 x 3857, 2.25 378 / 356; 32 x 2067, 0.56 68.8 / 60.4; but 96 x 942, 0.75 28.4 / 32.3; 160 x 1446, 1.88 130 / 142).
 static long work_units(long BH, long q_tiles, long D, int causal) {
     const long tiles = BH * q_tiles;
     bool pairs = causal && tiles > 256 && (D == 256 || tiles > 512 || q_tiles > 6);
+    const long count = BH * ((q_tiles + 1) / 2);
     if (D == 256 && pairs) {
-        const long count = BH * ((q_tiles + 1) / 2), last = count % 256;
+        const long last = count % 256;
         pairs = count >= 3 * 256 || last == 0 || last > 136 || (q_tiles % 2 && last <= 8);
+    } else if (pairs) {
+        const long last = count % 512;
+        pairs = count <= 512 ? count <= 256 || count > 344 : count >= 3 * 512 || last == 0 || last > 144;
     }
     return pairs ? (q_tiles + 1) / 2 : q_tiles;
 }

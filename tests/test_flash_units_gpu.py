@@ -36,3 +36,10 @@ def test_units_do_not_change_the_bits(dev, heads, s, d, mask):
 def test_units_of_rows_of_256(dev, heads, s):
     test_units_do_not_change_the_bits(dev, heads, s, 256, False)
     test_units_do_not_change_the_bits(dev, heads, s, 256, True)
+
+
+# rows of 64 and 128: just above one workgroup to a compute unit, and above two
+@pytest.mark.parametrize("heads,s,d", [(80, 790, 128), (90, 790, 128), (208, 615, 128), (224, 615, 64), (300, 140, 64)])
+def test_units_of_rows_of_64_and_128(dev, heads, s, d):
+    test_units_do_not_change_the_bits(dev, heads, s, d, False)
+    test_units_do_not_change_the_bits(dev, heads, s, d, True)
