@@ -8,8 +8,10 @@
 // and what streams is bounded by the bytes in flight per CU, i.e. by what the LDS holds: the next chunk's keys are
 // requested as soon as this one's are in registers, its values likewise, so that half of a wave's region is always
 // under way (32 pairs of 4096 keys, D = 128: 16.9 us with a launch for the merge, 18.1 where both were requested after the
-// products; 5 x 8 pairs of 3703, D = 256: 29.1 and 32.1).  Under a mask, and where the caches grow, a lane has other
-// loads or stores in the queue that the waits count: there a chunk is requested and awaited as a whole.
+// products; 5 x 8 pairs of 3703, D = 256: 29.1 and 32.1).  Under an additive mask, and where the caches grow, a lane has other
+// loads or stores in the queue that the waits count: there a chunk is requested and awaited as a whole.  A Bool mask's bytes are copied
+// to LDS in a fixed number of instructions a chunk, [slot][32 keys], for that reason (loaded per lane, with a chunk awaited as a whole / copied:
+// 32 pairs of 4096 keys 17.4 / 15.4 us, 64 x 22360 118 / 111, 128 x 2000, D = 256 48.4 / 44.6; 22 shapes 1.07 of the speed).
 // S^T = K Q^T on v_mfma_f32_16x16x32_bf16 (operand A: 16 keys x 32 d read back from LDS, rows swizzled by the key
 // so that the 16 rows of a read fall into different banks; operand B: the queries, 16 columns, loaded once;
 // queries beyond Sq repeat the last one and are not written; from 17 on a second block of 16 takes the same K and V
@@ -26,7 +28,7 @@
 // A pair is a (batch, head), or a (batch, run of consecutive heads) when those heads share their K and V (zero
 // head strides: multi-query / grouped-query attention): the run's heads then occupy the query slots together
 // and K and V are read once for all of them.  attn_mask (Bool bytes or additive bf16, any broadcast layout) and
-// softcap of the reference (transformer.rs:112-132) are template options: a lane loads the mask of its eight keys
+// softcap of the reference (transformer.rs:112-132) are template options: a lane has the mask of its eight keys
 // with the chunk's copies and applies it, then the cap, to its scores before the maximum.
 #include <hip/hip_runtime.h>
 
@@ -123,8 +125,12 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
     constexpr int kSlots = 16 * kQB;                     // query slots of a pair
     constexpr int kPartBytes = kQB * (kColBlocks * 1024 + 128);  // a wave's O blocks, then maximum and sum, per query block
     constexpr int kLds = kWaves * kWaveBytes > kWaves * kPartBytes ? kWaves * kWaveBytes : kWaves * kPartBytes;
-    static_assert(kLds <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(1024))) char smem[kLds];
+    // A Bool mask's bytes of a chunk, [query slot][32 keys], are copied like the keys, so that the next chunk can be under way here too
+    constexpr bool kPipe = kMask != 2 && !kAppend;
+    constexpr int kMaskCopies = kMask == 1 ? 2 * kQB : 0;  // of 64 words
+    constexpr int kMaskBytes = kMaskCopies * 256;
+    static_assert(kLds + kWaves * kMaskBytes <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char smem[kLds + kWaves * kMaskBytes];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int jl = lane & 15, blk = lane >> 4;
     const int bh = blockIdx.y, b = bh / lay.heads, h = (bh % lay.heads) * lay.group;  // h: the pair's first head
@@ -191,9 +197,27 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
                          : "m0", "memory");
         }
     };
-    constexpr bool kPipe = kMask == 0 && !kAppend;
+    const unsigned lds_m = (unsigned)(uintptr_t)MRK_FD_LDS(char, smem) + kLds + wave * kMaskBytes;
+    const char* mask_of[kMaskCopies ? kMaskCopies : 1];  // the mask row of the slot that a lane copies words of: slot 8 i + lane / 8, word lane % 8
+    auto copy_mask = [&](int ci) {
+        const int k0 = k_begin + ci * kChunkKeys, words = (k_end - k0) >> 2;  // (words past the end repeat the last one: those keys do not exist)
+        const int word = (lane & 7) < words ? lane & 7 : words - 1;
+#pragma unroll
+        for (int i = 0; i < kMaskCopies; i++) {
+            const char* at = mask_of[i] + k0 + 4 * word;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds_m + i * 256), "v"(at) : "m0", "memory");
+        }
+    };
+    if (kPipe && wave < chunks) copy(wave, lds_k, k_head, lay.k_row, k_piece);
+    if constexpr (kMask == 1) {
+#pragma unroll
+        for (int i = 0; i < kMaskCopies; i++) {
+            const int nq = Sq * lay.group, want = 8 * i + (lane >> 3), slot = want < nq ? want : nq - 1, qg = slot / Sq, qi = slot - qg * Sq;
+            mask_of[i] = static_cast<const char*>(dm.mask) + (b * dm.batch + (h + qg) * dm.head + qi * dm.row);
+        }
+    }
     if (kPipe && wave < chunks) {
-        copy(wave, lds_k, k_head, lay.k_row, k_piece);
+        if constexpr (kMask == 1) copy_mask(wave);
         copy(wave, lds_v, v_head, lay.v_row, v_piece);
     }
     // the queries: operand B, query slot 16 qb + jl (the last one again beyond the pair's slots), eight d at 32 s + 8 blk
@@ -209,8 +233,7 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
         const int slot = want < nq ? want : nq - 1;
         const int qg = slot / Sq, qi = slot - qg * Sq;
         mrow[qb] = nullptr;
-        if constexpr (kMask != 0)
-            mrow[qb] = static_cast<const char*>(dm.mask) + (b * dm.batch + (h + qg) * dm.head + qi * dm.row) * (kMask == 2 ? 2 : 1);
+        if constexpr (kMask == 2) mrow[qb] = static_cast<const char*>(dm.mask) + (b * dm.batch + (h + qg) * dm.head + qi * dm.row) * 2;
         const char* qrow = reinterpret_cast<const char*>(Q + b * lay.q_batch + (h + qg) * lay.q_head) + (size_t)qi * lay.q_row;
 #pragma unroll
         for (int s = 0; s < kSteps; s++) qf[qb][s] = *reinterpret_cast<const u32x4*>(qrow + 64 * s + 16 * blk);
@@ -250,22 +273,24 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
         for (int qb = 0; qb < kQB; qb++) {
             mb0[qb] = mb1[qb] = 0u;
             ma0[qb] = ma1[qb] = u32x2{0u, 0u};
-            if constexpr (kMask != 0) {
+            if constexpr (kMask == 2) {
                 const int g0 = k0 + 4 * blk, g1 = g0 + 16;
-                if constexpr (kMask == 1) {
-                    if (g0 < k_end) mb0[qb] = *reinterpret_cast<const unsigned*>(mrow[qb] + g0);
-                    if (g1 < k_end) mb1[qb] = *reinterpret_cast<const unsigned*>(mrow[qb] + g1);
-                } else {
-                    if (g0 < k_end) ma0[qb] = *reinterpret_cast<const u32x2*>(mrow[qb] + 2 * (size_t)g0);
-                    if (g1 < k_end) ma1[qb] = *reinterpret_cast<const u32x2*>(mrow[qb] + 2 * (size_t)g1);
-                }
+                if (g0 < k_end) ma0[qb] = *reinterpret_cast<const u32x2*>(mrow[qb] + 2 * (size_t)g0);
+                if (g1 < k_end) ma1[qb] = *reinterpret_cast<const u32x2*>(mrow[qb] + 2 * (size_t)g1);
             }
         }
         const bool more = ci + kWaves < chunks;
         if constexpr (kPipe)
-            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies) : "memory");  // the keys; the values may still be on their way
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies) : "memory");  // the keys (and their mask); the values may still be on their way
         else
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (kMask == 1) {
+#pragma unroll
+            for (int qb = 0; qb < kQB; qb++) {
+                mb0[qb] = *MRK_FD_LDS(unsigned, lds_m + (16 * qb + jl) * 32 + 4 * blk);
+                mb1[qb] = *MRK_FD_LDS(unsigned, lds_m + (16 * qb + jl) * 32 + 4 * blk + 16);
+            }
+        }
         if constexpr (kAppend) {
             // what this lane copied, to its place in the grown cache
 #pragma unroll
@@ -295,6 +320,7 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
         }
         if (kPipe && more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this chunk's keys are in registers
+            if constexpr (kMask == 1) copy_mask(ci + kWaves);
             copy(ci + kWaves, lds_k, k_head, lay.k_row, k_piece);
         }
         bf16x8 pb[kQB];
@@ -361,7 +387,7 @@ __global__ __launch_bounds__(decode_waves<kD>() * 64) void flash_decode_split(
             pb[qb] = __builtin_convertvector(p, bf16x8);
         }
         if constexpr (kPipe) {  // the values
-            if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies) : "memory");
+            if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kCopies + kMaskCopies) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
 #pragma unroll
