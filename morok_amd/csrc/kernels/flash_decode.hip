@@ -531,10 +531,23 @@ __global__ __launch_bounds__(256) void flash_decode_merge(const float* __restric
     fold_ranges<kD>([&](int s) { return src + s * slice; }, splits, O, bh, q, d, Sq, lay);
 }
 
+__global__ __launch_bounds__(256) void clear_words(unsigned* words, long n) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) words[i] = 0u;
+}
+
 }  // namespace mrk::dev
 
 namespace mrk {
 using namespace mrk::dev;
+
+int launch_clear_words(void* stream, void* words, long n) {
+    if (n <= 0) return 0;
+    if (n > 0x7fffffffL || !words) return (int)hipErrorInvalidValue;
+    (void)hipGetLastError();
+    clear_words<<<(unsigned)((n + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(static_cast<unsigned*>(words), n);
+    return (int)hipGetLastError();
+}
 
 // Shapes the split kernel takes and the number of key ranges it uses: up to 32 query slots of a pair (two blocks
 // of 16: 17 and more cost a second set of matrix instructions per chunk, still far from what the stream of K and V

@@ -158,6 +158,8 @@ int launch_flash_decode(void* stream, const void* q, const void* k, const void* 
                         float scale, const long* strides, long splits, long keys_per_split, void* W, const void* mask = nullptr,
                         int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f, long group = 1,
                         unsigned* arrivals = nullptr);
+// n words of zeros (a kernel's counters)
+int launch_clear_words(void* stream, void* words, long n);
 // One query per (batch, head) over past_k / past_v [B, H, Sk - 1, D] and one new key and value each (all bf16), which also writes the grown
 // caches k_out / v_out [B, H, Sk, D]: the bits of the copies followed by the attention over them.  strides (elements, multiples of
 // 8): q batch, head; new key batch, head; new value batch, head; o batch, head.  Workspace as flash_fwd_workspace_bytes says.

@@ -2411,15 +2411,24 @@ struct Scheduler {
     // A plan that outlives this call keeps a counter per pair for the attention that splits its keys, which spares it the launch that merges
     // the ranges (one query against 32 pairs of 4096 keys 16.9 -> 15.0 us).  They have to be zero at a launch and are again after it: memory of
     // the plan's own, not an intermediate that shares a block.  A realization would have to clear them first, as long a launch as the one
-    // it saves.
+    // it saves.  (One allocation with the scratch, cleared by a kernel: a second one and a memset made prepare() 25 us longer.)
     bool outlives = false;
-    int count_arrivals(int64_t pairs, std::vector<int64_t>* params, std::vector<std::shared_ptr<Buffer>>* bufs) {
-        if (!outlives || dry) return kOk;
-        BufferOptions zeros;
-        zeros.zero_init = true;
-        auto arrivals = std::make_shared<Buffer>(dev->allocator, static_cast<size_t>(pairs) * sizeof(unsigned), zeros);
-        MRK_TRY(arrivals->ensure_allocated());
-        bufs->push_back(arrivals);
+    int scratch_of_ranges(size_t ws, int64_t pairs, std::vector<int64_t>* params, std::vector<std::shared_ptr<Buffer>>* bufs) {
+        params->push_back(static_cast<int64_t>(ws));
+        if (!outlives || dry) {
+            bufs->push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
+            return kOk;
+        }
+        const Buffer whole(dev->allocator, ws + static_cast<size_t>(pairs) * sizeof(unsigned), BufferOptions());
+        MRK_TRY(whole.ensure_allocated());
+        std::unique_ptr<Buffer> ranges, arrivals;
+        MRK_TRY(whole.view(0, ws, &ranges));
+        MRK_TRY(whole.view(ws, static_cast<size_t>(pairs) * sizeof(unsigned), &arrivals));
+        void* at = nullptr;
+        MRK_TRY(arrivals->as_raw_ptr(&at));
+        MRK_HIP(launch_clear_words(dev->allocator->stream(), at, pairs), "clearing counters");
+        bufs->push_back(std::move(ranges));
+        bufs->push_back(std::move(arrivals));
         params->push_back(1);
         return kOk;
     }
@@ -2515,27 +2524,19 @@ struct Scheduler {
             bufs.push_back(has_mask ? mask_buf : bufs[1]);
             // a handful of queries without the causal rule: the kernel that splits the keys, with its scratch
             const size_t ws = flash_fwd_workspace_bytes(B * H, Sq, Sk, D, att->hint_causal ? 1 : 0);
-            if (ws) {
-                bufs.push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
-                params.push_back(static_cast<int64_t>(ws));
-                MRK_TRY(count_arrivals(B * H, &params, &bufs));
-            }
+            if (ws) MRK_TRY(scratch_of_ranges(ws, B * H, &params, &bufs));
             MRK_TRY(builtin("flash_fwd_bf16_ext", params, bufs));
         } else {
             // a handful of queries against a long key sequence: the keys are split over workgroups and the ranges'
             // partial results go through scratch, an intermediate of the plan like any other
             const size_t ws = flash_fwd_workspace_bytes(B * H, Sq, Sk, D, att->hint_causal ? 1 : 0);
-            if (ws) bufs.push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
             if (dense) {
                 params = {B * H, Sq, Sk, D, att->hint_causal ? 1 : 0, static_cast<int64_t>(bits)};
             } else {
                 params = {B, H, Sq, Sk, D, att->hint_causal ? 1 : 0, static_cast<int64_t>(bits), offsets[0], offsets[1], offsets[2], 0};
                 params.insert(params.end(), strides.begin(), strides.end());
             }
-            if (ws) {
-                params.push_back(static_cast<int64_t>(ws));
-                MRK_TRY(count_arrivals(B * H, &params, &bufs));
-            }
+            if (ws) MRK_TRY(scratch_of_ranges(ws, B * H, &params, &bufs));
             MRK_TRY(builtin(dense ? "flash_fwd_bf16" : "flash_fwd_bf16_strided", params, bufs));
         }
         dst->buffer = out;

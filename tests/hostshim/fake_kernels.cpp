@@ -123,6 +123,7 @@ int launch_gemm_f32(void* stream, const void*, const void*, void*, const void* a
     mrk_shim_note_launch(stream, add ? (add_is_row ? "gemm_f32_bias" : "gemm_f32_residual") : b_transposed ? "gemm_f32_nt" : "gemm_f32");
     return 0;
 }
+int launch_clear_words(void*, void*, long) { return 0; }
 int launch_fill(void* stream, void*, size_t, int, int, unsigned long long, unsigned long long, float, float) {
     mrk_shim_note_launch(stream, "fill");
     return 0;
