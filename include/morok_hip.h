@@ -448,8 +448,8 @@ int mrk_hip_gemm_bf16(int device_id, const void* a, const void* b, void* c, int6
 size_t mrk_hip_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t batch);
 /* Which kernel a bf16 or f16 product of this shape runs on, with aligned operands and the scratch above: out = {rows and columns of C
  * that a workgroup owns, ranges of K, stages of the small-tile kernel (0: the kernels of large tiles)}; rows 0 where up to 64 rows are
- * streamed.  b_transposed: second operand [N, K]; paired: with the gated or the rotary epilogue, n all of its columns
- * (a rotary product of more than 256 tiles of 128 x 256 runs on tiles of 256 x 256 whatever is reported). */
+ * streamed.  b_transposed: second operand [N, K]; paired: 0, or with the gated (1) or the rotary (2) epilogue, n all of
+ * its columns. */
 int mrk_hip_gemm_16bit_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int b_transposed, int paired, int64_t out[4]);
 /* c[M,N] = a[M,K] * bt[N,K]^T: the product with the second operand as it is stored by a Linear
  * layer (weight [out_features, in_features], tensor/src/nn/linear.rs:9-14, 39-41), read in place

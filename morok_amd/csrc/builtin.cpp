@@ -280,7 +280,7 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         if (!gemm_bf16_swiglu_supported(p[0], p[1], p[2], nt))
             return failf(kInvalidArgument, "%s: shape not covered (M, F, K > 0; F and K multiples of 8)", k.c_str());
         std::string name = k + "_" + std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]);
-        const int tile = gemm_bf16_paired_tile(p[0], 2 * p[1], p[2]);
+        const int tile = gemm_bf16_paired_tile(p[0], 2 * p[1], p[2], false);
         out->reset(new BuiltinProgram(device_id, stream, name, 3, p,
                                       [nt, tile](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                           return launch_gemm_bf16_swiglu(s, b[1], b[2], b[0], q[0], q[1], q[2], nt, tile);
@@ -295,7 +295,7 @@ int create_builtin_program(int device_id, ffi::Stream stream, const char* kind, 
         if (!gemm_bf16_rope_supported(p[0], p[1], p[2], p[3], p[4]))
             return fail(kInvalidArgument, k + ": shape not covered (K a multiple of 64, N of 8, split a multiple of 256 within N, seq > 0)");
         std::string name = k + "_" + std::to_string(p[0]) + "_" + std::to_string(p[1]) + "_" + std::to_string(p[2]) + "_s" + std::to_string(p[3]);
-        const int tile = gemm_bf16_paired_tile(p[0], p[1], p[2]);
+        const int tile = gemm_bf16_paired_tile(p[0], p[1], p[2], true);
         out->reset(new BuiltinProgram(device_id, stream, name, 6, p,
                                       [nt, tile](ffi::Stream s, void* const* b, const std::vector<int64_t>& q) {
                                           return launch_gemm_bf16_rope(s, b[1], b[2], b[0], b[3], q[0], q[1], q[2], q[3], b[4], b[5], q[4], nt, tile);

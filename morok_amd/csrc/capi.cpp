@@ -881,7 +881,7 @@ size_t mrk_hip_gemm_bf16_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_
 int mrk_hip_gemm_16bit_tile(int64_t m, int64_t n, int64_t k, int64_t batch, int b_transposed, int paired, int64_t out[4]) {
     MRK_NONNULL(out);
     if (m < 0 || n < 0 || k < 0 || batch < 1) return fail(kInvalidArgument, "gemm_16bit_tile: bad shape");
-    const ProductTile t = gemm_16bit_tile(m, n, k, batch, b_transposed != 0, paired != 0);
+    const ProductTile t = gemm_16bit_tile(m, n, k, batch, b_transposed != 0, paired);
     out[0] = t.rows, out[1] = t.cols, out[2] = t.k_ranges, out[3] = t.stages;
     return kOk;
 }

@@ -694,7 +694,8 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         const f32x8 x = __builtin_convertvector(__builtin_bit_cast(bf16x8, v[t]), f32x8);
                         const f32x8 y = __builtin_convertvector(__builtin_bit_cast(bf16x8, pv[t]), f32x8);
                         const f32x8 sn = lc < 8 ? -sn_cur[t] : sn_cur[t];  // first half: x1 cos - x2 sin; second half: x2 cos + x1 sin
-                        const f32x8 o = __builtin_elementwise_fma(y, sn, x * cs_cur[t]);
+                        // (which of the two products is rounded decides the last bit: the sine's in rows 0..3 of sixteen, the cosine's below)
+                        const f32x8 o = t == 0 ? __builtin_elementwise_fma(x, cs_cur[t], y * sn) : __builtin_elementwise_fma(y, sn, x * cs_cur[t]);
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
@@ -1058,12 +1059,12 @@ double large_tiles_us(long M, long N, long K, long batch, long splits, long kt_p
     return us + 6.5 + (splits > 1 ? 4.2 + 0.25 * splits + 0.06 * 4e-6 * splits * batch * M * N : 0.0);
 }
 // One pass of 256-row tiles, in us (tiles of 256 x 256: fitted to 39 shapes, 8 % off)
-double tiles256_us(long M, long N, long K) {
-    if (mid_pipelined(N, K) && mid_many_tiles(M, N, 1)) return large_pass_us(M, N, K, 1);
+double rounds256_us(long M, long N, long K) {
     const double rounds = (double)((((M + 255) / 256) * ((N + 255) / 256) + 255) / 256), mb = 2e-6 * ((double)M * K + (double)N * K + (double)M * N);
     const double us = rounds * (1.02 * ((K + 63) / 64) + 5.8);
     return 4.8 + (us > mb / 4.0 ? us : mb / 4.0);
 }
+double tiles256_us(long M, long N, long K) { return mid_pipelined(N, K) && mid_many_tiles(M, N, 1) ? large_pass_us(M, N, K, 1) : rounds256_us(M, N, K); }
 // Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both
 // decide, with a margin for their errors: against the large tiles alone 0.71 of the time over 1400 shapes (geometric mean), 2 of them
 // slower by more than 5 % (8 at most).  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
@@ -1091,14 +1092,27 @@ Route choose_route(long M, long N, long K, long batch) {
     if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
     return r;
 }
-// The gated (N = 2 F) and the rotary product: small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
+// The gated product (N = 2 F): small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
 // two rounds of 256, against 860 of 128 x 128).  A negative answer: tiles of 256 x 256.
-int choose_paired_tile(long M, long N, long K) {
-    const MidPlan p = plan_mid(M, N, K, 1, true, true);
+int gated_tile(const MidPlan& p, long M, long N, long K) {
     // (the kernel addresses B's columns from its first with 32-bit offsets)
     return p.tile >= 0 && (double)N * K < 1e9 && p.us < 0.95 * tiles256_us(M, N, K) ? p.tile : -1;
 }
-// Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form
+// The rotary product.  Tiles of 256 x 256 round the products of a rotation as they always have, small tiles as they do: which of the two a shape
+// runs on decides the last bit of a few results (16 of a million), so that is a matter of the estimates the number of K ranges follows from, and
+// those of gemm_mid.hip choose among the small tiles alone.  Where more than 256 tiles of 128 x 256 exist that is 128 x 128, taken in turn where
+// the pipeline is long enough for it, with two stages and two workgroups to a compute unit where it is not (us on 256 x 256 / on the one that
+// small tiles then run on: 2568 x 6144 x 2048 95.5 / 76.4, 5384 x 3072 x 1024 55.1 / 54.7, 2440 x 3112 x 384 22.3 / 16.8, 6531 x 2344 x 2432 100 / 78;
+// 4000 x 4608 x 256 35.9 / 29.6, 9149 x 5680 x 64 50.1 / 44.7 (60.9 with three stages); 80 shapes 0.84 in the geometric mean).  Up to 256 rows
+// tiles of 256 x 256 come out in as many or fewer rounds: 156 x 61680 x 1984 59.2 / 82.9, 230 x 59600 x 64 16.9 / 18.4, 183 x 35008 x 768 28.2 / 28.8.
+int rotary_tile(const MidPlan& p, long M, long N, long K) {
+    const bool many = mid_many_tiles(M, N, 1);
+    if (p.tile < 0 || (double)N * K >= 1e9 || (many && M <= 256) || p.ranges_us >= 0.95 * rounds256_us(M, N, K)) return -1;
+    return !many ? p.tile : mid_pipelined(N, K) ? kMidThreeStages : kMidTwoStages;
+}
+// Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form: against the
+// faster of its tiles by estimate, for the rotation too where it runs on the other ones.  (Against those, 3 of 1000 shapes more would be separate,
+// and 7 of 8 of them measured slower so: fused / product + rotation in us, 9053 x 2464 x 12928 498 / 553, 10868 x 4408 x 7680 595 / 601.)
 bool choose_separate(const Route& r, long M, long N, long K) {
     if (!r.mid) return r.splits > 1;  // (as large tiles: the fused forms are theirs)
     const MidPlan fused = plan_mid(M, N, K, 1, true, true);
@@ -1109,9 +1123,9 @@ bool choose_separate(const Route& r, long M, long N, long K) {
 // last shapes it met (pure functions of the shape).
 struct Chosen {
     long M = 0, N = 0, K = 0, batch = 0;
-    bool has_route = false, has_paired = false, has_separate = false, separate = false;
+    bool has_route = false, has_paired[2] = {}, has_separate = false, separate = false;
     Route route;
-    int paired = -1;
+    int paired[2] = {-1, -1};  // gated, rotary
 };
 Chosen& chosen(long M, long N, long K, long batch) {
     static thread_local Chosen kept[32];
@@ -1207,12 +1221,12 @@ size_t gemm_bf16_nt_workspace_bytes(long M, long N, long K, long batch) {
     return route_bytes(M, N, K, batch, true);
 }
 
-ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, bool paired) {
+ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, int paired) {
     using namespace mrk::dev;
     ProductTile t;
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return t;
     if (paired) {
-        const int tile = gemm_bf16_paired_tile(M, N, K);
+        const int tile = gemm_bf16_paired_tile(M, N, K, paired == 2);
         t.rows = kBM, t.cols = kBN;
         if (tile >= 0) mid_tile_shape(tile, &t.rows, &t.cols, &t.stages);
         return t;
@@ -1275,11 +1289,14 @@ bool gemm_bf16_separate_preferred(long M, long N, long K) {
     return e.separate;
 }
 
-int gemm_bf16_paired_tile(long M, long N, long K) {
+int gemm_bf16_paired_tile(long M, long N, long K, bool rotary) {
     if (M <= 0 || N <= 0 || K <= 0) return -1;
     Chosen& e = chosen(M, N, K, 1);
-    if (!e.has_paired) e.paired = choose_paired_tile(M, N, K), e.has_paired = true;
-    return e.paired;
+    if (!e.has_paired[rotary]) {
+        const MidPlan p = plan_mid(M, N, K, 1, true, true);
+        e.paired[rotary] = rotary ? rotary_tile(p, M, N, K) : gated_tile(p, M, N, K), e.has_paired[rotary] = true;
+    }
+    return e.paired[rotary];
 }
 
 int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C, long M, long F, long K, bool b_transposed, int tile) {
@@ -1291,7 +1308,7 @@ int launch_gemm_bf16_swiglu(void* stream, const void* A, const void* B, void* C,
     if (b_transposed && gemm_nt_swiglu_streamed(M, F, K)) return launch_gemm_nt_swiglu_streamed(stream, A, B, C, M, F, K);
     hipStream_t s = static_cast<hipStream_t>(stream);
     (void)hipGetLastError();
-    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, 2 * F, K);
+    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, 2 * F, K, false);
     if (tile >= 0) return launch_gemm_mid_paired(s, tile, A, B, C, M, 2 * F, K, b_transposed, nullptr);
     const long tn = (F + 127) / 128, tm = (M + kBM - 1) / kBM;
     const dim3 grid((unsigned)(tm * tn), 1);
@@ -1320,10 +1337,7 @@ int launch_gemm_bf16_rope(void* stream, const void* A, const void* B, void* C_ro
                           reinterpret_cast<uintptr_t>(C_rest) | reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin);
     if (all % 16 || reinterpret_cast<uintptr_t>(cos) % 32 || reinterpret_cast<uintptr_t>(sin) % 32) return (int)hipErrorInvalidValue;
     (void)hipGetLastError();
-    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, N, K);
-    // In several rounds of small tiles each waits for its rows' angles anew (8000 x 3072 x 1024: 64.3 us on 256 x 128, 61.0 on 256 x 256; gated
-    // products of such sizes gain, 4096 x 5632 x 1024 55.0 -> 48.9)
-    if (mid_many_tiles(M, N, 1)) tile = -1;
+    if (tile == kChooseTile) tile = gemm_bf16_paired_tile(M, N, K, true);
     if (tile >= 0) {
         const MidRope angles{static_cast<const float*>(cos), static_cast<const float*>(sin), C_rest, (int)seq, (int)split};
         return launch_gemm_mid_paired(static_cast<hipStream_t>(stream), tile, A, B, C_rot, M, N, K, b_transposed, &angles);

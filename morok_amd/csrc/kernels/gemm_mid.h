@@ -9,8 +9,9 @@ struct MidPlan {
     int tile = -1;
     long splits = 1, kt_per_split = 0;
     double us = 0.0;
-    double ranges_us = 0.0;  // what the number of ranges follows from (us, where that is more than one)
+    double ranges_us = 0.0;  // what the number of ranges follows from (us, where that is more than one), and the rounding of a rotation
 };
+constexpr int kMidTwoStages = 0, kMidThreeStages = 1;  // tiles of 128 x 128
 constexpr int kMidSmallest = 3, kMidUnaligned = 4;  // tiles of 64 x 64: rows of whole chunks; rows that start on any element
 constexpr int kMidTall = 5;                         // tiles of 256 x 128
 // The fastest by estimate.  whole_chunks: rows of both operands are whole 16-byte chunks on 16-byte bases, whichever way B is stored; else

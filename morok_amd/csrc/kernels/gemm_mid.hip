@@ -259,10 +259,10 @@ __global__ __launch_bounds__(kCopyWaves ? 512 : 256, !kCopyWaves || kTM * kTN >=
                         f32x4 first = x, second = y;
                         if (rotated) {
                             const f32x4 cs = *reinterpret_cast<const f32x4*>(rope.cos + pos + in_head), sn = *reinterpret_cast<const f32x4*>(rope.sin + pos + in_head);
-                            // (the product that is rounded is the cosine's, as in the tiles of 256 x 256: left to the compiler it was the sine's here,
-                            // and 386 of 25 million results an ulp from theirs)
-                            first = __builtin_elementwise_fma(y, -sn, x * cs);
-                            second = __builtin_elementwise_fma(x, sn, y * cs);
+                            // (the product that is rounded is the sine's; on tiles of 256 x 256 it is in a quarter of the rows, and some 12 of a
+                            // million results lie an ulp from these)
+                            first = __builtin_elementwise_fma(x, cs, y * -sn);
+                            second = __builtin_elementwise_fma(y, cs, x * sn);
                         }
                         // rotated columns: row pitch `split`; those behind: a matrix of their own
                         const size_t ldc = rotated ? (size_t)rope.split : (size_t)(N - rope.split);
@@ -679,8 +679,8 @@ void with_tile(int tile, F&& f) {
     using I64 = integral_constant<int, 64>;
     using I128 = integral_constant<int, 128>;
     switch (tile) {
-        case 0: f(I128{}, I128{}, integral_constant<int, 2>{}); break;
-        case 1: f(I128{}, I128{}, integral_constant<int, 3>{}); break;
+        case kMidTwoStages: f(I128{}, I128{}, integral_constant<int, 2>{}); break;
+        case kMidThreeStages: f(I128{}, I128{}, integral_constant<int, 3>{}); break;
         case 2: f(I128{}, I64{}, integral_constant<int, 3>{}); break;
         case kMidTall: f(integral_constant<int, 256>{}, I128{}, integral_constant<int, 3>{}); break;
         default: f(I64{}, I64{}, integral_constant<int, 3>{}); break;

@@ -97,7 +97,7 @@ bool gemm_bf16_separate_preferred(long M, long N, long K);
 // The tile the gated and the rotary product (N all of their columns) run on, for their last argument: a matter of the shape alone, so
 // a program asks once, when it is created; kChooseTile asks at the launch.
 constexpr int kChooseTile = -2;
-int gemm_bf16_paired_tile(long M, long N, long K);
+int gemm_bf16_paired_tile(long M, long N, long K, bool rotary);
 int launch_gemm_bf16_swiglu(void* stream, const void* a, const void* w, void* c, long M, long F, long K, bool b_transposed = false,
                             int tile = kChooseTile);
 // A packed projection whose first `split` columns are attention heads of 128 columns (q | k of a
@@ -117,13 +117,13 @@ int launch_gemm_bf16_rope(void* stream, const void* a, const void* b, void* c_ro
 size_t gemm_bf16_workspace_bytes(long M, long N, long K, long batch);
 // The tile of C that a workgroup of the product owns, given aligned operands and the scratch asked for above: rows, columns, ranges of K and
 // the stages of the small-tile kernel (0: the kernels of large tiles).  rows = 0: a streaming kernel (up to 64 rows).  paired: with the
-// gated or the rotary epilogue, N all of its columns (the [N, K] gated form streams up to 64 rows).
+// gated (1) or the rotary (2) epilogue, N all of its columns (the [N, K] gated form streams up to 64 rows).
 struct ProductTile {
     int rows = 0, cols = 0;
     long k_ranges = 1;
     int stages = 0;
 };
-ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, bool paired);
+ProductTile gemm_16bit_tile(long M, long N, long K, long batch, bool b_transposed, int paired);
 // The same product with the split-K partials in a file-scope device array instead of a
 // caller's workspace, for callers that must not allocate.  gemm_bf16_static_workspace_init
 // resolves the array's address on one device (that device current; once per device, at

@@ -17,7 +17,7 @@ int launch_softmax_half(void* stream, const void*, void*, long, long, bool f16) 
     return 0;
 }
 size_t gemm_bf16_workspace_bytes(long, long, long, long) { return 0; }
-ProductTile gemm_16bit_tile(long, long, long, long, bool, bool) { return ProductTile(); }
+ProductTile gemm_16bit_tile(long, long, long, long, bool, int) { return ProductTile(); }
 size_t gemm_bf16_nt_workspace_bytes(long, long, long, long) { return 0; }
 bool gemm_bf16_separate_preferred(long, long, long) { return false; }
 int launch_gemm_bf16(void* stream, const void*, const void*, void*, long, long, long, int, long, void*, size_t, bool b_transposed, bool f16) {
@@ -81,12 +81,12 @@ int launch_gemm_bf16_residual(void* stream, const void*, const void*, const void
 bool gemm_bf16_swiglu_supported(long M, long F, long K, bool) { return M > 0 && F > 0 && K > 0 && F % 8 == 0 && K % 8 == 0; }
 static std::atomic<size_t> g_tile_choices{0};
 extern "C" size_t mrk_shim_tile_choices() { return g_tile_choices; }
-int gemm_bf16_paired_tile(long, long, long) {
+int gemm_bf16_paired_tile(long, long, long, bool) {
     g_tile_choices++;
     return -1;
 }
 int launch_gemm_bf16_swiglu(void* stream, const void*, const void*, void*, long M, long F, long K, bool b_transposed, int tile) {
-    if (tile == kChooseTile) gemm_bf16_paired_tile(M, 2 * F, K);
+    if (tile == kChooseTile) gemm_bf16_paired_tile(M, 2 * F, K, false);
     mrk_shim_note_launch(stream, b_transposed ? "gemm_bf16_nt_swiglu" : "gemm_bf16_swiglu");
     return 0;
 }
@@ -94,7 +94,7 @@ bool gemm_bf16_rope_supported(long M, long N, long K, long split, long seq) {
     return M > 0 && N > 0 && K > 0 && seq > 0 && K % 64 == 0 && N % 8 == 0 && split > 0 && split <= N && split % 256 == 0;
 }
 int launch_gemm_bf16_rope(void* stream, const void*, const void*, void*, void*, long M, long N, long K, long, const void*, const void*, long, bool b_transposed, int tile) {
-    if (tile == kChooseTile) gemm_bf16_paired_tile(M, N, K);
+    if (tile == kChooseTile) gemm_bf16_paired_tile(M, N, K, true);
     mrk_shim_note_launch(stream, b_transposed ? "gemm_bf16_nt_rope" : "gemm_bf16_rope");
     return 0;
 }
