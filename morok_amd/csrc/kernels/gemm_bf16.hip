@@ -1067,14 +1067,17 @@ double rounds256_us(long M, long N, long K) {
 double tiles256_us(long M, long N, long K) { return mid_pipelined(N, K) && mid_many_tiles(M, N, 1) ? large_pass_us(M, N, K, 1) : rounds256_us(M, N, K); }
 // Where more than 256 tiles of 128 x 256 exist the large tiles win (2222 x 6144 x 2048 44 us against 66); below, the estimates of both
 // decide, with a margin for their errors: against the large tiles alone 0.71 of the time over 1400 shapes (geometric mean), 2 of them
-// slower by more than 5 % (8 at most).  Odd operands cost the large tiles a padded copy each (3.5 us and its traffic).
+// slower by more than 5 % (8 at most).  Above 256 the estimates of rounds decide for a single product whose pipeline is long enough; those count
+// on tiles taken in turn, which those of a batch are not (us on large tiles / as estimated: 8 x 1000 x 3000 x 384 31.1 / 38.5, 20 x 640 x 768 x 320
+// 16.0 / 20.5, 14 x 1627 x 384 x 512 18.7 / 25.0; 64 x 128 x 2048 x 320 34.1 / 32.1).  Odd operands cost the large tiles a padded copy each (3.5 us
+// and its traffic).
 Route choose_route(long M, long N, long K, long batch) {
     Route r;
     const SplitPlan sp = tile_addressable(M, N, K, batch) ? plan_split_k(M, N, K, batch) : SplitPlan();
     r.splits = sp.splits, r.kt_per_split = sp.kt_per_split;
     const long tiles = ((M + 127) / 128) * ((N + 255) / 256) * batch, kt = (K + 63) / 64;
     const bool pipelined = sp.splits == 1 && mid_pipelined(N, K);
-    if (tiles > 256 && !pipelined) return r;
+    if (tiles > 256 && (batch > 1 || !pipelined)) return r;
     const bool whole = N % 8 == 0 && K % 8 == 0;
     r.plan = plan_mid(M, N, K, batch, whole);
     if (r.plan.tile < 0) return r;
