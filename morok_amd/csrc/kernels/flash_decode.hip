@@ -595,6 +595,14 @@ size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal) 
     return most;
 }
 
+// The last workgroup of a pair folds its ranges where they fit the local memory a workgroup has anyway.  Its three trips to memory in a row
+// (results out, the count, results in) take less than a second launch (us with it / without: 32 pairs of 4096 keys 17.2 / 15.3, D = 64:
+// 16 x 4000 11.4 / 9.4, 4 x 30000 18.5 / 13.6; 8 slots of 32 x 2243 17.8 / 16.5), but for rows of 256 from five slots on, which four waves
+// fold (4 slots of 16 x 2000 17.6 / 16.7, 8 of 8 x 1500 15.3 / 17.0).
+bool flash_decode_folds(long splits, long slots, long D) {
+    return splits > 1 && splits * slots * (D + 2) * (long)sizeof(float) <= (D == 64 ? 64 : 128) * 1024 && (D != 256 || slots <= 4);
+}
+
 // strides: (batch, head, row) element strides of q, k, v and o (validated by the caller: multiples of 8, rows
 // addressable in 32 bits, pointers 16-byte aligned); W: splits * pairs * flash_decode_slot_capacity(group * Sq) * (D + 2)
 // floats, needed with several splits (pairs = B * H / group).
@@ -640,12 +648,7 @@ int launch_flash_decode(void* stream, const void* q, const void* k, const void* 
     const long quads = pairs * slots * (D / 4);
     const unsigned merge_blocks = (unsigned)((quads + 255) / 256);
     const int slot_cap = (int)flash_decode_slot_capacity(slots);
-    // The last workgroup of a pair folds its ranges where they fit the local memory a workgroup has anyway.  Its three trips to memory in a row
-    // (results out, the count, results in) take less than a second launch (us with it / without: 32 pairs of 4096 keys 17.2 / 15.3, D = 64:
-    // 16 x 4000 11.4 / 9.4, 4 x 30000 18.5 / 13.6; 8 slots of 32 x 2243 17.8 / 16.5), but for rows of 256 from five slots on, which four waves
-    // fold (4 slots of 16 x 2000 17.6 / 16.7, 8 of 8 x 1500 15.3 / 17.0).
-    const bool fold = splits * slots * (D + 2) * (long)sizeof(float) <= (D == 64 ? 64 : 128) * 1024 && (D != 256 || slots <= 4);
-    unsigned* counted = w && fold ? arrivals : nullptr;
+    unsigned* counted = w && flash_decode_folds(splits, slots, D) ? arrivals : nullptr;
 #define MRK_DECODE_QB(DIM, MASK, CAP, QB) \
     (counted ? flash_decode_split<DIM, MASK, CAP, QB, false, true> : flash_decode_split<DIM, MASK, CAP, QB>)<<<grid, decode_waves<DIM>() * 64, 0, s>>>(qp, kp, vp, op, w, (int)Sq, (int)Sk, (int)keys_per_split, scale_log2e, lay, dm, DecodeAppend{}, counted)
 #define MRK_DECODE(DIM, MASK)                              \

@@ -749,21 +749,29 @@ static long work_units(long BH, long q_tiles, long D, int causal) {
     return pairs ? (q_tiles + 1) / 2 : q_tiles;
 }
 
+// Heads that share K and V (zero head strides) become query slots of one pair: K and V are read once per batch
+// (runs of consecutive heads: the largest divisor of the head count that gives at most 32 slots).
+static long decode_group(long H, long Sq, const long* strides) {
+    if (H > 1 && strides[4] == 0 && strides[7] == 0 && Sq >= 1)
+        for (long g = 32 / Sq; g > 1; g--)
+            if (H % g == 0) return g;
+    return 1;
+}
+
+bool flash_fwd_counts_arrivals(long B, long H, long Sq, long Sk, long D, int causal, const long* strides) {
+    if (B <= 0 || H <= 0 || Sq <= 0) return false;
+    const long group = decode_group(H, Sq, strides);
+    long splits = 0, per = 0;
+    return flash_decode_plan(B * (H / group), group * Sq, Sk, D, causal, &splits, &per) && flash_decode_folds(splits, group * Sq, D);
+}
+
 // A handful of queries against a long key sequence: the kernel that splits the keys (flash_decode.hip), in as many
 // ranges as the workspace allows (one range needs none).
 static bool decode_route(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
                          float scale, int causal, const long* strides, void* workspace, size_t workspace_bytes, unsigned* arrivals, int* rc,
                          const void* mask = nullptr, int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f) {
     using namespace mrk::dev;
-    // heads that share K and V (zero head strides) become query slots of one pair: K and V are read once per batch
-    // (runs of consecutive heads: the largest divisor of the head count that gives at most 32 slots)
-    long group = 1;
-    if (H > 1 && strides[4] == 0 && strides[7] == 0 && Sq >= 1)
-        for (long g = 32 / Sq; g > 1; g--)
-            if (H % g == 0) {
-                group = g;
-                break;
-            }
+    const long group = decode_group(H, Sq, strides);
     const long pairs = B * (H / group), slots = group * Sq;
     long splits = 0, per = 0;
     if (!flash_decode_plan(pairs, slots, Sk, D, causal, &splits, &per)) return false;

@@ -154,6 +154,9 @@ inline bool flash_fwd_rows_addressable(long rows, long row_bytes, long D) {
 bool flash_decode_plan(long BH, long Sq, long Sk, long D, int causal, long* splits, long* keys_per_split);
 long flash_decode_slot_capacity(long slots);
 size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal);
+bool flash_decode_folds(long splits, long slots, long D);
+// Whether a launch with these (batch, head, row) strides of q, k, v and o, that workspace and counters would use the counters.
+bool flash_fwd_counts_arrivals(long B, long H, long Sq, long Sk, long D, int causal, const long* strides);
 int launch_flash_decode(void* stream, const void* q, const void* k, const void* v, void* o, long B, long H, long Sq, long Sk, long D,
                         float scale, const long* strides, long splits, long keys_per_split, void* W, const void* mask = nullptr,
                         int mask_kind = 0, const long* mask_strides = nullptr, float softcap = 0.0f, long group = 1,

@@ -2408,28 +2408,40 @@ struct Scheduler {
         return kOk;
     }
 
-    // A plan that outlives this call keeps a counter per pair for the attention that splits its keys, which spares it the launch that merges
-    // the ranges (one query against 32 pairs of 4096 keys 16.9 -> 15.0 us).  They have to be zero at a launch and are again after it: memory of
-    // the plan's own, not an intermediate that shares a block.  A realization would have to clear them first, as long a launch as the one
-    // it saves.  (One allocation with the scratch, cleared by a kernel: a second one and a memset made prepare() 25 us longer.)
+    // A plan that outlives this call keeps a counter per pair for the attention that splits its keys and folds them by counting, which spares it
+    // the launch that merges the ranges (one query against 32 pairs of 4096 keys 16.9 -> 15.0 us).  They have to be zero at a launch and are
+    // again after it: memory of the plan's own, not an intermediate that shares a block, as the ranges' partial results are.  A realization
+    // would have to clear them first, as long a launch as the one it saves.  (Words of one block for all of a plan's attentions, made and
+    // cleared by one kernel when the plan is accepted.)
     bool outlives = false;
-    int scratch_of_ranges(size_t ws, int64_t pairs, std::vector<int64_t>* params, std::vector<std::shared_ptr<Buffer>>* bufs) {
+    static constexpr size_t kCounterBlock = 0x1000;
+    std::vector<std::unique_ptr<Buffer>> counters;
+    size_t counters_used = 0;  // bytes of the last block
+    int scratch_of_ranges(size_t ws, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, bool causal, const std::vector<int64_t>& strides,
+                          std::vector<int64_t>* params, std::vector<std::shared_ptr<Buffer>>* bufs) {
         params->push_back(static_cast<int64_t>(ws));
-        if (!outlives || dry) {
-            bufs->push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
-            return kOk;
+        bufs->push_back(std::make_shared<Buffer>(dev->allocator, ws, BufferOptions()));
+        const std::vector<long> st(strides.begin(), strides.end());
+        if (!outlives || dry || !flash_fwd_counts_arrivals(B, H, Sq, Sk, D, causal ? 1 : 0, st.data())) return kOk;
+        const size_t bytes = static_cast<size_t>(B * H) * sizeof(unsigned);
+        if (counters.empty() || counters.back()->size() - counters_used < bytes) {
+            counters.emplace_back(new Buffer(dev->allocator, std::max(bytes, kCounterBlock), BufferOptions()));
+            counters_used = 0;
         }
-        const Buffer whole(dev->allocator, ws + static_cast<size_t>(pairs) * sizeof(unsigned), BufferOptions());
-        MRK_TRY(whole.ensure_allocated());
-        std::unique_ptr<Buffer> ranges, arrivals;
-        MRK_TRY(whole.view(0, ws, &ranges));
-        MRK_TRY(whole.view(ws, static_cast<size_t>(pairs) * sizeof(unsigned), &arrivals));
-        void* at = nullptr;
-        MRK_TRY(arrivals->as_raw_ptr(&at));
-        MRK_HIP(launch_clear_words(dev->allocator->stream(), at, pairs), "clearing counters");
-        bufs->push_back(std::move(ranges));
+        std::unique_ptr<Buffer> arrivals;
+        MRK_TRY(counters.back()->view(counters_used, bytes, &arrivals));
+        counters_used += bytes;
         bufs->push_back(std::move(arrivals));
         params->push_back(1);
+        return kOk;
+    }
+    int clear_counters() const {
+        for (const auto& block : counters) {
+            void* at = nullptr;
+            MRK_TRY(block->ensure_allocated());
+            MRK_TRY(block->as_raw_ptr(&at));
+            MRK_HIP(launch_clear_words(dev->allocator->stream(), at, static_cast<long>(block->size() / sizeof(unsigned))), "clearing counters");
+        }
         return kOk;
     }
 
@@ -2524,7 +2536,7 @@ struct Scheduler {
             bufs.push_back(has_mask ? mask_buf : bufs[1]);
             // a handful of queries without the causal rule: the kernel that splits the keys, with its scratch
             const size_t ws = flash_fwd_workspace_bytes(B * H, Sq, Sk, D, att->hint_causal ? 1 : 0);
-            if (ws) MRK_TRY(scratch_of_ranges(ws, B * H, &params, &bufs));
+            if (ws) MRK_TRY(scratch_of_ranges(ws, B, H, Sq, Sk, D, att->hint_causal, strides, &params, &bufs));
             MRK_TRY(builtin("flash_fwd_bf16_ext", params, bufs));
         } else {
             // a handful of queries against a long key sequence: the keys are split over workgroups and the ranges'
@@ -2536,7 +2548,7 @@ struct Scheduler {
                 params = {B, H, Sq, Sk, D, att->hint_causal ? 1 : 0, static_cast<int64_t>(bits), offsets[0], offsets[1], offsets[2], 0};
                 params.insert(params.end(), strides.begin(), strides.end());
             }
-            if (ws) MRK_TRY(scratch_of_ranges(ws, B * H, &params, &bufs));
+            if (ws) MRK_TRY(scratch_of_ranges(ws, B, H, Sq, Sk, D, att->hint_causal, strides, &params, &bufs));
             MRK_TRY(builtin(dense ? "flash_fwd_bf16" : "flash_fwd_bf16_strided", params, bufs));
         }
         dst->buffer = out;
@@ -3478,6 +3490,7 @@ int prepare_locked(const TensorRef& root, std::unique_ptr<ExecutionPlan>* out, s
         s.plan->set_outputs(outputs);
     }
     if (deferred && !deferred->empty()) return kCompileFirst;  // (the rollback returns every touched node to its lazy state)
+    MRK_TRY(s.clear_counters());
     // Intermediates share blocks by liveness (tensor/src/memory_planner.rs); their contents do
     // not outlive the plan's execution, so their nodes go back to being lazy: only the root, and
     // what the caller asked to keep of a realization, stay in memory.  MOROK_NO_MEMORY_PLANNER=1 keeps every intermediate resident.

@@ -102,6 +102,7 @@ int launch_gemm_bf16_rope(void* stream, const void*, const void*, void*, void*, 
 size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal) {
     return !causal && Sq >= 1 && Sq <= 16 && Sk >= 1024 && BH >= 1 && BH <= 96 ? (size_t)2 * BH * 16 * (D + 2) * 4 : 0;
 }
+bool flash_fwd_counts_arrivals(long, long, long Sq, long, long, int, const long*) { return Sq <= 4; }
 int launch_flash_fwd_bf16(void* stream, const void*, const void*, const void*, void*, long, long, long, long, float, int, void* ws, size_t, unsigned*) {
     mrk_shim_note_launch(stream, ws ? "flash_fwd_bf16_splitkv" : "flash_fwd_bf16");
     return 0;
@@ -123,7 +124,10 @@ int launch_gemm_f32(void* stream, const void*, const void*, void*, const void* a
     mrk_shim_note_launch(stream, add ? (add_is_row ? "gemm_f32_bias" : "gemm_f32_residual") : b_transposed ? "gemm_f32_nt" : "gemm_f32");
     return 0;
 }
-int launch_clear_words(void*, void*, long) { return 0; }
+int launch_clear_words(void* stream, void*, long) {
+    mrk_shim_note_launch(stream, "clear_words");
+    return 0;
+}
 int launch_fill(void* stream, void*, size_t, int, int, unsigned long long, unsigned long long, float, float) {
     mrk_shim_note_launch(stream, "fill");
     return 0;

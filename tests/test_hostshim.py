@@ -769,6 +769,42 @@ def test_memory_planner_reuses_intermediates(T, shim, monkeypatch):
     del out2
 
 
+def chained_attentions(T, sq, d=128, wide=None):
+    """Two attentions of `sq` queries, one's output the other's queries."""
+    from morok_amd import uop
+
+    bf = lambda *shape: zeros(T, shape, np.uint16, uop.BF16)
+    k, v = bf(1, 8, 2048, d), bf(1, 8, 2048, d)
+    x = bf(1, 8, sq, d).scaled_dot_product_attention(k, v)
+    if wide:
+        x = x.cast(uop.F32).try_add(wide).cast(uop.BF16).contiguous()  # (a generated kernel in between)
+    return x.scaled_dot_product_attention(k, v)
+
+
+@pytest.mark.parametrize("sq,counted", [(1, True), (8, False)])
+def test_a_plans_attentions_share_their_scratch(T, shim, sq, counted):
+    """The scratch of the split key sequence is an intermediate like any other, in a prepared plan as in a realization; the plan's own are the
+    counters, where its attentions use them, in one block that is cleared once."""
+    from morok_amd import tensor
+
+    chained_attentions(T, sq).realize()
+    want = tensor.last_intermediate_bytes(), tensor.last_memory_plan()
+    launches = shim.mrk_shim_launches()
+    morok_amd.Device("HIP").lru_clear()
+    root = chained_attentions(T, sq)
+    root.prepare()
+    assert (tensor.last_intermediate_bytes(), tensor.last_memory_plan()) == want and want[1][0] >= 1
+    assert shim.mrk_shim_launches() - launches == int(counted)
+    assert not counted or shim.mrk_shim_last_kernel() == b"clear_words"
+
+
+def test_counters_are_cleared_once_where_kernels_have_to_be_compiled_first(T, shim):
+    """(a schedule that finds kernels to compile is thrown away and made again)"""
+    launches = shim.mrk_shim_launches()
+    chained_attentions(T, 1, wide=0.8125).prepare()
+    assert shim.mrk_shim_launches() - launches == 1
+
+
 def test_planned_intermediates_become_lazy_again(T, shim):
     x = zeros(T, (64, 64))
     mid = x.try_add(1.0).contiguous()              # an intermediate of the first realization
