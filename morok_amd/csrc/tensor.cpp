@@ -2440,6 +2440,7 @@ struct Scheduler {
             void* at = nullptr;
             MRK_TRY(block->ensure_allocated());
             MRK_TRY(block->as_raw_ptr(&at));
+            MRK_HIP(ffi::set_device(dev->allocator->device_id()), "hipSetDevice");
             MRK_HIP(launch_clear_words(dev->allocator->stream(), at, static_cast<long>(block->size() / sizeof(unsigned))), "clearing counters");
         }
         return kOk;

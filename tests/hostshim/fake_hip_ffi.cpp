@@ -24,6 +24,8 @@ size_t g_in_use = 0, g_limit = ~size_t(0), g_alloc_calls = 0, g_free_calls = 0, 
 int g_devices = 1;
 unsigned g_last_grid[3], g_last_block[3];
 std::string g_last_kernel;
+thread_local int g_current_device = 0;
+int g_last_device = 0;  // current at the last kernel launch of a stand-in
 struct FakeModule {
     std::string image;
 };
@@ -100,6 +102,7 @@ size_t mrk_shim_alloc_calls() { return g_alloc_calls; }
 size_t mrk_shim_free_calls() { return g_free_calls; }
 size_t mrk_shim_launches() { return g_launches; }
 size_t mrk_shim_syncs() { return g_syncs; }
+int mrk_shim_last_device() { return g_last_device; }
 const char* mrk_shim_last_kernel() { return g_last_kernel.c_str(); }
 void mrk_shim_last_dims(unsigned* grid, unsigned* block) {
     std::memcpy(grid, g_last_grid, sizeof g_last_grid);
@@ -111,6 +114,7 @@ void mrk_shim_note_launch(void* stream, const char* name) {
     count_launch(stream);
     trace("launch:" + std::to_string(stream_no(stream)));
     g_last_kernel = name;
+    g_last_device = g_current_device;
 }
 }
 
@@ -122,7 +126,11 @@ int device_count(int* out) {
     *out = g_devices;
     return g_devices > 0 ? 0 : 100;  // hipErrorNoDevice
 }
-int set_device(int device_id) { return device_id >= 0 && device_id < g_devices ? 0 : kInvalidDevice; }
+int set_device(int device_id) {
+    if (device_id < 0 || device_id >= g_devices) return kInvalidDevice;
+    g_current_device = device_id;
+    return 0;
+}
 
 constexpr size_t kReservedOnly = size_t(8) << 30;
 int malloc_device(void** out, size_t bytes) {

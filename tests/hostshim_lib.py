@@ -40,6 +40,7 @@ def load():
         ("mrk_shim_syncs", C.c_size_t, []),
         ("mrk_shim_tile_choices", C.c_size_t, []),
         ("mrk_shim_last_kernel", C.c_char_p, []),
+        ("mrk_shim_last_device", C.c_int, []),
         ("mrk_shim_last_dims", None, [C.POINTER(C.c_uint * 3), C.POINTER(C.c_uint * 3)]),
     ]:
         fn = getattr(lib, name)

@@ -805,6 +805,23 @@ def test_counters_are_cleared_once_where_kernels_have_to_be_compiled_first(T, sh
     assert shim.mrk_shim_launches() - launches == 1
 
 
+def test_counters_are_cleared_on_their_plans_device(T, shim):
+    """(their block comes out of the allocator's cache, which makes no device current)"""
+    from morok_amd import uop
+
+    shim.mrk_shim_set_device_count(2)
+    bf = lambda *shape: T.Tensor.from_numpy(np.zeros(shape, np.uint16), uop.BF16, device_id=1)  # noqa: E731
+    k = bf(1, 8, 2048, 128)
+    attend = lambda: bf(1, 8, 1, 128).scaled_dot_product_attention(k, k)  # noqa: E731
+    attend().prepare()                          # its blocks go back to the cache
+    root = attend()
+    morok_amd.Buffer(64).copyin(np.zeros(64, np.uint8))  # device 0 is current
+    allocs = shim.mrk_shim_alloc_calls()
+    root.prepare()
+    assert shim.mrk_shim_alloc_calls() == allocs
+    assert shim.mrk_shim_last_kernel() == b"clear_words" and shim.mrk_shim_last_device() == 1
+
+
 def test_planned_intermediates_become_lazy_again(T, shim):
     x = zeros(T, (64, 64))
     mid = x.try_add(1.0).contiguous()              # an intermediate of the first realization
