@@ -22,6 +22,17 @@ PLAIN = {
     (2492, 3144, 328): (256, 128, 1, 3),
 }
 GATED = {(68, 144, 392): (64, 64, 1, 3), (147, 5456, 360): (128, 64, 1, 3), (2055, 912, 328): (128, 128, 1, 3), (2124, 2880, 328): (256, 128, 1, 3)}
+# More tiles than the 256 workgroups that take them in turn, two and three a workgroup: the copies run on into the next tile while the last is
+# stored.  Ragged rows and columns, and counts of steps (K) with every remainder by the ring's three stages, with a partial last step and without
+IN_TURN = {
+    (769, 9376, 352): (128, 128, 1, 3),   # six steps
+    (642, 11096, 280): (128, 128, 1, 3),  # five; 522 tiles
+    (790, 9776, 448): (128, 128, 1, 3),   # seven; 539 tiles
+    (1281, 10800, 520): (256, 128, 1, 3),  # nine
+    (1540, 9264, 512): (256, 128, 1, 3),  # eight
+    (4100, 5640, 448): (256, 128, 1, 3),  # seven; 765 tiles
+}
+IN_TURN_GATED = {(518, 10976, 328): (128, 128, 1, 3), (513, 10992, 448): (128, 128, 1, 3), (1281, 10768, 376): (256, 128, 1, 3), (4096, 5632, 1024): (256, 128, 1, 3)}
 ROTARY = {(67, 264, 384, 256, 50): (64, 64, 1, 3), (147, 5384, 384, 5120, 147): (128, 64, 1, 3), (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
           (2124, 2888, 384, 2816, 531): (256, 128, 1, 3)}
 
@@ -33,9 +44,13 @@ def test_shapes_reach_the_tiles_they_stand_for():
         for shape, tile in GATED.items():
             assert _tile(*shape, nt, True) == tile, shape
         for (m, n, k, _, _), tile in ROTARY.items():
-            assert _tile(m, n, k, nt, True) == tile, (m, n, k)
-        for m, tile in ((1830, (256, 128)), (732, (128, 128)), (61, (64, 64))):  # (of the last test)
-            assert _tile(m, 3112, 384, nt, True)[:2] == tile, m
+            assert _tile(m, n, k, nt, 2) == tile, (m, n, k)
+        for m, tile in ((2440, (128, 128)), (1830, (256, 128)), (732, (128, 128)), (61, (64, 64))):  # (of the last test)
+            assert _tile(m, 3112, 384, nt, 2)[:2] == tile, m
+        for shapes, paired in ((IN_TURN, 0), (IN_TURN_GATED, 1)):
+            for (m, n, k), tile in shapes.items():
+                assert _tile(m, n, k, nt, paired) == tile, (m, n, k)
+                assert -(-m // tile[0]) * -(-n // tile[1]) > 256, (m, n, k)
 
 
 @pytest.mark.gpu
@@ -44,6 +59,40 @@ def test_shapes_reach_the_tiles_they_stand_for():
 @pytest.mark.parametrize("shape", list(PLAIN))
 def test_plain_bias_and_residual_exact(dev, shape, nt, f16):
     _exact(dev, (*shape, 1), nt, f16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", list(IN_TURN))
+def test_tiles_in_turn_exact(dev, shape, nt, f16):
+    _exact(dev, (*shape, 1), nt, f16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("shape", list(IN_TURN_GATED))
+def test_gated_tiles_in_turn(dev, shape, nt):
+    """Against the same rows in products of few enough tiles for a workgroup each: the same bits, whichever tile those run on."""
+    m, n, k = shape
+    a, w = synth.normal_bf16((m, k), 41, 0), synth.normal_bf16((k, n), 41, 1, sigma=k ** -0.5)
+    ba = morok_amd.Buffer.from_numpy(a, dev.device_id)
+    bw = morok_amd.Buffer.from_numpy(np.ascontiguousarray(w.T) if nt else w, dev.device_id)
+    bc = morok_amd.Buffer.from_numpy(np.full(m * n // 2 + 64, 0x7FC0, np.uint16), dev.device_id)
+    kind = "gemm_bf16_nt_swiglu" if nt else "gemm_bf16_swiglu"
+    morok_amd.Program.builtin(kind, [m, n // 2, k], dev.device_id).execute([bc, ba, bw])
+    got = bc.copyout(np.uint16)
+    assert np.all(got[m * n // 2:] == 0x7FC0)
+    got = got[:m * n // 2].reshape(m, n // 2)
+    for first in range(0, m, 250):  # (more than the 64 rows that are streamed)
+        rows = min(250, m - first)
+        if rows < 65:
+            first, rows = m - 65, 65
+        tile = _tile(rows, n, k, nt, 1)
+        assert -(-rows // tile[0]) * -(-n // tile[1]) <= 256
+        part = dev.buffer(rows * n)
+        morok_amd.Program.builtin(kind, [rows, n // 2, k], dev.device_id).execute([part, ba.view(first * k * 2, rows * k * 2), bw])
+        assert np.array_equal(part.copyout(np.uint16, (rows, n // 2)), got[first:first + rows]), first
 
 
 @pytest.mark.gpu
@@ -69,7 +118,8 @@ def test_rotary_epilogue(dev, oracle, shape):
 @pytest.mark.gpu
 @pytest.mark.parametrize("nt", [False, True])
 def test_rotation_gives_the_same_bits_on_every_tile(dev, nt):
-    """The same rows in a product of each tile: 256 x 256 (2440 rows) rounds the products of a rotation as the small tiles do."""
+    """The same rows in products of each small tile and of more tiles than workgroups (2440 rows): all round the products of a rotation alike.
+    (Tiles of 256 x 256 do not: test_gemm_rotary_rounding_gpu.py.)"""
     n, k, split, seq = 3112, 384, 3072, 61
     rows = (2440, 1830, 732, 61)
     a, b = synth.normal_bf16((2440, k), 31, 0), synth.normal_bf16((k, n), 31, 1, sigma=k ** -0.5)
