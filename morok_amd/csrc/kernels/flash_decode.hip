@@ -603,6 +603,14 @@ bool flash_decode_folds(long splits, long slots, long D) {
     return splits > 1 && splits * slots * (D + 2) * (long)sizeof(float) <= (D == 64 ? 64 : 128) * 1024 && (D != 256 || slots <= 4);
 }
 
+// (rows of 256 in 17 and more slots are never folded by counting)
+template <int kD, int kMask, bool kCap, int kQB>
+static auto split_kernel(bool counted) {
+    auto kernel = flash_decode_split<kD, kMask, kCap, kQB>;
+    if constexpr (kD == 256 && kQB == 2) return kernel;
+    else return counted ? flash_decode_split<kD, kMask, kCap, kQB, false, true> : kernel;
+}
+
 // strides: (batch, head, row) element strides of q, k, v and o (validated by the caller: multiples of 8, rows
 // addressable in 32 bits, pointers 16-byte aligned); W: splits * pairs * flash_decode_slot_capacity(group * Sq) * (D + 2)
 // floats, needed with several splits (pairs = B * H / group).
@@ -650,7 +658,7 @@ int launch_flash_decode(void* stream, const void* q, const void* k, const void* 
     const int slot_cap = (int)flash_decode_slot_capacity(slots);
     unsigned* counted = w && flash_decode_folds(splits, slots, D) ? arrivals : nullptr;
 #define MRK_DECODE_QB(DIM, MASK, CAP, QB) \
-    (counted ? flash_decode_split<DIM, MASK, CAP, QB, false, true> : flash_decode_split<DIM, MASK, CAP, QB>)<<<grid, decode_waves<DIM>() * 64, 0, s>>>(qp, kp, vp, op, w, (int)Sq, (int)Sk, (int)keys_per_split, scale_log2e, lay, dm, DecodeAppend{}, counted)
+    split_kernel<DIM, MASK, CAP, QB>(counted != nullptr)<<<grid, decode_waves<DIM>() * 64, 0, s>>>(qp, kp, vp, op, w, (int)Sq, (int)Sk, (int)keys_per_split, scale_log2e, lay, dm, DecodeAppend{}, counted)
 #define MRK_DECODE(DIM, MASK)                              \
     do {                                                   \
         if (cap) {                                         \

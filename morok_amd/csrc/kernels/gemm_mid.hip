@@ -702,7 +702,7 @@ int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* 
     using namespace mrk::dev;
     if (p.tile < 0 || p.tile > kMidTall) return (int)hipErrorInvalidValue;
     const bool split = p.splits > 1;
-    if (split && (!W || batch * p.splits > 65535)) return (int)hipErrorInvalidValue;
+    if (split && (!W || batch * p.splits > 65535 || p.tile == kMidTall)) return (int)hipErrorInvalidValue;  // (256 x 128: one range of K)
     int rows = 0, cols = 0, stages = 0;
     mid_tile_shape(p.tile, &rows, &cols, &stages);
     const long tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols;
@@ -717,7 +717,9 @@ int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* 
             const bool copy_waves = kMay && (kAlways || (split ? p.kt_per_split : (K + 63) / 64) > kFewSteps);
             auto of = [&](auto waves) {
                 constexpr bool kWaves = decltype(waves)::value;
-                return split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true, kPlain, kWaves> : gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, false, kPlain, kWaves>;
+                auto whole = gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, false, kPlain, kWaves>;
+                if constexpr (kTM == 256) return whole;
+                else return split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true, kPlain, kWaves> : whole;
             };
             auto kernel = copy_waves ? of(std::integral_constant<bool, kMay>{}) : of(std::integral_constant<bool, kAlways>{});
             const bool in_turn = copy_waves && kTM * kTN >= 128 * 128 && !split && batch == 1 && tm * tn > 256;
