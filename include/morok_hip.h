@@ -209,7 +209,11 @@ void mrk_hip_program_destroy(mrk_program* p);
  *                     of q k v o into their buffers (4), (batch, head, row) element strides of
  *                     q k v o (12)}                                  buffers = {o, q, k, v}
  *                     (both: optionally one more parameter, the bytes of a scratch buffer that follows v:
- *                     mrk_hip_flash_attn_workspace_bytes, for a key sequence split over workgroups)
+ *                     mrk_hip_flash_attn_workspace_bytes, for a key sequence split over workgroups; behind it
+ *                     optionally 1, with one more buffer behind the scratch, B*H zeros of 32 bits: counters, with
+ *                     which the split kernel merges the ranges itself where that is faster, instead of a second
+ *                     launch.  Zero before the program's first execution, they are zero again after every one;
+ *                     executions that use the same counters have to follow each other, as those of one stream do)
  *   "flash_decode_append"  one query per head over a bf16 cache grown by one key (B*H <= 65535, Sk >= 256 with the new key):
  *                     params = {B, H, Sk, D, f32 bits of scale, element offsets of q, the new key and the new value into their
  *                     buffers (3), (batch, head) element strides of q, the new key, the new value and o (8), workspace bytes}
@@ -597,7 +601,8 @@ int mrk_hip_flash_attn_fwd_bf16_strided(int device_id, const void* q, const void
  * lengths decoding under a key-padding mask [batch, 1, 1, sk]) takes the kernel that splits the key sequence, like
  * the unmasked call, mask and softcap inside it; key ranges without a visible key weigh nothing.
  * Builtin Program kind "flash_fwd_bf16_ext" (29 params, buffers {o, q, k, v, mask}; optionally a 30th, the bytes
- * of a scratch buffer that follows the mask: mrk_hip_flash_attn_workspace_bytes). */
+ * of a scratch buffer that follows the mask: mrk_hip_flash_attn_workspace_bytes, and a 31st, 1, with zeroed
+ * counters behind that, as for "flash_fwd_bf16" (mrk_hip_program_builtin)). */
 int mrk_hip_flash_attn_fwd_bf16_ex(int device_id, const void* q, const void* k, const void* v, void* o, int64_t batch,
                                    int64_t heads, int64_t sq, int64_t sk, int64_t d, float scale, int causal,
                                    const int64_t* strides, const void* mask, int mask_kind, const int64_t* mask_strides,

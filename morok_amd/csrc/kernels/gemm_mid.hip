@@ -4,18 +4,21 @@
 // What bounds it: with one workgroup on a compute unit, the instruction stream of its four waves.  A copy of 1 KB into the LDS waits for its
 // turn on the vector-memory path (one takes 16 cycles, four waves ask at once), and the matrix instructions behind it wait as well: a K step
 // of a 128 x 128 tile, 512 cycles of matrix instructions, 512 of copies and 512 of LDS reads, took 0.49 us (1170 cycles).  Above four steps of
-// K, four more waves make the copies, two waves to a SIMD, and the four that multiply issue nothing else but their LDS reads: 0.38 to 0.41 us, and a
+// K, four more waves make the copies, two waves to a SIMD, and the four that multiply issue nothing else but their LDS reads: 0.38 to 0.42 us, and a
 // launch starts 1 to 2 us sooner.  A ring of four or five stages changes neither (0.49 / 0.46 without such waves, 0.38 to 0.41 with them).  With several
-// workgroups on a compute unit the path from the caches into the LDS bounds it (94 GB/s, 24 TB/s over the chip; profiles/gemm_mid_steps.txt), with
+// workgroups on a compute unit the path from the caches into the LDS bounds it (90 to 94 GB/s, 24 TB/s over the chip; profiles/gemm_mid_steps.txt), with
 // or without them.  Tiles of 128 x 128 and more leave room for one workgroup: it takes its tiles in turn, and the next one's copies run under the stores
-// of the last (3076 x 3072 x 1024 28.1 -> 25.4 us, 512 x 50257 x 768 65 -> 54 against a workgroup to each).
+// of the last (against a workgroup to each tile, us: 1639 x 10368 x 416 on 128 x 128 31.2 -> 25.4, 791 x 9248 x 384 12.0 -> 10.7; on 256 x 128
+// 1627 x 9296 x 320 19.9 -> 17.0, 4096 x 5632 x 512 35.3 -> 28.2).  A lane of 256 x 128 tiles has no registers left: 2 to 8 of its values, all of them
+// of the stores and of what is set up before the first step, lie in scratch (up to 5 in the plain and the gated product); the K loop touches none.
 // Hence smaller tiles for fewer rows and columns, K split over workgroups where even those are few, and the choice by an estimate of the
 // time (plan_mid).
 //
-// us on 128 x 256 tiles (split along K where that paid, padded copies of odd operands), on these tiles without and with copying waves:
-// 1024 x 1024 x 1024 12.3 / 7.0 / 5.5, 1000 x 3000 x 2048 [N, K] 22.9 / 20.3 / 16.7, 3076 x 1024 x 1024 20.3 / 15.1 / 9.8, 512 x 8192 x 8192 92 / 74 / 56;
-// [N, K] weights: 219 x 4288 x 3232 43.1 / 19.1, 700 x 700 x 4096 53.1 / 15.6, 75 x 1536 x 4576 18.7 / 11.5; odd: 300 x 3001 x 777 23.4 / 8.5,
-// 5 x 7152 x 1638 27.8 / 9.0.  500 random products: 1.05 of the speed without copying waves (geometric mean), one slower by more than 4 %.
+// us in a prepared plan against an [N, K] weight, two inputs in turn, without copying waves (large tiles in the last two) and now: 1024 x 1024 x 1024
+// 7.3 / 6.4, 198 x 3072 x 1024 7.0 / 6.2, 1000 x 3000 x 2048 19.1 / 15.8, 3076 x 1024 x 1024 11.8 / 10.5, 219 x 4288 x 3232 (three ranges) 18.5 / 17.5,
+// 512 x 8192 x 8192 75.6 / 73.2, 487 x 4920 x 13416 (three ranges) 121 / 124, 1639 x 10368 x 416 34.4 / 25.4, 1627 x 9296 x 320 24.2 / 17.3.
+// On 128 x 256 tiles, split along K where that paid, padded copies of odd operands, and on these: 700 x 700 x 4096 53.1 / 13.4, 75 x 1536 x 4576
+// 18.7 / 11.1; odd: 300 x 3001 x 777 23.4 / 9.3, 5 x 7152 x 1638 27.8 / 10.9.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -562,8 +565,8 @@ constexpr Tile kTiles[] = {
     {64, 64, 4, 2.4, 0.40, 0.27, 1.27, 50.0, 11.5},  // through registers
 };
 // The same with the gated or the rotary epilogue, where neither the depth nor the unevenness below is told apart: the choice against tiles of
-// 256 x 256 (tiles256_us) is as good without (over the widths of decoder blocks; 0.46 of the time of those tiles alone, none
-// slower by more than 12 % of 320).
+// 256 x 256 is as good without (over the widths of decoder blocks; 0.46 of the time of those tiles alone, none
+// slower by more than 12 % of 320).  Of gated products up to four steps of K; of rotary products against 256 x 256 at any K (ranges_us).
 constexpr Tile kPairedTiles[] = {
     {128, 128, 2, 2.7, 0.71, 0.50, 1.6, 5.7, 1e3},
     {128, 128, 1, 2.7, 0.31, 0.46, 1.6, 6.1, 1e3},

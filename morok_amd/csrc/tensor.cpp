@@ -2848,9 +2848,9 @@ struct Scheduler {
             todo.pop_back();
             if (std::find(found.begin(), found.end(), R) != found.end()) continue;
             if (!qualifies(R)) {
-                // Computed first, like any other input.  Directly under n only what reduces another tensor (a product whose rows are
-                // normalised: log_softmax of a classifier's 64 x 10 logits 3 launches, 1 now): a reduction of the row itself that has to be
-                // in memory anyway leaves this kernel less to keep.
+                // Computed first, like any other input (a product whose rows are normalised: log_softmax of a classifier's 64 x 10 logits
+                // 3 launches, 1 now).  Directly under n not what reduces a tensor of n's shape: of the row itself, which has to be in memory
+                // anyway and leaves this kernel less to keep, or of another one (not told apart: either keeps the separate kernels it had).
                 if (R->src.size() == 1 && R->src[0]->shape == n->shape && std::find(deps.begin(), deps.end(), R) != deps.end()) return {};
                 continue;
             }

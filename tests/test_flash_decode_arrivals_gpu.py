@@ -9,8 +9,6 @@ from morok_amd import tensor as T, uop
 from morok_amd._ffi import lib
 from tests.test_flash_decode_gpu import _attn, _check, _inputs
 
-pytestmark = pytest.mark.gpu
-
 
 def _build(B, H, group, Sq, Sk, d, mask, cap, seed):
     """group > 1: heads that share their keys."""
@@ -33,6 +31,7 @@ CASES = [(1, 32, False, 1, 4096, 128, False, None), (2, 3, False, 1, 1030, 64, F
          (2, 4, False, 2, 2048, 64, True, 20.0), (40, 4, False, 1, 513, 128, False, None), (1, 2, False, 1, 300, 128, False, None)]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(x) for x in c))
 def test_a_plans_executions_match_a_realization(dev, case):
     B, H, group, Sq, Sk, d, mask, cap = case
@@ -52,6 +51,7 @@ def test_a_plans_executions_match_a_realization(dev, case):
         assert np.all(other.try_mul(float(i)).sum(1).to_numpy() == 512.0 * i)  # (work of others in between)
 
 
+@pytest.mark.gpu
 def test_executions_that_follow_each_other_without_a_wait(dev):
     build = _build(2, 4, False, 1, 6000, 128, False, None, seed=32)
     want = build().realize().to_numpy()
@@ -64,17 +64,34 @@ def test_executions_that_follow_each_other_without_a_wait(dev):
         assert np.array_equal(r.buffer().copyout(np.uint16, want.shape), want)
 
 
-# rows of 256 in as many workgroups as there are compute units, or one more pair than that; three ranges a pair just above, first and last count
+# Pairs, query slots, keys, head dim: ranges a pair.  Rows of 256 in as many workgroups as there are compute units, or one more pair than that; more
+# ranges in a band of pairs above, its first and last count and the keys from which there are two and three
+RANGES = {(96, 1, 1231, 256): 2, (129, 1, 900, 256): 1, (257, 1, 1499, 256): 1, (257, 1, 1500, 256): 3, (320, 16, 1530, 256): 3, (321, 1, 1530, 256): 1,
+          (260, 17, 1500, 128): 1, (257, 1, 1499, 128): 1, (257, 1, 1500, 128): 2, (320, 1, 1535, 128): 2, (257, 1, 1536, 128): 3, (320, 16, 1601, 128): 3,
+          (321, 1, 1600, 128): 1, (256, 1, 1600, 128): 1, (257, 1, 1600, 64): 1}
+
+
+def test_ranges_of_a_pair():
+    for (pairs, slots, Sk, d), ranges in RANGES.items():
+        slice_bytes = pairs * (16 if slots <= 16 else 32) * (d + 2) * 4
+        got = lib.mrk_hip_flash_attn_workspace_bytes(1, pairs, slots, Sk, d, 0)
+        # (the scratch also holds what runs of heads that share their keys would take: less than two ranges of all pairs)
+        assert max(1, got // slice_bytes) == ranges, (pairs, slots, Sk, d)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(6, 16, 1, 1231, 256), (1, 129, 1, 900, 256), (1, 257, 1, 1500, 128), (10, 32, 1, 1501, 128), (1, 321, 1, 1500, 128),
-                                   (1, 260, 16, 1530, 256), (1, 260, 17, 1500, 128)])
+                                   (1, 260, 16, 1530, 256), (1, 260, 17, 1500, 128),
+                                   (1, 320, 1, 1535, 128), (1, 257, 1, 1536, 128), (2, 160, 2, 1601, 128)])
 def test_ranges_that_follow_the_count_of_compute_units(dev, oracle, shape):
     B, H, Sq, Sk, d = shape
     q, k, v = _inputs(B, H, Sq, Sk, d, seed=33)
     want = oracle.sdpa_bf16(q, k, v, float(d) ** -0.5, causal=False)
-    for mode in ("abi", "program"):
+    for mode in ("abi", "program", "program_ws"):
         _check(_attn(dev, q, k, v, float(d) ** -0.5, mode=mode), want)
 
 
+@pytest.mark.gpu
 def test_counters_come_with_a_workspace(dev):
     bits = int(np.float32(0.1).view(np.uint32))
     for params in ([8, 1, 2048, 128, 0, bits, 0, 1], [8, 1, 2048, 128, 0, bits, 1 << 20, 2]):
