@@ -1108,10 +1108,17 @@ int gated_tile(const MidPlan& p, long M, long N, long K) {
 // small tiles then run on: 2568 x 6144 x 2048 95.5 / 76.4, 5384 x 3072 x 1024 55.1 / 54.7, 2440 x 3112 x 384 22.3 / 16.8, 6531 x 2344 x 2432 100 / 78;
 // 4000 x 4608 x 256 35.9 / 29.6, 9149 x 5680 x 64 50.1 / 44.7 (60.9 with three stages); 80 shapes 0.84 in the geometric mean).  Up to 256 rows
 // tiles of 256 x 256 come out in as many or fewer rounds: 156 x 61680 x 1984 59.2 / 82.9, 230 x 59600 x 64 16.9 / 18.4, 183 x 35008 x 768 28.2 / 28.8.
+// A lane of a 256 x 128 tile rotates twice as many values as one of 128 x 128, with nothing beside it on the compute unit, which the estimates do not know:
+// up to twenty steps of K, those products run on 128 x 128 with two stages, two workgroups to a compute unit, one's stores beside the other's steps (us
+// on 256 x 128 / so, [K, N] and [N, K] weights: 1708 x 3072 x 1024 22.9 / 22.1 and 22.5 / 20.6, 1054 x 6144 x 640 20.3 / 17.8 and 20.0 / 16.5,
+// 2070 x 3072 x 1152 24.5 / 24.5 and 24.5 / 22.7, 1817 x 3072 x 1152 23.7 / 24.3 and 23.8 / 22.1, 964 x 6144 x 1280 25.9 / 25.6 and 25.7 / 23.9; behind
+// them 793 x 6144 x 1408 25.5 / 26.9 and 25.8 / 24.7, 368 x 12288 x 1664 27.4 / 29.2 and 27.4 / 26.8, 766 x 6144 x 2048 30.7 / 35.6 and 30.8 / 32.3).
+constexpr long kRotatedTall = 20 * 64;
 int rotary_tile(const MidPlan& p, long M, long N, long K) {
     const bool many = mid_many_tiles(M, N, 1);
     if (p.tile < 0 || (double)N * K >= 1e9 || (many && M <= 256) || p.ranges_us >= 0.95 * rounds256_us(M, N, K)) return -1;
-    return !many ? p.tile : mid_pipelined(N, K) ? kMidThreeStages : kMidTwoStages;
+    if (!many) return p.tile == kMidTall && K <= kRotatedTall ? kMidTwoStages : p.tile;
+    return mid_pipelined(N, K) ? kMidThreeStages : kMidTwoStages;
 }
 // Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form: against the
 // faster of its tiles by estimate, for the rotation too where it runs on the other ones.  (Against those, 3 of 1000 shapes more would be separate,

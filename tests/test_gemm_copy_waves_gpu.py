@@ -34,7 +34,7 @@ IN_TURN = {
 }
 IN_TURN_GATED = {(518, 10976, 328): (128, 128, 1, 3), (513, 10992, 448): (128, 128, 1, 3), (1281, 10768, 376): (256, 128, 1, 3), (4096, 5632, 1024): (256, 128, 1, 3)}
 ROTARY = {(67, 264, 384, 256, 50): (64, 64, 1, 3), (147, 5384, 384, 5120, 147): (128, 64, 1, 3), (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
-          (2124, 2888, 384, 2816, 531): (256, 128, 1, 3)}
+          (2124, 2888, 1344, 2816, 531): (256, 128, 1, 3)}
 
 
 def test_shapes_reach_the_tiles_they_stand_for():
@@ -45,8 +45,9 @@ def test_shapes_reach_the_tiles_they_stand_for():
             assert _tile(*shape, nt, True) == tile, shape
         for (m, n, k, _, _), tile in ROTARY.items():
             assert _tile(m, n, k, nt, 2) == tile, (m, n, k)
-        for m, tile in ((2440, (128, 128)), (1830, (256, 128)), (732, (128, 128)), (61, (64, 64))):  # (of the last test)
-            assert _tile(m, 3112, 384, nt, 2)[:2] == tile, m
+        for k, tall in ((384, (128, 128)), (1344, (256, 128))):  # (of the last test)
+            for m, tile in ((2440, (128, 128)), (1830, tall), (732, (128, 128)), (61, (64, 64))):
+                assert _tile(m, 3112, k, nt, 2)[:2] == tile, m
         for shapes, paired in ((IN_TURN, 0), (IN_TURN_GATED, 1)):
             for (m, n, k), tile in shapes.items():
                 assert _tile(m, n, k, nt, paired) == tile, (m, n, k)
@@ -117,10 +118,11 @@ def test_rotary_epilogue(dev, oracle, shape):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("nt", [False, True])
-def test_rotation_gives_the_same_bits_on_every_tile(dev, nt):
+@pytest.mark.parametrize("k", [384, 1344])
+def test_rotation_gives_the_same_bits_on_every_tile(dev, k, nt):
     """The same rows in products of each small tile and of more tiles than workgroups (2440 rows): all round the products of a rotation alike.
     (Tiles of 256 x 256 do not: test_gemm_rotary_rounding_gpu.py.)"""
-    n, k, split, seq = 3112, 384, 3072, 61
+    n, split, seq = 3112, 3072, 61
     rows = (2440, 1830, 732, 61)
     a, b = synth.normal_bf16((2440, k), 31, 0), synth.normal_bf16((k, n), 31, 1, sigma=k ** -0.5)
     angle = synth.uniform((seq, 64), 31, 2).astype(np.float64) * 3.0

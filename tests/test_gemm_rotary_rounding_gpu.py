@@ -20,7 +20,10 @@ SHAPES = {
     (8000, 3072, 1024, 2048, 2000): LARGE,
     (2068, 5776, 128, 5632, 100): LARGE,
     (140, 40000, 384, 39936, 140): LARGE,              # up to 256 rows
-    (2124, 2888, 384, 2816, 531): (256, 128, 1, 3),
+    (2124, 2888, 384, 2816, 531): (128, 128, 1, 2),    # too few steps of K for tiles of 256 x 128
+    (1708, 3072, 1024, 2048, 854): (128, 128, 1, 2),
+    (1153, 4616, 1280, 4608, 384): (128, 128, 1, 2),   # the last count of steps, and the first they are worth it from
+    (1153, 4616, 1344, 4608, 384): (256, 128, 1, 3),
     (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
     (147, 5384, 384, 5120, 147): (128, 64, 1, 3),
     (67, 264, 384, 256, 50): (64, 64, 1, 3),
