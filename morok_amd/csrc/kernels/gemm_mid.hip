@@ -4,7 +4,7 @@
 // What bounds it: with one workgroup on a compute unit, the instruction stream of its four waves.  A copy of 1 KB into the LDS waits for its
 // turn on the vector-memory path (one takes 16 cycles, four waves ask at once), and the matrix instructions behind it wait as well: a K step
 // of a 128 x 128 tile, 512 cycles of matrix instructions, 512 of copies and 512 of LDS reads, took 0.49 us (1170 cycles).  Above four steps of
-// K, four more waves make the copies, two waves to a SIMD, and the four that multiply issue nothing else but their LDS reads: 0.38 to 0.42 us, and a
+// K (copies_apart), four more waves make the copies, two waves to a SIMD, and the four that multiply issue nothing else but their LDS reads: 0.38 to 0.42 us, and a
 // launch starts 1 to 2 us sooner.  A ring of four or five stages changes neither (0.49 / 0.46 without such waves, 0.38 to 0.41 with them).  With several
 // workgroups on a compute unit the path from the caches into the LDS bounds it (90 to 94 GB/s, 24 TB/s over the chip; profiles/gemm_mid_steps.txt), with
 // or without them.  Tiles of 128 x 128 and more leave room for one workgroup: it takes its tiles in turn, and the next one's copies run under the stores
@@ -15,10 +15,10 @@
 // time (plan_mid).
 //
 // us in a prepared plan against an [N, K] weight, two inputs in turn, without copying waves (large tiles in the last two) and now: 1024 x 1024 x 1024
-// 7.3 / 6.4, 198 x 3072 x 1024 7.0 / 6.2, 1000 x 3000 x 2048 19.1 / 15.8, 3076 x 1024 x 1024 11.8 / 10.5, 219 x 4288 x 3232 (three ranges) 18.5 / 17.5,
-// 512 x 8192 x 8192 75.6 / 73.2, 487 x 4920 x 13416 (three ranges) 121 / 124, 1639 x 10368 x 416 34.4 / 25.4, 1627 x 9296 x 320 24.2 / 17.3.
-// On 128 x 256 tiles, split along K where that paid, padded copies of odd operands, and on these: 700 x 700 x 4096 53.1 / 13.4, 75 x 1536 x 4576
-// 18.7 / 11.1; odd: 300 x 3001 x 777 23.4 / 9.3, 5 x 7152 x 1638 27.8 / 10.9.
+// 7.2 / 6.3, 198 x 3072 x 1024 7.0 / 6.1, 1000 x 3000 x 2048 19.2 / 15.9, 3076 x 1024 x 1024 11.8 / 10.6, 512 x 8192 x 8192 76 to 79 / 73 to 74,
+// 1639 x 10368 x 416 34.4 / 25.4, 1627 x 9296 x 320 24.2 / 17.3.
+// On 128 x 256 tiles, split along K where that paid, padded copies of odd operands, and on these: 219 x 4288 x 3232 43.1 / 17.7, 700 x 700 x 4096
+// 53.1 / 13.4, 75 x 1536 x 4576 18.7 / 10.7; odd: 300 x 3001 x 777 23.4 / 9.2, 5 x 7152 x 1638 27.8 / 10.3.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -549,6 +549,16 @@ namespace {
 // Up to four steps of K the multiplying waves copy as well: 1.5 to 2.5 us of copies in flight hide nothing, and starting four more waves costs 0.15 to
 // 0.25 us (541 x 1216 x 192 3.47 us / 3.73 with them, 567 x 512 x 256 3.65 / 3.81; 384 deep and more is faster with them).
 constexpr long kFewSteps = 4;
+// So they do up to eight steps on tiles of 64 x 64, and on more of those than compute units, which take the copies of one workgroup beside the steps of
+// another anyway (without / with copying waves, us: 266 x 80 x 384 3.82 / 4.05, 806 x 984 x 384 4.26 / 4.44, 273 x 200 x 752 5.28 / 5.13, 2045 x 304 x 1384
+// 7.6 / 7.1; 145 x 8392 x 384 4.85 / 5.20, 144 x 9392 x 2368 18.2 / 18.7; 21 such products 1.4 % faster without), and in ranges of K, whose
+// workgroups are as many (23 products 1 to 4 % faster without: 1163 x 680 x 4512 19.7 / 20.2, 826 x 240 x 2080 8.7 / 8.9).
+constexpr long kFewSteps64 = 8;
+bool copies_apart(long rows, long cols, long groups, long kt, bool split) {
+    if (rows == 256) return true;  // (built in this form alone)
+    if (split || kt <= kFewSteps) return false;
+    return rows * cols > 64 * 64 || (kt > kFewSteps64 && groups <= 256);
+}
 // The tiles and what one costs in us, fitted to 25000 timings of every tile and number of ranges over 950 shapes (10 to 12 % off,
 // root mean square): start of a launch, step of K that waits for its data (any number of workgroups resident at
 // once), step of one workgroup more on the same compute unit, start and end of a workgroup, TB/s of the operands, TB/s of what all
@@ -715,14 +725,14 @@ int launch_gemm_mid(hipStream_t s, const MidPlan& p, const void* A, const void* 
         constexpr bool kDirect = decltype(direct)::value;
         auto pick = [&](auto bt, auto half) {
             constexpr bool kBT = decltype(bt)::value, kF16 = decltype(half)::value;
-            // waves of their own copy in more than four steps; tiles of 128 x 128 and more, one workgroup to a compute unit, are taken in turn
+            // (tiles of 128 x 128 and more, one workgroup to a compute unit, are taken in turn)
             constexpr bool kMay = kDirect && kAhead == 3, kAlways = kTM == 256;
-            const bool copy_waves = kMay && (kAlways || (split ? p.kt_per_split : (K + 63) / 64) > kFewSteps);
+            const bool copy_waves = kMay && copies_apart(kTM, kTN, tm * tn * batch, (K + 63) / 64, split);
             auto of = [&](auto waves) {
                 constexpr bool kWaves = decltype(waves)::value;
                 auto whole = gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, false, kPlain, kWaves>;
-                if constexpr (kTM == 256) return whole;
-                else return split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true, kPlain, kWaves> : whole;
+                if constexpr (kWaves) return whole;
+                else return split ? gemm_mid<kTM, kTN, kAhead, kBT, kF16, kDirect, true> : whole;
             };
             auto kernel = copy_waves ? of(std::integral_constant<bool, kMay>{}) : of(std::integral_constant<bool, kAlways>{});
             const bool in_turn = copy_waves && kTM * kTN >= 128 * 128 && !split && batch == 1 && tm * tn > 256;
@@ -753,7 +763,7 @@ int launch_gemm_mid_paired(hipStream_t s, int tile, const void* A, const void* B
     with_tile(tile, [&](auto tile_m, auto tile_n, auto stages) {
         constexpr int kTM = decltype(tile_m)::value, kTN = decltype(tile_n)::value, kStages = decltype(stages)::value;
         constexpr bool kMay = kStages == 3, kAlways = kTM == 256;
-        const bool copy_waves = kMay && (kAlways || K > 64 * kFewSteps), in_turn = copy_waves && kTM * kTN >= 128 * 128 && tm * tn > 256;
+        const bool copy_waves = kMay && copies_apart(kTM, kTN, tm * tn, (K + 63) / 64, false), in_turn = copy_waves && kTM * kTN >= 128 * 128 && tm * tn > 256;
         auto of = [&](auto waves) {
             constexpr bool kWaves = decltype(waves)::value;
             return rope ? (b_transposed ? gemm_mid<kTM, kTN, kStages, true, false, true, false, kRotate, kWaves> : gemm_mid<kTM, kTN, kStages, false, false, true, false, kRotate, kWaves>)

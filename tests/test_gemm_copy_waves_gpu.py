@@ -1,5 +1,5 @@
-"""16-bit products whose copies are made by waves of their own, in one range of K long enough for the pipeline (more than four steps): every
-tile such a product can be sent to, with ragged rows and columns, whole and partial last steps of K.  As in test_gemm_routes_gpu.py each
+"""16-bit products whose copies are made by waves of their own, in one range of K long enough for the pipeline (more than four steps; tiles
+of 64 x 64 more than eight, and no more of them than compute units, with shapes on either side): every tile such a product can be sent to, with ragged rows and columns, whole and partial last steps of K.  As in test_gemm_routes_gpu.py each
 shape states its tile, checked on the CPU; the checks themselves are those of the tests imported here."""
 import numpy as np
 import pytest
@@ -14,6 +14,10 @@ from tests.test_gemm_routes_gpu import _tile
 
 PLAIN = {
     (65, 72, 328): (64, 64, 1, 3),        # one row and one chunk of columns past a tile
+    (65, 72, 584): (64, 64, 1, 3),        # the same, ten steps: with such waves
+    (256, 2048, 576): (64, 64, 1, 3),     # nine, the first with them
+    (1024, 1024, 640): (64, 64, 1, 3),    # as many tiles as compute units
+    (147, 9392, 1160): (64, 64, 1, 3),    # more
     (256, 2048, 512): (64, 64, 1, 3),     # whole tiles
     (129, 5592, 360): (128, 64, 1, 3),
     (384, 3072, 1024): (128, 64, 1, 3),
@@ -21,7 +25,7 @@ PLAIN = {
     (1541, 4968, 328): (128, 128, 1, 3),  # more than 256 tiles of 128 x 256
     (2492, 3144, 328): (256, 128, 1, 3),
 }
-GATED = {(68, 144, 392): (64, 64, 1, 3), (147, 5456, 360): (128, 64, 1, 3), (2055, 912, 328): (128, 128, 1, 3), (2124, 2880, 328): (256, 128, 1, 3)}
+GATED = {(68, 144, 392): (64, 64, 1, 3), (68, 144, 584): (64, 64, 1, 3), (147, 5456, 360): (128, 64, 1, 3), (2055, 912, 328): (128, 128, 1, 3), (2124, 2880, 328): (256, 128, 1, 3)}
 # More tiles than the 256 workgroups that take them in turn, two and three a workgroup: the copies run on into the next tile while the last is
 # stored.  Ragged rows and columns, and counts of steps (K) with every remainder by the ring's three stages, with a partial last step and without
 IN_TURN = {
@@ -33,7 +37,7 @@ IN_TURN = {
     (4100, 5640, 448): (256, 128, 1, 3),  # seven; 765 tiles
 }
 IN_TURN_GATED = {(518, 10976, 328): (128, 128, 1, 3), (513, 10992, 448): (128, 128, 1, 3), (1281, 10768, 376): (256, 128, 1, 3), (4096, 5632, 1024): (256, 128, 1, 3)}
-ROTARY = {(67, 264, 384, 256, 50): (64, 64, 1, 3), (147, 5384, 384, 5120, 147): (128, 64, 1, 3), (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
+ROTARY = {(67, 264, 384, 256, 50): (64, 64, 1, 3), (67, 264, 704, 256, 50): (64, 64, 1, 3), (147, 5384, 384, 5120, 147): (128, 64, 1, 3), (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
           (2124, 2888, 1344, 2816, 531): (256, 128, 1, 3)}
 
 
