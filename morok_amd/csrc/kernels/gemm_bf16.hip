@@ -532,7 +532,6 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     const bool col_ok = col0 + lc * 8 + 8 <= (size_t)N;
     // columns of this lane's chunk inside C when the chunk is the partial last one of a row (kAny: N % 8 of them), else 0
     const int col_tail = kAny && !col_ok && col0 + lc * 8 < (size_t)N ? (int)((size_t)N - (col0 + lc * 8)) : 0;
-    const bool inside = rows_here == 128 && col0 + kJ * 32 <= (size_t)N;  // the whole wave's tile
     auto store_any = [&](__bf16* dst, const u32x4& v, bool row_ok) {
         if (col_ok && row_ok) *reinterpret_cast<u32x4_any*>(dst) = v;
         else if (row_ok) {
@@ -551,8 +550,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
             const __bf16* src = Rl + (size_t)(it * kRowsPerIt) * r_pitch;
             if constexpr (kAny) {
                 const bool row_ok = it * kRowsPerIt + lr < rows_here;
-                if (inside) res[it] = *reinterpret_cast<const u32x4_any*>(src);
-                else if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
+                if (col_ok && row_ok) res[it] = *reinterpret_cast<const u32x4_any*>(src);
                 else if (row_ok) {
                     bf16x8 e8 = __builtin_bit_cast(bf16x8, res[it]);
 #pragma unroll
@@ -568,8 +566,9 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
     {
         using Last = std::true_type;
         int kt = 0;
-        // (512 x 50264 x 776 with the choice of the source in every step 52.6 us, 49.6 so; 4096 x 4096 x 4088 107.6 / 94.4; odd columns, which
-        // have no partial step, 512 x 50257 x 768 47.1 / 43.7 with whole tiles stored without a test, 1000 x 30001 x 2048 103.7 / 90.0)
+        // (us with the choice of the source in every step / so: 512 x 50264 x 776 52.6 / 49.6, 4096 x 4096 x 4088 107.6 / 94.4; odd columns, which have
+        // no partial step, 512 x 50257 x 768 47.2 / 44.1, 1000 x 30001 x 2048 107 / 97.  Stores of whole tiles without a test beside them are not worth
+        // the longer code: 2600 x 4127 x 256 17.6, 16.9 without; 3000 x 8193 x 264 44.3 / 42.7, 1322 x 6672 x 72 13.8 / 12.9; level in long K.)
         if constexpr (kAny) {
             const int whole = has_last ? KT - 3 : KT;  // the first step that copies tile KT - 1, clamped to which those behind it do as well
             for (; kt + 1 < whole; kt += 2) {
@@ -699,10 +698,7 @@ __device__ __forceinline__ void gemm_tile_body(const __bf16* __restrict__ A, con
                         v[t] = __builtin_bit_cast(u32x4, __builtin_convertvector(o, bf16x8));
                     }
                 }
-                if constexpr (kAny) {
-                    if (inside) *reinterpret_cast<u32x4_any*>(Cl + (size_t)r * ldc) = v[t];
-                    else store_any(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
-                }
+                if constexpr (kAny) store_any(Cl + (size_t)r * ldc, v[t], r + lr < rows_here);
                 else if (col_ok && r + lr < rows_here) *reinterpret_cast<u32x4*>(Cl + (size_t)r * ldc) = v[t];
             }
         }
