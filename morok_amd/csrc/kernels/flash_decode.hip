@@ -597,12 +597,17 @@ size_t flash_fwd_workspace_bytes(long BH, long Sq, long Sk, long D, int causal) 
     return most;
 }
 
-// The last workgroup of a pair folds its ranges where they fit the local memory a workgroup has anyway.  Its three trips to memory in a row
-// (results out, the count, results in) take less than a second launch (us with it / without: 32 pairs of 4096 keys 17.2 / 15.3, D = 64:
-// 16 x 4000 11.4 / 9.4, 4 x 30000 18.5 / 13.6; 8 slots of 32 x 2243 17.8 / 16.5), but for rows of 256 from five slots on, which four waves
-// fold (4 slots of 16 x 2000 17.6 / 16.7, 8 of 8 x 1500 15.3 / 17.0).
+// The last workgroup of a pair folds its ranges where its three trips to memory in a row (results out, the count, results in) take less than a second
+// launch, which folds a query's ranges one behind the other in as many threads as there are results.  By what a pair's ranges leave (us with the
+// launch / without): 32 pairs of 4096 keys, 3 KB 16.6 / 14.8, 16 slots of 64 x 4096, 24 KB 25.9 / 25.2, 8 of 16 x 4096, 32 KB 12.5 / 12.7, 16 of 16 x
+// 12000, 98 KB 21.7 / 23.9, 24 of 8 x 4096, 98 KB 14.1 / 16.7; many ranges of few slots are a long chain for the launch: 8 of 4 x 12000, 23 ranges,
+// 93 KB 15.3 / 14.8, D = 64 13.3 / 10.9.  Rows of 256, which four waves fold: 2 of 32 x 4096, 16 KB 28.3 / 27.8, 3 of 32 x 4096, 24 KB level, 2 of
+// 8 x 12000, 64 KB 25.7 / 26.3, 4 of 8 x 4096, 64 KB 15.5 / 17.8; one slot of 4 x 12000, 42 KB 21.9 / 19.2.
 bool flash_decode_folds(long splits, long slots, long D) {
-    return splits > 1 && splits * slots * (D + 2) * (long)sizeof(float) <= (D == 64 ? 64 : 128) * 1024 && (D != 256 || slots <= 4);
+    const long bytes = splits * slots * (D + 2) * (long)sizeof(float);
+    if (splits <= 1 || bytes > (D == 64 ? 64 : 128) * 1024) return false;  // (the local memory a workgroup has anyway)
+    if (D == 256) return slots == 1 || (slots <= 4 && bytes <= 17 * 1024);
+    return bytes <= 25 * 1024 || (splits >= 20 && slots <= 8);
 }
 
 // (rows of 256 in 17 and more slots are never folded by counting)

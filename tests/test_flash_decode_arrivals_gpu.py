@@ -28,7 +28,10 @@ def _build(B, H, group, Sq, Sk, d, mask, cap, seed):
 CASES = [(1, 32, False, 1, 4096, 128, False, None), (2, 3, False, 1, 1030, 64, False, None), (1, 1, False, 1, 70000, 128, False, None),
          (1, 4, False, 3, 5000, 256, False, None), (1, 2, False, 32, 16384, 128, False, None), (1, 1, False, 17, 2000, 64, False, None),
          (4, 8, True, 1, 9000, 128, False, None), (3, 12, True, 2, 3000, 256, False, None), (2, 4, True, 1, 5000, 256, False, None), (3, 4, False, 1, 4100, 128, True, None),
-         (2, 4, False, 2, 2048, 64, True, 20.0), (40, 4, False, 1, 513, 128, False, None), (1, 2, False, 1, 300, 128, False, None)]
+         (2, 4, False, 2, 2048, 64, True, 20.0), (40, 4, False, 1, 513, 128, False, None), (1, 2, False, 1, 300, 128, False, None),
+         # (more partial results than are folded by counting, and just as many: many ranges of few slots, two blocks of slots, rows of 256)
+         (2, 8, True, 1, 12000, 128, False, None), (1, 8, True, 1, 12000, 64, False, None), (2, 4, False, 24, 1500, 128, False, None), (1, 8, False, 8, 4096, 128, False, None),
+         (16, 4, False, 3, 1500, 256, False, None), (2, 4, False, 4, 1500, 256, False, None), (1, 3, False, 1, 12000, 256, True, None)]
 
 
 @pytest.mark.gpu
