@@ -567,10 +567,11 @@ bool flash_decode_plan(long BH, long Sq, long Sk, long D, int causal, long* spli
     // 1500 40.7 / 28.4, 72 x 2500 47.2 / 34.3, 160 x 700 33.4 / 23.5, 20 x 4000 30.4 / 23.0).
     long want = D == 256 ? target / BH : (target + BH / 2) / BH;
     // A few pairs more than compute units, each of which holds one workgroup of these: three shorter ranges a pair instead of a second round for
-    // those few (us in one / three: 288 x 4000 114 / 98, x 2000 60 / 57, x 1000 level; 257 x 1600 46.1 / 44.3, 320 x 1600 49.3 / 49.1; 272 x 2500,
-    // D = 256 144 / 125, 257 x 1500 87.6 / 80.9; 384 x 2500 78 / 82).  Rows of 128 of fewer than 1536 keys have room for two (in one / two: 257 x
-    // 1500 44.5 / 43.1, 288 x 1500 46.6 / 45.8, 320 x 1530 49.1 / 48.1).
-    if (D != 64 && Sq <= 16 && BH > 256 && BH <= 320 && Sk >= 1500) want = 3;
+    // those few, from where the rounds are longer than three sets of partial results, which grow with the slots (us in one / three: one slot of 288 x 4000
+    // 114 / 98, 257 x 1600 46.1 / 44.3; 16 of 320 x 1500 47.9 / 52.8, x 2500 76.2 / 78.2, x 5000 147 / 141; 8 of 288 x 1500 46.4 / 47.8, x 2500 74.2 / 70.4;
+    // D = 256 one of 257 x 1500 87.6 / 79.8, 8 of 320 x 1500 92.9 / 91.6, 16 of 320 x 1500 93.7 / 97.6, x 2500 150.5 / 149; 384 x 2500 78 / 82).  One slot
+    // of fewer than 1536 keys of 128 has room for two ranges (in one / two: 257 x 1500 44.5 / 43.1, 320 x 1530 49.1 / 48.1).
+    if (D != 64 && Sq <= 16 && BH > 256 && BH <= 320 && Sk >= (D == 128 ? 1400 + 100 * Sq : Sq <= 8 ? 1500 : 2500)) want = 3;
     want = want < max_splits ? want : max_splits;
     want = want < 1 ? 1 : want;
     const long per = ((Sk + want - 1) / want + kChunkKeys - 1) / kChunkKeys * kChunkKeys;

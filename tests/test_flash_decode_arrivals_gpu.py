@@ -68,9 +68,9 @@ def test_executions_that_follow_each_other_without_a_wait(dev):
 
 
 # Pairs, query slots, keys, head dim: ranges a pair.  Rows of 256 in as many workgroups as there are compute units, or one more pair than that; more
-# ranges in a band of pairs above, its first and last count and the keys from which there are two and three
-RANGES = {(96, 1, 1231, 256): 2, (129, 1, 900, 256): 1, (257, 1, 1499, 256): 1, (257, 1, 1500, 256): 3, (320, 16, 1530, 256): 3, (321, 1, 1530, 256): 1,
-          (260, 17, 1500, 128): 1, (257, 1, 1499, 128): 1, (257, 1, 1500, 128): 2, (320, 1, 1535, 128): 2, (257, 1, 1536, 128): 3, (320, 16, 1601, 128): 3,
+# ranges in a band of pairs above, its first and last count and the keys, by slots, from which there are two and three
+RANGES = {(96, 1, 1231, 256): 2, (129, 1, 900, 256): 1, (257, 1, 1499, 256): 1, (257, 1, 1500, 256): 3, (320, 8, 1500, 256): 3, (320, 16, 2499, 256): 1, (320, 16, 2500, 256): 3, (321, 1, 1530, 256): 1,
+          (260, 17, 1500, 128): 1, (257, 1, 1499, 128): 1, (257, 1, 1500, 128): 2, (320, 1, 1535, 128): 2, (257, 1, 1536, 128): 3, (288, 8, 2199, 128): 1, (288, 8, 2200, 128): 3, (320, 16, 2999, 128): 1, (320, 16, 3000, 128): 3,
           (321, 1, 1600, 128): 1, (256, 1, 1600, 128): 1, (257, 1, 1600, 64): 1}
 
 
@@ -85,7 +85,7 @@ def test_ranges_of_a_pair():
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(6, 16, 1, 1231, 256), (1, 129, 1, 900, 256), (1, 257, 1, 1500, 128), (10, 32, 1, 1501, 128), (1, 321, 1, 1500, 128),
                                    (1, 260, 16, 1530, 256), (1, 260, 17, 1500, 128),
-                                   (1, 320, 1, 1535, 128), (1, 257, 1, 1536, 128), (2, 160, 2, 1601, 128)])
+                                   (1, 320, 1, 1535, 128), (1, 257, 1, 1536, 128), (2, 160, 2, 1601, 128), (1, 257, 8, 1500, 256)])
 def test_ranges_that_follow_the_count_of_compute_units(dev, oracle, shape):
     B, H, Sq, Sk, d = shape
     q, k, v = _inputs(B, H, Sq, Sk, d, seed=33)
