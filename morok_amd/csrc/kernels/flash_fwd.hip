@@ -728,26 +728,32 @@ namespace mrk {
 // there are more tiles than run at once (one or two to a compute unit).  Where there are not, a pair is a longer chain and a second start and end:
 // 80 heads x 169, D = 128 12.2 us in pairs, 7.6 as tiles; 32 x 700 22.3 / 15.4, D = 256 41.4 / 28.5.  With two to a compute unit the
 // longest tiles share one, and short sequences alone gain (64 x 700, 384 tiles 23.3 / 20.2; 32 x 1500, as many 34.4 / 35.6).
-// Rows of 256, one workgroup to a compute unit: tiles take about half a round of pairs longer than evenly spread work would, the more the more rounds
-// there are; pairs take the rest of their last round.  Tiles below three rounds where the last is filled to half or less (us in pairs / as
-// tiles: 32 x 3000, 1.5 rounds 213 / 187; 24 x 6437, 2.44 626 / 562; 160 x 378, 1.25 62 / 41; but 72 x 1500, 1.69 128 / 137; 128 x 1000, 2 107 / 132;
-// 208 x 952, 3.25 206 / 219), unless all that is left for it are the unpaired middle tiles of an odd count (88 x 628, 1.03 41.5 / 50.4).
-// Rows of 64 and 128, two workgroups to a compute unit, which have the longer of them to themselves at the end: tiles where pairs fill a quarter of their
-// last round, or put a second workgroup on up to a third of the compute units (us in pairs / as tiles: 88 x 1516, 1.03 rounds 99.1 / 85.7; 128 x 1046, 1.25
-// 77.3 / 70.5; 72 x 3857, 2.25 378 / 356; 32 x 2067, 0.56 68.8 / 60.4; but 96 x 942, 0.75 28.4 / 32.3; 160 x 1446, 1.88 130 / 142).
-static long work_units(long BH, long q_tiles, long D, int causal) {
-    const long tiles = BH * q_tiles;
-    bool pairs = causal && tiles > 256 && (D == 256 || tiles > 512 || q_tiles > 6);
-    const long count = BH * ((q_tiles + 1) / 2);
-    if (D == 256 && pairs) {
-        const long last = count % 256;
-        pairs = count >= 3 * 256 || last == 0 || last > 136 || (q_tiles % 2 && last <= 8);
-    } else if (pairs) {
-        const long last = count % 512;
-        pairs = count <= 512 ? count <= 256 || count > 344 : count >= 3 * 512 || last == 0 || last > 144;
+// Pairs cost the same each and so take all of their last round, however little of it they fill; tiles end with the shorter ones.  Below three
+// rounds tiles are faster where pairs fill little of the last round (us in pairs / as tiles).  Not with four tiles to a head, whose pairs hardly differ
+// from what a round of tiles takes (168 heads x 512, D = 64 18.2 / 20.6, 264 x 507, D = 256 118 / 130).  Not where heads are no multiple of the XCDs and
+// tiles of a head are: every head's longest tile then falls on the same XCD (69 x 986, D = 128 40.7 / 51.4; 33 x 2048, D = 64 39.4 / 57.0; 97 x 1024,
+// D = 256 114 / 165).  And not for the unpaired middle tiles of an odd count alone (88 x 628, D = 256, 1.03 rounds 41.5 / 50.4).
+// Rows of 256, one workgroup to a compute unit: last round filled to three eighths, to half with an odd count (an unpaired tile in it) or many tiles,
+// to a quarter with eight (odd: 162 x 384, 1.27 65.5 / 44.3; 72 x 806, 1.12 88.6 / 60.6; even: 88 x 728, 1.03 81.7 / 58.9;
+// 56 x 1446, 1.31 132 / 129; 32 x 3000, 1.5 213 / 187; but 96 x 919, 1.5 103 / 110; 88 x 1019, 1.38 108 / 112; 108 x 1496, 1.53 223 / 232).
+// Rows of 64 and 128, two workgroups to a compute unit, which have the longer of them to themselves at the end: last round filled to a quarter (an eighth
+// with eight tiles), or a second workgroup on a sixth of the compute units, a third with an odd count (D = 128: 176 x 728, 1.03 rounds 53.5 / 43.3; 144 x 984, 1.12
+// 69.1 / 63.3; 72 x 3857, 2.25 378 / 356; 56 x 1190, 0.55 42.7 / 34.7; but 160 x 1019, D = 64, 1.25 42.3 / 44.2; 56 x 1496, D = 64, 0.66 31.7 / 34.9).
+// 254 shapes on the tiles' side of any of these lines: 174 on tiles, 0.89 of the time of pairs (worst 1.04), the others' pairs as fast or faster.
+static bool causal_pairs(long BH, long q_tiles, long D) {
+    const long tiles = BH * q_tiles, pairs = BH * ((q_tiles + 1) / 2), held = D == 256 ? 256 : 512, last = pairs % held;
+    if (tiles <= 256 || (D != 256 && tiles <= 512 && q_tiles <= 6)) return false;
+    const bool odd = q_tiles % 2;
+    if (q_tiles == 4 || (BH % 8 && q_tiles % 8 == 0)) return true;
+    if (pairs >= 3 * held || last == 0 || (odd && pairs > held && last <= 8)) return true;
+    if (D == 256) {
+        if (pairs < 256) return q_tiles < 12 || pairs > 136;
+        return last > (odd || (q_tiles >= 18 && BH % 8 == 0) ? 136 : q_tiles == 8 ? 64 : 96);
     }
-    return pairs ? (q_tiles + 1) / 2 : q_tiles;
+    if (pairs < 512) return pairs <= 256 || pairs > (odd ? 344 : 296);
+    return last > (q_tiles == 8 ? 64 : 144);
 }
+static long work_units(long BH, long q_tiles, long D, int causal) { return causal && causal_pairs(BH, q_tiles, D) ? (q_tiles + 1) / 2 : q_tiles; }
 
 // Heads that share K and V (zero head strides) become query slots of one pair: K and V are read once per batch
 // (runs of consecutive heads: the largest divisor of the head count that gives at most 32 slots).

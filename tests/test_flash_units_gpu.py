@@ -43,3 +43,10 @@ def test_units_of_rows_of_256(dev, heads, s):
 def test_units_of_rows_of_64_and_128(dev, heads, s, d):
     test_units_do_not_change_the_bits(dev, heads, s, d, False)
     test_units_do_not_change_the_bits(dev, heads, s, d, True)
+
+
+# heads that are a multiple of the XCDs and that are not, with eight tiles a head; four tiles a head; even counts with little left for the last round
+@pytest.mark.parametrize("heads,s,d", [(69, 986, 128), (144, 984, 128), (97, 1001, 256), (72, 930, 256), (168, 512, 64), (88, 728, 256), (56, 1190, 128)])
+@pytest.mark.parametrize("mask", [False, True])
+def test_units_of_even_counts(dev, heads, s, d, mask):
+    test_units_do_not_change_the_bits(dev, heads, s, d, mask)
