@@ -739,7 +739,7 @@ namespace mrk {
 // Rows of 64 and 128, two workgroups to a compute unit, which have the longer of them to themselves at the end: last round filled to a quarter (an eighth
 // with eight tiles), or a second workgroup on a sixth of the compute units, a third with an odd count (D = 128: 176 x 728, 1.03 rounds 53.5 / 43.3; 144 x 984, 1.12
 // 69.1 / 63.3; 72 x 3857, 2.25 378 / 356; 56 x 1190, 0.55 42.7 / 34.7; but 160 x 1019, D = 64, 1.25 42.3 / 44.2; 56 x 1496, D = 64, 0.66 31.7 / 34.9).
-// 254 shapes on the tiles' side of any of these lines: 174 on tiles, 0.89 of the time of pairs (worst 1.04), the others' pairs as fast or faster.
+// 254 shapes on the tiles' side of any of these lines: 174 on tiles, 0.89 of the time of pairs (worst 1.05), the others' pairs as fast or faster.
 static bool causal_pairs(long BH, long q_tiles, long D) {
     const long tiles = BH * q_tiles, pairs = BH * ((q_tiles + 1) / 2), held = D == 256 ? 256 : 512, last = pairs % held;
     if (tiles <= 256 || (D != 256 && tiles <= 512 && q_tiles <= 6)) return false;
