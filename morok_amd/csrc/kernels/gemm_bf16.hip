@@ -1091,11 +1091,24 @@ Route choose_route(long M, long N, long K, long batch) {
     if (r.mid) r.splits = r.plan.splits, r.kt_per_split = r.plan.kt_per_split;
     return r;
 }
+// What the estimates of paired products do not know is their epilogue.  On 256 x 128, a lane gates or rotates twice as many values as on 128 x 128, with
+// nothing beside it on the compute unit, and so it is where workgroups take two tiles of 128 x 128 in turn.  Up to `tall_from` of K, and 2048 in the second
+// case, such products (up to 256 tiles of 128 x 256) run on 128 x 128 with two stages, two workgroups to a compute unit, one's epilogue beside the other's
+// steps (us as estimated / so, [K, N] and [N, K] weights).  Gated: 438 x 11904 x 288 10.8 / 8.9 and 10.9 / 8.4, 751 x 9200 x 408 13.5 / 11.8 and 13.1 / 11.4,
+// 664 deep 15.7 / 15.3 and 15.7 / 13.5, but 824 deep 16.7 / 17.4 and 16.7 / 17.1; in turn 348 x 19264 x 504 13.7 / 12.4, 1589 x 4672 x 1440 31.2 / 28.7.
+// Rotary: 1708 x 3072 x 1024 22.9 / 22.1 and 22.5 / 20.6, 1054 x 6144 x 640 20.3 / 17.8 and 20.0 / 16.5, 1817 x 3072 x 1152 23.7 / 24.3 and 23.8 / 22.1,
+// 964 x 6144 x 1280 25.9 / 25.6 and 25.7 / 23.9, but 793 x 6144 x 1408 25.5 / 26.9 and 25.8 / 24.7; in turn 815 x 9216 x 1600 33.2 / 31.4 and 31.2 / 29.8.
+constexpr long kGatedTall = 11 * 64, kRotatedTall = 20 * 64;
+int paired_beside(int tile, long M, long N, long K, long tall_from) {
+    if (!mid_pipelined(N, K) || mid_many_tiles(M, N, 1)) return tile;
+    const bool in_turn = tile == kMidThreeStages && ((M + 127) / 128) * ((N + 127) / 128) > 256;
+    return (tile == kMidTall && K <= tall_from) || (in_turn && K <= 2048) ? kMidTwoStages : tile;
+}
 // The gated product (N = 2 F): small tiles where they are faster by estimate (557 x 22016 x 4096: 258 tiles of 256 x 256,
 // two rounds of 256, against 860 of 128 x 128).  A negative answer: tiles of 256 x 256.
 int gated_tile(const MidPlan& p, long M, long N, long K) {
     // (the kernel addresses B's columns from its first with 32-bit offsets)
-    return p.tile >= 0 && (double)N * K < 1e9 && p.us < 0.95 * tiles256_us(M, N, K) ? p.tile : -1;
+    return p.tile >= 0 && (double)N * K < 1e9 && p.us < 0.95 * tiles256_us(M, N, K) ? paired_beside(p.tile, M, N, K, kGatedTall) : -1;
 }
 // The rotary product.  Tiles of 256 x 256 round the products of a rotation as they always have, small tiles as they do: which of the two a shape
 // runs on decides the last bit of a few results (16 of a million), so that is a matter of the estimates the number of K ranges follows from, and
@@ -1104,16 +1117,10 @@ int gated_tile(const MidPlan& p, long M, long N, long K) {
 // small tiles then run on: 2568 x 6144 x 2048 95.5 / 76.4, 5384 x 3072 x 1024 55.1 / 54.7, 2440 x 3112 x 384 22.3 / 16.8, 6531 x 2344 x 2432 100 / 78;
 // 4000 x 4608 x 256 35.9 / 29.6, 9149 x 5680 x 64 50.1 / 44.7 (60.9 with three stages); 80 shapes 0.84 in the geometric mean).  Up to 256 rows
 // tiles of 256 x 256 come out in as many or fewer rounds: 156 x 61680 x 1984 59.2 / 82.9, 230 x 59600 x 64 16.9 / 18.4, 183 x 35008 x 768 28.2 / 28.8.
-// A lane of a 256 x 128 tile rotates twice as many values as one of 128 x 128, with nothing beside it on the compute unit, which the estimates do not know:
-// up to twenty steps of K, those products run on 128 x 128 with two stages, two workgroups to a compute unit, one's stores beside the other's steps (us
-// on 256 x 128 / so, [K, N] and [N, K] weights: 1708 x 3072 x 1024 22.9 / 22.1 and 22.5 / 20.6, 1054 x 6144 x 640 20.3 / 17.8 and 20.0 / 16.5,
-// 2070 x 3072 x 1152 24.5 / 24.5 and 24.5 / 22.7, 1817 x 3072 x 1152 23.7 / 24.3 and 23.8 / 22.1, 964 x 6144 x 1280 25.9 / 25.6 and 25.7 / 23.9; behind
-// them 793 x 6144 x 1408 25.5 / 26.9 and 25.8 / 24.7, 368 x 12288 x 1664 27.4 / 29.2 and 27.4 / 26.8, 766 x 6144 x 2048 30.7 / 35.6 and 30.8 / 32.3).
-constexpr long kRotatedTall = 20 * 64;
 int rotary_tile(const MidPlan& p, long M, long N, long K) {
     const bool many = mid_many_tiles(M, N, 1);
     if (p.tile < 0 || (double)N * K >= 1e9 || (many && M <= 256) || p.ranges_us >= 0.95 * rounds256_us(M, N, K)) return -1;
-    if (!many) return p.tile == kMidTall && K <= kRotatedTall ? kMidTwoStages : p.tile;
+    if (!many) return paired_beside(p.tile, M, N, K, kRotatedTall);
     return mid_pipelined(N, K) ? kMidThreeStages : kMidTwoStages;
 }
 // Whether the product alone, on the tiles of its route, and a kernel for the gate or the rotation are faster than the fused form: against the

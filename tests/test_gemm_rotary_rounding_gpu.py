@@ -22,6 +22,7 @@ SHAPES = {
     (140, 40000, 384, 39936, 140): LARGE,              # up to 256 rows
     (2124, 2888, 384, 2816, 531): (128, 128, 1, 2),    # too few steps of K for tiles of 256 x 128
     (1708, 3072, 1024, 2048, 854): (128, 128, 1, 2),
+    (815, 9216, 1600, 6144, 815): (128, 128, 1, 2),    # more tiles of 128 x 128 than compute units
     (1153, 4616, 1280, 4608, 384): (128, 128, 1, 2),   # the last count of steps, and the first they are worth it from
     (1153, 4616, 1344, 4608, 384): (256, 128, 1, 3),
     (706, 3216, 384, 3072, 100): (128, 128, 1, 3),
